@@ -83,16 +83,14 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
                          int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb,
                          int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb, int64_t o_st,
                          int64_t g_sb, const FeatArgs& fa, void* ws, int64_t ws_bytes,
-                         void* psi_buf, float* F_out, int64_t f_sb, int phases,
-                         hipStream_t stream);
+                         void* psi_buf, hipStream_t stream);
 int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p);
 int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void* vb,
                          const float* Y, const float* gate, float* out, int nb, int T, int n,
                          int C, int r, int p, int64_t q_sb, int64_t q_st, int64_t k_sb,
                          int64_t k_st, int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st,
                          int64_t o_sb, int64_t o_st, int64_t g_sb, int write_H, void* ws,
-                         int64_t ws_bytes, hipStream_t stream, float* F_out = nullptr,
-                         int64_t f_sb = 0, int phases = 3);
+                         int64_t ws_bytes, hipStream_t stream);
 
 // Workspace carve-up, each region 256-byte aligned.  The fused causal pass
 // (chunk <= 128, no H requested) needs only its group states; the staged one
@@ -105,6 +103,12 @@ struct FwdLayout {
 static inline int64_t al256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 // Row stride of the long-range term Y: 16-byte rows for vector access.
 static inline int64_t y_stride(int p) { return (p + 3) & ~3; }
+
+// Every recent row reads the state of all landmark tokens: the identity
+// incidence (no table) over one profile, no global channel.
+static bool one_state(const void* idx, int N0, int B, int n_P) {
+  return !idx && N0 == 1 && B == 1 && n_P == 0;
+}
 
 static FwdLayout fwd_layout(int nb, int T, int n, int N0, int B, int n_P, int C, int r, int p,
                             bool want_H) {
@@ -239,13 +243,18 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
   const int64_t yst = y_stride(p);
   int rc;
 
-  // One profile holding every landmark token (d = 1, no global channel, the
-  // identity incidence): its pool is the sum of the causal pass's group sums
-  // over the tokens [0, n), so the causal pass's summaries run first and no
-  // pool pass is made.
-  // (the group sums are added as float4, so r*p is a multiple of 4)
-  const bool pool_from_prepass =
-      L.fused && T_R > 0 && !idx && N0 == 1 && n_P == 0 && n > 0 && rp % 4 == 0;
+  // One profile holding every landmark token and one row type reading it (d = 1,
+  // no global channel, the identity incidence): U = F is the state at n, so
+  // adding Phi F to the recent rows is the scan carried on past n without its
+  // reset.  The causal pass over one segment is the whole forward: no pool, no
+  // query (198 us at 8 x 131072 tokens of head size 128) and no Y (0.55 GB
+  // there): 699 -> 459 us.
+  if (L.fused && one_state(idx, N0, B, n_P)) {
+    StageScope stage(3);
+    return causal_scan_dispatch(dtype, phi, psi, vb, nullptr, g, out, nb, T, 0, C, r, p, q_sb,
+                                q_st, k_sb, k_st, v_sb, v_st, 0, 0, o_sb, o_st, g_sb, 0,
+                                ws + L.scan, L.part - L.scan, st);
+  }
 
   // ---- long range: S^T, then C, then R ---------------------------------
   if (T_R > 0) {
@@ -257,13 +266,8 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
     const int64_t ld = idx && plane_code && profiled ? incidence_plane_ld(q, N0, B, rp) : rp;
     {
       StageScope stage(0);
-      if (pool_from_prepass)
-        rc = causal_scan_dispatch(dtype, phi, psi, vb, nullptr, g, out, nb, T, n, C, r, p, q_sb,
-                                  q_st, k_sb, k_st, v_sb, v_st, (int64_t)T_R * yst, yst, o_sb,
-                                  o_st, g_sb, 0, ws + L.scan, L.part - L.scan, st, F, ld, 1);
-      else
-        rc = pool_dispatch(dtype, psi, vb, F, Fg, nb, n_P, n, N0, r, p, k_sb, k_st, v_sb, v_st,
-                           part, part_bytes, st, ld);
+      rc = pool_dispatch(dtype, psi, vb, F, Fg, nb, n_P, n, N0, r, p, k_sb, k_st, v_sb, v_st,
+                         part, part_bytes, st, ld);
     }
     if (rc) return rc;
     const float* Uq = U;
@@ -292,8 +296,7 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
     // one kernel: segmented scan, + Y on recent rows, normalise, gate
     return causal_scan_dispatch(dtype, phi, psi, vb, T_R > 0 ? Y : nullptr, g, out, nb, T, n, C,
                                 r, p, q_sb, q_st, k_sb, k_st, v_sb, v_st, (int64_t)T_R * yst, yst,
-                                o_sb, o_st, g_sb, 0, ws + L.scan, L.part - L.scan, st, nullptr,
-                                0, pool_from_prepass ? 2 : 3);
+                                o_sb, o_st, g_sb, 0, ws + L.scan, L.part - L.scan, st);
   }
   // staged: chunk summaries, segmented scan, chunk-local pass into H, normalise
   float* D = (float*)(ws + L.D);
@@ -440,21 +443,19 @@ extern "C" int smat_forward_fused(int dtype, const void* q, const void* k, const
   int rc;
 
   void* psi_rows = ws + L.total + fused_phi_bytes(nb, T, n, B);
-  // One profile holding every landmark token (d = 1, no global channel, the
-  // identity incidence): its pool is the sum of the causal pass's group sums
-  // over the tokens [0, n), so the prepass runs first and no pool pass is made.
-  const bool pool_from_prepass = T_R > 0 && !idx && N0 == 1 && n_P == 0 && n > 0;
+  // One state (d = 1): the causal pass without its reset, as in smat_forward.
+  if (one_state(idx, N0, B, n_P)) {
+    StageScope stage(3);
+    return causal_scan_run_feat(dtype, q, k, v, nullptr, g, out, nb, T, 0, C, q_sb, q_st, k_sb,
+                                k_st, v_sb, v_st, 0, 0, o_sb, o_st, g_sb, fa, ws + L.scan,
+                                L.part - L.scan, psi_rows, st);
+  }
   if (T_R > 0) {
     const bool profiled = n > n_P;
     // row stride of F and U
     const int64_t ld =
         idx && plane_code && profiled ? incidence_plane_ld(field_q, N0, B, rp) : rp;
-    if (pool_from_prepass) {
-      StageScope stage(0);
-      rc = causal_scan_run_feat(dtype, q, k, v, nullptr, g, out, nb, T, n, C, q_sb, q_st, k_sb,
-                                k_st, v_sb, v_st, (int64_t)T_R * yst, yst, o_sb, o_st, g_sb, fa,
-                                ws + L.scan, L.part - L.scan, psi_rows, F, ld, 1, st);
-    } else {
+    {
       GramItems it{};
       it.mode = 1;
       it.n_P = n_P;
@@ -501,6 +502,5 @@ extern "C" int smat_forward_fused(int dtype, const void* q, const void* k, const
   StageScope stage(3);
   return causal_scan_run_feat(dtype, q, k, v, T_R > 0 ? Y : nullptr, g, out, nb, T, n, C, q_sb,
                               q_st, k_sb, k_st, v_sb, v_st, (int64_t)T_R * yst, yst, o_sb, o_st,
-                              g_sb, fa, ws + L.scan, L.part - L.scan, psi_rows, nullptr, 0,
-                              pool_from_prepass ? 2 : 3, st);
+                              g_sb, fa, ws + L.scan, L.part - L.scan, psi_rows, st);
 }

@@ -468,57 +468,23 @@ static int scan_group_chunks(int nb, int nc) {
   return K;
 }
 
-// F[b] = sum of the group sums G[b][g], g < ng0 (the tokens [0, n)).  A
-// block takes 64 float4 columns of the r*p floats; its four waves sum every
-// fourth group (each wave's loads independent of one another), then wave 0
-// adds the other three partial sums in wave order.
-__global__ __launch_bounds__(256) void group_sum_kernel(const float* __restrict__ G,
-                                                        float* __restrict__ F, int ng0,
-                                                        int64_t rp4, int64_t g_sb,
-                                                        int64_t f_sb) {
-  __shared__ float4 part[3][64];
-  const int64_t b = blockIdx.y;
-  const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
-  const int64_t e = (int64_t)blockIdx.x * 64 + lane;
-  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (e < rp4) {
-    const float4* Gb = reinterpret_cast<const float4*>(G + b * g_sb) + e;
-#pragma unroll 4
-    for (int g = w; g < ng0; g += 4) {
-      const float4 x = Gb[(int64_t)g * rp4];
-      acc.x += x.x;
-      acc.y += x.y;
-      acc.z += x.z;
-      acc.w += x.w;
-    }
-  }
-  if (w > 0) part[w - 1][lane] = acc;
-  __syncthreads();
-  if (w == 0 && e < rp4) {
-    for (int k = 0; k < 3; ++k) {
-      const float4 x = part[k][lane];
-      acc.x += x.x;
-      acc.y += x.y;
-      acc.z += x.z;
-      acc.w += x.w;
-    }
-    reinterpret_cast<float4*>(F + b * f_sb)[e] = acc;
-  }
+static int64_t al256(int64_t x) { return (x + 255) & ~(int64_t)255; }
+// Bytes of the summaries, or of the states, of groups of K chunks (+1: the
+// segment split may add a group).
+static int64_t group_bytes(int nb, int nc, int K, int r, int p) {
+  return al256((int64_t)nb * ((nc + K - 1) / K + 1) * r * p * 4);
 }
 
 int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
-                    const float* gate, float* out, int nb, int T, int n, int C, int K, int r,
-                    int p, int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb,
-                    int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb, int64_t o_st,
-                    int64_t g_sb, int write_H, void* ws, float* F_out, int64_t f_sb,
-                    int phases, hipStream_t stream);
+                    const float* gate, float* out, int nb, int T, int n, int C, int K, int r, int p,
+                    int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st,
+                    int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb,
+                    int64_t o_st, int64_t g_sb, int write_H, void* ws, hipStream_t stream);
 
 int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p) {
   const int nc = (T + C - 1) / C;
   const int K = scan_group_chunks(nb, nc);
-  const int ng = (nc + K - 1) / K + 1;             // +1: the segment split may add a group
-  return 2 * (((int64_t)nb * ng * r * p * 4 + 255) & ~(int64_t)255);
+  return 2 * group_bytes(nb, nc, K, r, p);
 }
 
 int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void* vb,
@@ -526,8 +492,7 @@ int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void
                          int C, int r, int p, int64_t q_sb, int64_t q_st, int64_t k_sb,
                          int64_t k_st, int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st,
                          int64_t o_sb, int64_t o_st, int64_t g_sb, int write_H, void* ws,
-                         int64_t ws_bytes, hipStream_t stream, float* F_out, int64_t f_sb,
-                         int phases) {
+                         int64_t ws_bytes, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
   const int nc = (T + C - 1) / C;
   const int K = scan_group_chunks(nb, nc);
@@ -537,47 +502,26 @@ int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void
               (long long)ws_bytes);
     return SMAT_EINVAL;
   }
-  return causal_scan_run(dtype, phi, psi, vb, Y, gate, out, nb, T, n, C, K, r, p, q_sb, q_st,
-                         k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb, o_st, g_sb, write_H, ws,
-                         F_out, f_sb, phases, stream);
+  return causal_scan_run(dtype, phi, psi, vb, Y, gate, out, nb, T, n, C, K, r, p,
+                         q_sb, q_st, k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb, o_st, g_sb,
+                         write_H, ws, stream);
 }
 
-// The causal pass with groups of K chunks; ws holds 2 * al256(nb * ng * r * p
-// floats) bytes (ng = ceil(nc / K) + 1): the group summaries, then their scan.
+// The causal pass with groups of K chunks; ws holds twice group_bytes: the
+// summaries, then the states.
 int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
-                    const float* gate, float* out, int nb, int T, int n, int C, int K, int r,
-                    int p, int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb,
-                    int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb, int64_t o_st,
-                    int64_t g_sb, int write_H, void* ws, float* F_out, int64_t f_sb,
-                    int phases, hipStream_t stream) {
+                    const float* gate, float* out, int nb, int T, int n, int C, int K, int r, int p,
+                    int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st,
+                    int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb,
+                    int64_t o_st, int64_t g_sb, int write_H, void* ws, hipStream_t stream) {
   const int nc = (T + C - 1) / C;
-  const int ng_max = (nc + K - 1) / K + 1;
   float* G = (float*)ws;
-  float* Sg = (float*)((char*)ws + (((int64_t)nb * ng_max * r * p * 4 + 255) & ~(int64_t)255));
-  // the group layout chunk_states_dispatch uses: groups of K chunks over
-  // [0, n), then over [n, T)
-  const int ng0 = (n / C + K - 1) / K;
-  const int ng = ng0 + (nc - n / C + K - 1) / K;
-  const int64_t rp = (int64_t)r * p;
-  int rc = SMAT_OK;
-  if (phases & 1) {
-    int ng_d = 0, ng0_d = 0;
-    rc = chunk_states_dispatch(dtype, psi, vb, G, nb, T, C, K, n, r, p, k_sb, k_st, v_sb, v_st,
-                               nullptr, 0, stream, &ng_d, &ng0_d);
-    if (rc) return rc;
-    SMAT_REQUIRE(ng_d == ng && ng0_d == ng0, SMAT_EINVAL,
-                 "smat_causal_scan: group layout %d/%d, expected %d/%d", ng_d, ng0_d, ng, ng0);
-    if (F_out) {
-      SMAT_REQUIRE(rp % 4 == 0 && f_sb % 4 == 0, SMAT_EINVAL,
-                   "smat_forward: group sums need r*p and the row stride of F a multiple of 4");
-      smat::launch(group_sum_kernel, dim3((unsigned)((rp / 4 + 63) / 64), (unsigned)nb),
-                   dim3(256), 0, stream, (const float*)G, F_out, ng0, rp / 4, (int64_t)ng * rp,
-                   f_sb);
-      rc = launch_status("smat_forward");
-      if (rc) return rc;
-    }
-  }
-  if (!(phases & 2)) return SMAT_OK;
+  float* Sg = (float*)((char*)ws + group_bytes(nb, nc, K, r, p));
+  // groups over [0, n), then over [n, T)
+  int ng = 0, ng0 = 0;
+  int rc = chunk_states_dispatch(dtype, psi, vb, G, nb, T, C, K, n, r, p, k_sb, k_st, v_sb, v_st,
+                                 nullptr, 0, stream, &ng, &ng0);
+  if (rc) return rc;
   rc = segment_scan_dispatch(G, Sg, nb, ng, ng0, (int64_t)r * p, stream);
   if (rc) return rc;
   ScanArgs a{};
@@ -621,18 +565,13 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
 // and the scan form Psi (and Phi) tiles in LDS from the DMA'd K (and Q) rows,
 // and Vb = [V, 1] from V.  Same workspace as causal_scan_dispatch.  With
 // psi_buf (nb x T rows of 128, 16-bit) the prepass also stores the Psi tiles
-// it forms there and the scan reads them, forming only Phi.  phases: 1 the
-// prepass (and, with F_out, F_out[b] = the sum over the tokens [0, n) of
-// Psi^T Vb, from its group sums: one profile's pool), 2 the segment scan and
-// the streaming scan, 3 both; a call of phase 2 follows one of phase 1 with
-// the same workspace.
+// it forms there and the scan reads them, forming only Phi.
 int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v, const float* Y,
                          const float* gate, float* out, int nb, int T, int n, int C,
                          int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb,
                          int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb, int64_t o_st,
                          int64_t g_sb, const FeatArgs& fa, void* ws, int64_t ws_bytes,
-                         void* psi_buf, float* F_out, int64_t f_sb, int phases,
-                         hipStream_t stream) {
+                         void* psi_buf, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
   constexpr int r = 128, p = 129;
   const int64_t rp = (int64_t)r * p;
@@ -644,9 +583,8 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
               (long long)need, (long long)ws_bytes);
     return SMAT_EINVAL;
   }
-  const int ng_max = (nc + K - 1) / K + 1;
   float* G = (float*)ws;
-  float* Sg = (float*)((char*)ws + (((int64_t)nb * ng_max * rp * 4 + 255) & ~(int64_t)255));
+  float* Sg = (float*)((char*)ws + group_bytes(nb, nc, K, r, p));
   GramItems it{};
   it.mode = 0;
   it.T = T;
@@ -661,21 +599,9 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
   FeatArgs fp = fa;
   fp.psi_out = psi_buf;
   fp.psi_sb = (int64_t)T * 128;
-  int rc = SMAT_OK;
-  if (phases & 1) {
-    rc = gram_stream_launch_feat(dtype, k, v, G, nullptr, it, ng, nb, k_sb, k_st, v_sb, v_st,
-                                 (int64_t)ng * rp, rp, 0, fp, stream, "smat_forward_fused");
-    if (rc) return rc;
-    if (F_out) {
-      const int64_t rp4 = rp / 4;
-      smat::launch(group_sum_kernel, dim3((unsigned)((rp4 + 63) / 64), (unsigned)nb),
-                   dim3(256), 0, stream, (const float*)G, F_out, it.ng0, rp4,
-                   (int64_t)ng * rp, f_sb);
-      rc = launch_status("smat_forward_fused");
-      if (rc) return rc;
-    }
-  }
-  if (!(phases & 2)) return SMAT_OK;
+  int rc = gram_stream_launch_feat(dtype, k, v, G, nullptr, it, ng, nb, k_sb, k_st, v_sb, v_st,
+                                   (int64_t)ng * rp, rp, 0, fp, stream, "smat_forward_fused");
+  if (rc) return rc;
   rc = segment_scan_dispatch(G, Sg, nb, ng, it.ng0, rp, stream);
   if (rc) return rc;
   ScanArgs a{};
@@ -747,18 +673,12 @@ static int scratch_for_current_device(void** out) {
   return SMAT_OK;
 }
 
-// Scratch bytes for group size K (as causal_scan_workspace_bytes at its K).
-static int64_t scan_scratch_bytes(int nb, int nc, int K, int r, int p) {
-  const int ng = (nc + K - 1) / K + 1;
-  return 2 * (((int64_t)nb * ng * r * p * 4 + 255) & ~(int64_t)255);
-}
-
 // The group size of the allocating entry point when its scratch fits the
 // array, else the least power-of-two multiple of it that fits (larger groups,
 // fewer summaries; 0 when not even one group per segment fits).
 static int noalloc_group_chunks(int nb, int nc, int r, int p) {
   int K = scan_group_chunks(nb, nc);
-  while (scan_scratch_bytes(nb, nc, K, r, p) > kNoAllocScratchBytes) {
+  while (2 * group_bytes(nb, nc, K, r, p) > kNoAllocScratchBytes) {
     if (K >= nc) return 0;
     K *= 2;
   }
@@ -803,7 +723,7 @@ extern "C" int smat_causal_scan_noalloc(int dtype, const void* phi, const void* 
   if (rc) return rc;
   return causal_scan_run(dtype, phi, psi, vb, Y, gate, out, nb, T, n, C, K, r, p, q_sb, q_st,
                          k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb, o_st, g_sb, write_H, ws,
-                         nullptr, 0, 3, (hipStream_t)stream);
+                         (hipStream_t)stream);
 }
 
 extern "C" int64_t smat_causal_scan_workspace_bytes(int nb, int T, int C, int r, int p) {
@@ -834,5 +754,5 @@ extern "C" int smat_causal_scan(int dtype, const void* phi, const void* psi, con
                "smat_causal_scan: workspace must be 256-byte aligned");
   return causal_scan_dispatch(dtype, phi, psi, vb, Y, gate, out, nb, T, n, C, r, p, q_sb, q_st,
                               k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb, o_st, g_sb, write_H,
-                              workspace, workspace_bytes, (hipStream_t)stream, nullptr, 0, 3);
+                              workspace, workspace_bytes, (hipStream_t)stream);
 }

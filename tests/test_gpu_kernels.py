@@ -486,6 +486,34 @@ def test_forward_fp32_small(T, d, n_P):
     _check_forward(spec, Phi, Psi, Vb, dt=torch.float32, g=g, label=f"T={T} d={d}")
 
 
+@pytest.mark.parametrize("T,hd,dt,gate", [(1024, 64, torch.float32, True),
+                                          (1000, 32, torch.float32, False),
+                                          (2048 + 64, 128, torch.bfloat16, False),
+                                          (1337, 96, torch.float16, True),
+                                          (640, 128, torch.float16, True)])
+def test_forward_one_state(T, hd, dt, gate):
+    """d = 1: the forward is the causal pass over one segment (every recent row
+    reads the state of all landmark tokens); against plain causal attention in
+    fp64, scores rounded to the input type as the reference rounds them (ragged
+    lengths, the last chunk short; streaming, wide and narrow scans)."""
+    _say("forward one state", T, hd, dt, gate)
+    spec = build_mask(T, 1, chunk=128)
+    Phi, Psi, Vb = _feats(3, T, hd, dt, seed=31)
+    g = (torch.rand(3, T, generator=torch.Generator().manual_seed(32)) + 0.5) if gate else None
+    got = A.smat_attention(*(x.to(DEV) for x in (Phi, Psi, Vb)), spec,
+                           g=None if g is None else g.to(DEV))
+    S = Phi.double() @ Psi.double().transpose(1, 2).contiguous()
+    H = S.tril() @ Vb.double()
+    want = H[..., :-1] / H[..., -1:]
+    want = want if g is None else want * g.double().unsqueeze(-1)
+    # fp32: the suite's bar; 16-bit: scores rounded to half an ulp (2^-9 bf16,
+    # 2^-12 fp16, at most doubled by the division), of values up to max |V|
+    tol = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dt]
+    e = (got.double().cpu() - want).abs().max().item() / Vb[..., :-1].abs().max().item()
+    _say(f"  rel {e:.2e}")
+    assert e < tol * (1.5 if gate else 1.0)
+
+
 def test_forward_single_gpu_d2_bf16():
     """nb=32 (B=4, H=8), T=8192, d=2, head_dim=64, bf16, q,k,v ~ N(0,1)/sqrt(64)."""
     _say("forward T=8192 d=2 nb=32 hd=64 bf16")
