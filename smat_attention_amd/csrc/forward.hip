@@ -84,13 +84,13 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
                          int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb, int64_t o_st,
                          int64_t g_sb, const FeatArgs& fa, void* ws, int64_t ws_bytes,
                          void* psi_buf, hipStream_t stream);
-int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p);
+int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, bool forward);
 int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void* vb,
                          const float* Y, const float* gate, float* out, int nb, int T, int n,
                          int C, int r, int p, int64_t q_sb, int64_t q_st, int64_t k_sb,
                          int64_t k_st, int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st,
                          int64_t o_sb, int64_t o_st, int64_t g_sb, int write_H, void* ws,
-                         int64_t ws_bytes, hipStream_t stream);
+                         int64_t ws_bytes, bool forward, hipStream_t stream);
 
 // Workspace carve-up, each region 256-byte aligned.  The fused causal pass
 // (chunk <= 128, no H requested) needs only its group states; the staged one
@@ -126,7 +126,7 @@ static FwdLayout fwd_layout(int nb, int T, int n, int N0, int B, int n_P, int C,
   L.U = off;   off += al256((int64_t)nb * B * ld * 4);
   L.Y = off;   off += al256((int64_t)nb * T_R * y_stride(p) * 4);
   if (L.fused) {
-    L.scan = off; off += al256(causal_scan_workspace_bytes(nb, T, C, r, p));
+    L.scan = off; off += al256(causal_scan_workspace_bytes(nb, T, C, r, p, true));
   } else {
     L.D = off;   off += al256((int64_t)nb * nc * rp * 4);
     L.Sin = off; off += al256((int64_t)nb * nc * rp * 4);
@@ -253,7 +253,7 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
     StageScope stage(3);
     return causal_scan_dispatch(dtype, phi, psi, vb, nullptr, g, out, nb, T, 0, C, r, p, q_sb,
                                 q_st, k_sb, k_st, v_sb, v_st, 0, 0, o_sb, o_st, g_sb, 0,
-                                ws + L.scan, L.part - L.scan, st);
+                                ws + L.scan, L.part - L.scan, true, st);
   }
 
   // ---- long range: S^T, then C, then R ---------------------------------
@@ -296,7 +296,7 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
     // one kernel: segmented scan, + Y on recent rows, normalise, gate
     return causal_scan_dispatch(dtype, phi, psi, vb, T_R > 0 ? Y : nullptr, g, out, nb, T, n, C,
                                 r, p, q_sb, q_st, k_sb, k_st, v_sb, v_st, (int64_t)T_R * yst, yst,
-                                o_sb, o_st, g_sb, 0, ws + L.scan, L.part - L.scan, st);
+                                o_sb, o_st, g_sb, 0, ws + L.scan, L.part - L.scan, true, st);
   }
   // staged: chunk summaries, segmented scan, chunk-local pass into H, normalise
   float* D = (float*)(ws + L.D);

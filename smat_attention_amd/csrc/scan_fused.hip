@@ -460,12 +460,36 @@ int gram_stream_launch_feat(int dtype, const void* k, const void* v, float* G, f
                             int64_t gl_sb, const FeatArgs& fa, hipStream_t stream,
                             const char* who);
 
-// Group size: enough workgroups to fill the GPU (one per CU at a time), and
-// no more than needed so the prepass stays small.
-static int scan_group_chunks(int nb, int nc) {
-  int K = 8;
-  while (K > 1 && (int64_t)nb * ((nc + K - 1) / K) < 1024) K >>= 1;
-  return K;
+// Chunks a group, at most kmax.  A group costs its chunks plus the summary it
+// writes, the two passes of the scan over groups and the state it loads -- four
+// r x p tables, about what one of its chunks moves in all -- and the launch runs
+// in rounds of as many groups as the GPU works on at once, so K minimises rounds
+// x (K + 1), the smallest such K.  The rounds: a workgroup a CU at head size 128
+// (8 sequences of 32768 tokens: forward 641 -> 599 us with 256 groups in place
+// of 1024, 613 with 512), four for the narrow shape (8192 tokens, 32 sequences:
+// 164.0 us with 1024 groups, 166.2 with 512).  n is not an argument (the
+// workspace is sized without it): the groups are counted as if it split the
+// chunks in half, where build_mask puts it.
+//
+// The one-call forwards take up to kForwardK: past 32 the uneven halves (only
+// recent rows read Y) cost more than the states (524288 tokens: 5810 us at 32,
+// 5850 at 64; 8 x 131072 tokens at d = 1: 408 us at 32, 428 at 16).  The scan
+// called alone keeps to kScanK: it also serves the H-writing general kernel,
+// whose groups overlap less.
+constexpr int kForwardK = 32, kScanK = 16;
+static int scan_group_chunks(int nb, int nc, int r, int p, int kmax) {
+  const int64_t slots = r <= 64 && p <= 80 ? 1024 : 256;
+  int best = 1;
+  int64_t best_cost = INT64_MAX;
+  for (int K = 1; K <= kmax && K <= nc; ++K) {
+    const int64_t groups = (int64_t)nb * 2 * (((nc + 1) / 2 + K - 1) / K);
+    const int64_t cost = (groups + slots - 1) / slots * (K + 1);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = K;
+    }
+  }
+  return best;
 }
 
 static int64_t al256(int64_t x) { return (x + 255) & ~(int64_t)255; }
@@ -481,9 +505,10 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
                     int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb,
                     int64_t o_st, int64_t g_sb, int write_H, void* ws, hipStream_t stream);
 
-int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p) {
+// forward: the causal pass of a one-call forward (groups of up to kForwardK).
+int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, bool forward) {
   const int nc = (T + C - 1) / C;
-  const int K = scan_group_chunks(nb, nc);
+  const int K = scan_group_chunks(nb, nc, r, p, forward ? kForwardK : kScanK);
   return 2 * group_bytes(nb, nc, K, r, p);
 }
 
@@ -492,11 +517,11 @@ int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void
                          int C, int r, int p, int64_t q_sb, int64_t q_st, int64_t k_sb,
                          int64_t k_st, int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st,
                          int64_t o_sb, int64_t o_st, int64_t g_sb, int write_H, void* ws,
-                         int64_t ws_bytes, hipStream_t stream) {
+                         int64_t ws_bytes, bool forward, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
   const int nc = (T + C - 1) / C;
-  const int K = scan_group_chunks(nb, nc);
-  const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p);
+  const int K = scan_group_chunks(nb, nc, r, p, forward ? kForwardK : kScanK);
+  const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, forward);
   if (ws_bytes < need) {
     set_error("smat_causal_scan: workspace of %lld bytes needed, %lld given", (long long)need,
               (long long)ws_bytes);
@@ -563,7 +588,8 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
 // The streaming causal pass with the feature map computed inside the kernels:
 // q, k, v are the Q, K, V rows (r = d_qk = d_v = 128); the prepass Gram sums
 // and the scan form Psi (and Phi) tiles in LDS from the DMA'd K (and Q) rows,
-// and Vb = [V, 1] from V.  Same workspace as causal_scan_dispatch.  With
+// and Vb = [V, 1] from V.  Same workspace as causal_scan_dispatch's
+// with forward.  With
 // psi_buf (nb x T rows of 128, 16-bit) the prepass also stores the Psi tiles
 // it forms there and the scan reads them, forming only Phi.
 int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v, const float* Y,
@@ -576,8 +602,8 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
   constexpr int r = 128, p = 129;
   const int64_t rp = (int64_t)r * p;
   const int nc = (T + C - 1) / C;
-  const int K = scan_group_chunks(nb, nc);
-  const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p);
+  const int K = scan_group_chunks(nb, nc, r, p, kForwardK);
+  const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, true);
   if (ws_bytes < need) {
     set_error("smat_forward_fused: causal-pass workspace of %lld bytes needed, %lld given",
               (long long)need, (long long)ws_bytes);
@@ -677,7 +703,7 @@ static int scratch_for_current_device(void** out) {
 // array, else the least power-of-two multiple of it that fits (larger groups,
 // fewer summaries; 0 when not even one group per segment fits).
 static int noalloc_group_chunks(int nb, int nc, int r, int p) {
-  int K = scan_group_chunks(nb, nc);
+  int K = scan_group_chunks(nb, nc, r, p, kScanK);
   while (2 * group_bytes(nb, nc, K, r, p) > kNoAllocScratchBytes) {
     if (K >= nc) return 0;
     K *= 2;
@@ -728,7 +754,7 @@ extern "C" int smat_causal_scan_noalloc(int dtype, const void* phi, const void* 
 
 extern "C" int64_t smat_causal_scan_workspace_bytes(int nb, int T, int C, int r, int p) {
   if (nb <= 0 || T <= 0 || C <= 0 || r <= 0 || p <= 0) return 0;
-  return smat::causal_scan_workspace_bytes(nb, T, C, r, p);
+  return smat::causal_scan_workspace_bytes(nb, T, C, r, p, false);
 }
 
 extern "C" int smat_causal_scan(int dtype, const void* phi, const void* psi, const void* vb,
@@ -754,5 +780,5 @@ extern "C" int smat_causal_scan(int dtype, const void* phi, const void* psi, con
                "smat_causal_scan: workspace must be 256-byte aligned");
   return causal_scan_dispatch(dtype, phi, psi, vb, Y, gate, out, nb, T, n, C, r, p, q_sb, q_st,
                               k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb, o_st, g_sb, write_H,
-                              workspace, workspace_bytes, (hipStream_t)stream);
+                              workspace, workspace_bytes, false, (hipStream_t)stream);
 }

@@ -382,6 +382,20 @@ def test_causal_scan_fused(dt, T, n, C, hd):
     assert (out.double().cpu() - want).abs().max().item() < tol * max(1.0, want.abs().max().item())
 
 
+@pytest.mark.parametrize("nb,T,n,C,r", [(8, 32768, 16384, 8, 8), (4, 4096, 56, 8, 72),
+                                        (3, 4096 + 5, 2048, 8, 72), (1, 64, 64, 8, 72),
+                                        (5, 2049, 0, 8, 8)])
+def test_causal_scan_group_sizes(nb, T, n, C, r):
+    """The causal pass with many chunks a group (both tile shapes), groups cut
+    short by n and by T, and n far from the half the grouping assumes, against
+    fp64."""
+    _say("causal scan groups", nb, T, n, C, r)
+    Phi, Psi, Vb = _feats(nb, T, r, torch.float32, seed=33)
+    H = K.causal_scan(Phi.to(DEV), Psi.to(DEV), Vb.to(DEV), n, C, write_H=True)
+    ref = O.segmented_causal_scan(Phi.double(), Psi.double(), Vb.double(), n, chunk=C)
+    assert _rel(H, ref) < 1e-5
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,n,C", [(4096, 2048, 128), (8192, 0, 128), (4096, 4096, 128),
                                    (4096, 1024, 64), (2048 + 64, 1024, 128), (16384, 8192, 128)])
