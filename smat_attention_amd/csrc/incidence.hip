@@ -335,23 +335,37 @@ static int launch_plane(const float* F, const float* F_glob, const int* code, in
 // eight adds.  Steps are issued two at a time with three pairs in flight.
 // Lanes past q in a direction's last group read in bounds and store nothing.
 //
-// The panel (4 x kPlane entries, 147 KB) leaves no room for a second one, so
+// The panel (4 x kPlane entries, 147 KB at q = 41) leaves no room for a second one, so
 // the workgroup is persistent and prefetches the next item's panel into
 // registers while it sums the current one.  Nothing in the summing loop may
 // wait on the vector memory counter, which counts those loads too: the kernel
 // fits 128 VGPRs without spilling (a spill reload waits for every load issued
 // before it), the chunk map is recomputed per item rather than kept live.
 namespace iw {
-constexpr int kThreads = 1024;
-constexpr int kWaves = kThreads / 64;
 constexpr int kE = 16;            // floats of r*p per item (four planes)
 constexpr int kPlanes = kE / 4;
-constexpr int kPF = 7;            // panel chunks each thread prefetches (N0 <= 1792)
 constexpr int kGroup = 16;        // lines per row
-constexpr int kCW = 56;           // entries per column: >= q + 15
-constexpr int kQMax = kCW - 15;   // largest q the layout holds
-constexpr int kPlane = (kCW * kQMax + 15) / 16 * 16;   // 2304 entries
-constexpr int kPlaneBytes = kPlane * 16;               // 36864: fits the 16-bit offset
+constexpr int kQMax = 41;         // largest q whose four planes fit the LDS
+// A small field's panel leaves room for more workgroups on a CU, and its few
+// wave tasks an item (7 at q = 13, 11 at q = 19) idle most of sixteen waves: 256
+// threads and four workgroups (three at q = 19) up to q = 19, 512 and two at
+// q = 23.  One workgroup's staging and barriers then pass under another's sums
+// and more items' loads are in flight: 193 -> 149 us at q = 13 (96 sequences,
+// head size 64), 160 -> 150 us at q = 23 (8 of 128).  Two workgroups at q = 29
+// (the panels fill the LDS exactly) ran as one does, 234 us.
+template <int Q>
+struct Shape {
+  static constexpr int kThreads = Q <= 19 ? 256 : Q <= 23 ? 512 : 1024;
+  static constexpr int kWaves = kThreads / 64;
+  static constexpr int kWgs = Q <= 17 ? 4 : Q <= 19 ? 3 : Q <= 23 ? 2 : 1;   // on a CU
+  static constexpr int kPF = (Q * Q * kPlanes + kThreads - 1) / kThreads;   // chunks a thread
+  static constexpr int kCW = (Q + 15 + 1) / 2 * 2;       // entries per column: even, >= q + 15
+  static constexpr int kPlane = (kCW * Q + 15) / 16 * 16;
+  static constexpr int kPlaneBytes = kPlane * 16;        // fits the 16-bit read offset
+  static constexpr int kLdsBytes = kPlanes * kPlaneBytes;
+  static_assert(kPlaneBytes < 65536 && kWgs * kLdsBytes <= 160 * 1024, "panels fit the LDS");
+  static_assert(Q * (Q + 1) * 2 <= kLdsBytes, "the line table fits the panel");
+};
 }  // namespace iw
 
 // Lane n of each sixteen-lane row of v, broadcast to the whole row (DPP row_newbcast).
@@ -375,18 +389,18 @@ __device__ __forceinline__ void swap_halves(int& x, int& y) {
 }
 
 // Step N: both planes of the pair at the lane part plus the row part of step N.
-template <int N>
+template <int Q, int N>
 __device__ __forceinline__ void lg_issue(float4* v, const char* vb, const int* ot) {
   const char* a = vb + row_bcast<N % 16>(ot[N / 16]);
   v[0] = *reinterpret_cast<const float4*>(a);
-  v[1] = *reinterpret_cast<const float4*>(a + iw::kPlaneBytes);
+  v[1] = *reinterpret_cast<const float4*>(a + iw::Shape<Q>::kPlaneBytes);
 }
 
 // Pair K of steps (2K, 2K + 1), into buffer K mod 3.
 template <int Q, int K>
 __device__ __forceinline__ void lg_issue_pair(float4 (&buf)[3][4], const char* vb, const int* ot) {
-  if constexpr (2 * K < Q) lg_issue<2 * K>(&buf[K % 3][0], vb, ot);
-  if constexpr (2 * K + 1 < Q) lg_issue<2 * K + 1>(&buf[K % 3][2], vb, ot);
+  if constexpr (2 * K < Q) lg_issue<Q, 2 * K>(&buf[K % 3][0], vb, ot);
+  if constexpr (2 * K + 1 < Q) lg_issue<Q, 2 * K + 1>(&buf[K % 3][2], vb, ot);
 }
 
 // The sums so far are materialised here and no memory access moves across:
@@ -498,24 +512,19 @@ struct LgGroup {
 };
 
 // Panel chunk u of thread tid: plane kx = (tid >> 4) & 3 and slot
-// ps = 16 * (wave + 16 u) + (tid & 15) in column-major point order
+// ps = 16 * (wave + kWaves u) + (tid & 15) in column-major point order
 // (x1 = ps / q, x0 = ps mod q), so the sixteen lanes of a row write sixteen
 // consecutive entries of one plane.  Its F offset in bytes (4 N0 rp < 2^32,
 // checked on the host) is 4 (x*rp + 4*kx) for the point x = x0*q + x1; its LDS
 // entry is kx*kPlane + kCW*x1 + x0, with copies at + q, + 2q, ... below q + 15.
 template <int Q>
-using LgSlot = LgDiv<Q, 16 * iw::kWaves * iw::kPF>;
+using LgSlot = LgDiv<Q, 16 * iw::Shape<Q>::kWaves * iw::Shape<Q>::kPF>;
 
 // Byte offsets into one sequence's F panel rows and U type rows are 32-bit;
 // ld is their row stride in floats.
 static bool wave_kernel_fits(int q, int N0, int B, int64_t ld) {
-  return q >= 2 && q <= iw::kQMax && N0 == q * q &&
-         (int64_t)N0 * iw::kPlanes <= (int64_t)iw::kPF * iw::kThreads &&
-         (int64_t)N0 * ld < (1ll << 30) && (int64_t)B * ld < (1ll << 30);
-}
-
-static int64_t wave_lds_bytes(int q) {
-  return (int64_t)iw::kPlanes * iw::kPlane * 16 + (((int64_t)q * (q + 1) * 2 + 15) & ~15);
+  return q >= 2 && q <= iw::kQMax && N0 == q * q && (int64_t)N0 * ld < (1ll << 30) &&
+         (int64_t)B * ld < (1ll << 30);
 }
 
 // A line of its own per lane (the last q mod 16 lines of each direction, when
@@ -540,17 +549,18 @@ __device__ __forceinline__ float4 lds_at(uint32_t addr) {
   return make_float4(v.x, v.y, v.z, v.w);
 }
 // pb: the panel's LDS address
-template <int N>
+template <int Q, int N>
 __device__ __forceinline__ void lw_issue(float4 (&v)[4], uint32_t pb, LrLane& ln) {
+  constexpr int kPB = iw::Shape<Q>::kPlaneBytes;
   const uint32_t a = pb + __umul24(ln.c16, (uint32_t)N) + ln.s16;
   // planes 2 and 3 from a second base: opaque, so plane 3 stays an immediate
   // offset from it rather than a third address
-  uint32_t a2 = a + 2 * iw::kPlaneBytes;
+  uint32_t a2 = a + 2 * kPB;
   asm volatile("" : "+v"(a2));
   v[0] = lds_at(a);
-  v[1] = lds_at(a + iw::kPlaneBytes);
+  v[1] = lds_at(a + kPB);
   v[2] = lds_at(a2);
-  v[3] = lds_at(a2 + iw::kPlaneBytes);
+  v[3] = lds_at(a2 + kPB);
   const uint32_t c = ln.s16 + ln.qm16;
   ln.s16 = min(c, c - ln.m16);
 }
@@ -576,7 +586,7 @@ __device__ __forceinline__ void lw_pipe(float4 (&a)[4], float4 (&buf)[4], uint32
     }
     lw_fence(a);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (N + 1 < Q) lw_issue<N + 1>(buf, pb, ln);
+    if constexpr (N + 1 < Q) lw_issue<Q, N + 1>(buf, pb, ln);
     __builtin_amdgcn_sched_barrier(0);
     lw_pipe<Q, N + 1>(a, buf, pb, ln);
   }
@@ -585,7 +595,7 @@ __device__ __forceinline__ void lw_pipe(float4 (&a)[4], float4 (&buf)[4], uint32
 template <int Q>
 __device__ __forceinline__ void lw_line_sums(float4 (&a)[4], uint32_t pb, LrLane ln) {
   float4 buf[4];
-  lw_issue<0>(buf, pb, ln);
+  lw_issue<Q, 0>(buf, pb, ln);
   __builtin_amdgcn_sched_barrier(0);
   lw_pipe<Q, 0>(a, buf, pb, ln);
 }
@@ -609,11 +619,17 @@ __device__ __forceinline__ LrLane own_lane(int li, int& code) {
 }
 
 template <int Q, bool HasG>
-__global__ __launch_bounds__(iw::kThreads, 1) void incidence_wave_kernel(
+__global__ __launch_bounds__(iw::Shape<Q>::kThreads,
+                             iw::Shape<Q>::kWgs * iw::Shape<Q>::kWaves / 4)
+void incidence_wave_kernel(
     const float* __restrict__ F, const float* __restrict__ Fg, const int* __restrict__ code,
     float* __restrict__ U, int B, int64_t rp, int64_t ld, int nslices, int64_t total,
     int64_t per_xcd) {
   using namespace iw;
+  typedef Shape<Q> Sh;
+  constexpr int kThreads = Sh::kThreads, kWaves = Sh::kWaves, kPF = Sh::kPF, kCW = Sh::kCW;
+  constexpr int kPlane = Sh::kPlane, kPlaneBytes = Sh::kPlaneBytes;
+  constexpr uint32_t kSlots = kThreads / 4;          // slots from one chunk to the next
   constexpr int q = Q;
   constexpr int N0 = Q * Q;
   constexpr int nlines = Q * (Q + 1);
@@ -631,7 +647,7 @@ __global__ __launch_bounds__(iw::kThreads, 1) void incidence_wave_kernel(
   static_assert(!kOwn || (NT - 1) / kWaves == kOwnK, "lines of their own in one task slot");
   constexpr int NR = (Q + 15) / 16;                  // runs of sixteen steps
   extern __shared__ float4 smem[];
-  short* line_type = reinterpret_cast<short*>(smem + (size_t)kPlanes * kPlane);
+  short* line_type = reinterpret_cast<short*>(smem);   // until the first panel
   const int tid = threadIdx.x;
   const int lane = lane_id();
   const int wv = __builtin_amdgcn_readfirstlane(wave_id());
@@ -667,12 +683,12 @@ __global__ __launch_bounds__(iw::kThreads, 1) void incidence_wave_kernel(
     const bool in = e0 + 4 * kx < rp;
 #pragma unroll
     for (int u = 0; u < kPF; ++u)
-      pf[u] = (ps0 + 256u * u < (uint32_t)N0 && in)
+      pf[u] = (ps0 + kSlots * u < (uint32_t)N0 && in)
                   ? *reinterpret_cast<const float4*>(Fb + src[u])
                   : make_float4(0.f, 0.f, 0.f, 0.f);
   };
 #pragma unroll
-  for (int u = 0; u < kPF; ++u) src[u] = chunk_src(ps0 + 256u * u);
+  for (int u = 0; u < kPF; ++u) src[u] = chunk_src(ps0 + kSlots * u);
   prefetch(first);
 
   // Row roles: group A or B of the wave's task, plane pair (0, 1) or (2, 3).
@@ -685,7 +701,7 @@ __global__ __launch_bounds__(iw::kThreads, 1) void incidence_wave_kernel(
   const uint32_t splane16 = 16u * splane;
 
   // The lane state of each of the wave's tasks is the same for every item, so
-  // it is worked out once: tasks wv, wv + 16, ... (kTasks at most); for each,
+  // it is worked out once: tasks wv, wv + kWaves, ... (kTasks at most); for each,
   // the lane part of the read address, the row parts ot[] of the q steps, and
   // the byte offsets in an item's U rows of the two lines this lane stores
   // after the half exchange (kNoLine: none).
@@ -746,6 +762,7 @@ __global__ __launch_bounds__(iw::kThreads, 1) void incidence_wave_kernel(
     tsA[k] = hA >= 0 ? (uint32_t)hA * ld4 + splane16 : kNoLine;
     tsB[k] = hB >= 0 ? (uint32_t)hB * ld4 + splane16 : kNoLine;
   }
+  lds_barrier();                                     // the line table's readers are done
 
   for (int64_t item = first; item < end; item += nk) {
     {
@@ -753,7 +770,7 @@ __global__ __launch_bounds__(iw::kThreads, 1) void incidence_wave_kernel(
       asm volatile("" : "+v"(p0));
 #pragma unroll
       for (int u = 0; u < kPF; ++u) {
-        const uint32_t ps = p0 + 256u * u;
+        const uint32_t ps = p0 + kSlots * u;
         const uint32_t x1 = LgSlot<Q>::div(ps), x0 = ps - Q * x1;
         if (ps < (uint32_t)N0) {
           float4* e = smem + (kx * kPlane + kCW * x1 + x0);
@@ -764,7 +781,7 @@ __global__ __launch_bounds__(iw::kThreads, 1) void incidence_wave_kernel(
         src[u] = __umul24(x0 * Q + x1, ld4) + 16u * kx;
       }
     }
-    lds_barrier();                                   // panel (and line table) complete
+    lds_barrier();                                   // panel complete
     const int64_t b = item / nslices;
     const int64_t e0 = (item - b * nslices) * kE;
     if (item + nk < end) prefetch(item + nk);        // lands while this item is summed
@@ -834,9 +851,9 @@ static int launch_wave_q(const float* F, const float* F_glob, const int* code, f
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   const int64_t per_xcd = (total + inc::kXCD - 1) / inc::kXCD;
-  const int64_t per_xcd_wgs = std::max<int64_t>(1, std::min<int64_t>(ncu / inc::kXCD, per_xcd));
+  const int64_t per_xcd_wgs = std::max<int64_t>(1, std::min<int64_t>((int64_t)ncu * Shape<Q>::kWgs / inc::kXCD, per_xcd));
   const unsigned grid = (unsigned)(per_xcd_wgs * inc::kXCD);
-  const size_t smem = (size_t)wave_lds_bytes(Q);
+  const size_t smem = (size_t)Shape<Q>::kLdsBytes;
   static bool attr_set[2] = {false, false};
   auto kern = F_glob ? incidence_wave_kernel<Q, true> : incidence_wave_kernel<Q, false>;
   if (!attr_set[F_glob ? 1 : 0]) {
@@ -844,7 +861,7 @@ static int launch_wave_q(const float* F, const float* F_glob, const int* code, f
                               inc::kPlaneLdsBudget);
     attr_set[F_glob ? 1 : 0] = true;
   }
-  smat::launch(kern, dim3(grid), dim3(kThreads), smem, stream, F, F_glob, code, U, B, rp, ld,
+  smat::launch(kern, dim3(grid), dim3(Shape<Q>::kThreads), smem, stream, F, F_glob, code, U, B, rp, ld,
                      nslices, total, per_xcd);
   return launch_status("smat_incidence_plane");
 }

@@ -352,6 +352,61 @@ def test_line_group_incidence_reads_each_line_once_in_bounds(q):
     assert sorted(stored) == list(range(q * (q + 1))) and set(stored.values()) == {1}
 
 
+def _line_group_shape(q):
+    """(threads, workgroups a CU, chunks a thread, kCW, kPlane) of iw::Shape<q>."""
+    threads = 256 if q <= 19 else 512 if q <= 23 else 1024
+    wgs = 4 if q <= 17 else 3 if q <= 19 else 2 if q <= 23 else 1
+    cw = (q + 15 + 1) // 2 * 2
+    return threads, wgs, -(-q * q * 4 // threads), cw, -(-cw * q // 16) * 16
+
+
+@pytest.mark.parametrize("q", _WAVE_Q)
+def test_line_group_incidence_shapes_by_field_size(q, monkeypatch):
+    """The panel shape and thread count of each field size: the panels of a CU's
+    workgroups fit its 160 KB of LDS and the 16-bit read offset, the line table
+    (which shares the panel's first bytes before the first item) fits a panel,
+    the staging covers every (point, plane) once, and every read lands on a
+    staged entry, each line on its own q points."""
+    threads, wgs, pf, cw, plane = _line_group_shape(q)
+    waves = threads // 64
+    monkeypatch.setitem(globals(), "_KCW", cw)
+    monkeypatch.setitem(globals(), "_KPLANE", plane)
+    assert wgs * 4 * plane * 16 <= 160 * 1024 and plane * 16 < 65536
+    assert q * (q + 1) * 2 <= 4 * plane * 16 and cw % 2 == 0
+    M, S = _lgdiv(q, 16 * waves * pf)
+    panel, seen = {}, set()
+    for tid in range(threads):
+        kx = (tid >> 4) & 3
+        for u in range(pf):
+            ps = 16 * (tid >> 6) + (tid & 15) + threads // 4 * u
+            if ps >= q * q:
+                continue
+            x1 = (ps * M) >> S
+            x0 = ps - q * x1
+            assert (x1, x0) == divmod(ps, q) and (kx, ps) not in seen
+            seen.add((kx, ps))
+            for c in range((q + 15 + q - 1) // q):
+                if x0 + c * q < q + 15:
+                    e = kx * plane + cw * x1 + x0 + c * q
+                    assert e not in panel and e < 4 * plane
+                    panel[e] = x0 * q + x1
+    assert len(seen) == 4 * q * q
+    P, G, NTG, R, NOL = _wave_plan(q)
+    NT = NTG + (NOL + 63) // 64
+    assert NOL == 0 or (NT - 1) // waves == NTG // waves
+    got = {}
+    for grp, j, pl, pp, t, e, lc in _wave_reads(q):
+        assert e in panel and e // plane == pl
+        if lc is not None:
+            got.setdefault((lc, pl), []).append(panel[e])
+    for e in range(q + 1):
+        for b in range(q):
+            pts = sorted(x0 * q + b for x0 in range(q)) if e == 0 else \
+                sorted(((b - (e - 1) * t) % q) * q + t for t in range(q))
+            for pl in range(4):
+                assert sorted(got[e * q + b, pl]) == pts
+
+
 @pytest.mark.parametrize("q", [17, 29, 37, 41])
 def test_line_group_incidence_rows_read_one_bank_phase_each(q):
     """At every step the sixteen lanes of a row read sixteen distinct 16-byte
