@@ -453,7 +453,7 @@ int scan_stream_launch(int dtype, const void* phi, const void* psi, const void* 
 int scan_stream_launch_feat(int dtype, const void* q, const void* k, const void* v,
                             const float* Sg, const float* Y, const float* gate, float* out,
                             int nb, int ng, const ScanArgs& a, const FeatArgs& fa,
-                            bool psi_formed, hipStream_t stream);
+                            hipStream_t stream);
 int gram_stream_launch_feat(int dtype, const void* k, const void* v, float* G, float* G_last,
                             const GramItems& it, int nitems, int nb, int64_t k_sb, int64_t k_st,
                             int64_t v_sb, int64_t v_st, int64_t g_sb, int64_t g_si,
@@ -588,10 +588,9 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
 // The streaming causal pass with the feature map computed inside the kernels:
 // q, k, v are the Q, K, V rows (r = d_qk = d_v = 128); the prepass Gram sums
 // and the scan form Psi (and Phi) tiles in LDS from the DMA'd K (and Q) rows,
-// and Vb = [V, 1] from V.  Same workspace as causal_scan_dispatch's
-// with forward.  With
-// psi_buf (nb x T rows of 128, 16-bit) the prepass also stores the Psi tiles
-// it forms there and the scan reads them, forming only Phi.
+// and Vb = [V, 1] from V.  Same workspace as causal_scan_dispatch's with
+// forward.  The prepass also stores the Psi tiles it forms to psi_buf (nb x T
+// rows of 128, 16-bit) and the scan reads them, forming only Phi.
 int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v, const float* Y,
                          const float* gate, float* out, int nb, int T, int n, int C,
                          int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb,
@@ -642,8 +641,8 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
   a.p = p;
   a.q_sb = q_sb;
   a.q_st = q_st;
-  a.k_sb = psi_buf ? fp.psi_sb : k_sb;
-  a.k_st = psi_buf ? 128 : k_st;
+  a.k_sb = fp.psi_sb;
+  a.k_st = 128;
   a.v_sb = v_sb;
   a.v_st = v_st;
   a.y_sb = y_sb;
@@ -652,8 +651,7 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
   a.o_st = o_st;
   a.g_sb = g_sb;
   a.write_H = 0;
-  return scan_stream_launch_feat(dtype, q, psi_buf ? psi_buf : k, v, Sg, Y, gate, out, nb, ng, a,
-                                 fa, psi_buf != nullptr, stream);
+  return scan_stream_launch_feat(dtype, q, psi_buf, v, Sg, Y, gate, out, nb, ng, a, fa, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -1,9 +1,11 @@
-// The causal pass of the schedule for the common head shape -- 16-bit inputs,
-// r = 128 features, p = 129 value columns (head_dim 128 plus the ones column),
-// T and n multiples of 64 -- streamed through LDS.  Same contract as the
-// normalising mode of scan_fused_kernel (src/smat/attention.py:134-192 and
+// The causal pass of the schedule for the common head shapes -- 16-bit inputs,
+// r = 64, 80, 96, 112 or 128 features, p = r + 1 value columns (the head's plus
+// the ones column), n and the chunk multiples of 64 -- streamed through LDS.
+// Same contract as scan_fused_kernel (src/smat/attention.py:134-192 and
 // :446-453): segmented chunked scan with one reset at n, the long-range term
-// Y added to recent rows, division by the normaliser column, optional gate.
+// Y added to recent rows, division by the normaliser column, optional gate; or
+// H itself.  The description below is of r = 128, eight waves; r = 16 NW takes
+// NW waves and NW column tiles, rows of eight chunks and two buffers at r = 64.
 //
 //   * One workgroup of eight waves walks one group of chunks; the group's
 //     incoming state comes from the same prepass (Gram sums per group, shifted
@@ -61,7 +63,24 @@ constexpr int kTileChunks = kStep * kRowChunks;    // 1024
 constexpr int kVbTileChunks = kTileChunks + kStep; // + columns 128..135, one chunk a row
 constexpr int kPhiLoads = kTileChunks / 64;        // wave-wide DMA loads per tile: 16
 constexpr int kVbLoads = kVbTileChunks / 64;       // 17
-constexpr int kLoads = 2 * kPhiLoads + kVbLoads;   // 49 per step, over eight waves
+
+// The scan at r = 16 NW features: NW waves, one 16-column tile of Vb each.
+// LDS rows hold 16 chunks of 16 bytes (r > 64, of which 2 NW are used) or 8.
+// kLoads wave-wide copies bring a step's rows (Phi, Psi, Vb and Vb's
+// normaliser chunks); copy I goes to wave I % NW, so wave w issues kBase of
+// them, one more for w < kExtra.  Three row buffers at r > 64 (a workgroup a
+// CU); two at r = 64, whose 59 KB let two workgroups share a CU.
+template <int NW, bool FEAT>
+struct Scan {
+  static constexpr int kThreads = 64 * NW;
+  static constexpr int kRC = NW > 4 ? 16 : 8;
+  static constexpr int kTile = kStep * kRC;
+  static constexpr int kVbTile = kTile + kStep;
+  static constexpr int kLoads = 3 * kRC + (FEAT ? 0 : 1);
+  static constexpr int kBase = kLoads / NW, kExtra = kLoads % NW;
+  static constexpr int kSlots = (kLoads + NW - 1) / NW;
+  static constexpr int kBufs = NW > 4 ? 3 : 2;
+};
 }  // namespace ss
 
 #define SMAT_LDS __attribute__((address_space(3)))
@@ -71,6 +90,13 @@ __device__ __forceinline__ int swz16(int t) {
   return (((t & 7) << 1) | ((t >> 3) & 1)) ^ (t & 8);
 }
 __device__ __forceinline__ int swz8(int t) { return (t >> 1) & 7; }
+// The same for rows of eight chunks (r = 64): t's bits 2, 1, 3, so that the
+// even (and the odd) rows of a phase of any of the three reads take distinct
+// slots beside their neighbours' half of the banks.
+template <int RC>
+__device__ __forceinline__ int swz_row(int t) {
+  return RC == 16 ? swz16(t) : ((t >> 2) & 1) | (t & 2) | ((t >> 1) & 4);
+}
 // Float index of wave w's normaliser partial of row t: 8 floats a row, the two
 // 4-float halves swapped in rows 8..15 of every 16.
 __device__ __forceinline__ int norm_slot(int t, int w) {
@@ -99,18 +125,17 @@ __device__ __forceinline__ uint32_t load_u16_untracked(const void* p) {
   return v;
 }
 
-// 8 bytes of a swizzled 256-byte row (t, chunk k, half h).
-template <typename In>
+// 8 bytes of a swizzled row of RC chunks (t, chunk k, half h).
+template <typename In, int RC>
 __device__ __forceinline__ typename Traits<In>::half_frag row_half(const uint4* tile, int t, int k,
                                                                     int h) {
-  const char* p = reinterpret_cast<const char*>(tile + t * ss::kRowChunks + (k ^ swz16(t))) + 8 * h;
+  const char* p = reinterpret_cast<const char*>(tile + t * RC + (k ^ swz_row<RC>(t))) + 8 * h;
   return *reinterpret_cast<const typename Traits<In>::half_frag*>(p);
 }
-// 16 bytes (one chunk) of a swizzled 256-byte row.
-template <typename In>
+// 16 bytes (one chunk) of a swizzled row.
+template <typename In, int RC>
 __device__ __forceinline__ typename Traits<In>::frag row_chunk(const uint4* tile, int t, int k) {
-  return *reinterpret_cast<const typename Traits<In>::frag*>(tile + t * ss::kRowChunks +
-                                                              (k ^ swz16(t)));
+  return *reinterpret_cast<const typename Traits<In>::frag*>(tile + t * RC + (k ^ swz_row<RC>(t)));
 }
 
 template <typename In>
@@ -134,7 +159,7 @@ __device__ __forceinline__ typename Traits<In>::frag join(typename Traits<In>::h
 
 // A fragment of Psi^T (rows a = 16*at + lane%16, k-slots = tokens
 // 32*ks + 8*grp + j) from a swizzled Psi tile, by two transposing reads.
-template <typename In>
+template <typename In, int RC = ss::kRowChunks>
 __device__ __forceinline__ typename Traits<In>::frag psi_tr(const uint4* tile, int at, int ks,
                                                             int lane) {
   const int r16 = lane & 15, g = lane >> 4;
@@ -144,95 +169,102 @@ __device__ __forceinline__ typename Traits<In>::frag psi_tr(const uint4* tile, i
     const int row = 32 * ks + 8 * g + 4 * h + (r16 >> 2);
     const int k = 2 * at + ((r16 & 3) >> 1);
     const char* p =
-        reinterpret_cast<const char*>(tile + row * ss::kRowChunks + (k ^ swz16(row))) +
-        8 * (r16 & 1);
+        reinterpret_cast<const char*>(tile + row * RC + (k ^ swz_row<RC>(row))) + 8 * (r16 & 1);
     h2[h] = tr_read<In>(p);
   }
   return join<In>(h2[0], h2[1]);
 }
 
-// Fragment of Vb along tokens (column 16*ct + lane%16, k-slots = tokens
-// 32*ks + 8*grp + j): the B operand of the state update and the A operand
-// (Vb^T) of the within-step product.  Column tiles 0..7 are read like Psi's;
-// tile 8 (columns 128..143) comes from the 16-byte rows of columns 128..135,
-// and its lanes 8..15 repeat columns 128..135 in place of 136..143, which
-// no caller keeps.
-template <typename In>
-__device__ __forceinline__ typename Traits<In>::frag vb_tr(const uint4* tile, int ct, int ks,
-                                                           int lane) {
-  if (ct < 8) return psi_tr<In>(tile, ct, ks, lane);
+// The normaliser tile of Vb along tokens (column d_v + lane%16, k-slots =
+// tokens 32*ks + 8*grp + j) from the 16-byte rows of columns d_v .. d_v + 7 after
+// the tile: the ones column and seven columns of padding; lanes 8..15 repeat
+// them in place of columns no caller keeps.
+template <typename In, int RC = ss::kRowChunks>
+__device__ __forceinline__ typename Traits<In>::frag vb_norm_tr(const uint4* tile, int ks,
+                                                                int lane) {
   const int r16 = lane & 15, g = lane >> 4;
   typename Traits<In>::half_frag h2[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int row = 32 * ks + 8 * g + 4 * h + (r16 >> 2);
-    const char* p = reinterpret_cast<const char*>(tile + ss::kTileChunks + row) + 8 * (r16 & 1);
+    const char* p = reinterpret_cast<const char*>(tile + ss::kStep * RC + row) + 8 * (r16 & 1);
     h2[h] = tr_read<In>(p);
   }
   return join<In>(h2[0], h2[1]);
 }
 
 // The DMA of one step's Phi, Psi and Vb rows [ts, ts + 64) into one buffer.
-// Load I of the 49 goes to wave I % 8 as its slot u = I / 8: slots 0-1 are
-// Phi's loads 0-15, slots 2-3 Psi's, slots 4-5 Vb's columns 0..127, and slot
-// 6 (wave 0 only) Vb's columns 128..135, lane = row (wave 0 issues seven
-// loads, the others six).  Each load moves 64 x 16 bytes to 1 KB of
-// consecutive LDS; which global chunk a lane fetches implements the swizzle.
-// That choice does not depend on the step, so a lane's byte offset from the
-// step's first row is computed once per slot (dma_offsets); a step adds it
-// to the wave-uniform row base of the slot's tensor.
+// Copy I of the kLoads goes to wave I % NW as its slot u = I / NW: kRC copies of
+// Phi, of Psi, of Vb's columns below r, then (not FEAT) one of the normaliser
+// chunks, lane = row.  Each moves 64 x 16 bytes to 1 KB of consecutive LDS;
+// which global chunk a lane fetches implements the swizzle (chunks past the
+// row's 2 NW re-read one of its own).  That choice does not depend on the
+// step, so a lane's byte offset from the step's first row is computed once per
+// slot; a step adds it to the wave-uniform row base of the slot's tensor.
+template <int NW, bool FEAT>
 struct DmaOffsets {
-  uint32_t off[7];
+  uint32_t off[ss::Scan<NW, FEAT>::kSlots];
 };
 
-template <typename In>
-__device__ __forceinline__ void dma_offsets(DmaOffsets& d, const ScanArgs& a, int w, int lane) {
-#pragma unroll
-  for (int u = 0; u < 7; ++u) {
-    const int I = w + 8 * u;
-    int64_t e = 0;                                   // element offset from row ts
-    if (u < 6) {
-      const int li = I & 15;
-      const int row = 4 * li + (lane >> 4);
-      const int k = (lane & 15) ^ swz16(row);
-      e = (int64_t)row * (u < 2 ? a.q_st : u < 4 ? a.k_st : a.v_st) + 8 * k;
-    } else if (I < ss::kLoads) {
-      e = (int64_t)lane * a.v_st + 128;              // columns 128..135 of row = lane
-    }
-    d.off[u] = (uint32_t)(e * (int64_t)sizeof(In));
-  }
+// Which tensor copy NW u + w belongs to (0 Phi, 1 Psi, 2 Vb): known at compile
+// time unless the slot's copies straddle two tensors.
+template <int NW, int RC>
+__device__ __forceinline__ int dma_tensor(int u, int w) {
+  const int lo = NW * u, hi = NW * u + NW - 1;
+  if (hi < RC) return 0;
+  if (lo >= RC && hi < 2 * RC) return 1;
+  if (lo >= 2 * RC) return 2;
+  const int I = NW * u + w;
+  return I < RC ? 0 : I < 2 * RC ? 1 : 2;
 }
 
-// FEAT: the rows are Q, K and V (the feature map runs in LDS afterwards), and
-// the ninth Vb tile is the constant [1, 0, ...] written once: six loads a wave.
-template <typename In, bool FEAT, bool UNTRACKED>
+// last: the last row to fetch (rows past it re-read it).
+template <typename In, int NW, bool FEAT>
+__device__ __forceinline__ uint32_t dma_offset(const ScanArgs& a, int u, int w, int lane,
+                                               int last) {
+  typedef ss::Scan<NW, FEAT> Sh;
+  constexpr int RC = Sh::kRC;
+  const int I = w + NW * u;
+  if (I >= 3 * RC)                                   // the normaliser chunk of row = lane
+    return (uint32_t)(((int64_t)min(lane, last) * a.v_st + 16 * NW) * (int64_t)sizeof(In));
+  const int t = dma_tensor<NW, RC>(u, w);
+  const int row = (64 / RC) * (I - t * RC) + lane / RC;
+  int k = (lane % RC) ^ swz_row<RC>(row);
+  if (2 * NW < RC && k >= 2 * NW) k -= 8;
+  const int64_t st = t == 0 ? a.q_st : t == 1 ? a.k_st : a.v_st;
+  return (uint32_t)((min(row, last) * st + 8 * k) * (int64_t)sizeof(In));
+}
+
+// FEAT: the rows are Q, Psi and V (the feature map runs in LDS afterwards), and
+// the normaliser tile is the constant [1, 0, ...] written once.  RAG: T is not a
+// multiple of 64, and the step that crosses it fetches row T - 1 in place of
+// rows past it.
+template <typename In, int NW, bool FEAT, bool RAG>
 __device__ __forceinline__ void issue_step(uint4* dphi, uint4* dpsi, uint4* dvb, const In* phib,
                                            const In* psib, const In* vbb, int64_t ts,
-                                           const ScanArgs& a, int w, const DmaOffsets& d) {
+                                           const ScanArgs& a, int w, int lane,
+                                           const DmaOffsets<NW, FEAT>& d) {
+  typedef ss::Scan<NW, FEAT> Sh;
+  constexpr int RC = Sh::kRC;
   const char* bphi = reinterpret_cast<const char*>(phib + ts * a.q_st);
   const char* bpsi = reinterpret_cast<const char*>(psib + ts * a.k_st);
   const char* bvb = reinterpret_cast<const char*>(vbb + ts * a.v_st);
+  const int last = (int)min<int64_t>(ss::kStep, a.T - ts) - 1;
 #pragma unroll
-  for (int u = 0; u < (FEAT ? 6 : 7); ++u) {
-    const int I = w + 8 * u;
-    if (I < ss::kLoads) {
-      const char* base = u < 2 ? bphi : u < 4 ? bpsi : bvb;
-      uint4* dst = u < 2 ? dphi + 64 * I
-                 : u < 4 ? dpsi + 64 * (I - ss::kPhiLoads)
-                         : dvb + 64 * (I - 2 * ss::kPhiLoads);
-      lds_dma16<UNTRACKED>(reinterpret_cast<const void*>(base + d.off[u]), dst);
+  for (int u = 0; u < Sh::kSlots; ++u) {
+    const int I = w + NW * u;
+    if (I < Sh::kLoads) {
+      const int t = dma_tensor<NW, RC>(u, w);
+      const char* base = t == 0 ? bphi : t == 1 ? bpsi : bvb;
+      uint4* dst = t == 0 ? dphi : t == 1 ? dpsi : dvb;
+      const uint32_t off = RAG && last < ss::kStep - 1
+                               ? dma_offset<In, NW, FEAT>(a, u, w, lane, last)
+                               : d.off[u];
+      lds_dma16<true>(reinterpret_cast<const void*>(base + off), dst + 64 * (I - t * RC));
     }
   }
 }
 
-struct YRegs {
-  float4 y[4];      // Y[t][16w + 4g .. +3] for the step's four row tiles
-  float y8[4];      // Y[t][p - 1]
-  float gv[4];      // gate
-};
-
-// Twelve loads, always issued (dummy in-bounds addresses when a term is
-// absent), so the compiler's waits on them count a fixed number of loads.
 // Per-lane byte offsets of the step's Y and output rows from row ts (the
 // lane's rows 16 tt + lane % 16 at columns 16 w + 4 g), computed once; a step
 // adds them to wave-uniform row bases.  y8 is the normaliser column's offset
@@ -252,21 +284,6 @@ __device__ __forceinline__ void row_offsets(RowOffsets& R, const ScanArgs& a, in
   R.y8 = (a.p - 1 - 16 * w - 4 * g) * 4;
 }
 
-__device__ __forceinline__ void issue_y(YRegs& R, const float* Yb, const float* gb,
-                                       const float* dummy, int64_t ts, const ScanArgs& a,
-                                       const RowOffsets& ro, int lane) {
-  const int r16 = lane & 15;
-  const bool rec = Yb != nullptr && ts >= a.n;
-  const char* yb = rec ? reinterpret_cast<const char*>(Yb + (ts - a.n) * a.y_st) : nullptr;
-#pragma unroll
-  for (int tt = 0; tt < 4; ++tt) {
-    const char* yc = rec ? yb + ro.y[tt] : reinterpret_cast<const char*>(dummy);
-    R.y[tt] = *reinterpret_cast<const float4*>(yc);
-    R.y8[tt] = rec ? *reinterpret_cast<const float*>(yc + ro.y8) : 0.f;
-    R.gv[tt] = gb ? gb[ts + 16 * tt + r16] : 1.f;
-  }
-}
-
 __device__ __forceinline__ f32x4 mma16(f32x4 c, bf16x4 a, bf16x4 b) {
   typedef short s4 __attribute__((ext_vector_type(4)));
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s4, a),
@@ -276,42 +293,60 @@ __device__ __forceinline__ f32x4 mma16(f32x4 c, f16x4 a, f16x4 b) {
   return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
 }
 
-// FEAT = 1: phi, psi and vb are Q, K and V rows (v_st may be 128); each
-// step's Phi and Psi tiles are formed from the DMA'd Q and K tiles into two
-// more tiles, phiF and psiF (feat_rows, W in registers), the key gate applied
-// to Psi.  A step's reads of phiF and psiF end before the barrier after its
-// state update, so the next step's features overwrite them safely.
-// FEAT = 2: psi holds Psi rows already (gate applied), only Phi is formed,
-// in place over the DMA'd Q tile, with three row buffers.
-template <typename In, int FEAT, int NBUF, bool TERMS>
-__global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
+// The step's Y rows, its normaliser column and gates in registers, loaded
+// untracked (used after a wait that covers them).
+struct YRegs {
+  f32x4 y[4];      // Y[t][16w + 4g .. +3] for the step's four row tiles
+  float y8[4];     // Y[t][p - 1]
+  float gv[4];     // gate
+};
+
+// NW: r = 16 NW features, p = 16 NW + 1.  FEAT (NW = 8): phi, psi and vb are Q,
+// Psi (formed by the prepass, gate applied) and V rows; Phi is formed in place
+// over the copied Q tile.  TERMS = false compiles Y and the gate out (launches
+// with neither): their pointers and flags would otherwise spill scalar
+// registers every step.  RAG: T is not a multiple of 64.  WH: out is H
+// (unnormalised, p columns, rows of any alignment).
+//
+// What bounds it: HBM at r = 128 (4.6 TB/s).  At r = 64 .. 112 it took the place
+// of the general kernel, which stages rows through registers into two LDS
+// layouts and stores 4-byte elements: forward of 32 x 8192 tokens at r = 64
+// 164 -> 119 us, of 12 x 10007 (ragged) at r = 96 403 -> 317 us, the positional
+// training step's (H, r = 64) 1825 -> 1766 us.
+template <typename In, int NW, bool FEAT, bool TERMS, bool RAG, bool WH>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
     const In* __restrict__ phi, const In* __restrict__ psi, const In* __restrict__ vb,
     const float* __restrict__ Sg, const float* __restrict__ Y, const float* __restrict__ gate,
     float* __restrict__ out, ScanArgs a, FeatArgs fa) {
   using namespace ss;
+  typedef Scan<NW, FEAT> Sh;
   typedef typename Traits<In>::frag Frag;
   typedef typename Traits<In>::half_frag Half;
-  __shared__ __attribute__((aligned(16))) uint4 phi0[kTileChunks];
-  __shared__ __attribute__((aligned(16))) uint4 psi0[kTileChunks];
-  __shared__ __attribute__((aligned(16))) uint4 vb0[kVbTileChunks];
-  __shared__ __attribute__((aligned(16))) uint4 phi1[kTileChunks];
-  __shared__ __attribute__((aligned(16))) uint4 psi1[kTileChunks];
-  __shared__ __attribute__((aligned(16))) uint4 vb1[kVbTileChunks];
-  // NBUF = 3 (no Psi formed here): a third buffer (160 768 bytes of LDS in
-  // all) keeps the rows of steps s + 1 and s + 2 in flight while step s
-  // computes.
-  // Y and the gate are then loaded untracked and waited for by count.
-  // TERMS = false compiles Y and the gate out (launches with neither): their
-  // pointers and flags would otherwise spill scalar registers every step.
-  static_assert(NBUF == 2 || (NBUF == 3 && FEAT != 1), "three buffers only without Psi formed here");
-  __shared__ __attribute__((aligned(16))) uint4 phi2[NBUF == 3 ? kTileChunks : 1];
-  __shared__ __attribute__((aligned(16))) uint4 psi2[NBUF == 3 ? kTileChunks : 1];
-  __shared__ __attribute__((aligned(16))) uint4 vb2[NBUF == 3 ? kVbTileChunks : 1];
+  constexpr int RC = Sh::kRC, NBUF = Sh::kBufs, NKB = NW / 2;
+  // An odd NW's last 16 features are a k-block whose other half is zero, on the
+  // same MFMA as the others: a chain that went on from the 16 x 16 x 32 form to
+  // the 16 x 16 x 16 one lost terms of its accumulator (seen on gfx950).
+  constexpr bool kOdd = NW % 2 != 0;
+  constexpr int kSteps = NKB + (kOdd ? 1 : 0);
+  constexpr int kBase = Sh::kBase, kExtra = Sh::kExtra;
+  static_assert(!FEAT || (NW == 8 && !RAG && !WH), "the feature map is 128 x 128");
+  static_assert(!(WH && TERMS), "H carries no Y and no gate");
+  __shared__ __attribute__((aligned(16))) uint4 phi0[Sh::kTile];
+  __shared__ __attribute__((aligned(16))) uint4 psi0[Sh::kTile];
+  __shared__ __attribute__((aligned(16))) uint4 vb0[Sh::kVbTile];
+  __shared__ __attribute__((aligned(16))) uint4 phi1[Sh::kTile];
+  __shared__ __attribute__((aligned(16))) uint4 psi1[Sh::kTile];
+  __shared__ __attribute__((aligned(16))) uint4 vb1[Sh::kVbTile];
+  // Three buffers (160 768 bytes of LDS in all) keep the rows of steps s + 1
+  // and s + 2 in flight while step s computes; with two, step s + 2's copy is
+  // issued once every wave is past step s's rows.  Y and
+  // the gate are loaded untracked and waited for by count.
+  __shared__ __attribute__((aligned(16))) uint4 phi2[NBUF == 3 ? Sh::kTile : 1];
+  __shared__ __attribute__((aligned(16))) uint4 psi2[NBUF == 3 ? Sh::kTile : 1];
+  __shared__ __attribute__((aligned(16))) uint4 vb2[NBUF == 3 ? Sh::kVbTile : 1];
   __shared__ __attribute__((aligned(16))) uint4 share[kStep * 8];
   // normaliser partials: wave w's share of H[t][p-1] at normp[norm_slot(t, w)]
   __shared__ __attribute__((aligned(16))) float normp[kStep * 8];
-  __shared__ __attribute__((aligned(16))) uint4 phiF[FEAT && NBUF == 2 ? kTileChunks : 1];
-  __shared__ __attribute__((aligned(16))) uint4 psiF[FEAT == 1 ? kTileChunks : 1];
 
   // Groups run last sequence first, last group first: the prepass just read
   // the same Psi and Vb rows in the opposite order, so the first groups here
@@ -323,9 +358,7 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
   // scalar branch.  (Under a vector condition the compiler masks EXEC around
   // an MFMA without branching past it, and MFMAs execute regardless of EXEC.)
   const int w = __builtin_amdgcn_readfirstlane(wave_id());
-  // Eight waves: the DMA's loads 0..47 are then unconditional, and the
-  // compiler's count of loads issued after the Y loads is exact.
-  __builtin_assume(w >= 0 && w < 8);
+  __builtin_assume(w >= 0 && w < NW);
   const int lane = lane_id();
   const int r16 = lane & 15, g = lane >> 4;
 
@@ -339,7 +372,7 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
   }
   const int64_t tk0 = (int64_t)c0 * a.C;
   const int64_t tk1 = min((int64_t)c1 * a.C, (int64_t)a.T);
-  const int nsteps = (int)((tk1 - tk0) / kStep);
+  const int nsteps = (int)((tk1 - tk0 + (RAG ? kStep - 1 : 0)) / kStep);
 
   const In* phib = phi + b * a.q_sb;
   const In* psib = psi + b * a.k_sb;
@@ -347,55 +380,97 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
   const float* Yb = (TERMS && Y) ? Y + b * a.y_sb : nullptr;
   const float* gb = (TERMS && gate) ? gate + b * a.g_sb : nullptr;
   float* outb = out + b * a.o_sb;
-  const float* Sb = Sg + ((int64_t)b * gridDim.x + grp) * (int64_t)128 * a.p;
+  const float* Sb = Sg + ((int64_t)b * gridDim.x + grp) * (int64_t)(16 * NW) * a.p;
 
-  DmaOffsets dmo;
-  dma_offsets<In>(dmo, a, w, lane);
+  DmaOffsets<NW, FEAT> dmo;
+#pragma unroll
+  for (int u = 0; u < Sh::kSlots; ++u)
+    dmo.off[u] = w + NW * u < Sh::kLoads ? dma_offset<In, NW, FEAT>(a, u, w, lane, kStep - 1) : 0;
   RowOffsets rof;
   row_offsets(rof, a, w, lane);
-  if (nsteps > 0) issue_step<In, FEAT != 0, NBUF == 3>(phi0, psi0, vb0, phib, psib, vbb, tk0, a, w, dmo);
+  if (nsteps > 0)
+    issue_step<In, NW, FEAT, RAG>(phi0, psi0, vb0, phib, psib, vbb, tk0, a, w, lane, dmo);
   Frag wa[4];
-  const In* hb = nullptr;
   if constexpr (FEAT) {
     feat_w_load<In>(wa, (const In*)fa.W, w, lane);
-    feat_ones_tile<In>(vb0 + kTileChunks, threadIdx.x, kThreads);
-    feat_ones_tile<In>(vb1 + kTileChunks, threadIdx.x, kThreads);
-    if (NBUF == 3) feat_ones_tile<In>(vb2 + kTileChunks, threadIdx.x, kThreads);
-    if (FEAT == 1) hb = fa.h ? (const In*)fa.h + b * fa.h_sb : nullptr;
+    feat_ones_tile<In>(vb0 + Sh::kTile, threadIdx.x, Sh::kThreads);
+    feat_ones_tile<In>(vb1 + Sh::kTile, threadIdx.x, Sh::kThreads);
+    feat_ones_tile<In>(vb2 + Sh::kTile, threadIdx.x, Sh::kThreads);
+  }
+  // The score tiles (1, 0) and (3, 2) stay zero, and so do the normaliser
+  // partials of waves that do not exist (published by step 0's first barrier).
+  for (int e = threadIdx.x; e < kStep * 8; e += Sh::kThreads) {
+    share[e] = make_uint4(0, 0, 0, 0);
+    normp[e] = 0.f;
   }
 
   // incoming state: S[a][16w + lane%16] for all a, and the normaliser column
-  // block S[a][128 + lane%16] for this wave's rows a in [16w, 16w + 16)
-  const int cn = a.p - 1 - 128;            // normaliser's row in the ninth tile
-  f32x4 accS[8], accS8;
+  // S[a][16 NW] (in lanes % 16 = 0) for this wave's rows a in [16w, 16w + 16)
+  f32x4 accS[NW], accS8;
 #pragma unroll
-  for (int at = 0; at < 8; ++at)
+  for (int at = 0; at < NW; ++at)
 #pragma unroll
     for (int i = 0; i < 4; ++i) accS[at][i] = Sb[(int64_t)(16 * at + 4 * g + i) * a.p + 16 * w + r16];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int c8 = 128 + r16;
-    const float v8 = Sb[(int64_t)(16 * w + 4 * g + i) * a.p + (c8 < a.p ? c8 : 0)];
-    accS8[i] = c8 < a.p ? v8 : 0.f;
+    const float v8 = Sb[(int64_t)(16 * w + 4 * g + i) * a.p + (r16 == 0 ? 16 * NW : 0)];
+    accS8[i] = r16 == 0 ? v8 : 0.f;
   }
   // Consume the state (and W) loads here, so that no wait for them is placed
-  // inside the loop.  With three buffers the copies are untracked and the
-  // compiler's wait here is vmcnt(0), which lands step 0's rows too; step
-  // 1's copy goes out after it.
+  // inside the loop.  The copies are untracked and the compiler's wait here is
+  // vmcnt(0), which lands step 0's rows too; step 1's copy goes out after it.
 #pragma unroll
-  for (int at = 0; at < 8; ++at) asm volatile("" : "+v"(accS[at]));
+  for (int at = 0; at < NW; ++at) asm volatile("" : "+v"(accS[at]));
   asm volatile("" : "+v"(accS8));
   if constexpr (FEAT) {
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) asm volatile("" : "+v"(wa[kb]));
   }
-  if (NBUF == 3 && nsteps > 1)
-    issue_step<In, FEAT != 0, true>(phi1, psi1, vb1, phib, psib, vbb, tk0 + kStep, a, w, dmo);
+
+  // Rows of the step at ts that exist (all 64 except across a ragged T).
+  auto rows_left = [&](int64_t ts) { return RAG ? (int)min<int64_t>(kStep, a.T - ts) : kStep; };
+  // The Y rows and gates of the step at ts (rows past a ragged T re-read row
+  // T - 1's).
+  auto issue_y = [&](YRegs& R, int64_t ts) {
+    const bool rec = Yb != nullptr && ts >= a.n;
+    const int left = rows_left(ts);
+    if (rec) {
+      const char* yb = reinterpret_cast<const char*>(Yb + (ts - a.n) * a.y_st);
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) {
+        uint32_t off = rof.y[tt];
+        if (RAG && left < kStep)
+          off = (uint32_t)((min(16 * tt + r16, left - 1) * a.y_st + 16 * w + 4 * g) * 4);
+        R.y[tt] = load4_untracked(yb + off);
+        R.y8[tt] = load1_untracked(yb + off + rof.y8);
+      }
+    }
+    if (gb) {
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) {
+        const int t = RAG ? min(16 * tt + r16, left - 1) : 16 * tt + r16;
+        R.gv[tt] = load1_untracked(gb + ts + t);
+      }
+    }
+  };
+  // Until only the step's copy issued last is outstanding (its count differs by
+  // one between the waves), or nothing when none was issued.
+  auto wait_dma = [&](bool issued) {
+    if (!issued)
+      wait_vmcnt<0>();
+    else if (w < kExtra)
+      wait_vmcnt<kBase + 1>();
+    else
+      wait_vmcnt<kBase>();
+  };
+  if constexpr (NBUF == 2) wait_vmcnt<0>();
+  if (nsteps > 1)
+    issue_step<In, NW, FEAT, RAG>(phi1, psi1, vb1, phib, psib, vbb, tk0 + kStep, a, w, lane, dmo);
 
   auto step = [&](auto BUFC, int s) {
     constexpr int BUF = decltype(BUFC)::value;
-    const uint4* tphi = FEAT && NBUF == 2 ? phiF : BUF == 2 ? phi2 : BUF ? phi1 : phi0;
-    const uint4* tpsi = FEAT == 1 ? psiF : BUF == 2 ? psi2 : BUF ? psi1 : psi0;
+    const uint4* tphi = BUF == 2 ? phi2 : BUF ? phi1 : phi0;
+    const uint4* tpsi = BUF == 2 ? psi2 : BUF ? psi1 : psi0;
     const uint4* tvb = BUF == 2 ? vb2 : BUF ? vb1 : vb0;
     const int64_t ts = tk0 + (int64_t)s * kStep;
     // An opaque copy of the lane index per step: the LDS addresses derived
@@ -405,87 +480,33 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
     int lane = lane_id();
     asm volatile("" : "+v"(lane));
     const int r16 = lane & 15, g = lane >> 4;
-    float hv[4] = {1.f, 1.f, 1.f, 1.f};    // FEAT = 1: the key gate of the lane's four rows
-    if constexpr (FEAT == 1) {
-#pragma unroll
-      for (int tt = 0; tt < 4; ++tt) hv[tt] = hb ? to_f32(hb[ts + 16 * tt + r16]) : 1.f;
-    }
-    static_assert(kLoads / 8 == 6 && kLoads % 8 == 1, "seven loads on wave 0, six on the rest");
-    if constexpr (NBUF == 3) {
-      // Issued after this step's DMA: the previous step's output stores and the
-      // next step's DMA, seven loads on wave 0 and six on the rest (six on every
-      // wave with the feature map).  Loads complete in order, so waiting down
-      // to that many lands this step's rows.
-      if (s + 1 < nsteps) {
-        if (!FEAT && w == 0)
-          wait_vmcnt<7>();
-        else
-          wait_vmcnt<6>();
-      } else {
-        wait_vmcnt<0>();
-      }
-    } else if (s + 1 < nsteps) {
-      issue_step<In, FEAT != 0, NBUF == 3>(BUF ? phi0 : phi1, BUF ? psi0 : psi1, BUF ? vb0 : vb1, phib, psib,
-                           vbb, ts + kStep, a, w, dmo);
-      // the gate loads (issued first) are older than this step's six DMA loads
-      if (!FEAT && w == 0)
-        wait_vmcnt<7>();
-      else
-        wait_vmcnt<6>();
-    } else {
-      wait_vmcnt<0>();
-    }
+    // Loads complete in order, so waiting until only the next step's copy is
+    // outstanding lands this step's.  (Two buffers: the previous step's (e), or
+    // the prologue, has waited for it.)
+    if constexpr (NBUF == 3) wait_dma(s + 1 < nsteps);
     lds_barrier();      // every wave's DMA of this step has landed
-    if constexpr (FEAT && NBUF == 3) {
+    if constexpr (FEAT) {
       // in place: feat_rows reads every wave's rows, then waits, then writes
+      const float none[4] = {1.f, 1.f, 1.f, 1.f};
       const auto sw = [](int t) { return swz16(t); };
       uint4* tq = BUF == 2 ? phi2 : BUF ? phi1 : phi0;
-      feat_rows<In, 4>(tq, tq, 0, true, wa, w, fa.kind, false, hv, lane, sw);
+      feat_rows<In, 4>(tq, tq, 0, true, wa, w, fa.kind, false, none, lane, sw);
       lds_barrier();    // the step's Phi tile is complete
-    } else if constexpr (FEAT) {
-      const auto sw = [](int t) { return swz16(t); };
-      feat_rows<In, 4>(BUF ? phi1 : phi0, phiF, 0, true, wa, w, fa.kind, false, hv, lane, sw);
-      if constexpr (FEAT == 1)
-        feat_rows<In, 4>(BUF ? psi1 : psi0, psiF, 0, true, wa, w, fa.kind, hb != nullptr, hv, lane,
-                         sw);
-      lds_barrier();    // the step's Phi (and Psi) tiles are complete
     }
-    YRegs yr;
-    if constexpr (NBUF == 2) issue_y(yr, Yb, gb, Sb, ts, a, rof, lane);
-    // Three buffers: the step's Y rows and gates, untracked; the only vector
-    // memory issued after them before (e) is the DMA of step s + 2.
+    // The step's Y rows and gates; the only vector memory issued after them
+    // before (e) is the DMA of step s + 2.
     const bool rec = Yb != nullptr && ts >= a.n;
-    f32x4 ya[4];
-    float y8a[4], ga[4];
-    if constexpr (NBUF == 3) {
-      if (rec) {
-        const char* yb = reinterpret_cast<const char*>(Yb + (ts - a.n) * a.y_st);
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
-          ya[tt] = load4_untracked(yb + rof.y[tt]);
-          y8a[tt] = load1_untracked(yb + rof.y[tt] + rof.y8);
-        }
-      }
-      if (gb) {
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) ga[tt] = load1_untracked(gb + ts + 16 * tt + r16);
-      }
-    }
+    YRegs yr;
+    if constexpr (TERMS) issue_y(yr, ts);
 
     // (a) this wave's share of the causal score tiles A^T = Psi Phi^T
-    //     entries 0..9: (ut, tt) with ut <= tt; 10, 11: zero tiles (1,0), (3,2).
-    //     Wave w takes entry w and, for w < 4, entry w + 8: waves 0, 1 two
-    //     products, whose fragments are all read first and whose MFMA chains
-    //     interleave; waves 2, 3 a product and a zero tile.
+    //     entries 0..9: (ut, tt) with ut <= tt.  Wave w takes entries w, w + NW,
+    //     ...; the fragments of its (up to three) products are read first and
+    //     their MFMA chains interleave.
     {
       auto entry = [](int e, int& ut, int& tt) {
-        if (e < 10) {
-          tt = e < 1 ? 0 : e < 3 ? 1 : e < 6 ? 2 : 3;
-          ut = e - (tt * (tt + 1)) / 2;
-        } else {
-          ut = e == 10 ? 1 : 3;
-          tt = e == 10 ? 0 : 2;
-        }
+        tt = e < 1 ? 0 : e < 3 ? 1 : e < 6 ? 2 : 3;
+        ut = e - (tt * (tt + 1)) / 2;
       };
       // acc[i] = A^T[t' = 16ut + 4g + i][t = 16tt + r16] = A[t][t'], masked,
       // rounded to the input type and stored to the share
@@ -501,36 +522,52 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
         char* p = reinterpret_cast<char*>(share + t * 8 + (k ^ swz8(t))) + 8 * (g & 1);
         *reinterpret_cast<Half*>(p) = hv;
       };
-      int ut0, tt0, ut1, tt1;
-      entry(w, ut0, tt0);
-      entry(w + 8, ut1, tt1);
-      Frag fa0[4], fb0[4];
+      struct Prod {
+        Frag fa[kSteps], fb[kSteps];
+        int ut, tt;
+      };
+      auto read = [&](Prod& q, int e) {
+        entry(e, q.ut, q.tt);
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        fa0[kk] = row_chunk<In>(tpsi, 16 * ut0 + r16, 4 * kk + g);
-        fb0[kk] = row_chunk<In>(tphi, 16 * tt0 + r16, 4 * kk + g);
-      }
-      f32x4 acc0 = zero4();
-      if (w < 2) {
-        Frag fa1[4], fb1[4];
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          fa1[kk] = row_chunk<In>(tpsi, 16 * ut1 + r16, 4 * kk + g);
-          fb1[kk] = row_chunk<In>(tphi, 16 * tt1 + r16, 4 * kk + g);
+        for (int kk = 0; kk < NKB; ++kk) {
+          q.fa[kk] = row_chunk<In, RC>(tpsi, 16 * q.ut + r16, 4 * kk + g);
+          q.fb[kk] = row_chunk<In, RC>(tphi, 16 * q.tt + r16, 4 * kk + g);
         }
-        f32x4 acc1 = zero4();
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          acc0 = mma(acc0, fa0[kk], fb0[kk]);
-          acc1 = mma(acc1, fa1[kk], fb1[kk]);
+        if constexpr (kOdd) {
+          const int kl = 2 * (NW - 1) + (g >> 1);
+          q.fa[NKB] = join<In>(row_half<In, RC>(tpsi, 16 * q.ut + r16, kl, g & 1), Half{});
+          q.fb[NKB] = join<In>(row_half<In, RC>(tphi, 16 * q.tt + r16, kl, g & 1), Half{});
         }
-        put(acc1, ut1, tt1);
+      };
+      auto mul = [&](f32x4& acc, const Prod& q, int kk) { acc = mma(acc, q.fa[kk], q.fb[kk]); };
+      constexpr int kMax = (10 + NW - 1) / NW;       // products a wave: at most 2 or 3
+      // wave w has kMax products if w + NW (kMax - 1) < 10, else one fewer
+      Prod q0, q1, q2;
+      f32x4 s0 = zero4(), s1 = zero4(), s2 = zero4();
+      read(q0, w);
+      if constexpr (kMax == 3) read(q1, w + NW);
+      if (w + NW * (kMax - 1) < 10) {
+        if constexpr (kMax == 3)
+          read(q2, w + 2 * NW);
+        else
+          read(q1, w + NW);
+#pragma unroll
+        for (int kk = 0; kk < kSteps; ++kk) {
+          mul(s0, q0, kk);
+          mul(s1, q1, kk);
+          if constexpr (kMax == 3) mul(s2, q2, kk);
+        }
+        put(s1, q1.ut, q1.tt);
+        if constexpr (kMax == 3) put(s2, q2.ut, q2.tt);
       } else {
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) acc0 = mma(acc0, fa0[kk], fb0[kk]);
-        if (w < 4) put(zero4(), ut1, tt1);
+        for (int kk = 0; kk < kSteps; ++kk) {
+          mul(s0, q0, kk);
+          if constexpr (kMax == 3) mul(s1, q1, kk);
+        }
+        if constexpr (kMax == 3) put(s1, q1.ut, q1.tt);
       }
-      put(acc0, ut0, tt0);
+      put(s0, q0.ut, q0.tt);
     }
 
     // Three buffers: step s + 2's rows go to the buffer step s - 1 used, free
@@ -539,9 +576,10 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
     if constexpr (NBUF == 3) {
       constexpr int NB = (BUF + 2) % 3;
       if (s + 2 < nsteps)
-        issue_step<In, FEAT != 0, NBUF == 3>(NB == 2 ? phi2 : NB ? phi1 : phi0, NB == 2 ? psi2 : NB ? psi1 : psi0,
-                             NB == 2 ? vb2 : NB ? vb1 : vb0, phib, psib, vbb, ts + 2 * kStep, a,
-                             w, dmo);
+        issue_step<In, NW, FEAT, RAG>(NB == 2 ? phi2 : NB ? phi1 : phi0,
+                                      NB == 2 ? psi2 : NB ? psi1 : psi0,
+                                      NB == 2 ? vb2 : NB ? vb1 : vb0, phib, psib, vbb,
+                                      ts + 2 * kStep, a, w, lane, dmo);
     }
 
     // (b) O^T = S^T Phi^T with the state before this step; the normaliser
@@ -550,18 +588,18 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) accO[tt] = zero4();
     // Row t = 16 tt + r16 of the Phi tile, one opaque base per tt.  Rows t and
-    // t + 16 sit at the same swizzle 4096 bytes apart; seen as such, their two
+    // t + 16 sit at the same swizzle a constant apart; seen as such, their two
     // 8-byte reads are fused into one ds_read2st64_b64, which the LDS serves at
     // half the rate of two ds_read_b64 and with this pattern's lanes in
     // conflict.  With opaque bases every read stays a ds_read_b64.
     const char* prow[4];
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) {
-      uint32_t off = (uint32_t)(16 * tt + r16) * (ss::kRowChunks * 16);
+      uint32_t off = (uint32_t)(16 * tt + r16) * (RC * 16);
       asm volatile("" : "+v"(off));
       prow[tt] = reinterpret_cast<const char*>(tphi) + off;
     }
-    const int sw = swz16(r16);
+    const int sw = swz_row<RC>(r16);
     auto phi_half = [&](int tt, int k) {
       return *reinterpret_cast<const Half*>(prow[tt] + ((k ^ sw) * 16 + 8 * (g & 1)));
     };
@@ -576,8 +614,8 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
     };
     read_bf(bfs[0], 0);
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      if (kk + 1 < 4) read_bf(bfs[(kk + 1) & 1], kk + 1);
+    for (int kk = 0; kk < NKB; ++kk) {
+      if (kk + 1 < NKB) read_bf(bfs[(kk + 1) & 1], kk + 1);
       Half h0, l0, h1, l1;
       split4<In>(accS[2 * kk], h0, l0);
       split4<In>(accS[2 * kk + 1], h1, l1);
@@ -586,6 +624,19 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
       for (int tt = 0; tt < 4; ++tt) accO[tt] = mma(accO[tt], shi, bfs[kk & 1][tt]);
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) accO[tt] = mma(accO[tt], slo, bfs[kk & 1][tt]);
+    }
+    if constexpr (kOdd) {
+      Half hi, lo;
+      Frag bh[4];
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt)
+        bh[tt] = join<In>(phi_half(tt, 2 * (NW - 1) + (g >> 1)), Half{});
+      split4<In>(accS[NW - 1], hi, lo);
+      const Frag shi = join<In>(hi, Half{}), slo = join<In>(lo, Half{});
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) accO[tt] = mma(accO[tt], shi, bh[tt]);
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) accO[tt] = mma(accO[tt], slo, bh[tt]);
     }
     float own = 0.f;                       // wave w < 4: its row tile's value, finished in (d)
     {
@@ -598,42 +649,50 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
       for (int tt = 0; tt < 4; ++tt) pn[tt] = mma16(zero4(), s8hi, bfn[tt]);
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) pn[tt] = mma16(pn[tt], s8lo, bfn[tt]);
-      if (g == (cn >> 2)) {
+      if (g == 0) {                        // the normaliser's row of the tile: 0
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt) {
           if (tt == w)
-            own = pn[tt][cn & 3];
+            own = pn[tt][0];
           else
-            normp[norm_slot(16 * tt + r16, w)] = pn[tt][cn & 3];
+            normp[norm_slot(16 * tt + r16, w)] = pn[tt][0];
         }
       }
     }
 
     // (c) S += Psi^T Vb over the step's 64 tokens
-    // The ninth tile's rows of this wave take the Psi fragment of row tile w
-    // once more, outside the loop: a branch on at == w inside it would split
+    // The normaliser tile's rows of this wave take the Psi fragment of row tile
+    // w once more, outside the loop: a branch on at == w inside it would split
     // the loop into blocks the compiler cannot move a read across.
-    // The sixteen (ks, at) products run in order with the Psi fragments of the
-    // next two read ahead (sched barriers keep the compiler from sinking the
-    // reads to their MFMAs).
+    // The (ks, at) products run in order with the Psi fragments of the next two
+    // read ahead (sched barriers keep the compiler from sinking the reads to
+    // their MFMAs).
     Frag vbw[2], vb8[2], pa[3];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      vbw[ks] = vb_tr<In>(tvb, w, ks, lane);
-      vb8[ks] = vb_tr<In>(tvb, 8, ks, lane);
+      vbw[ks] = psi_tr<In, RC>(tvb, w, ks, lane);
+      vb8[ks] = vb_norm_tr<In, RC>(tvb, ks, lane);
     }
-    pa[0] = psi_tr<In>(tpsi, 0, 0, lane);
-    pa[1] = psi_tr<In>(tpsi, 1, 0, lane);
+    pa[0] = psi_tr<In, RC>(tpsi, 0, 0, lane);
+    pa[1] = psi_tr<In, RC>(tpsi, 1, 0, lane);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      if (i + 2 < 16) pa[(i + 2) % 3] = psi_tr<In>(tpsi, (i + 2) & 7, (i + 2) >> 3, lane);
+    for (int i = 0; i < 2 * NW; ++i) {
+      if (i + 2 < 2 * NW)
+        pa[(i + 2) % 3] = psi_tr<In, RC>(tpsi, (i + 2) % NW, (i + 2) / NW, lane);
       __builtin_amdgcn_sched_barrier(0);
-      accS[i & 7] = mma(accS[i & 7], pa[i % 3], vbw[i >> 3]);
+      accS[i % NW] = mma(accS[i % NW], pa[i % 3], vbw[i / NW]);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) accS8 = mma(accS8, psi_tr<In>(tpsi, w, ks, lane), vb8[ks]);
+    for (int ks = 0; ks < 2; ++ks) accS8 = mma(accS8, psi_tr<In, RC>(tpsi, w, ks, lane), vb8[ks]);
     lds_barrier();       // the score share is complete
+    // Two buffers: every wave is past its reads of this step's rows, so step
+    // s + 2's go there, a whole step before (e) of step s + 1 waits for them.
+    if constexpr (NBUF == 2) {
+      if (s + 2 < nsteps)
+        issue_step<In, NW, FEAT, RAG>(BUF ? phi1 : phi0, BUF ? psi1 : psi0, BUF ? vb1 : vb0, phib,
+                                      psib, vbb, ts + 2 * kStep, a, w, lane, dmo);
+    }
 
     // (d) O^T += Vb^T A^T within the step; waves 0..3 add the row sums of A
     //     (the ones column) to their row tile's normaliser
@@ -655,54 +714,54 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
       const int t = 16 * w + r16;
       f32x4 p8 = mma(zero4(), vb8[0], share_bf(t, 0));
       if (w >= 2) p8 = mma(p8, vb8[1], share_bf(t, 1));
-      if (g == (cn >> 2)) normp[norm_slot(t, w)] = own + p8[cn & 3];
+      if (g == 0) normp[norm_slot(t, w)] = own + p8[0];
     }
     lds_barrier();
 
     // (e) long-range term, normalise, store four columns per lane per row tile
-    if constexpr (NBUF == 3) {
-      if (rec || gb) {
-        // everything issued after the Y and gate loads: step s + 2's DMA
-        if (s + 2 < nsteps) {
-          if (!FEAT && w == 0)
-            wait_vmcnt<7>();
-          else
-            wait_vmcnt<6>();
-        } else {
-          wait_vmcnt<0>();
-        }
-        asm volatile("" : "+v"(ya[0]), "+v"(ya[1]), "+v"(ya[2]), "+v"(ya[3]), "+v"(y8a[0]),
-                     "+v"(y8a[1]), "+v"(y8a[2]), "+v"(y8a[3]));
-        asm volatile("" : "+v"(ga[0]), "+v"(ga[1]), "+v"(ga[2]), "+v"(ga[3]));
-      }
+    // Issued after the Y and gate loads: step s + 2's copy.  With two buffers
+    // this wait also lands step s + 1's rows.
+    if (NBUF == 2 || (TERMS && (rec || gb))) wait_dma(s + 2 < nsteps);
+    if (TERMS && (rec || gb)) {
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt)
+        asm volatile("" : "+v"(yr.y[tt]), "+v"(yr.y8[tt]), "+v"(yr.gv[tt]));
     }
+    const int left = rows_left(ts);
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) {
       const int t = 16 * tt + r16;
       const float4 n0 = *reinterpret_cast<const float4*>(normp + norm_slot(t, 0));
-      const float4 n1 = *reinterpret_cast<const float4*>(normp + norm_slot(t, 4));
-      float den = ((n0.x + n0.y) + (n0.z + n0.w)) + ((n1.x + n1.y) + (n1.z + n1.w));
+      float den = (n0.x + n0.y) + (n0.z + n0.w);
+      if constexpr (NW > 4) {
+        const float4 n1 = *reinterpret_cast<const float4*>(normp + norm_slot(t, 4));
+        den += (n1.x + n1.y) + (n1.z + n1.w);
+      }
       float4 o;
       o.x = accO[tt][0];
       o.y = accO[tt][1];
       o.z = accO[tt][2];
       o.w = accO[tt][3];
-      if (rec) {
-        if constexpr (NBUF == 3) {
-          den += y8a[tt];
-          o.x += ya[tt][0];
-          o.y += ya[tt][1];
-          o.z += ya[tt][2];
-          o.w += ya[tt][3];
-        } else {
-          den += yr.y8[tt];
-          o.x += yr.y[tt].x;
-          o.y += yr.y[tt].y;
-          o.z += yr.y[tt].z;
-          o.w += yr.y[tt].w;
+      if constexpr (WH) {
+        if (!RAG || t < left) {
+          float* h = reinterpret_cast<float*>(reinterpret_cast<char*>(outb + ts * a.o_st) +
+                                              rof.o[tt]);
+          h[0] = o.x;
+          h[1] = o.y;
+          h[2] = o.z;
+          h[3] = o.w;
+          if (tt % NW == w && g == 0) outb[(ts + t) * a.o_st + 16 * NW] = den;
         }
+        continue;
       }
-      const float num = NBUF == 3 ? (gb ? ga[tt] : 1.f) : yr.gv[tt];   // the gate (1 without)
+      if (TERMS && rec) {
+        den += yr.y8[tt];
+        o.x += yr.y[tt][0];
+        o.y += yr.y[tt][1];
+        o.z += yr.y[tt][2];
+        o.w += yr.y[tt][3];
+      }
+      const float num = TERMS && gb ? yr.gv[tt] : 1.f;   // the gate (1 without)
       // the reciprocal (1 ulp) in place of the IEEE division's ten-instruction
       // sequence; the product below rounds once more either way
       const float inv = num * __builtin_amdgcn_rcpf(den);
@@ -710,7 +769,8 @@ __global__ __launch_bounds__(ss::kThreads, 1) void scan_stream_kernel(
       o.y *= inv;
       o.z *= inv;
       o.w *= inv;
-      *reinterpret_cast<float4*>(reinterpret_cast<char*>(outb + ts * a.o_st) + rof.o[tt]) = o;
+      if (!RAG || t < left)
+        *reinterpret_cast<float4*>(reinterpret_cast<char*>(outb + ts * a.o_st) + rof.o[tt]) = o;
     }
   };
 
@@ -916,8 +976,8 @@ __global__ __launch_bounds__(ss::kThreads, (ONE && !FEAT) ? 3 : 2) void gram_str
     const int nvalid = count - s * kStep;        // rows of this step holding tokens
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      Frag vbw = vb_tr<In>(tvb, w, ks, lane);
-      Frag vb8 = vb_tr<In>(tvb, 8, ks, lane);
+      Frag vbw = psi_tr<In>(tvb, w, ks, lane);
+      Frag vb8 = vb_norm_tr<In>(tvb, ks, lane);
       if (nvalid < kStep) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -1078,12 +1138,14 @@ int gram_stream_launch_feat(int dtype, const void* k, const void* v, float* G, f
 bool scan_stream_ok(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
                     const float* out, const ScanArgs& a) {
   if (dtype != SMAT_BF16 && dtype != SMAT_F16) return false;
-  if (a.write_H || a.r != 128 || a.p != 129) return false;
-  if (a.C % ss::kStep || a.T % ss::kStep || a.n % ss::kStep) return false;
+  if (a.r % 16 || a.r < 64 || a.r > 128 || a.p != a.r + 1) return false;
+  if (a.C % ss::kStep || a.n % ss::kStep) return false;
   if (!rows_vec_ok(phi, a.q_sb, a.q_st, 2) || !rows_vec_ok(psi, a.k_sb, a.k_st, 2) ||
-      !rows_vec_ok(vb, a.v_sb, a.v_st, 2) || a.v_st < 136)
+      !rows_vec_ok(vb, a.v_sb, a.v_st, 2) || a.v_st < a.r + 8)
     return false;
-  if (!rows_vec_ok(out, a.o_sb, a.o_st, 4)) return false;
+  // H only at r = 64, the width of the fused backward; the wider general kernel
+  // gives a training step the same bits for every row stride of Vb
+  if (a.write_H ? a.r != 64 : !rows_vec_ok(out, a.o_sb, a.o_st, 4)) return false;
   if (Y && !rows_vec_ok(Y, a.y_sb, a.y_st, 4)) return false;
   // per-lane row offsets are 32-bit bytes over 64 rows
   constexpr int64_t kMaxSt = 1 << 20;
@@ -1093,53 +1155,78 @@ bool scan_stream_ok(int dtype, const void* phi, const void* psi, const void* vb,
   return variant(SMAT_VARIANT_SCAN) == 0;
 }
 
-template <typename In, int FEAT>
+template <typename In, int NW>
 static void scan_stream_kernel_launch(const void* phi, const void* psi, const void* vb,
                                       const float* Sg, const float* Y, const float* gate,
-                                      float* out, dim3 grid, const ScanArgs& a, const FeatArgs& fa,
+                                      float* out, dim3 grid, const ScanArgs& a,
                                       hipStream_t stream) {
   const In* q = (const In*)phi;
   const In* k = (const In*)psi;
   const In* v = (const In*)vb;
-  if constexpr (FEAT != 0)
-    smat::launch((scan_stream_kernel<In, FEAT, FEAT == 2 ? 3 : 2, true>), grid,
-                 dim3(ss::kThreads), 0, stream, q, k, v, Sg, Y, gate, out, a, fa);
+  const dim3 blk(64 * NW);
+  const FeatArgs fa{};
+  if constexpr (NW == 4) {
+    if (a.write_H) {
+      smat::launch((scan_stream_kernel<In, NW, false, false, true, true>), grid, blk, 0, stream,
+                   q, k, v, Sg, Y, gate, out, a, fa);
+      return;
+    }
+  }
+  if (a.T % ss::kStep)
+    smat::launch((scan_stream_kernel<In, NW, false, true, true, false>), grid, blk, 0, stream, q,
+                 k, v, Sg, Y, gate, out, a, fa);
   else if (Y || gate)
-    smat::launch((scan_stream_kernel<In, 0, 3, true>), grid, dim3(ss::kThreads), 0,
-                       stream, q, k, v, Sg, Y, gate, out, a, fa);
+    smat::launch((scan_stream_kernel<In, NW, false, true, false, false>), grid, blk, 0, stream, q,
+                 k, v, Sg, Y, gate, out, a, fa);
   else
-    smat::launch((scan_stream_kernel<In, 0, 3, false>), grid, dim3(ss::kThreads), 0,
-                       stream, q, k, v, Sg, Y, gate, out, a, fa);
+    smat::launch((scan_stream_kernel<In, NW, false, false, false, false>), grid, blk, 0, stream,
+                 q, k, v, Sg, Y, gate, out, a, fa);
 }
 
-template <int FEAT>
-static int scan_stream_go(int dtype, const void* phi, const void* psi, const void* vb,
-                          const float* Sg, const float* Y, const float* gate, float* out, int nb,
-                          int ng, const ScanArgs& a, const FeatArgs& fa, hipStream_t stream) {
-  dim3 grid((unsigned)ng, (unsigned)nb);
-  if (dtype == SMAT_BF16)
-    scan_stream_kernel_launch<bf16, FEAT>(phi, psi, vb, Sg, Y, gate, out, grid, a, fa, stream);
-  else
-    scan_stream_kernel_launch<f16, FEAT>(phi, psi, vb, Sg, Y, gate, out, grid, a, fa, stream);
-  return launch_status("smat_causal_scan");
+template <typename In>
+static void scan_stream_shape(const void* phi, const void* psi, const void* vb, const float* Sg,
+                              const float* Y, const float* gate, float* out, dim3 grid,
+                              const ScanArgs& a, hipStream_t stream) {
+  switch (a.r / 16) {
+    case 4:
+      return scan_stream_kernel_launch<In, 4>(phi, psi, vb, Sg, Y, gate, out, grid, a, stream);
+    case 5:
+      return scan_stream_kernel_launch<In, 5>(phi, psi, vb, Sg, Y, gate, out, grid, a, stream);
+    case 6:
+      return scan_stream_kernel_launch<In, 6>(phi, psi, vb, Sg, Y, gate, out, grid, a, stream);
+    case 7:
+      return scan_stream_kernel_launch<In, 7>(phi, psi, vb, Sg, Y, gate, out, grid, a, stream);
+    default:
+      return scan_stream_kernel_launch<In, 8>(phi, psi, vb, Sg, Y, gate, out, grid, a, stream);
+  }
 }
 
 int scan_stream_launch(int dtype, const void* phi, const void* psi, const void* vb,
                        const float* Sg, const float* Y, const float* gate, float* out, int nb,
                        int ng, const ScanArgs& a, hipStream_t stream) {
-  return scan_stream_go<0>(dtype, phi, psi, vb, Sg, Y, gate, out, nb, ng, a, FeatArgs{},
-                           stream);
+  const dim3 grid((unsigned)ng, (unsigned)nb);
+  if (dtype == SMAT_BF16)
+    scan_stream_shape<bf16>(phi, psi, vb, Sg, Y, gate, out, grid, a, stream);
+  else
+    scan_stream_shape<f16>(phi, psi, vb, Sg, Y, gate, out, grid, a, stream);
+  return launch_status("smat_causal_scan");
 }
 
-// The streaming causal pass with the feature map in place: q and v are Q
-// and V rows (the shapes scan_stream_ok accepts, with V rows of 128); k is
-// K rows, or the Psi rows (key gate applied) when psi_formed.
-int scan_stream_launch_feat(int dtype, const void* q, const void* k, const void* v,
+// The streaming causal pass with the feature map in place: q and v are Q and V
+// rows (r = 128, T a multiple of 64, V rows of 128); psi is the Psi rows (key
+// gate applied).
+int scan_stream_launch_feat(int dtype, const void* q, const void* psi, const void* v,
                             const float* Sg, const float* Y, const float* gate, float* out,
                             int nb, int ng, const ScanArgs& a, const FeatArgs& fa,
-                            bool psi_formed, hipStream_t stream) {
-  if (psi_formed) return scan_stream_go<2>(dtype, q, k, v, Sg, Y, gate, out, nb, ng, a, fa, stream);
-  return scan_stream_go<1>(dtype, q, k, v, Sg, Y, gate, out, nb, ng, a, fa, stream);
+                            hipStream_t stream) {
+  const dim3 grid((unsigned)ng, (unsigned)nb), blk(64 * 8);
+  if (dtype == SMAT_BF16)
+    smat::launch((scan_stream_kernel<bf16, 8, true, true, false, false>), grid, blk, 0, stream,
+                 (const bf16*)q, (const bf16*)psi, (const bf16*)v, Sg, Y, gate, out, a, fa);
+  else
+    smat::launch((scan_stream_kernel<f16, 8, true, true, false, false>), grid, blk, 0, stream,
+                 (const f16*)q, (const f16*)psi, (const f16*)v, Sg, Y, gate, out, a, fa);
+  return launch_status("smat_causal_scan");
 }
 
 }  // namespace smat

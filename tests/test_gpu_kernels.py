@@ -477,6 +477,52 @@ def _check_forward(spec, Phi, Psi, Vb, *, dt, g=None, label=""):
     return out
 
 
+@pytest.mark.parametrize("hd,T,n,C,dt", [
+    (64, 1024, 512, 128, torch.bfloat16), (64, 64, 0, 64, torch.float16),
+    (64, 8192 + 1, 4096, 128, torch.bfloat16), (64, 1023, 1023 // 64 * 64, 64, torch.bfloat16),
+    (80, 2048, 1024, 128, torch.float16), (80, 1000, 512, 64, torch.bfloat16),
+    (96, 3 * 128 + 17, 128, 128, torch.float16), (96, 2048, 2048, 128, torch.bfloat16),
+    (112, 640 + 63, 256, 128, torch.bfloat16), (112, 1024, 0, 128, torch.float16),
+    (128, 1000, 512, 128, torch.bfloat16), (128, 65, 64, 64, torch.float16)])
+def test_causal_scan_streaming_widths(hd, T, n, C, dt):
+    """The streaming scan at every head width it takes (r = 64 .. 128 by 16: four to
+    eight waves, an odd k-block of 16 features at 80 and 112) and at lengths that
+    are no multiple of its 64-token step: normalised with Y and the gate, with
+    neither, and H itself, against the general kernel and the oracle's path."""
+    _say("causal scan widths", hd, T, n, C, dt)
+    Phi, Psi, Vb = _feats(3, T, hd, dt, seed=41)
+    P, pad = hd + 1, hd + 8
+    g = torch.Generator().manual_seed(42)
+    Y = torch.rand(3, T - n, P, generator=g)
+    gate = (torch.rand(3, T, generator=g) + 0.5).to(DEV)
+    Vp = torch.full((3, T, pad), float("nan"), dtype=dt)      # the row padding is never data
+    Vp[..., :P] = Vb
+    Yp = torch.full((3, T - n, (P + 3) // 4 * 4), float("nan"))
+    Yp[..., :P] = Y
+    Pd, Sd, Vd = Phi.to(DEV), Psi.to(DEV), Vp.to(DEV)[..., :P]
+    Yd = Yp.to(DEV)[..., :P] if T > n else None
+    runs = (dict(Y=Yd, g=gate), dict(Y=Yd), dict(), dict(write_H=True))
+    got = [K.causal_scan(Pd, Sd, Vd, n, C, **kw) for kw in runs]
+    with general_kernel("scan"):
+        old = [K.causal_scan(Pd, Sd, Vd, n, C, **kw) for kw in runs]
+    torch.cuda.synchronize()
+    H64 = O.segmented_causal_scan(Phi.double(), Psi.double(), Vb.double(), n, chunk=C)
+    Hy = H64.clone()
+    if T > n:
+        Hy[:, n:] += Y.double()
+    norm = lambda H: H[..., :-1] / H[..., -1:]
+    want = (norm(Hy) * gate.double().cpu().unsqueeze(-1), norm(Hy), norm(H64), H64)
+    for name, a, b, w in zip(("Y, gate", "Y", "plain", "H"), got, old, want):
+        scale = w.abs().max().item()
+        e_new = (a.double().cpu() - w).abs().max().item() / scale
+        e_old = (b.double().cpu() - w).abs().max().item() / scale
+        _say(f"  {name}: streaming {e_new:.2e} general {e_old:.2e}")
+        assert torch.isfinite(a).all()
+        # both round the scores to the input type once; the streaming kernel
+        # fewer of them (64-token steps against whole chunks)
+        assert e_new <= 1.5 * e_old + 1e-6
+
+
 def test_forward_plumbing_config_fp32():
     """nb=4 (B=1, H=4), T=1024, d=2, head_dim=64, fp32, q,k,v ~ N(0,1) seed 0."""
     _say("forward T=1024 d=2 nb=4 hd=64 fp32")
