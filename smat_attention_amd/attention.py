@@ -707,8 +707,9 @@ def smat_attention_fused(Q, K, V, phi, spec: MaskSpec, *, g=None, h=None, chunk:
     query, the prepass and the scan form ``Phi = map(Q W^T)``, ``Psi = h
     map(K W^T)`` and ``Vb = [V, 1]`` in LDS from the Q, K, V tiles they stream
     (``smat_forward_fused``), bitwise the features :func:`featurise` writes,
-    so the output equals the unfused path's while Phi, Psi and Vb never reach
-    memory (where a row type has more than 64 recent rows, the recent rows'
+    so the output is the unfused path's (at lengths where that one takes larger
+    chunk groups, up to the order of the fp32 state sums) while Phi, Psi and Vb
+    never reach memory (where a row type has more than 64 recent rows, the recent rows'
     Phi alone is featurised for the general query kernel; at d = 1 the causal
     pass without its reset is the whole forward).  Other inputs --
     other widths and dtypes, fewer than 256 (sequence, profile) pools with

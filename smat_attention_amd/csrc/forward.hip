@@ -84,13 +84,13 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
                          int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb, int64_t o_st,
                          int64_t g_sb, const FeatArgs& fa, void* ws, int64_t ws_bytes,
                          void* psi_buf, hipStream_t stream);
-int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, bool forward);
+int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, int kmax);
 int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void* vb,
                          const float* Y, const float* gate, float* out, int nb, int T, int n,
                          int C, int r, int p, int64_t q_sb, int64_t q_st, int64_t k_sb,
                          int64_t k_st, int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st,
                          int64_t o_sb, int64_t o_st, int64_t g_sb, int write_H, void* ws,
-                         int64_t ws_bytes, bool forward, hipStream_t stream);
+                         int64_t ws_bytes, int kmax, hipStream_t stream);
 
 // Workspace carve-up, each region 256-byte aligned.  The fused causal pass
 // (chunk <= 128, no H requested) needs only its group states; the staged one
@@ -110,8 +110,9 @@ static bool one_state(const void* idx, int N0, int B, int n_P) {
   return !idx && N0 == 1 && B == 1 && n_P == 0;
 }
 
+// kmax: the causal pass's largest group, kForwardK or kFeatK.
 static FwdLayout fwd_layout(int nb, int T, int n, int N0, int B, int n_P, int C, int r, int p,
-                            bool want_H) {
+                            bool want_H, int kmax) {
   FwdLayout L{};
   const int64_t rp = (int64_t)r * p;
   const int nc = (T + C - 1) / C;
@@ -126,7 +127,7 @@ static FwdLayout fwd_layout(int nb, int T, int n, int N0, int B, int n_P, int C,
   L.U = off;   off += al256((int64_t)nb * B * ld * 4);
   L.Y = off;   off += al256((int64_t)nb * T_R * y_stride(p) * 4);
   if (L.fused) {
-    L.scan = off; off += al256(causal_scan_workspace_bytes(nb, T, C, r, p, true));
+    L.scan = off; off += al256(causal_scan_workspace_bytes(nb, T, C, r, p, kmax));
   } else {
     L.D = off;   off += al256((int64_t)nb * nc * rp * 4);
     L.Sin = off; off += al256((int64_t)nb * nc * rp * 4);
@@ -191,8 +192,8 @@ extern "C" int smat_set_variant(int which, int value) {
 extern "C" int64_t smat_forward_workspace_bytes(int nb, int T, int n, int N0, int B, int n_P,
                                                 int C, int r, int p) {
   if (nb <= 0 || T <= 0 || C <= 0 || N0 <= 0 || B <= 0 || r <= 0 || p <= 0) return 0;
-  const smat::FwdLayout a = smat::fwd_layout(nb, T, n, N0, B, n_P, C, r, p, false);
-  const smat::FwdLayout b = smat::fwd_layout(nb, T, n, N0, B, n_P, C, r, p, true);
+  const smat::FwdLayout a = smat::fwd_layout(nb, T, n, N0, B, n_P, C, r, p, false, smat::kForwardK);
+  const smat::FwdLayout b = smat::fwd_layout(nb, T, n, N0, B, n_P, C, r, p, true, smat::kForwardK);
   return a.total > b.total ? a.total : b.total;
 }
 
@@ -224,7 +225,8 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
                "smat_forward: a row stride is shorter than its row");
   SMAT_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, SMAT_EINVAL,
                "smat_forward: workspace must be 256-byte aligned");
-  const FwdLayout L = fwd_layout(nb, T, n, N0, B, n_P, C, r, p, H_out != nullptr);
+  const FwdLayout L =
+      fwd_layout(nb, T, n, N0, B, n_P, C, r, p, H_out != nullptr, kForwardK);
   SMAT_REQUIRE(workspace_bytes >= L.total, SMAT_EINVAL,
                "smat_forward: workspace of %lld bytes needed, %lld given", (long long)L.total,
                (long long)workspace_bytes);
@@ -253,7 +255,7 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
     StageScope stage(3);
     return causal_scan_dispatch(dtype, phi, psi, vb, nullptr, g, out, nb, T, 0, C, r, p, q_sb,
                                 q_st, k_sb, k_st, v_sb, v_st, 0, 0, o_sb, o_st, g_sb, 0,
-                                ws + L.scan, L.part - L.scan, true, st);
+                                ws + L.scan, L.part - L.scan, kForwardK, st);
   }
 
   // ---- long range: S^T, then C, then R ---------------------------------
@@ -296,7 +298,7 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
     // one kernel: segmented scan, + Y on recent rows, normalise, gate
     return causal_scan_dispatch(dtype, phi, psi, vb, T_R > 0 ? Y : nullptr, g, out, nb, T, n, C,
                                 r, p, q_sb, q_st, k_sb, k_st, v_sb, v_st, (int64_t)T_R * yst, yst,
-                                o_sb, o_st, g_sb, 0, ws + L.scan, L.part - L.scan, true, st);
+                                o_sb, o_st, g_sb, 0, ws + L.scan, L.part - L.scan, kForwardK, st);
   }
   // staged: chunk summaries, segmented scan, chunk-local pass into H, normalise
   float* D = (float*)(ws + L.D);
@@ -366,7 +368,7 @@ static int64_t fused_phi_bytes(int nb, int T, int n, int B) {
   return fused_query_staged(T, n, B) ? al256((int64_t)nb * (T - n) * 128 * 2) : 0;
 }
 static int64_t fused_workspace_bytes(int nb, int T, int n, int N0, int B, int n_P, int C) {
-  const FwdLayout L = fwd_layout(nb, T, n, N0, B, n_P, C, 128, 129, false);
+  const FwdLayout L = fwd_layout(nb, T, n, N0, B, n_P, C, 128, 129, false, kFeatK);
   return L.total + fused_phi_bytes(nb, T, n, B) + al256((int64_t)nb * T * 128 * 2);
 }
 }  // namespace smat
@@ -425,7 +427,7 @@ extern "C" int smat_forward_fused(int dtype, const void* q, const void* k, const
                SMAT_EUNSUPPORTED, "smat_forward_fused: rows and W must be 16-byte aligned");
   SMAT_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, SMAT_EINVAL,
                "smat_forward_fused: workspace must be 256-byte aligned");
-  const FwdLayout L = fwd_layout(nb, T, n, N0, B, n_P, C, r, p, false);
+  const FwdLayout L = fwd_layout(nb, T, n, N0, B, n_P, C, r, p, false, kFeatK);
   const int64_t need = fused_workspace_bytes(nb, T, n, N0, B, n_P, C);
   SMAT_REQUIRE(workspace_bytes >= need, SMAT_EINVAL,
                "smat_forward_fused: workspace of %lld bytes needed, %lld given",

@@ -471,12 +471,14 @@ int gram_stream_launch_feat(int dtype, const void* k, const void* v, float* G, f
 // workspace is sized without it): the groups are counted as if it split the
 // chunks in half, where build_mask puts it.
 //
-// The one-call forwards take up to kForwardK: past 32 the uneven halves (only
+// The one-call forward takes up to kForwardK: past 32 the uneven halves (only
 // recent rows read Y) cost more than the states (524288 tokens: 5810 us at 32,
-// 5850 at 64; 8 x 131072 tokens at d = 1: 408 us at 32, 428 at 16).  The scan
-// called alone keeps to kScanK: it also serves the H-writing general kernel,
-// whose groups overlap less.
-constexpr int kForwardK = 32, kScanK = 16;
+// 5850 at 64; 8 x 131072 tokens at d = 1: 408 us at 32, 428 at 16).  The forward
+// from q, k, v keeps to kFeatK, whose 512 groups there let two workgroups of the
+// prepass share a CU and hide each other's feature map (1776 us at 16, 1809 at
+// 32); the scan called alone to kScanK: it also serves the H-writing general
+// kernel, whose groups overlap less.
+constexpr int kScanK = 16;
 static int scan_group_chunks(int nb, int nc, int r, int p, int kmax) {
   const int64_t slots = r <= 64 && p <= 80 ? 1024 : 256;
   int best = 1;
@@ -505,10 +507,9 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
                     int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb,
                     int64_t o_st, int64_t g_sb, int write_H, void* ws, hipStream_t stream);
 
-// forward: the causal pass of a one-call forward (groups of up to kForwardK).
-int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, bool forward) {
+int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, int kmax) {
   const int nc = (T + C - 1) / C;
-  const int K = scan_group_chunks(nb, nc, r, p, forward ? kForwardK : kScanK);
+  const int K = scan_group_chunks(nb, nc, r, p, kmax);
   return 2 * group_bytes(nb, nc, K, r, p);
 }
 
@@ -517,11 +518,11 @@ int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void
                          int C, int r, int p, int64_t q_sb, int64_t q_st, int64_t k_sb,
                          int64_t k_st, int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st,
                          int64_t o_sb, int64_t o_st, int64_t g_sb, int write_H, void* ws,
-                         int64_t ws_bytes, bool forward, hipStream_t stream) {
+                         int64_t ws_bytes, int kmax, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
   const int nc = (T + C - 1) / C;
-  const int K = scan_group_chunks(nb, nc, r, p, forward ? kForwardK : kScanK);
-  const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, forward);
+  const int K = scan_group_chunks(nb, nc, r, p, kmax);
+  const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, kmax);
   if (ws_bytes < need) {
     set_error("smat_causal_scan: workspace of %lld bytes needed, %lld given", (long long)need,
               (long long)ws_bytes);
@@ -588,9 +589,10 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
 // The streaming causal pass with the feature map computed inside the kernels:
 // q, k, v are the Q, K, V rows (r = d_qk = d_v = 128); the prepass Gram sums
 // and the scan form Psi (and Phi) tiles in LDS from the DMA'd K (and Q) rows,
-// and Vb = [V, 1] from V.  Same workspace as causal_scan_dispatch's with
-// forward.  The prepass also stores the Psi tiles it forms to psi_buf (nb x T
-// rows of 128, 16-bit) and the scan reads them, forming only Phi.
+// and Vb = [V, 1] from V.  The workspace is
+// causal_scan_workspace_bytes' at kFeatK.  The prepass also stores the Psi
+// tiles it forms to psi_buf (nb x T rows of 128, 16-bit) and the scan reads
+// them, forming only Phi.
 int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v, const float* Y,
                          const float* gate, float* out, int nb, int T, int n, int C,
                          int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb,
@@ -601,8 +603,8 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
   constexpr int r = 128, p = 129;
   const int64_t rp = (int64_t)r * p;
   const int nc = (T + C - 1) / C;
-  const int K = scan_group_chunks(nb, nc, r, p, kForwardK);
-  const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, true);
+  const int K = scan_group_chunks(nb, nc, r, p, kFeatK);
+  const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, kFeatK);
   if (ws_bytes < need) {
     set_error("smat_forward_fused: causal-pass workspace of %lld bytes needed, %lld given",
               (long long)need, (long long)ws_bytes);
@@ -752,7 +754,7 @@ extern "C" int smat_causal_scan_noalloc(int dtype, const void* phi, const void* 
 
 extern "C" int64_t smat_causal_scan_workspace_bytes(int nb, int T, int C, int r, int p) {
   if (nb <= 0 || T <= 0 || C <= 0 || r <= 0 || p <= 0) return 0;
-  return smat::causal_scan_workspace_bytes(nb, T, C, r, p, false);
+  return smat::causal_scan_workspace_bytes(nb, T, C, r, p, smat::kScanK);
 }
 
 extern "C" int smat_causal_scan(int dtype, const void* phi, const void* psi, const void* vb,
@@ -778,5 +780,5 @@ extern "C" int smat_causal_scan(int dtype, const void* phi, const void* psi, con
                "smat_causal_scan: workspace must be 256-byte aligned");
   return causal_scan_dispatch(dtype, phi, psi, vb, Y, gate, out, nb, T, n, C, r, p, q_sb, q_st,
                               k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb, o_st, g_sb, write_H,
-                              workspace, workspace_bytes, false, (hipStream_t)stream);
+                              workspace, workspace_bytes, kScanK, (hipStream_t)stream);
 }

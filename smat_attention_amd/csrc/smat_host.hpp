@@ -92,6 +92,10 @@ struct ScanArgs {
   int write_H;          // 1: out is H (nb, T, p) unnormalised, no Y / gate
 };
 
+// Most chunks a group of the causal pass takes in smat_forward and in
+// smat_forward_fused (scan_group_chunks, scan_fused.hip).
+constexpr int kForwardK = 32, kFeatK = 16;
+
 // Token progressions summed by the Gram kernels (gram.hip, scan_stream.hip).
 struct GramItems {
   int mode;        // 0: chunk groups, 1: profiles (+ optional global channel)
