@@ -56,11 +56,10 @@
 namespace smat {
 
 namespace ss {
-constexpr int kThreads = 512;
 constexpr int kStep = 64;                      // tokens per step
-constexpr int kRowChunks = 16;                 // 16-byte chunks per Phi/Psi/Vb row
+constexpr int kRowChunks = 16;                 // 16-byte chunks per LDS row of the Gram sums
 constexpr int kTileChunks = kStep * kRowChunks;    // 1024
-constexpr int kVbTileChunks = kTileChunks + kStep; // + columns 128..135, one chunk a row
+constexpr int kVbTileChunks = kTileChunks + kStep; // + the normaliser chunk of each row
 constexpr int kPhiLoads = kTileChunks / 64;        // wave-wide DMA loads per tile: 16
 constexpr int kVbLoads = kVbTileChunks / 64;       // 17
 
@@ -793,15 +792,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
 // prepass of the causal pass, and the profile pool), same machinery: rows
 // of 64 tokens at a time copied HBM -> LDS by DMA (double-buffered), read
 // along tokens by transposing LDS reads, wave w accumulating G[:, 16w ..
-// 16w+15] and rows [16w, 16w+16) of the ninth column tile.  Rows past the end
-// of a progression are fetched from its first token (in bounds) and zeroed in
-// the Vb fragment, so they add nothing.
+// 16w+15] and rows [16w, 16w+16) of the normaliser column's tile.  r = 16 NW
+// takes NW waves, as in the scan.  Rows past the end of a progression are
+// fetched from its first token (in bounds) and zeroed in the Vb fragment, so
+// they add nothing.
 // ---------------------------------------------------------------------------
 
 // Issue one step's DMA: Psi (16 loads) and Vb (17) for rows
-// tok(row) = start + stride * (base + row), row < 64; wave 0 issues five
-// loads, the others four.
-// FEAT: K and V rows; the ninth Vb tile is constant, so 32 loads, four a wave.
+// tok(row) = start + stride * (base + row), row < 64, load I on wave I % NW
+// (chunks past the row's 2 NW re-read one of its own).
+// FEAT: K and V rows; the normaliser tile is constant, so 32 loads, four a wave.
 // Token of term idx: LIST (mode 2) reads it from the item's column list; the
 // other modes compute it, with no index loads whose waits (vmcnt(0), placed by
 // the compiler at every join after them) would drain the DMA in flight.
@@ -814,30 +814,31 @@ __device__ __forceinline__ int64_t gram_token_of(const GramItems& it, int item, 
     return start + (int64_t)idx * stride;
 }
 
-template <typename In, bool FEAT, bool LIST>
+template <typename In, int NW, bool FEAT, bool LIST>
 __device__ __forceinline__ void issue_gram(uint4* dpsi, uint4* dvb, const In* psib,
                                            const In* vbb, const GramItems& it, int item,
                                            int64_t start, int64_t stride, int base, int count,
                                            int64_t k_st, int64_t v_st, int w, int lane) {
   constexpr int kL = ss::kPhiLoads + ss::kVbLoads - (FEAT ? 1 : 0);     // 33 or 32
+  const auto chunk = [](int k) { return 2 * NW < ss::kRowChunks && k >= 2 * NW ? k - 8 : k; };
 #pragma unroll
-  for (int u = 0; u < 5; ++u) {
-    const int I = w + 8 * u;
+  for (int u = 0; u < (kL + NW - 1) / NW; ++u) {
+    const int I = w + NW * u;
     if (I < kL) {
       const In* src;
       uint4* dst;
       if (I < ss::kPhiLoads) {
         const int row = 4 * I + (lane >> 4);
-        const int k = (lane & 15) ^ swz16(row);
+        const int k = chunk((lane & 15) ^ swz16(row));
         const int64_t tok =
             gram_token_of<LIST>(it, item, start, stride, base + row < count ? base + row : 0);
         src = psib + tok * k_st + 8 * k;
         dst = dpsi + 64 * I;
       } else {
-        // Vb columns 0..127 swizzled like Psi, then columns 128..135, lane = row
+        // Vb's value columns swizzled like Psi, then the normaliser chunks, lane = row
         const int li = I - ss::kPhiLoads;
         const int row = li < ss::kPhiLoads ? 4 * li + (lane >> 4) : lane;
-        const int col = li < ss::kPhiLoads ? 8 * ((lane & 15) ^ swz16(row)) : 128;
+        const int col = li < ss::kPhiLoads ? 8 * chunk((lane & 15) ^ swz16(row)) : 16 * NW;
         const int64_t tok =
             gram_token_of<LIST>(it, item, start, stride, base + row < count ? base + row : 0);
         src = vbb + tok * v_st + col;
@@ -858,16 +859,20 @@ __device__ __forceinline__ void issue_gram(uint4* dpsi, uint4* dvb, const In* ps
 // FEAT: psi and vb are K and V rows; each step's Psi tile is formed in place
 // from the DMA'd K tile (feat_rows, W in registers, two halves of 32 rows),
 // times the key gate.
-template <typename In, bool ONE, bool FEAT, bool LIST>
-__global__ __launch_bounds__(ss::kThreads, (ONE && !FEAT) ? 3 : 2) void gram_stream_kernel(
+template <typename In, int NW, bool ONE, bool FEAT, bool LIST>
+__global__ __launch_bounds__(64 * NW, (ONE && !FEAT) ? 3 : 2) void gram_stream_kernel(
     const In* __restrict__ psi, const In* __restrict__ vb, float* __restrict__ G,
-    float* __restrict__ G_last, GramItems it, int p, int64_t k_sb, int64_t k_st, int64_t v_sb,
+    float* __restrict__ G_last, GramItems it, int64_t k_sb, int64_t k_st, int64_t v_sb,
     int64_t v_st, int64_t g_sb, int64_t g_si, int64_t gl_sb, FeatArgs fa) {
   using namespace ss;
   typedef typename Traits<In>::frag Frag;
+  constexpr int kThreads = 64 * NW;
+  constexpr int kP = 16 * NW + 1;                    // = p
+  constexpr int kL = kPhiLoads + kVbLoads - (FEAT ? 1 : 0);
+  static_assert(!FEAT || NW == 8, "the feature map is 128 x 128");
   // psi0 and vb0 are one array: after the last step it stages the output
   __shared__ __attribute__((aligned(16))) uint4 stage0[kTileChunks + kVbTileChunks];
-  static_assert((kTileChunks + kVbTileChunks) * 16 >= 64 * 129 * 4, "stage holds 64 rows of G");
+  static_assert((kTileChunks + kVbTileChunks) * 16 >= 64 * kP * 4, "stage holds 64 rows of G");
   uint4* psi0 = stage0;
   uint4* vb0 = stage0 + kTileChunks;
   __shared__ __attribute__((aligned(16))) uint4 psi1[ONE ? 1 : kTileChunks];
@@ -885,7 +890,7 @@ __global__ __launch_bounds__(ss::kThreads, (ONE && !FEAT) ? 3 : 2) void gram_str
     item = (int)(lin / gridDim.y);
   }
   const int w = __builtin_amdgcn_readfirstlane(wave_id());
-  __builtin_assume(w >= 0 && w < 8);                 // eight waves
+  __builtin_assume(w >= 0 && w < NW);
   int64_t start, stride;
   int count;
   gram_item(it, item, start, stride, count);
@@ -894,11 +899,11 @@ __global__ __launch_bounds__(ss::kThreads, (ONE && !FEAT) ? 3 : 2) void gram_str
   float* Gout = (it.mode == 1 && item == it.N0) ? G_last + b * gl_sb : G + b * g_sb + item * g_si;
   const int nsteps = (count + kStep - 1) / kStep;
 
-  f32x4 accS[8], accS8 = zero4();
+  f32x4 accS[NW], accS8 = zero4();
 #pragma unroll
-  for (int at = 0; at < 8; ++at) accS[at] = zero4();
+  for (int at = 0; at < NW; ++at) accS[at] = zero4();
   if (nsteps > 0)
-    issue_gram<In, FEAT, LIST>(psi0, vb0, psib, vbb, it, item, start, stride, 0, count, k_st, v_st, w,
+    issue_gram<In, NW, FEAT, LIST>(psi0, vb0, psib, vbb, it, item, start, stride, 0, count, k_st, v_st, w,
                          lane_id());
   Frag wa[4];
   const In* hb = nullptr;
@@ -935,14 +940,13 @@ __global__ __launch_bounds__(ss::kThreads, (ONE && !FEAT) ? 3 : 2) void gram_str
       }
     }
     if (!ONE && s + 1 < nsteps) {
-      issue_gram<In, FEAT, LIST>(BUF ? psi0 : psi1, BUF ? vb0 : vb1, psib, vbb, it, item, start, stride,
+      issue_gram<In, NW, FEAT, LIST>(BUF ? psi0 : psi1, BUF ? vb0 : vb1, psib, vbb, it, item, start, stride,
                            (s + 1) * kStep, count, k_st, v_st, w, lane);
-      static_assert(kPhiLoads + kVbLoads == 33, "five loads on wave 0, four on the rest");
       // the gate loads (issued first) are older than this step's DMA loads
-      if (!FEAT && w == 0)
-        wait_vmcnt<5>();
+      if (w < kL % NW)
+        wait_vmcnt<kL / NW + 1>();
       else
-        wait_vmcnt<4>();
+        wait_vmcnt<kL / NW>();
     } else {
       wait_vmcnt<0>();
     }
@@ -987,7 +991,7 @@ __global__ __launch_bounds__(ss::kThreads, (ONE && !FEAT) ? 3 : 2) void gram_str
         }
       }
 #pragma unroll
-      for (int at = 0; at < 8; ++at) {
+      for (int at = 0; at < NW; ++at) {
         const Frag pa = psi_tr<In>(tpsi, at, ks, lane);
         accS[at] = mma(accS[at], pa, vbw);
         if (at == w) accS8 = mma(accS8, pa, vb8);
@@ -1006,30 +1010,33 @@ __global__ __launch_bounds__(ss::kThreads, (ONE && !FEAT) ? 3 : 2) void gram_str
 
   const int lane = lane_id();
   const int r16 = lane & 15, g = lane >> 4;
-  if (p == 129 && (reinterpret_cast<uintptr_t>(Gout) & 15) == 0) {
-    // The r x p result is one contiguous block.  Stage it 64 rows (33 KB) at
-    // a time in the idle tile buffer and store each half as consecutive
-    // 16-byte stores: whole cache lines, instead of 64-byte runs of
+  if ((reinterpret_cast<uintptr_t>(Gout) & 15) == 0) {
+    // The r x p result is one contiguous block.  Stage it 64 rows (33 KB at
+    // r = 128) at a time in the idle tile buffer and store each part as
+    // consecutive 16-byte stores: whole cache lines, instead of 64-byte runs of
     // 516-byte rows.  Non-temporal: the table (888 MB for the long-prefill
     // pool) is far larger than the last-level cache and is read back only by
     // the next kernel.
     float* st = reinterpret_cast<float*>(stage0);
-    constexpr int kHalf = 64 * 129;                  // floats
-    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int h = 0; h < (NW + 3) / 4; ++h) {
+      const int tiles = min(4, NW - 4 * h);          // row tiles of this part
       lds_barrier();                                 // the tile buffer is free
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4)
+      for (int q4 = 0; q4 < 4; ++q4) {
+        if (4 * h + q4 >= NW) continue;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          st[(16 * q4 + 4 * g + i) * 129 + 16 * w + r16] = accS[4 * h + q4][i];
-      if ((w >> 2) == h && r16 == 0) {               // column 128: rows 16 w + 4 g + i
+          st[(16 * q4 + 4 * g + i) * kP + 16 * w + r16] = accS[4 * h + q4][i];
+      }
+      if ((w >> 2) == h && r16 == 0) {               // the last column: rows 16 w + 4 g + i
 #pragma unroll
-        for (int i = 0; i < 4; ++i) st[(16 * (w & 3) + 4 * g + i) * 129 + 128] = accS8[i];
+        for (int i = 0; i < 4; ++i) st[(16 * (w & 3) + 4 * g + i) * kP + kP - 1] = accS8[i];
       }
       lds_barrier();
       const float4* src = reinterpret_cast<const float4*>(st);
-      float4* dst = reinterpret_cast<float4*>(Gout + h * kHalf);
-      for (int e = threadIdx.x; e < kHalf / 4; e += kThreads) {
+      float4* dst = reinterpret_cast<float4*>(Gout + h * 64 * kP);
+      for (int e = threadIdx.x; e < tiles * 4 * kP; e += kThreads) {
         const float4 v = src[e];
         __builtin_nontemporal_store(v.x, &dst[e].x);
         __builtin_nontemporal_store(v.y, &dst[e].y);
@@ -1040,12 +1047,13 @@ __global__ __launch_bounds__(ss::kThreads, (ONE && !FEAT) ? 3 : 2) void gram_str
     return;
   }
 #pragma unroll
-  for (int at = 0; at < 8; ++at)
+  for (int at = 0; at < NW; ++at)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) Gout[(int64_t)(16 * at + 4 * g + i) * p + 16 * w + r16] = accS[at][i];
-  if (128 + r16 < p) {
+    for (int i = 0; i < 4; ++i)
+      Gout[(int64_t)(16 * at + 4 * g + i) * kP + 16 * w + r16] = accS[at][i];
+  if (r16 == 0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) Gout[(int64_t)(16 * w + 4 * g + i) * p + 128 + r16] = accS8[i];
+    for (int i = 0; i < 4; ++i) Gout[(int64_t)(16 * w + 4 * g + i) * kP + kP - 1] = accS8[i];
   }
 }
 
@@ -1053,69 +1061,81 @@ bool gram_stream_ok(int dtype, const void* psi, const void* vb, int r, int p, in
                     int64_t k_st, int64_t v_sb, int64_t v_st, const GramItems& it, int nitems,
                     int nb) {
   if (dtype != SMAT_BF16 && dtype != SMAT_F16) return false;
-  if (r != 128 || p != 129 || it.nsplit > 1) return false;
+  if (r % 16 || r < 80 || r > 128 || p != r + 1 || it.nsplit > 1) return false;
+  if (r < 128 && it.mode == 2) return false;           // lists: compiled for r = 128
   if ((int64_t)nitems * nb < 256) return false;        // few, long items: the split-K kernel
-  if (!rows_vec_ok(psi, k_sb, k_st, 2) || !rows_vec_ok(vb, v_sb, v_st, 2) || v_st < 136)
+  if (!rows_vec_ok(psi, k_sb, k_st, 2) || !rows_vec_ok(vb, v_sb, v_st, 2) || v_st < r + 8)
     return false;
   return variant(SMAT_VARIANT_GRAM) == 0;
 }
 
-template <typename In, bool FEAT>
+template <typename In, int NW, bool FEAT>
 static void gram_stream_kernel_launch(const void* psi, const void* vb, float* G, float* G_last,
-                                      const GramItems& it, dim3 grid, bool one, int p,
-                                      int64_t k_sb, int64_t k_st, int64_t v_sb, int64_t v_st,
-                                      int64_t g_sb, int64_t g_si, int64_t gl_sb,
-                                      const FeatArgs& fa, hipStream_t stream) {
+                                      const GramItems& it, dim3 grid, bool one, int64_t k_sb,
+                                      int64_t k_st, int64_t v_sb, int64_t v_st, int64_t g_sb,
+                                      int64_t g_si, int64_t gl_sb, const FeatArgs& fa,
+                                      hipStream_t stream) {
   const In* k = (const In*)psi;
   const In* v = (const In*)vb;
-  const dim3 blk(ss::kThreads);
-  // the feature map runs for profiles and chunk groups only: no list form
-  if (!FEAT && it.mode == 2) {
-    if (one)
-      smat::launch((gram_stream_kernel<In, true, false, true>), grid, blk, 0, stream, k, v,
-                         G, G_last, it, p, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
-    else
-      smat::launch((gram_stream_kernel<In, false, false, true>), grid, blk, 0, stream, k, v,
-                         G, G_last, it, p, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
-  } else if (one) {
-    smat::launch((gram_stream_kernel<In, true, FEAT, false>), grid, blk, 0, stream, k, v, G,
-                       G_last, it, p, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
-  } else {
-    smat::launch((gram_stream_kernel<In, false, FEAT, false>), grid, blk, 0, stream, k, v,
-                       G, G_last, it, p, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
+  const dim3 blk(64 * NW);
+  // lists (r = 128) have no form with the feature map
+  if constexpr (!FEAT && NW == 8) {
+    if (it.mode == 2) {
+      if (one)
+        smat::launch((gram_stream_kernel<In, 8, true, false, true>), grid, blk, 0, stream, k, v,
+                     G, G_last, it, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
+      else
+        smat::launch((gram_stream_kernel<In, 8, false, false, true>), grid, blk, 0, stream, k, v,
+                     G, G_last, it, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
+      return;
+    }
   }
+  if (one)
+    smat::launch((gram_stream_kernel<In, NW, true, FEAT, false>), grid, blk, 0, stream, k, v, G,
+                 G_last, it, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
+  else
+    smat::launch((gram_stream_kernel<In, NW, false, FEAT, false>), grid, blk, 0, stream, k, v, G,
+                 G_last, it, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
 }
 
-template <bool FEAT>
-static int gram_stream_go(int dtype, const void* psi, const void* vb, float* G, float* G_last,
-                          const GramItems& it, int nitems, int nb, int p, int64_t k_sb,
-                          int64_t k_st, int64_t v_sb, int64_t v_st, int64_t g_sb, int64_t g_si,
-                          int64_t gl_sb, const FeatArgs& fa, hipStream_t stream,
-                          const char* who) {
-  dim3 grid((unsigned)nitems, (unsigned)nb);
-  // the longest item: a profile has ceil((n - n_P) / N0) terms, the global
-  // channel (item N0, when launched) n_P
-  bool one = false;
-  if (it.mode == 1) {
-    int64_t maxc = it.N0 > 0 ? ((int64_t)it.n - it.n_P + it.N0 - 1) / it.N0 : 0;
-    if (nitems > it.N0) maxc = maxc > it.n_P ? maxc : it.n_P;
-    one = maxc <= ss::kStep;
-  }
-  if (dtype == SMAT_BF16)
-    gram_stream_kernel_launch<bf16, FEAT>(psi, vb, G, G_last, it, grid, one, p, k_sb, k_st, v_sb,
-                                          v_st, g_sb, g_si, gl_sb, fa, stream);
-  else
-    gram_stream_kernel_launch<f16, FEAT>(psi, vb, G, G_last, it, grid, one, p, k_sb, k_st, v_sb,
-                                         v_st, g_sb, g_si, gl_sb, fa, stream);
-  return launch_status(who);
+// Whether every item fits one step: a profile has ceil((n - n_P) / N0) terms,
+// the global channel (item N0, when launched) n_P.
+static bool gram_one_step(const GramItems& it, int nitems) {
+  if (it.mode != 1) return false;
+  int64_t maxc = it.N0 > 0 ? ((int64_t)it.n - it.n_P + it.N0 - 1) / it.N0 : 0;
+  if (nitems > it.N0) maxc = maxc > it.n_P ? maxc : it.n_P;
+  return maxc <= ss::kStep;
 }
 
 int gram_stream_launch(int dtype, const void* psi, const void* vb, float* G, float* G_last,
                        const GramItems& it, int nitems, int nb, int p, int64_t k_sb,
                        int64_t k_st, int64_t v_sb, int64_t v_st, int64_t g_sb, int64_t g_si,
                        int64_t gl_sb, hipStream_t stream, const char* who) {
-  return gram_stream_go<false>(dtype, psi, vb, G, G_last, it, nitems, nb, p, k_sb, k_st, v_sb,
-                               v_st, g_sb, g_si, gl_sb, FeatArgs{}, stream, who);
+  const dim3 grid((unsigned)nitems, (unsigned)nb);
+  const bool one = gram_one_step(it, nitems);
+  const FeatArgs fa{};
+#define SMAT_GRAM_NW(NWV)                                                                      \
+  case NWV:                                                                                    \
+    if (dtype == SMAT_BF16)                                                                    \
+      gram_stream_kernel_launch<bf16, NWV, false>(psi, vb, G, G_last, it, grid, one, k_sb,     \
+                                                  k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa,     \
+                                                  stream);                                     \
+    else                                                                                       \
+      gram_stream_kernel_launch<f16, NWV, false>(psi, vb, G, G_last, it, grid, one, k_sb,      \
+                                                 k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa,      \
+                                                 stream);                                      \
+    break;
+  switch (p / 16) {
+    SMAT_GRAM_NW(5)
+    SMAT_GRAM_NW(6)
+    SMAT_GRAM_NW(7)
+    SMAT_GRAM_NW(8)
+    default:
+      set_error("%s: no streaming Gram kernel for p=%d", who, p);
+      return SMAT_EUNSUPPORTED;
+  }
+#undef SMAT_GRAM_NW
+  return launch_status(who);
 }
 
 // The Gram sums with the feature map in place: k, v are K and V rows
@@ -1130,8 +1150,15 @@ int gram_stream_launch_feat(int dtype, const void* k, const void* v, float* G, f
     set_error("%s: the feature map is not fused into list Gram sums", who);
     return SMAT_EUNSUPPORTED;
   }
-  return gram_stream_go<true>(dtype, k, v, G, G_last, it, nitems, nb, 129, k_sb, k_st, v_sb, v_st,
-                              g_sb, g_si, gl_sb, fa, stream, who);
+  const dim3 grid((unsigned)nitems, (unsigned)nb);
+  const bool one = gram_one_step(it, nitems);
+  if (dtype == SMAT_BF16)
+    gram_stream_kernel_launch<bf16, 8, true>(k, v, G, G_last, it, grid, one, k_sb, k_st, v_sb,
+                                             v_st, g_sb, g_si, gl_sb, fa, stream);
+  else
+    gram_stream_kernel_launch<f16, 8, true>(k, v, G, G_last, it, grid, one, k_sb, k_st, v_sb,
+                                            v_st, g_sb, g_si, gl_sb, fa, stream);
+  return launch_status(who);
 }
 
 // The shapes this kernel serves; everything else runs scan_fused_kernel.

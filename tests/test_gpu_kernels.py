@@ -477,6 +477,36 @@ def _check_forward(spec, Phi, Psi, Vb, *, dt, g=None, label=""):
     return out
 
 
+@pytest.mark.parametrize("hd", [80, 96, 112])
+@pytest.mark.parametrize("T,n_P,n,N0,nb", [(2048, 0, 1024, 121, 3), (2048, 16, 1000, 90, 3),
+                                           (9000, 64, 8000, 50, 6), (640, 0, 640, 640, 1)])
+def test_gram_streaming_widths(hd, T, n_P, n, N0, nb):
+    """The streaming Gram sums between head sizes 64 and 128 (five to seven waves):
+    profiles of one step and of several, a short last step, one token a profile,
+    the global channel, and chunk groups, from rows whose padding is NaN, against
+    fp64."""
+    _say("gram widths", hd, T, n_P, n, N0, nb)
+    Phi, Psi, Vb = _feats(nb, T, hd, torch.bfloat16, seed=51)
+    Vp = torch.full((nb, T, hd + 8), float("nan"), dtype=torch.bfloat16)
+    Vp[..., :hd + 1] = Vb
+    Sd, Vd = Psi.to(DEV), Vp.to(DEV)[..., :hd + 1]
+    glob = torch.empty(nb, hd, hd + 1, device=DEV) if n_P else None
+    F = K.pool(Sd, Vd, n_P, n, N0, F_glob=glob)
+    S64, V64 = Psi.double(), Vb.double()
+    for x in (0, 1, (n - n_P) % N0 - 1, N0 - 1):
+        rows = slice(n_P + x % N0, n, N0)
+        want = S64[:, rows].transpose(1, 2).contiguous() @ V64[:, rows]
+        assert _rel(F[:, x % N0], want) < 1e-5
+    if n_P:
+        want = S64[:, :n_P].transpose(1, 2).contiguous() @ V64[:, :n_P]
+        assert _rel(glob, want) < 1e-5
+    C = 64 if nb == 1 else 8
+    D = K.chunk_states(Sd, Vd, C)
+    pad = torch.nn.functional.pad
+    c64 = lambda t: pad(t, (0, 0, 0, -T % C)).reshape(nb, -1, C, t.shape[-1])
+    assert _rel(D, c64(S64).transpose(2, 3).contiguous() @ c64(V64)) < 1e-5
+
+
 @pytest.mark.parametrize("hd,T,n,C,dt", [
     (64, 1024, 512, 128, torch.bfloat16), (64, 64, 0, 64, torch.float16),
     (64, 8192 + 1, 4096, 128, torch.bfloat16), (64, 1023, 1023 // 64 * 64, 64, torch.bfloat16),
