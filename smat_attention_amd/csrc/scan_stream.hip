@@ -851,8 +851,9 @@ __device__ __forceinline__ void issue_gram(uint4* dpsi, uint4* dvb, const In* ps
   }
 }
 
-// ONE: every item of the launch has at most kStep terms (the profile pool at
-// long T: (n - n_P) / N0 tokens a profile), so one buffer suffices.  Its
+// ONE: the profiles of the launch have at most kStep terms (the profile pool at
+// long T: (n - n_P) / N0 tokens a profile), so one buffer suffices -- a global
+// channel's few steps wait for their rows one by one.  Its
 // 35 KB of LDS let three workgroups share a CU instead of two, which is what
 // a launch of one-step items -- a load latency, a few MFMAs and a 66 KB
 // store each -- is limited by.
@@ -980,6 +981,7 @@ __global__ __launch_bounds__(64 * NW, (ONE && !FEAT) ? 3 : 2) void gram_stream_k
     const int nvalid = count - s * kStep;        // rows of this step holding tokens
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
+      if (32 * ks >= nvalid) continue;
       Frag vbw = psi_tr<In>(tvb, w, ks, lane);
       Frag vb8 = vb_norm_tr<In>(tvb, ks, lane);
       if (nvalid < kStep) {
@@ -997,10 +999,13 @@ __global__ __launch_bounds__(64 * NW, (ONE && !FEAT) ? 3 : 2) void gram_stream_k
         if (at == w) accS8 = mma(accS8, pa, vb8);
       }
     }
-    lds_barrier();     // this buffer is free for the DMA issued next step
+    lds_barrier();     // this buffer is free for the next DMA
+    if (ONE && s + 1 < nsteps)
+      issue_gram<In, NW, FEAT, LIST>(psi0, vb0, psib, vbb, it, item, start, stride,
+                                     (s + 1) * kStep, count, k_st, v_st, w, lane);
   };
   if constexpr (ONE) {
-    if (nsteps > 0) step(std::integral_constant<int, 0>{}, 0);     // nsteps <= 1
+    for (int s = 0; s < nsteps; ++s) step(std::integral_constant<int, 0>{}, s);
   } else {
     for (int s = 0; s < nsteps; s += 2) {
       step(std::integral_constant<int, 0>{}, s);
@@ -1063,7 +1068,8 @@ bool gram_stream_ok(int dtype, const void* psi, const void* vb, int r, int p, in
   if (dtype != SMAT_BF16 && dtype != SMAT_F16) return false;
   if (r % 16 || r < 80 || r > 128 || p != r + 1 || it.nsplit > 1) return false;
   if (r < 128 && it.mode == 2) return false;           // lists: compiled for r = 128
-  if ((int64_t)nitems * nb < 256) return false;        // few, long items: the split-K kernel
+  // few, long profiles: the split-K kernel (chunk groups are not split)
+  if (it.mode != 0 && (int64_t)nitems * nb < 256) return false;
   if (!rows_vec_ok(psi, k_sb, k_st, 2) || !rows_vec_ok(vb, v_sb, v_st, 2) || v_st < r + 8)
     return false;
   return variant(SMAT_VARIANT_GRAM) == 0;
@@ -1098,13 +1104,14 @@ static void gram_stream_kernel_launch(const void* psi, const void* vb, float* G,
                  G_last, it, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
 }
 
-// Whether every item fits one step: a profile has ceil((n - n_P) / N0) terms,
-// the global channel (item N0, when launched) n_P.
+// Whether the profiles, of ceil((n - n_P) / N0) terms, fit one step, and the
+// global channel (item N0, when launched), of n_P, a few: 128 of them beside
+// profiles of 14 tokens in two buffers held the pool of 12 x 10007 tokens of 96
+// to 72 us.
 static bool gram_one_step(const GramItems& it, int nitems) {
   if (it.mode != 1) return false;
-  int64_t maxc = it.N0 > 0 ? ((int64_t)it.n - it.n_P + it.N0 - 1) / it.N0 : 0;
-  if (nitems > it.N0) maxc = maxc > it.n_P ? maxc : it.n_P;
-  return maxc <= ss::kStep;
+  const int64_t maxc = it.N0 > 0 ? ((int64_t)it.n - it.n_P + it.N0 - 1) / it.N0 : 0;
+  return maxc <= ss::kStep && (nitems <= it.N0 || it.n_P <= 8 * ss::kStep);
 }
 
 int gram_stream_launch(int dtype, const void* psi, const void* vb, float* G, float* G_last,
