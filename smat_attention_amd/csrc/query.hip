@@ -157,6 +157,144 @@ __global__ __launch_bounds__(qy::kThreads) void query_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// Heads of 64 to 112 (16-bit inputs, r = 16 NW, p = r + 1): one workgroup of
+// NW + 1 waves per (sequence, row type, 64 rows).  U_h (17 KB at r = 64, 37 KB at
+// 96) and the rows are copied HBM -> LDS whole and multiplied as in the
+// streaming kernel below; the other workgroups of the CU (six at r = 64, three
+// at 96) hide each other's copies, which a walk through one U_h after another
+// would need a ring for.  What bounds it: HBM (4.9 TB/s at r = 96).  The general
+// kernel, whose lanes load U one element at a time, took 62 us where this takes
+// 42 (12 x 10007 tokens, r = 96), 26 where this takes 19 (32 x 8192, r = 64) and
+// 120 where this takes 82 (96 x 4096, d = 3).
+// ---------------------------------------------------------------------------
+
+namespace qt {
+template <int NW>
+struct Shape {
+  static constexpr int kR = 16 * NW, kP = 16 * NW + 1;
+  static constexpr int kWaves = NW + 1;                      // the last: column r alone
+  static constexpr int kRC = NW > 4 ? 16 : 8;                // 16-byte chunks a Phi row
+  static constexpr int kUChunks = kR * kP / 4;
+  static constexpr int kULoads = (kUChunks + 63) / 64;       // wave-wide copies of U_h
+  static constexpr int kPLoads = qy::kRowsPerWG * kRC / 64;  // and of the rows
+};
+// Slot of chunk k of row t: the eight rows a read phase covers, at chunks k and
+// k + 2 (the permuted k groups below), take distinct banks.
+template <int RC>
+__device__ __forceinline__ int swz(int t) { return RC == 16 ? t & 15 : (t >> 1) & 7; }
+}  // namespace qt
+
+template <typename In, int NW>
+__global__ __launch_bounds__(64 * (NW + 1)) void query_tile_kernel(
+    const In* __restrict__ phi, const float* __restrict__ U, float* __restrict__ Y, int T_R, int B,
+    int64_t u_ld, int64_t q_sb, int64_t q_st, int64_t y_sb, int64_t y_st, int nrb) {
+  typedef qt::Shape<NW> Sh;
+  typedef typename Traits<In>::frag Frag;
+  typedef typename Traits<In>::half_frag Half;
+  constexpr int RC = Sh::kRC, kP = Sh::kP;
+  __shared__ __attribute__((aligned(16))) float us[Sh::kULoads * 256];
+  __shared__ __attribute__((aligned(16))) uint4 ps[Sh::kPLoads * 64];
+  const int h = blockIdx.x / nrb;
+  const int k0 = (blockIdx.x - h * nrb) * qy::kRowsPerWG;
+  const int64_t b = blockIdx.y;
+  const int cnt = (h < T_R ? (T_R - h + B - 1) / B : 0) - k0;   // rows of this block
+  if (cnt <= 0) return;
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  __builtin_assume(w >= 0 && w < Sh::kWaves);
+  const int lane = lane_id();
+  const float* Uh = U + (b * B + h) * u_ld;
+  const In* phih = phi + b * q_sb + ((int64_t)h + (int64_t)k0 * B) * q_st;
+#pragma unroll
+  for (int u = 0; u < (Sh::kULoads + Sh::kWaves - 1) / Sh::kWaves; ++u) {
+    const int I = w + Sh::kWaves * u;
+    if (I < Sh::kULoads) {
+      const int c = 64 * I + lane;
+      lds_dma16<true>(Uh + 4 * (c < Sh::kUChunks ? c : 0), us + 256 * I);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < (Sh::kPLoads + Sh::kWaves - 1) / Sh::kWaves; ++u) {
+    const int I = w + Sh::kWaves * u;
+    if (I < Sh::kPLoads) {
+      const int row = (64 / RC) * I + lane / RC;
+      int k = (lane % RC) ^ qt::swz<RC>(row);
+      if (2 * NW < RC && k >= 2 * NW) k -= 8;        // past the row: one of its own
+      lds_dma16<true>(phih + (int64_t)(row < cnt ? row : 0) * B * q_st + 8 * k, ps + 64 * I);
+    }
+  }
+  wait_vmcnt<0>();
+  lds_barrier();
+
+  const int r16 = lane & 15, g = lane >> 4;
+  const int c = 16 * w + r16;
+  // Lane group g takes the k-slots of feature group pg of each 32, as in the
+  // streaming kernel (rows of U_h 16 apart fall on disjoint banks: 16 p is 16
+  // modulo the 64 banks at every one of these widths).
+  const int pg = (g >> 1) | ((g & 1) << 1);
+  f32x4 acc[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[t] = zero4();
+  // the hi and lo parts of n <= 8 rows of U_h from row a
+  auto u_frag = [&](Frag& ah, Frag& al, int a, int n) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float uv = e < n && c < kP ? us[(a + e) * kP + c] : 0.f;
+      In hh, ll;
+      split2<In>(uv, hh, ll);
+      ah[e] = hh;
+      al[e] = ll;
+    }
+  };
+#pragma unroll
+  for (int kb = 0; kb < NW / 2; ++kb) {
+    Frag ah, al;
+    u_frag(ah, al, 32 * kb + 8 * pg, 8);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int row = 16 * t + r16;
+      const Frag pb =
+          *reinterpret_cast<const Frag*>(ps + row * RC + ((4 * kb + pg) ^ qt::swz<RC>(row)));
+      acc[t] = mma(acc[t], ah, pb);
+      acc[t] = mma(acc[t], al, pb);
+    }
+  }
+  if constexpr (NW % 2 != 0) {
+    // the last 16 features: a k-block whose upper halves are zero
+    Frag ah, al;
+    u_frag(ah, al, 16 * (NW - 1) + 4 * g, 4);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int row = 16 * t + r16;
+      const char* src = reinterpret_cast<const char*>(
+          ps + row * RC + ((2 * (NW - 1) + (g >> 1)) ^ qt::swz<RC>(row)));
+      const Half ph = *reinterpret_cast<const Half*>(src + 8 * (g & 1));
+      Frag pb;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        pb[e] = ph[e];
+        pb[4 + e] = from_f32<In>(0.f);
+      }
+      acc[t] = mma(acc[t], ah, pb);
+      acc[t] = mma(acc[t], al, pb);
+    }
+  }
+  float* Yb = Y + b * y_sb;
+  const int c0 = 16 * w + 4 * g;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int k = 16 * t + r16;
+    if (k < cnt) {
+      float* yrow = Yb + ((int64_t)h + (int64_t)(k0 + k) * B) * y_st;
+      if (w < NW)
+        *reinterpret_cast<float4*>(yrow + c0) =
+            make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+      else if (g == 0)
+        yrow[c0] = acc[t][0];
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Head-dim-128 variant (16-bit inputs, r = 128, p = 129): persistent
 // workgroups of nine waves walk the (sequence, row type) items, MT 16-row
 // tiles an item (MT = 3: up to 48 rows a type, MT = 4: up to 64).  The product
@@ -516,8 +654,45 @@ int query_stream_launch_feat(int dtype, const void* q, const float* U, float* Y,
                                stream);
 }
 
+// The widths of query_tile_kernel, rows and U_h 16-byte aligned.
+static bool query_tile_ok(int dtype, const void* phi, const float* U, const float* Y, int r, int p,
+                          int64_t u_ld, int64_t q_sb, int64_t q_st, int64_t y_sb, int64_t y_st) {
+  if (dtype != SMAT_BF16 && dtype != SMAT_F16) return false;
+  if (r % 16 || r < 64 || r > 112 || p != r + 1 || u_ld % 4) return false;
+  if (!rows_vec_ok(phi, q_sb, q_st, 2) || !aligned16(U) || !rows_vec_ok(Y, y_sb, y_st, 4))
+    return false;
+  return variant(SMAT_VARIANT_QUERY) == 0;
+}
+
+template <typename In>
+static int launch_query_tile(const void* phi, const float* U, float* Y, int nb, int T_R, int B,
+                             int r, int64_t u_ld, int64_t q_sb, int64_t q_st, int64_t y_sb,
+                             int64_t y_st, hipStream_t stream) {
+  const int maxcnt = (T_R + B - 1) / B;
+  const int nrb = (maxcnt + qy::kRowsPerWG - 1) / qy::kRowsPerWG;
+  const int64_t gx = (int64_t)B * nrb;
+  if (gx >= (1ll << 31)) {
+    set_error("smat_query: problem too large");
+    return SMAT_EUNSUPPORTED;
+  }
+  const dim3 grid((unsigned)gx, (unsigned)nb);
+#define SMAT_QT(NWV)                                                                           \
+  case NWV:                                                                                    \
+    smat::launch((query_tile_kernel<In, NWV>), grid, dim3(64 * (NWV + 1)), 0, stream,          \
+                 (const In*)phi, U, Y, T_R, B, u_ld, q_sb, q_st, y_sb, y_st, nrb);             \
+    break;
+  switch (r / 16) {
+    SMAT_QT(4)
+    SMAT_QT(5)
+    SMAT_QT(6)
+    SMAT_QT(7)
+  }
+#undef SMAT_QT
+  return launch_status("smat_query");
+}
+
 // U: (nb, B) rows of r * p floats, u_ld floats apart (u_ld % 4 == 0 for the
-// streaming kernel's 16-byte copies).
+// streaming kernels' 16-byte copies).
 int query_dispatch(int dtype, const void* phi, const float* U, float* Y, int nb, int T_R, int B,
                    int r, int p, int64_t u_ld, int64_t q_sb, int64_t q_st, int64_t y_sb,
                    int64_t y_st, hipStream_t stream) {
@@ -525,6 +700,12 @@ int query_dispatch(int dtype, const void* phi, const float* U, float* Y, int nb,
   if (u_ld % 4 == 0 && query_stream_ok(dtype, phi, U, Y, T_R, B, r, p, q_sb, q_st, y_sb, y_st))
     return launch_query_stream(dtype, phi, U, Y, nb, T_R, B, u_ld, q_sb, q_st, y_sb, y_st,
                                stream);
+  if (query_tile_ok(dtype, phi, U, Y, r, p, u_ld, q_sb, q_st, y_sb, y_st))
+    return dtype == SMAT_BF16
+               ? launch_query_tile<bf16>(phi, U, Y, nb, T_R, B, r, u_ld, q_sb, q_st, y_sb, y_st,
+                                         stream)
+               : launch_query_tile<f16>(phi, U, Y, nb, T_R, B, r, u_ld, q_sb, q_st, y_sb, y_st,
+                                        stream);
   switch (dtype) {
     case SMAT_BF16:
       return launch_query<bf16>(phi, U, Y, nb, T_R, B, r, p, u_ld, q_sb, q_st, y_sb, y_st,

@@ -507,6 +507,27 @@ def test_gram_streaming_widths(hd, T, n_P, n, N0, nb):
     assert _rel(D, c64(S64).transpose(2, 3).contiguous() @ c64(V64)) < 1e-5
 
 
+@pytest.mark.parametrize("hd", [64, 80, 96, 112])
+@pytest.mark.parametrize("T_R,B", [(1024, 47), (300, 132), (1000, 7), (5, 9), (64, 1), (130, 2)])
+def test_query_tile_widths(hd, T_R, B):
+    """The query between head sizes 64 and 128 (U_h and 64 rows in LDS): several
+    row blocks a type, short last blocks, types without a row, against the general
+    kernel and fp64 (U split in two 16-bit parts: 2^-15 of the sum of products)."""
+    _say("query tile", hd, T_R, B)
+    g = torch.Generator().manual_seed(61)
+    Phi = (torch.rand(3, T_R, hd, generator=g) + 0.1).to(torch.bfloat16)
+    U = torch.randn(3, B, hd, hd + 1, generator=g)
+    Pd, Ud = Phi.to(DEV), U.to(DEV)
+    got = K.query(Pd, Ud)
+    with general_kernel("query"):
+        old = K.query(Pd, Ud)
+    Ui = U.double()[:, torch.arange(T_R) % B]
+    want = (Phi.double().unsqueeze(2) @ Ui).squeeze(2)
+    bound = (Phi.double().unsqueeze(2) @ Ui.abs()).squeeze(2) * 2.0 ** -15
+    assert ((got.double().cpu() - want).abs() <= bound).all()
+    assert _rel(got, old) < 1e-5
+
+
 @pytest.mark.parametrize("hd,T,n,C,dt", [
     (64, 1024, 512, 128, torch.bfloat16), (64, 64, 0, 64, torch.float16),
     (64, 8192 + 1, 4096, 128, torch.bfloat16), (64, 1023, 1023 // 64 * 64, 64, torch.bfloat16),
