@@ -20,6 +20,7 @@
 // hi/lo 16-bit parts for 16-bit inputs, as the B operand of the next chunk's
 // Phi S.  Psi and Vb are staged once per 64-token block and feed both the
 // intra-chunk product and the update.
+#include <algorithm>
 #include <mutex>
 
 #include "feat_map.hpp"
@@ -347,7 +348,9 @@ __global__ __launch_bounds__(sf::kThreads, kRK <= 2 ? 2 : 1) void scan_fused_ker
         }
       }
 
-      // state update: S += Psi_blk^T Vb_blk (this wave's rows of S)
+      // state update: S += Psi_blk^T Vb_blk (this wave's rows of S); nothing
+      // reads the state after the group's last chunk
+      if (ch + 1 < c1)
 #pragma unroll
       for (int kk = 0; kk < kBN / 32; ++kk) {
         if (n0 + 32 * kk >= Cv) continue;
@@ -501,16 +504,36 @@ static int64_t group_bytes(int nb, int nc, int K, int r, int p) {
   return al256((int64_t)nb * ((nc + K - 1) / K + 1) * r * p * 4);
 }
 
+// The chunk a small causal pass runs at: C halved while fewer than 256 chunks
+// would leave CUs without one, down to 32 tokens (64 for the streaming kernel's
+// widths in 16 bits: its step).  A group is then the smaller part of a longer
+// chain, and a 16-bit score that falls outside its chunk is not rounded.
+// Forward of 4 x 1024 tokens of 64: fp32 62 -> 40 us, bf16 43 -> 28 us; of 8 x
+// 1024 of 128 at d = 3 121 -> 88 us; of 32 x 4096 of 64 in fp32 (1024 chunks: as
+// before) 175 -> 165 us, from the last update that is now left out.
+static int scan_chunk(int dtype, int nb, int T, int C, int r, int p) {
+  const bool steps = dtype != SMAT_F32 && r % 16 == 0 && r >= 64 && p == r + 1;
+  const int least = steps ? 64 : 32;
+  while (C % (2 * least) == 0 && (int64_t)nb * ((T + C - 1) / C) < 256) C /= 2;
+  return C;
+}
+
 int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
                     const float* gate, float* out, int nb, int T, int n, int C, int K, int r, int p,
                     int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st,
                     int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb,
                     int64_t o_st, int64_t g_sb, int write_H, void* ws, hipStream_t stream);
 
+// The most any input type's chunk needs (the type is not an argument).
 int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, int kmax) {
-  const int nc = (T + C - 1) / C;
-  const int K = scan_group_chunks(nb, nc, r, p, kmax);
-  return 2 * group_bytes(nb, nc, K, r, p);
+  int64_t most = 0;
+  for (const int dtype : {SMAT_F32, SMAT_BF16}) {
+    const int c = scan_chunk(dtype, nb, T, C, r, p);
+    const int nc = (T + c - 1) / c;
+    const int K = scan_group_chunks(nb, nc, r, p, kmax);
+    most = std::max(most, 2 * group_bytes(nb, nc, K, r, p));
+  }
+  return most;
 }
 
 int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void* vb,
@@ -520,9 +543,9 @@ int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void
                          int64_t o_sb, int64_t o_st, int64_t g_sb, int write_H, void* ws,
                          int64_t ws_bytes, int kmax, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
-  const int nc = (T + C - 1) / C;
-  const int K = scan_group_chunks(nb, nc, r, p, kmax);
   const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, kmax);
+  C = scan_chunk(dtype, nb, T, C, r, p);
+  const int K = scan_group_chunks(nb, (T + C - 1) / C, r, p, kmax);
   if (ws_bytes < need) {
     set_error("smat_causal_scan: workspace of %lld bytes needed, %lld given", (long long)need,
               (long long)ws_bytes);
@@ -602,9 +625,10 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
   if (nb == 0 || T == 0) return SMAT_OK;
   constexpr int r = 128, p = 129;
   const int64_t rp = (int64_t)r * p;
+  const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, kFeatK);
+  C = scan_chunk(dtype, nb, T, C, r, p);
   const int nc = (T + C - 1) / C;
   const int K = scan_group_chunks(nb, nc, r, p, kFeatK);
-  const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, kFeatK);
   if (ws_bytes < need) {
     set_error("smat_forward_fused: causal-pass workspace of %lld bytes needed, %lld given",
               (long long)need, (long long)ws_bytes);

@@ -477,6 +477,22 @@ def _check_forward(spec, Phi, Psi, Vb, *, dt, g=None, label=""):
     return out
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nb,T,n,hd", [(64, 600, 256, 16), (31, 1000, 512, 16), (63, 130, 128, 64),
+                                       (128, 256, 128, 64), (1, 127, 0, 64), (2, 4096, 2048, 64)])
+def test_causal_scan_small_batches(dt, nb, T, n, hd):
+    """The causal pass at chunk 128 on both sides of the line under which it runs
+    halved chunks (fewer than 256 of them; 31 x 8 halves once, 64 x 5 not at all),
+    short last chunks included, against fp64 (scores rounded once in 16 bits)."""
+    _say("causal scan small batches", dt, nb, T, n, hd)
+    Phi, Psi, Vb = _feats(nb, T, hd, dt, seed=71)
+    Vp = torch.zeros(nb, T, hd + 8, dtype=dt)
+    Vp[..., :hd + 1] = Vb
+    H = K.causal_scan(Phi.to(DEV), Psi.to(DEV), Vp.to(DEV)[..., :hd + 1], n, 128, write_H=True)
+    ref = O.segmented_causal_scan(Phi.double(), Psi.double(), Vb.double(), n, chunk=128)
+    assert _rel(H, ref) < (1e-5 if dt == torch.float32 else 2.0 ** -8)
+
+
 @pytest.mark.parametrize("hd", [80, 96, 112])
 @pytest.mark.parametrize("T,n_P,n,N0,nb", [(2048, 0, 1024, 121, 3), (2048, 16, 1000, 90, 3),
                                            (9000, 64, 8000, 50, 6), (640, 0, 640, 640, 1)])
