@@ -221,8 +221,10 @@ def stage_events(events):
 
 
 def stream_of(t: torch.Tensor) -> int:
-    """hipStream_t of torch's current stream on ``t``'s device, as an integer."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """hipStream_t of torch's current stream on ``t``'s device, as an integer
+    (the handle alone: building the Stream object around it takes 1.8 us, a
+    decode step's launch 3.6)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def ptr(t) -> int:

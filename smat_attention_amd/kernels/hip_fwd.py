@@ -70,6 +70,8 @@ def _shape(who: str, name: str, t: torch.Tensor, want) -> None:
     """Raise ValueError unless ``t.shape`` equals ``want`` (``None`` entries match
     any size).  The kernels trust these sizes: a short buffer would be read past
     its end."""
+    if t.shape == want:
+        return
     got = tuple(t.shape)
     if len(got) != len(want) or any(w is not None and g != w for g, w in zip(got, want)):
         shown = tuple("*" if w is None else w for w in want)
@@ -600,15 +602,23 @@ def forward_fused(W, kind: str, Q, K, V, h, idx, deg: int, *, n: int, n_P: int, 
 def decode_step(Phi_t, Psi_t, Vb_t, S_in, S_out, U, step: int, *, out=None, o_full=None):
     """One decode step for a batch; returns fp32 ``(nb, p-1)`` and writes ``S_out``."""
     who = "decode_step"
-    _on_gpu(who, Phi_t, Psi_t, Vb_t, S_in, S_out, U)
+    if not (Phi_t.is_cuda and Psi_t.is_cuda and Vb_t.is_cuda and S_in.is_cuda
+            and S_out.is_cuda and U.is_cuda):
+        _on_gpu(who, Phi_t, Psi_t, Vb_t, S_in, S_out, U)
+    # a step is a launch of a few microseconds: the sizes are compared in place,
+    # and the helpers that word the errors are called only when one is wrong
     nb, R = Phi_t.shape
-    _shape(who, "U", U, (nb, None, R, None))
-    B, P = U.shape[1], U.shape[3]
-    _shape(who, "Psi_t", Psi_t, (nb, R))
-    _shape(who, "Vb_t", Vb_t, (nb, P))
-    _shape(who, "S_in", S_in, (nb, R, P))
-    _shape(who, "S_out", S_out, (nb, R, P))
-    _shape(who, "U", U, (nb, B, R, P))
+    sizes = U.shape
+    if len(sizes) != 4 or sizes[0] != nb or sizes[2] != R:
+        _shape(who, "U", U, (nb, None, R, None))
+    B, P = sizes[1], sizes[3]
+    state = (nb, R, P)
+    if Psi_t.shape != (nb, R) or Vb_t.shape != (nb, P) or S_in.shape != state \
+            or S_out.shape != state:
+        _shape(who, "Psi_t", Psi_t, (nb, R))
+        _shape(who, "Vb_t", Vb_t, (nb, P))
+        _shape(who, "S_in", S_in, state)
+        _shape(who, "S_out", S_out, state)
     if B < 1:
         raise ValueError(f"{who}: U has no row types")
     if S_in.data_ptr() == S_out.data_ptr():
@@ -620,12 +630,13 @@ def decode_step(Phi_t, Psi_t, Vb_t, S_in, S_out, U, step: int, *, out=None, o_fu
             _code(t, who)
         Phi_t, Psi_t, Vb_t = Phi_t.float(), Psi_t.float(), Vb_t.float()
     code = _code(Phi_t, who)
-    for t in (Phi_t, Psi_t, Vb_t):
-        if t.stride(-1) != 1:
-            raise ValueError(f"{who}: feature rows must be contiguous")
-    for t in (S_in, S_out, U):
-        if not t.is_contiguous() or t.dtype != torch.float32:
-            raise ValueError(f"{who}: S and U must be contiguous fp32")
+    (q_sb, q_s1), (k_sb, k_s1), (v_sb, v_s1) = Phi_t.stride(), Psi_t.stride(), Vb_t.stride()
+    if not q_s1 == k_s1 == v_s1 == 1:
+        raise ValueError(f"{who}: feature rows must be contiguous")
+    f32 = torch.float32
+    if not (S_in.is_contiguous() and S_out.is_contiguous() and U.is_contiguous()
+            and S_in.dtype == S_out.dtype == U.dtype == f32):
+        raise ValueError(f"{who}: S and U must be contiguous fp32")
     if out is None:
         out = torch.empty(nb, P - 1, device=Phi_t.device, dtype=torch.float32)
     elif out.shape != (nb, P - 1) or out.dtype != torch.float32 or not out.is_contiguous():
@@ -635,5 +646,5 @@ def decode_step(Phi_t, Psi_t, Vb_t, S_in, S_out, U, step: int, *, out=None, o_fu
         raise ValueError(f"{who}: o_full must be contiguous fp32 {(nb, P)}")
     call("smat_decode_step", code, Phi_t.data_ptr(), Psi_t.data_ptr(), Vb_t.data_ptr(),
          S_in.data_ptr(), S_out.data_ptr(), U.data_ptr(), out.data_ptr(), ptr(o_full), nb, B, R,
-         P, int(step), Phi_t.stride(0), Psi_t.stride(0), Vb_t.stride(0), stream_of(U))
+         P, int(step), q_sb, k_sb, v_sb, stream_of(U))
     return out
