@@ -14,8 +14,10 @@
 // reference fuses the same products in src/smat/kernels/triton_bwd.py:49-147
 // as a row-parallel dPhi kernel and a column-parallel dPsi/dVb kernel.)
 //
-// One workgroup of eight waves per (sequence, chunk).  The chunk's Phi, Psi,
-// Vb, dH, Sin and Q are staged in LDS once.  Wave w then does two passes:
+// One persistent workgroup of eight waves per CU walks the (sequence, chunk)
+// list.  The chunk's Phi, Psi, Vb, dH, Sin and Q are staged in LDS once, and
+// the next chunk's loads are in flight in registers during its products.
+// Wave w does two passes:
 //
 //   * row pass, row tile i = w (tokens 16w .. 16w+15): for every column tile
 //     s <= i it forms the 16 x 16 block of dA^T = Vb dH^T in MFMA
@@ -40,21 +42,30 @@
 // Precision: Phi, Psi and Vb are exact in the MFMA's 16-bit inputs; every
 // fp32 operand (dH, Sin, Q, A, dA) goes in as hi + lo (about 2^-17
 // relative), and a product of two fp32 operands takes hi.hi + hi.lo + lo.hi.
-// Value column 64 (the ones column) is the K = 16 tail of the contractions
-// over p and a fifth output column tile of dVb.
+// Value column 64 (the ones column) stays fp32: its rank-1 terms start the
+// accumulators of the contractions over p, and dVb's column 64 is summed
+// lane by lane from the blocks of A.
 //
-// LDS: Phi, Psi and Vb columns 0..63 as 128 rows of 128 bytes, 16-byte chunk
-// k of row t at k ^ (t & 6), which keeps both the row-wise 16-byte reads and
-// the transposing reads free of bank conflicts; Vb column 64 on its own; dH,
-// Sin and Q as fp32 rows of 68 floats (column reads by sixteen lanes of rows
-// 4 or 8 apart fall on disjoint banks).
+// LDS: columns 0..63 of every operand as 16-bit rows of 128 bytes (dH, Sin
+// and Q once as hi and once as lo), 16-byte chunk k of row t at k ^ (t & 6),
+// which keeps both the row-wise 16-byte reads and the transposing reads free
+// of bank conflicts; the columns 64 as fp32 arrays.
+//
+// Bound by HBM: 1.7 KB of operands and gradients a token, more with added
+// terms.  One workgroup a chunk, all of whose loads ended before its products
+// began, each fp32 value placed in LDS by itself, took 254 us with added
+// terms and 237 without at 96 sequences of 4096 tokens; the prefetch and the
+// row-wise staging 198 and 179; column 64 off the MFMA tails, four values a
+// split and one LDS address per operand and pass 185 and 165 (143 with the
+// passes over the tiles left out; the bytes at a copy's rate: 136 and 105).
 #include "bwd_common.hpp"
 
 namespace smat {
 
+constexpr int kBwdCUs = 256;   // one persistent workgroup per CU
+
 struct ChunkBwdArgs {
-  int nc;                       // chunks per sequence
-  int vec_dh, vec_vb;           // dH / Vb staged in 16-byte loads (see the kernel)
+  int nb, nc;                   // sequences, chunks per sequence
   int64_t q_sb, q_st, k_sb, k_st, v_sb, v_st;   // Phi, Psi, Vb (elements)
   int64_t h_sb, h_st;           // dH (floats)
   int64_t d_sb, d_st;           // dPhi and dPsi (elements of Out)
@@ -69,6 +80,53 @@ struct ChunkBwdArgs {
   int64_t add_split, add_end;
 };
 
+// One thread's share of a chunk, in flight between global memory and LDS: the
+// 16-byte pieces (row, k) = (u / 8, u % 8), u = tid + 512 i, of Phi, Psi and Vb
+// and the eight floats there of dH (i < 2) and of Sin and Q (i < 1); and one
+// value each of the columns 64: fp32 of dH (tid < 128), Sin (128 .. 191) or
+// Q (192 .. 255), and Vb's.  The fp32 rows lie at any float stride: their
+// sixteen-byte loads need only the floats' own alignment.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <typename In>
+struct ChunkBwdStage {
+  typedef typename Traits<In>::frag Frag;
+  typedef typename Traits<In>::half_frag Half;
+  Frag phi[2], psi[2], vb[2];
+  f32x4 dh[4], sn[2], qq[2];
+  float c64;
+  In v64;
+
+  __device__ __forceinline__ void load(const In* phib, const In* psib, const In* vbb,
+                                       const float* dHb, const float* Sinb, const float* Qb,
+                                       const ChunkBwdArgs& a, int tid) {
+    using namespace cb;
+    const int k = tid & 7;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int row = (tid >> 3) + 64 * u;
+      phi[u] = *reinterpret_cast<const Frag*>(phib + row * a.q_st + 8 * k);
+      psi[u] = *reinterpret_cast<const Frag*>(psib + row * a.k_st + 8 * k);
+      const In* v = vbb + row * a.v_st + 8 * k;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) vb[u][e] = v[e];   // one 16-byte load
+      const float* y = dHb + row * a.h_st + 8 * k;
+      dh[2 * u] = *reinterpret_cast<const f32x4u*>(y);
+      dh[2 * u + 1] = *reinterpret_cast<const f32x4u*>(y + 4);
+    }
+    const int o = (tid >> 3) * kP + 8 * k;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      sn[e] = *reinterpret_cast<const f32x4u*>(Sinb + o + 4 * e);
+      qq[e] = *reinterpret_cast<const f32x4u*>(Qb + o + 4 * e);
+    }
+    const int r = tid & (kR - 1);
+    const float* c = tid < 128 ? dHb + tid * a.h_st : (tid < 192 ? Sinb : Qb) + r * kP;
+    c64 = c[64];
+    v64 = vbb[(tid & (kC - 1)) * a.v_st + 64];
+  }
+};
+
 template <typename In, typename Out>
 __global__ __launch_bounds__(cb::kThreads, 1) void chunk_bwd_kernel(
     const In* __restrict__ phi, const In* __restrict__ psi, const In* __restrict__ vb,
@@ -77,369 +135,301 @@ __global__ __launch_bounds__(cb::kThreads, 1) void chunk_bwd_kernel(
   using namespace cb;
   typedef typename Traits<In>::frag Frag;
   typedef typename Traits<In>::half_frag Half;
-  __shared__ __attribute__((aligned(16))) uint4 sPhi[kC * kRowChunks];
+  // Phi's and dH's tiles end in sixteen rows of zeros: the row tile past the
+  // last one, where a pair of row tiles has no second
+  __shared__ __attribute__((aligned(16))) uint4 sPhi[(kC + 16) * kRowChunks];
   __shared__ __attribute__((aligned(16))) uint4 sPsi[kC * kRowChunks];
   __shared__ __attribute__((aligned(16))) uint4 sVb[kC * kRowChunks];
   // the fp32 operands split once into 16-bit hi and lo tiles, laid out as the
-  // 16-bit ones (columns 0..63 swizzled, column 64 on its own)
-  __shared__ __attribute__((aligned(16))) uint4 sdHh[kC * kRowChunks];
-  __shared__ __attribute__((aligned(16))) uint4 sdHl[kC * kRowChunks];
+  // 16-bit ones (columns 0..63 swizzled)
+  __shared__ __attribute__((aligned(16))) uint4 sdHh[(kC + 16) * kRowChunks];
+  __shared__ __attribute__((aligned(16))) uint4 sdHl[(kC + 16) * kRowChunks];
   __shared__ __attribute__((aligned(16))) uint4 sSinh[kR * kRowChunks];
   __shared__ __attribute__((aligned(16))) uint4 sSinl[kR * kRowChunks];
   __shared__ __attribute__((aligned(16))) uint4 sQh[kR * kRowChunks];
   __shared__ __attribute__((aligned(16))) uint4 sQl[kR * kRowChunks];
-  __shared__ In sVb64[kC], sdH64h[kC], sdH64l[kC];
-  __shared__ In sSin64h[kR], sSin64l[kR], sQ64h[kR], sQ64l[kR];
+  // columns 64, fp32
+  __shared__ __attribute__((aligned(16))) float sVb64[kC], sdH64[kC + 16], sSin64[kR], sQ64[kR];
 
-  const int c = blockIdx.x;
-  const int64_t b = blockIdx.y;
-  const int tid = threadIdx.x;
-  const int64_t t0 = (int64_t)c * kC;
-  const In* phib = phi + b * a.q_sb + t0 * a.q_st;
-  const In* psib = psi + b * a.k_sb + t0 * a.k_st;
-  const In* vbb = vb + b * a.v_sb + t0 * a.v_st;
-  const float* dHb = dH + b * a.h_sb + t0 * a.h_st;
-  const int64_t st_off = ((int64_t)b * a.nc + c) * (kR * kP);
-  const float* Sinb = Sin + st_off;
-  const float* Qb = Qs + st_off;
-
-  // ---- stage the chunk in LDS -------------------------------------------
-  // Phi and Psi rows: 64 elements, 16-byte aligned (checked on the host).
-  // Sin and Q (64 x 65 floats, contiguous) as float4s.  dH as float4s of the
-  // chunk's contiguous block when its rows are 65 floats apart (vec_dh); Vb
-  // as nine 16-byte pieces a row (columns 0..71: 64 to the swizzled rows,
-  // column 64 from the ninth) when its rows are 16-byte aligned and at least
-  // 72 elements apart (vec_vb); otherwise element-wise, consecutive threads
-  // on consecutive elements.  All loads are issued before the first LDS
-  // write.
-  constexpr int kVbN = kC * kP;                     // 8320
-  constexpr int kVbIt = (kVbN + kThreads - 1) / kThreads;   // 17
-  constexpr int kS4 = kR * kP / 4;                  // 1040 float4s of Sin / Q
-  constexpr int kS4It = (kS4 + kThreads - 1) / kThreads;    // 3
-  constexpr int kH4 = kVbN / 4;                     // 2080 float4s of dH
-  constexpr int kH4It = (kH4 + kThreads - 1) / kThreads;    // 5
-  constexpr int kV16 = kC * 9;                      // 1152 16-byte pieces of Vb
-  constexpr int kV16It = (kV16 + kThreads - 1) / kThreads;  // 3
-  uint4 rphi[2], rpsi[2];
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int e = tid + kThreads * u;              // chunk of 8 elements, < 1024
-    const int row = e >> 3, k = e & 7;
-    rphi[u] = *reinterpret_cast<const uint4*>(phib + row * a.q_st + 8 * k);
-    rpsi[u] = *reinterpret_cast<const uint4*>(psib + row * a.k_st + 8 * k);
-  }
-  float4 rsin[kS4It], rq[kS4It];
-#pragma unroll
-  for (int u = 0; u < kS4It; ++u) {
-    const int e4 = tid + kThreads * u;
-    const int ee = e4 < kS4 ? e4 : 0;
-    rsin[u] = reinterpret_cast<const float4*>(Sinb)[ee];
-    rq[u] = reinterpret_cast<const float4*>(Qb)[ee];
-  }
-  // element e of a row-major block of rows of kP floats, split hi/lo, to its
-  // place in a pair of 16-bit tiles (and their column-64 arrays)
-  auto put = [](uint4* th, uint4* tl, In* h64, In* l64, int e, In h, In l) {
-    const int row = e / kP, col = e - row * kP;
-    if (col < 64) {
-      reinterpret_cast<In*>(th + cb_slot(row, col >> 3))[col & 7] = h;
-      reinterpret_cast<In*>(tl + cb_slot(row, col >> 3))[col & 7] = l;
-    } else {
-      h64[row] = h;
-      l64[row] = l;
-    }
+  ChunkBwdStage<In> sg;
+  auto load = [&](int64_t b, int c, int tid) {
+    const int64_t t0 = (int64_t)c * kC;
+    const int64_t so = (b * a.nc + c) * (kR * kP);
+    sg.load(phi + b * a.q_sb + t0 * a.q_st, psi + b * a.k_sb + t0 * a.k_st,
+            vb + b * a.v_sb + t0 * a.v_st, dH + b * a.h_sb + t0 * a.h_st, Sin + so, Qs + so, a,
+            tid);
   };
-  auto put4 = [&](uint4* th, uint4* tl, In* h64, In* l64, int e, const float4& v) {
-    Half h, l;
-    split4<In>(f32x4{v.x, v.y, v.z, v.w}, h, l);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) put(th, tl, h64, l64, e + q, h[q], l[q]);
-  };
-  if (a.vec_dh) {
-    float4 rdh[kH4It];
-#pragma unroll
-    for (int u = 0; u < kH4It; ++u) {
-      const int e4 = tid + kThreads * u;
-      rdh[u] = reinterpret_cast<const float4*>(dHb)[e4 < kH4 ? e4 : 0];
-    }
-#pragma unroll
-    for (int u = 0; u < kH4It; ++u) {
-      const int e4 = tid + kThreads * u;
-      if (e4 < kH4) put4(sdHh, sdHl, sdH64h, sdH64l, 4 * e4, rdh[u]);
-    }
-  } else {
-    float rdh[kVbIt];
-#pragma unroll
-    for (int u = 0; u < kVbIt; ++u) {
-      const int e = tid + kThreads * u;
-      const int ee = e < kVbN ? e : 0;
-      const int row = ee / kP, col = ee - row * kP;
-      rdh[u] = dHb[row * a.h_st + col];
-    }
-#pragma unroll
-    for (int u = 0; u < kVbIt; ++u) {
-      const int e = tid + kThreads * u;
-      if (e < kVbN) {
-        In h, l;
-        split2<In>(rdh[u], h, l);
-        put(sdHh, sdHl, sdH64h, sdH64l, e, h, l);
-      }
-    }
-  }
-  if (a.vec_vb) {
-    uint4 rvb[kV16It];
-#pragma unroll
-    for (int u = 0; u < kV16It; ++u) {
-      const int q = tid + kThreads * u;
-      const int qq = q < kV16 ? q : 0;
-      const int row = qq / 9, k = qq - 9 * row;
-      rvb[u] = *reinterpret_cast<const uint4*>(vbb + row * a.v_st + 8 * k);
-    }
-#pragma unroll
-    for (int u = 0; u < kV16It; ++u) {
-      const int q = tid + kThreads * u;
-      if (q < kV16) {
-        const int row = q / 9, k = q - 9 * row;
-        if (k < 8)
-          sVb[cb_slot(row, k)] = rvb[u];
-        else
-          sVb64[row] = __builtin_bit_cast(Frag, rvb[u])[0];
-      }
-    }
-  } else {
-    In rvb[kVbIt];
-#pragma unroll
-    for (int u = 0; u < kVbIt; ++u) {
-      const int e = tid + kThreads * u;
-      const int ee = e < kVbN ? e : 0;
-      const int row = ee / kP, col = ee - row * kP;
-      rvb[u] = vbb[row * a.v_st + col];
-    }
-#pragma unroll
-    for (int u = 0; u < kVbIt; ++u) {
-      const int e = tid + kThreads * u;
-      if (e < kVbN) {
-        const int row = e / kP, col = e - row * kP;
-        if (col < 64)
-          reinterpret_cast<In*>(sVb + cb_slot(row, col >> 3))[col & 7] = rvb[u];
-        else
-          sVb64[row] = rvb[u];
-      }
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int e = tid + kThreads * u;
-    const int row = e >> 3, k = e & 7;
-    sPhi[cb_slot(row, k)] = rphi[u];
-    sPsi[cb_slot(row, k)] = rpsi[u];
-  }
-#pragma unroll
-  for (int u = 0; u < kS4It; ++u) {
-    const int e4 = tid + kThreads * u;
-    if (e4 < kS4) {
-      put4(sSinh, sSinl, sSin64h, sSin64l, 4 * e4, rsin[u]);
-      put4(sQh, sQl, sQ64h, sQ64l, 4 * e4, rq[u]);
-    }
-  }
-  __syncthreads();
-
-  const int w = __builtin_amdgcn_readfirstlane(wave_id());
-  const int lane = lane_id();
-  const int r16 = lane & 15, g = lane >> 4;
-  const Half hzero = {};
-  // the K = 16 tail over value columns 64..79: column 64 in k-slot 0 of lane
-  // group 0
-  auto tail16 = [&](const In* h64, const In* l64, int row, Half& hi, Half& lo) {
-    hi = hzero;
-    lo = hzero;
-    if (g == 0) {
-      hi[0] = h64[row];
-      lo[0] = l64[row];
-    }
-  };
-  // A operand down 8 consecutive rows row0 + 8g .. +7 of a 16-bit tile: lane
-  // (m = 16 ct + lane % 16, g), k-slot e <- column m of row row0 + 8g + e
-  auto col8 = [&](const uint4* tile, int row0, int ct) {
-    const int k = 2 * ct + ((r16 & 3) >> 1), half = r16 & 1;
-    const Half lo4 = cb_tr<In>(tile, row0 + 8 * g + (r16 >> 2), k, half);
-    const Half hi4 = cb_tr<In>(tile, row0 + 8 * g + 4 + (r16 >> 2), k, half);
-    Frag f;
+  auto split8 = [](const f32x4& x, const f32x4& y, uint4& hi, uint4& lo) {
+    Half h0, l0, h1, l1;
+    split4<In>(x, h0, l0);
+    split4<In>(y, h1, l1);
+    Frag h, l;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      f[e] = lo4[e];
-      f[4 + e] = hi4[e];
+      h[e] = h0[e];
+      h[4 + e] = h1[e];
+      l[e] = l0[e];
+      l[4 + e] = l1[e];
     }
-    return f;
+    hi = __builtin_bit_cast(uint4, h);
+    lo = __builtin_bit_cast(uint4, l);
   };
 
-  // ---- row pass: dPhi rows of tile i = w ----------------------------------
-  {
-    const int i = w;
-    const int trow = 16 * i + r16;
-    Frag dh_hi[2], dh_lo[2];
-    Half dht_hi, dht_lo;
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  // the chunks blockIdx.x, + gridDim.x, ... of the (sequence, chunk) list
+  const int step_b = (int)gridDim.x / a.nc, step_c = (int)gridDim.x - step_b * a.nc;
+  int64_t b = (int)blockIdx.x / a.nc;
+  int c = (int)blockIdx.x - (int)b * a.nc;
+  if (b < a.nb) load(b, c, threadIdx.x);
+  if (threadIdx.x < 16 * kRowChunks) {
+    const int z = kC * kRowChunks + (int)threadIdx.x;
+    sPhi[z] = sdHh[z] = sdHl[z] = make_uint4(0, 0, 0, 0);
+    if (threadIdx.x < 16) sdH64[kC + threadIdx.x] = 0.f;
+  }
+  while (b < a.nb) {
+    // opaque to the compiler, so that the LDS addresses of a whole pass are
+    // formed in it instead of held in registers across all of them
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
+    const int r16 = lane & 15, g = lane >> 4;
+    // byte offsets in a 16-bit tile of this lane's row-wise operand (row r16,
+    // chunk 4 kc + g; see cb_row) and of its transposing read (cb_tr_pair);
+    // row tile t lies 2048 t bytes on
+    int off_r[2], off_t[4];
 #pragma unroll
-    for (int kc = 0; kc < 2; ++kc) {
-      dh_hi[kc] = cb_row<In>(sdHh, i, kc, lane);
-      dh_lo[kc] = cb_row<In>(sdHl, i, kc, lane);
-    }
-    tail16(sdH64h, sdH64l, trow, dht_hi, dht_lo);
+    for (int kc = 0; kc < 2; ++kc) off_r[kc] = 16 * cb_slot(r16, 4 * kc + g);
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct)
+      off_t[ct] = 16 * cb_slot(4 * g + (r16 >> 2), 2 * ct + ((r16 & 3) >> 1)) + 8 * (r16 & 1);
+    auto row_op = [&](const uint4* tile, int t, int kc) {
+      return *reinterpret_cast<const Frag*>(reinterpret_cast<const char*>(tile) + off_r[kc] +
+                                            2048 * t);
+    };
+    auto tr_op = [&](const uint4* tile, int t0, int t1, int ct) {
+      typedef short short4v __attribute__((ext_vector_type(4)));
+      typedef __attribute__((address_space(3))) short4v* lds4;
+      const char* p = reinterpret_cast<const char*>(tile) + off_t[ct];
+      const Half x = __builtin_bit_cast(
+          Half, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (lds4)(__attribute__((address_space(3))) char*)(p + 2048 * t0)));
+      const Half y = __builtin_bit_cast(
+          Half, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (lds4)(__attribute__((address_space(3))) char*)(p + 2048 * t1)));
+      return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    // B operand hi/lo from two accumulator tiles (k-slot 4h + e <- tile h, entry e)
+    auto split_pair = [](const f32x4& x, const f32x4& y, Frag& hi, Frag& lo) {
+      Half h0, l0, h1, l1;
+      split4<In>(x, h0, l0);
+      split4<In>(y, h1, l1);
+      hi = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+      lo = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    auto four = [](const float* t, int row) { return *reinterpret_cast<const f32x4*>(t + row); };
+    // A operand down 8 consecutive rows row0 + 8g .. +7 of a 16-bit tile: lane
+    // (m = 16 ct + lane % 16, g), k-slot e <- column m of row row0 + 8g + e
+    auto col8 = [&](const uint4* tile, int row0, int ct) {
+      const int k = 2 * ct + ((r16 & 3) >> 1), half = r16 & 1;
+      const Half lo4 = cb_tr<In>(tile, row0 + 8 * g + (r16 >> 2), k, half);
+      const Half hi4 = cb_tr<In>(tile, row0 + 8 * g + 4 + (r16 >> 2), k, half);
+      Frag f;
+  #pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f[e] = lo4[e];
+        f[4 + e] = hi4[e];
+      }
+      return f;
+    };
 
-    f32x4 acc[4];
-    // dPhi^T += Sin dH^T: A = Sin rows a (k = value column), B = dH^T
+    const int64_t t0 = (int64_t)c * kC;
+    {
+      const int k = tid & 7;
+  #pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int s = cb_slot((tid >> 3) + 64 * u, k);
+        sPhi[s] = __builtin_bit_cast(uint4, sg.phi[u]);
+        sPsi[s] = __builtin_bit_cast(uint4, sg.psi[u]);
+        sVb[s] = __builtin_bit_cast(uint4, sg.vb[u]);
+        split8(sg.dh[2 * u], sg.dh[2 * u + 1], sdHh[s], sdHl[s]);
+      }
+      const int s = cb_slot(tid >> 3, k);
+      split8(sg.sn[0], sg.sn[1], sSinh[s], sSinl[s]);
+      split8(sg.qq[0], sg.qq[1], sQh[s], sQl[s]);
+      if (tid < 128) {
+        sdH64[tid] = sg.c64;
+        sVb64[tid] = to_f32(sg.v64);
+      } else if (tid < 192) {
+        sSin64[tid - 128] = sg.c64;
+      } else if (tid < 256) {
+        sQ64[tid - 192] = sg.c64;
+      }
+    }
+    __syncthreads();
+    // the added terms of this lane's token row (row 16w + r16 of the chunk in
+    // both passes): dPhi's from row add_split on, dPsi's and dVb's before it
+    const int64_t row = t0 + 16 * w + r16;
+    const bool head = row < a.add_split;
+    const float* ad1 = nullptr;
+    if (head && a.add_psi != nullptr) ad1 = a.add_psi + b * a.ak_sb + row * a.ak_st;
+    if (!head && row < a.add_end && a.add_phi != nullptr)
+      ad1 = a.add_phi + b * a.ap_sb + row * a.ap_st;
+    f32x4 add1[4], add2[4];
+    float add64 = 0.f;
 #pragma unroll
-    for (int at = 0; at < 4; ++at) {
-      f32x4 s = zero4();
-      const int arow = 16 * at + r16;
+    for (int at = 0; at < 4; ++at) add1[at] = add2[at] = zero4();
+    if (ad1 != nullptr) {
+#pragma unroll
+      for (int at = 0; at < 4; ++at)
+        add1[at] = *reinterpret_cast<const f32x4*>(ad1 + 16 * at + 4 * g);
+    }
+    if (head && a.add_vb != nullptr) {
+      const float* ad2 = a.add_vb + b * a.av_sb + row * a.av_st;
+#pragma unroll
+      for (int ct = 0; ct < 4; ++ct)
+        add2[ct] = *reinterpret_cast<const f32x4u*>(ad2 + 16 * ct + 4 * g);
+      add64 = ad2[64];
+    }
+    // the next chunk's loads, in flight during this one's products
+    int64_t nxt_b = b + step_b;
+    int nxt_c = c + step_c;
+    if (nxt_c >= a.nc) {
+      nxt_c -= a.nc;
+      ++nxt_b;
+    }
+    if (nxt_b < a.nb) load(nxt_b, nxt_c, tid);
+
+    // ---- row pass: dPhi rows of tile i = w ----------------------------------
+    {
+      const int i = w;
+      Frag dh_hi[2], dh_lo[2];
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc) {
-        const Frag hi = cb_row<In>(sSinh, at, kc, lane);
-        const Frag lo = cb_row<In>(sSinl, at, kc, lane);
-        s = mma(s, hi, dh_hi[kc]);
-        s = mma(s, hi, dh_lo[kc]);
-        s = mma(s, lo, dh_hi[kc]);
+        dh_hi[kc] = row_op(sdHh, i, kc);
+        dh_lo[kc] = row_op(sdHl, i, kc);
       }
-      Half thi, tlo;
-      tail16(sSin64h, sSin64l, arow, thi, tlo);
-      s = mma_k16(s, thi, dht_hi);
-      s = mma_k16(s, thi, dht_lo);
-      s = mma_k16(s, tlo, dht_hi);
-      acc[at] = s;
-    }
-    // dPhi^T += Psi^T dA^T over column tiles s <= i, two at a time
-    for (int sp = 0; 2 * sp <= i; ++sp) {
-      f32x4 dat[2];
+      const float dh64 = sdH64[16 * i + r16];
+
+      f32x4 acc[4];
+      // dPhi^T += Sin dH^T: A = Sin rows a (k = value column), B = dH^T
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int st = 2 * sp + h;
-        f32x4 d = zero4();
-        if (st <= i) {
-          // dA^T[s][t] = sum_c Vb[s][c] dH[t][c]: A = Vb rows s, B = dH^T
+      for (int at = 0; at < 4; ++at) {
+        f32x4 s = four(sSin64, 16 * at + 4 * g) * dh64;
+#pragma unroll
+        for (int kc = 0; kc < 2; ++kc) {
+          const Frag hi = row_op(sSinh, at, kc);
+          const Frag lo = row_op(sSinl, at, kc);
+          s = mma(s, hi, dh_hi[kc]);
+          s = mma(s, hi, dh_lo[kc]);
+          s = mma(s, lo, dh_hi[kc]);
+        }
+        acc[at] = s;
+      }
+      // dPhi^T += Psi^T dA^T over column tiles s <= i, two at a time
+      for (int sp = 0; 2 * sp <= i; ++sp) {
+        f32x4 dat[2];
+        // dA^T[s][t] = sum_c Vb[s][c] dH[t][c]: A = Vb rows s, B = dH^T
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          f32x4 d = four(sVb64, 32 * sp + 16 * h + 4 * g) * dh64;
 #pragma unroll
           for (int kc = 0; kc < 2; ++kc) {
-            const Frag vf = cb_row<In>(sVb, st, kc, lane);
+            const Frag vf = row_op(sVb, 2 * sp + h, kc);
             d = mma(d, vf, dh_hi[kc]);
             d = mma(d, vf, dh_lo[kc]);
           }
-          Half vt = hzero;
-          if (g == 0) vt[0] = sVb64[16 * st + r16];
-          d = mma_k16(d, vt, dht_hi);
-          d = mma_k16(d, vt, dht_lo);
-          if (st == i) {
-            // lane (t = r16, g) holds s = 16 st + 4g + e: keep s <= t
-#pragma unroll
-            for (int e = 0; e < 4; ++e) d[e] = 4 * g + e <= r16 ? d[e] : 0.f;
-          }
+          dat[h] = d;
         }
-        dat[h] = d;
-      }
-      Frag bh, bl;
-      cb_split_pair<In>(dat[0], dat[1], bh, bl);
-      const int st1 = 2 * sp + 1 < 8 ? 2 * sp + 1 : 2 * sp;
+        if (2 * sp + 1 >= i) {
+          // lane (t = r16, g) holds s = 16 (2 sp + h) + 4g + e: keep s <= t
+          const int t = 16 * (i - 2 * sp) + r16;
 #pragma unroll
-      for (int at = 0; at < 4; ++at) {
-        const Frag pa = cb_tr_pair<In>(sPsi, 2 * sp, st1, at, lane);
-        acc[at] = mma(acc[at], pa, bh);
-        acc[at] = mma(acc[at], pa, bl);
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dat[h][e] = 16 * h + 4 * g + e <= t ? dat[h][e] : 0.f;
+        }
+        Frag bh, bl;
+        split_pair(dat[0], dat[1], bh, bl);
+#pragma unroll
+        for (int at = 0; at < 4; ++at) {
+          const Frag pa = tr_op(sPsi, 2 * sp, 2 * sp + 1, at);
+          acc[at] = mma(acc[at], pa, bh);
+          acc[at] = mma(acc[at], pa, bl);
+        }
       }
+      // lane (t, g) holds dPhi[t][16 at + 4g + e]
+      if (!head) {
+#pragma unroll
+        for (int at = 0; at < 4; ++at) acc[at] += add1[at];
+      }
+      Out* out = dPhi + b * a.d_sb + row * a.d_st;
+  #pragma unroll
+      for (int at = 0; at < 4; ++at) store_grad4(out + 16 * at + 4 * g, acc[at]);
     }
-    // lane (t, g) holds dPhi[t][16 at + 4g + e]
-    const int64_t row = t0 + trow;
-    if (a.add_phi != nullptr && row >= a.add_split && row < a.add_end) {
-      const float* ad = a.add_phi + b * a.ap_sb + row * a.ap_st + 4 * g;
-#pragma unroll
-      for (int at = 0; at < 4; ++at) {
-        const float4 v = *reinterpret_cast<const float4*>(ad + 16 * at);
-        acc[at][0] += v.x;
-        acc[at][1] += v.y;
-        acc[at][2] += v.z;
-        acc[at][3] += v.w;
-      }
-    }
-    Out* out = dPhi + b * a.d_sb + row * a.d_st;
-#pragma unroll
-    for (int at = 0; at < 4; ++at) store_grad4(out + 16 * at + 4 * g, acc[at]);
-  }
 
-  // ---- column pass: dPsi and dVb rows of tile j = w -----------------------
-  {
-    const int j = w;
-    const int srow = 16 * j + r16;
-    Frag vf[2], pf[2];
-#pragma unroll
-    for (int kc = 0; kc < 2; ++kc) {
-      vf[kc] = cb_row<In>(sVb, j, kc, lane);
-      pf[kc] = cb_row<In>(sPsi, j, kc, lane);
-    }
-    Half vt = hzero;
-    if (g == 0) vt[0] = sVb64[srow];
-
-    f32x4 accq[4], accv[5];
-    // dPsi^T += Q Vb^T: A = Q rows a, B = Vb^T
-#pragma unroll
-    for (int at = 0; at < 4; ++at) {
-      f32x4 s = zero4();
-      const int arow = 16 * at + r16;
+    // ---- column pass: dPsi and dVb rows of tile j = w -----------------------
+    {
+      const int j = w;
+      Frag vf[2], pf[2];
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc) {
-        s = mma(s, cb_row<In>(sQh, at, kc, lane), vf[kc]);
-        s = mma(s, cb_row<In>(sQl, at, kc, lane), vf[kc]);
+        vf[kc] = row_op(sVb, j, kc);
+        pf[kc] = row_op(sPsi, j, kc);
       }
-      Half thi, tlo;
-      tail16(sQ64h, sQ64l, arow, thi, tlo);
-      s = mma_k16(s, thi, vt);
-      s = mma_k16(s, tlo, vt);
-      accq[at] = s;
-    }
-    // dVb^T += Q^T Psi^T: A = Q^T (rows = value column c, k = feature a)
+      const float vb64 = sVb64[16 * j + r16];
+
+      f32x4 accq[4], accv[4];
+      // dPsi^T += Q Vb^T: A = Q rows a, B = Vb^T
 #pragma unroll
-    for (int ct = 0; ct < 5; ++ct) {
-      f32x4 s = zero4();
-      const bool okc = 16 * ct + r16 < kP;
+      for (int at = 0; at < 4; ++at) {
+        f32x4 s = four(sQ64, 16 * at + 4 * g) * vb64;
 #pragma unroll
-      for (int ka = 0; ka < 2; ++ka) {
-        // A = Q^T: lane (c, g), k-slot e <- Q[32 ka + 8g + e][c]
-        Frag hi, lo;
-        if (ct < 4) {
-          hi = col8(sQh, 32 * ka, ct);
-          lo = col8(sQl, 32 * ka, ct);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            hi[e] = okc ? sQ64h[32 * ka + 8 * g + e] : from_f32<In>(0.f);
-            lo[e] = okc ? sQ64l[32 * ka + 8 * g + e] : from_f32<In>(0.f);
-          }
+        for (int kc = 0; kc < 2; ++kc) {
+          s = mma(s, row_op(sQh, at, kc), vf[kc]);
+          s = mma(s, row_op(sQl, at, kc), vf[kc]);
         }
-        s = mma(s, hi, pf[ka]);
-        s = mma(s, lo, pf[ka]);
+        accq[at] = s;
       }
-      accv[ct] = s;
-    }
-    // over row tiles t >= j, two at a time
-    for (int tp = 0; j + 2 * tp < 8; ++tp) {
-      const int tt0 = j + 2 * tp;
-      const int tt1 = tt0 + 1 < 8 ? tt0 + 1 : tt0;
-      const bool has1 = tt0 + 1 < 8;
-      f32x4 da[2], aa[2];
+      // dVb^T += Q^T Psi^T: A = Q^T (rows = value column c, k = feature a):
+      // lane (c, g), k-slot e <- Q[32 ka + 8g + e][c]
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int tt = h ? tt1 : tt0;
-        f32x4 d = zero4(), s = zero4();
-        if (h == 0 || has1) {
-          const int trow = 16 * tt + r16;
+      for (int ct = 0; ct < 4; ++ct) {
+        f32x4 s = zero4();
+#pragma unroll
+        for (int ka = 0; ka < 2; ++ka) {
+          s = mma(s, col8(sQh, 32 * ka, ct), pf[ka]);
+          s = mma(s, col8(sQl, 32 * ka, ct), pf[ka]);
+        }
+        accv[ct] = s;
+      }
+      // dVb's column 64, summed over this lane's features and row-tile entries
+      // and at the end over the lane groups
+      float v64 = 0.f;
+#pragma unroll
+      for (int ka = 0; ka < 2; ++ka)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 q = four(sQ64, 32 * ka + 8 * g + 4 * h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v64 += to_f32(pf[ka][4 * h + e]) * q[e];
+        }
+      // over row tiles t >= j, two at a time
+      for (int tp = 0; j + 2 * tp < 8; ++tp) {
+        const int tt = j + 2 * tp;
+        f32x4 da[2], aa[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 y = four(sdH64, 16 * (tt + h) + 4 * g);
+          f32x4 d = y * vb64, s = zero4();
           // dA[t][s] = sum_c dH[t][c] Vb[s][c]: A = dH rows t, B = Vb^T
+          // A[t][s] = sum_a Phi[t][a] Psi[s][a]
 #pragma unroll
           for (int kc = 0; kc < 2; ++kc) {
-            d = mma(d, cb_row<In>(sdHh, tt, kc, lane), vf[kc]);
-            d = mma(d, cb_row<In>(sdHl, tt, kc, lane), vf[kc]);
-            // A[t][s] = sum_a Phi[t][a] Psi[s][a]
-            s = mma(s, cb_row<In>(sPhi, tt, kc, lane), pf[kc]);
+            d = mma(d, row_op(sdHh, tt + h, kc), vf[kc]);
+            s = mma(s, row_op(sPhi, tt + h, kc), pf[kc]);
+            d = mma(d, row_op(sdHl, tt + h, kc), vf[kc]);
           }
-          Half thi, tlo;
-          tail16(sdH64h, sdH64l, trow, thi, tlo);
-          d = mma_k16(d, thi, vt);
-          d = mma_k16(d, tlo, vt);
-          if (tt == j) {
+          if (h == 0 && tp == 0) {
             // lane (s = r16, g) holds t = 16 tt + 4g + e: keep t >= s
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -448,79 +438,58 @@ __global__ __launch_bounds__(cb::kThreads, 1) void chunk_bwd_kernel(
               s[e] = keep ? s[e] : 0.f;
             }
           }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v64 += s[e] * y[e];
+          da[h] = d;
+          aa[h] = s;
         }
-        da[h] = d;
-        aa[h] = s;
-      }
-      Frag dah, dal, aah, aal;
-      cb_split_pair<In>(da[0], da[1], dah, dal);
-      cb_split_pair<In>(aa[0], aa[1], aah, aal);
-      // dPsi^T += Phi^T dA
+        Frag dah, dal, aah, aal;
+        split_pair(da[0], da[1], dah, dal);
+        split_pair(aa[0], aa[1], aah, aal);
+        // dPsi^T += Phi^T dA
 #pragma unroll
-      for (int at = 0; at < 4; ++at) {
-        const Frag pa = cb_tr_pair<In>(sPhi, tt0, tt1, at, lane);
-        accq[at] = mma(accq[at], pa, dah);
-        accq[at] = mma(accq[at], pa, dal);
-      }
-      // dVb^T += dH^T A: A operand = dH^T (rows = value column c, k = token t)
-#pragma unroll
-      for (int ct = 0; ct < 5; ++ct) {
-        // A = dH^T: lane (c, g), k-slot 4h + e <- dH[16 tile[h] + 4g + e][c]
-        Frag hi, lo;
-        if (ct < 4) {
-          hi = cb_tr_pair<In>(sdHh, tt0, tt1, ct, lane);
-          lo = cb_tr_pair<In>(sdHl, tt0, tt1, ct, lane);
-        } else {
-          const bool okc = r16 == 0;                 // column 64
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int trr = 16 * (e < 4 ? tt0 : tt1) + 4 * g + (e & 3);
-            hi[e] = okc ? sdH64h[trr] : from_f32<In>(0.f);
-            lo[e] = okc ? sdH64l[trr] : from_f32<In>(0.f);
-          }
+        for (int at = 0; at < 4; ++at) {
+          const Frag pa = tr_op(sPhi, tt, tt + 1, at);
+          accq[at] = mma(accq[at], pa, dah);
+          accq[at] = mma(accq[at], pa, dal);
         }
-        if (!has1) {
+        // dVb^T += dH^T A: A operand = dH^T (rows = value column c, k = token t)
 #pragma unroll
-          for (int e = 4; e < 8; ++e) {
-            hi[e] = from_f32<In>(0.f);
-            lo[e] = from_f32<In>(0.f);
-          }
+        for (int ct = 0; ct < 4; ++ct) {
+          const Frag hi = tr_op(sdHh, tt, tt + 1, ct);
+          const Frag lo = tr_op(sdHl, tt, tt + 1, ct);
+          accv[ct] = mma(accv[ct], hi, aah);
+          accv[ct] = mma(accv[ct], hi, aal);
+          accv[ct] = mma(accv[ct], lo, aah);
         }
-        accv[ct] = mma(accv[ct], hi, aah);
-        accv[ct] = mma(accv[ct], hi, aal);
-        accv[ct] = mma(accv[ct], lo, aah);
       }
-    }
-    // lane (s, g) holds dPsi[s][16 at + 4g + e] and dVb[s][16 ct + 4g + e]
-    const int64_t row = t0 + srow;
-    if (a.add_psi != nullptr && row < a.add_split) {
-      const float* ad = a.add_psi + b * a.ak_sb + row * a.ak_st + 4 * g;
+      v64 = cb_sum_groups(v64);
+      // lane (s, g) holds dPsi[s][16 at + 4g + e] and dVb[s][16 ct + 4g + e]
+      if (head) {
 #pragma unroll
-      for (int at = 0; at < 4; ++at) {
-        const float4 v = *reinterpret_cast<const float4*>(ad + 16 * at);
-        accq[at][0] += v.x;
-        accq[at][1] += v.y;
-        accq[at][2] += v.z;
-        accq[at][3] += v.w;
+        for (int at = 0; at < 4; ++at) {
+          accq[at] += add1[at];
+          accv[at] += add2[at];
+        }
+        v64 += add64;
       }
+      Out* op = dPsi + b * a.d_sb + row * a.d_st;
+  #pragma unroll
+      for (int at = 0; at < 4; ++at) store_grad4(op + 16 * at + 4 * g, accq[at]);
+      Out* ov = dVb + b * a.e_sb + row * a.e_st;
+#pragma unroll
+      for (int ct = 0; ct < 4; ++ct) {
+        typedef Out out4u __attribute__((ext_vector_type(4), aligned(sizeof(Out))));
+        out4u o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = from_f32<Out>(accv[ct][e]);
+        *reinterpret_cast<out4u*>(ov + 16 * ct + 4 * g) = o;
+      }
+      if (g == 0) ov[64] = from_f32<Out>(v64);
     }
-    if (a.add_vb != nullptr && row < a.add_split) {
-      const float* ad = a.add_vb + b * a.av_sb + row * a.av_st;
-#pragma unroll
-      for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) accv[ct][e] += ad[16 * ct + 4 * g + e];
-      if (g == 0) accv[4][0] += ad[64];
-    }
-    Out* op = dPsi + b * a.d_sb + row * a.d_st;
-#pragma unroll
-    for (int at = 0; at < 4; ++at) store_grad4(op + 16 * at + 4 * g, accq[at]);
-    Out* ov = dVb + b * a.e_sb + row * a.e_st;
-#pragma unroll
-    for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ov[16 * ct + 4 * g + e] = from_f32<Out>(accv[ct][e]);
-    if (g == 0) ov[64] = from_f32<Out>(accv[4][0]);
+    b = nxt_b;
+    c = nxt_c;
+    __syncthreads();                                   // this chunk's readers are done
   }
 }
 
@@ -538,8 +507,10 @@ bool chunk_bwd_ok(int dtype, int out_dtype, const void* phi, const void* psi, in
 template <typename In, typename Out>
 static void chunk_bwd_launch(const void* phi, const void* psi, const void* vb, const float* dH,
                              const float* Sin, const float* Q, void* dPhi, void* dPsi, void* dVb,
-                             const ChunkBwdArgs& a, dim3 grid, hipStream_t st) {
-  hipLaunchKernelGGL((chunk_bwd_kernel<In, Out>), grid, dim3(cb::kThreads), 0, st,
+                             const ChunkBwdArgs& a, hipStream_t st) {
+  const int64_t items = (int64_t)a.nb * a.nc;
+  const int grid = (int)(items < kBwdCUs ? items : kBwdCUs);
+  hipLaunchKernelGGL((chunk_bwd_kernel<In, Out>), dim3(grid), dim3(cb::kThreads), 0, st,
                      (const In*)phi, (const In*)psi, (const In*)vb, dH, Sin, Q, (Out*)dPhi,
                      (Out*)dPsi, (Out*)dVb, a);
 }
@@ -719,22 +690,17 @@ extern "C" int smat_chunk_backward(int dtype, int out_dtype, const void* phi, co
   if (nb == 0 || nc == 0) return SMAT_OK;
   SMAT_REQUIRE(aligned16(Sin) && aligned16(Q), SMAT_EINVAL,
                "smat_chunk_backward: Sin and Q must be 16-byte aligned");
-  // dH: the chunk's 128 rows of 65 floats are one 16-byte aligned block
-  const int vec_dh = h_st == p && h_sb % 4 == 0 && aligned16(dH);
-  // Vb: nine 16-byte pieces a row stay inside the row's stride
-  const int vec_vb = v_st >= 72 && v_st % 8 == 0 && v_sb % 8 == 0 && aligned16(vb);
-  ChunkBwdArgs a{nc,    vec_dh, vec_vb, q_sb,  q_st,    k_sb,    k_st,   v_sb,  v_st,
-                 h_sb,  h_st,   d_sb,   d_st,  e_sb,    e_st,    add_phi, add_psi, add_vb,
-                 ap_sb, ap_st,  ak_sb,  ak_st, av_sb,   av_st,   add_split, add_end};
-  const dim3 grid((unsigned)nc, (unsigned)nb);
+  ChunkBwdArgs a{nb,    nc,     q_sb,  q_st,  k_sb,    k_st,    v_sb,    v_st,
+                 h_sb,  h_st,   d_sb,  d_st,  e_sb,    e_st,    add_phi, add_psi, add_vb,
+                 ap_sb, ap_st,  ak_sb, ak_st, av_sb,   av_st,   add_split, add_end};
   hipStream_t st = (hipStream_t)stream;
   const bool f32 = out_dtype == SMAT_F32;
   if (dtype == SMAT_BF16)
     (f32 ? chunk_bwd_launch<bf16, float> : chunk_bwd_launch<bf16, bf16>)(
-        phi, psi, vb, dH, Sin, Q, dPhi, dPsi, dVb, a, grid, st);
+        phi, psi, vb, dH, Sin, Q, dPhi, dPsi, dVb, a, st);
   else
     (f32 ? chunk_bwd_launch<f16, float> : chunk_bwd_launch<f16, f16>)(
-        phi, psi, vb, dH, Sin, Q, dPhi, dPsi, dVb, a, grid, st);
+        phi, psi, vb, dH, Sin, Q, dPhi, dPsi, dVb, a, st);
   return launch_status("smat_chunk_backward");
 }
 

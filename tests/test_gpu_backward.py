@@ -425,6 +425,51 @@ def test_fused_chunk_backward(T, n):
         assert a.dtype == bf and torch.equal(a, b.to(bf)), name
 
 
+@pytest.mark.parametrize("nb,nc,pad,split", [(1, 1, 0, 0), (5, 77, 0, 77 * 128), (3, 129, 7, 4130),
+                                             (257, 2, 3, 100)])
+def test_chunk_backward_walks_every_chunk(nb, nc, pad, split):
+    """smat_chunk_backward at one chunk, at lists of chunks that do not divide by
+    the 256 workgroups that walk them, with rows of Vb and dH at odd strides and the
+    added terms split inside a row tile: sampled sequences against fp64 products
+    of the same values, within 2e-5 of the largest entry (three or four operands
+    split hi/lo, about 2^-17 relative each)."""
+    from smat_attention_amd.kernels.hip_fwd import call, stream_of
+    r, p, C = 64, 65, 128
+    T = nc * C
+    gen = torch.Generator().manual_seed(94)
+    bf = torch.bfloat16
+    Ph = (torch.rand(nb, T, r, generator=gen) + 0.1).to(bf)
+    Ps = (torch.rand(nb, T, r, generator=gen) + 0.1).to(bf)
+    Vv = torch.randn(nb, T, p + pad, generator=gen).to(bf)[..., :p]
+    dH = torch.randn(nb, T, p + pad, generator=gen)[..., :p]
+    S = torch.randn(nb, nc, r, p, generator=gen)
+    Q = torch.randn(nb, nc, r, p, generator=gen)
+    aP, aS = torch.randn(nb, T, r, generator=gen), torch.randn(nb, T, r, generator=gen)
+    aV = torch.randn(nb, T, p, generator=gen)
+    x = [t.to(DEV) for t in (Ph, Ps, Vv, dH, S, Q, aP, aS, aV)]
+    x[2] = torch.empty(nb, T, p + pad, device=DEV, dtype=bf)[..., :p].copy_(x[2])
+    x[3] = torch.empty(nb, T, p + pad, device=DEV)[..., :p].copy_(x[3])
+    g = [torch.full((nb, T, w), float("nan"), device=DEV) for w in (r, r, p)]
+    st = [v for t in x[:4] + [g[0], g[2]] for v in (t.stride(0), t.stride(1))]
+    call("smat_chunk_backward", 0, 2, *(t.data_ptr() for t in x[:6]), *(t.data_ptr() for t in g),
+         nb, nc, r, p, C, *st, *(t.data_ptr() for t in x[6:]), T * r, r, T * r, r, T * p, p, split,
+         T, stream_of(g[0]))
+    for i in sorted({0, nb // 2, nb - 1}):
+        ph, ps, v, y = (t[i].double().view(nc, C, -1) for t in (Ph, Ps, Vv, dH))
+        s, q = S[i].double(), Q[i].double()
+        A = torch.tril(ph @ ps.transpose(1, 2))
+        dA = torch.tril(y @ v.transpose(1, 2))
+        ref = [dA @ ps + y @ s.transpose(1, 2), dA.transpose(1, 2) @ ph + v @ q.transpose(1, 2),
+               A.transpose(1, 2) @ y + ps @ q]
+        ref = [t.reshape(T, -1) for t in ref]
+        ref[0][split:] += aP[i, split:].double()
+        ref[1][:split] += aS[i, :split].double()
+        ref[2][:split] += aV[i, :split].double()
+        for name, a, b in zip(("dPhi", "dPsi", "dVb"), g, ref):
+            err = (a[i].cpu().double() - b).abs().max() / b.abs().max()
+            assert err < 2e-5, (name, i, err)
+
+
 @pytest.mark.parametrize("vb_pad", [False, True])
 def test_chunk_state_gradients(vb_pad):
     """smat_chunk_dstates: Dr_c = Phi_c^T dH_c for every (sequence, chunk), bf16
