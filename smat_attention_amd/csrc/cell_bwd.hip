@@ -18,11 +18,15 @@
 // staged in LDS once.  Four workgroups share a CU (registers capped at 128
 // a lane): their waves spend most of their time waiting on the gathers, and
 // a fourth workgroup hides more of it (the read kernel ran 430 us at three,
-// 367 us at four at C4 d = 3).  The products against the table run on fp32 MFMA
-// (v_mfma_f32_16x16x4_f32; frag element j holds k = 4j + g): their sums over
+// 367 us at four at C4 d = 3).  Rows are gathered eight values a load and read
+// back from LDS four at a time, the next step's entry ids a step ahead: at 96
+// sequences of 4096 tokens, d = 2, the read takes 87 us and the pool 92 (140
+// and 107 with single values).  The products against the table run on fp32 MFMA
+// (v_mfma_f32_16x16x4_f32; frag element j holds column 32 kc + 8g + j): their sums over
 // value columns cancel the normaliser column against the values, which a
 // hi/lo 16-bit split would not resolve.  dF, a sum over tokens per column,
-// runs on 16-bit MFMA with dy split hi/lo, like the pool.
+// runs on 16-bit MFMA with dy split hi/lo, like the pool; its column 64, and
+// dVb's, are fp32 sums by the threads that gather.
 #include "bwd_common.hpp"
 
 namespace smat {
@@ -41,7 +45,7 @@ constexpr int kStep = 32;                 // entries a step (read backward)
 // Phi . v over the lane groups and, through LDS, the waves.  The dF Gram over
 // the step's pair-0 entries follows (A = Phi^T by transposing reads, B = dy
 // columns split hi/lo, zero for other pairs): wave w owns value-column tile
-// w, wave 0 also tile 4 (column 64).
+// w.
 // ---------------------------------------------------------------------------
 template <typename In, typename Out>
 __global__ __launch_bounds__(cw::kThreads, 4) void cell_read_bwd_kernel(
@@ -67,7 +71,11 @@ __global__ __launch_bounds__(cw::kThreads, 4) void cell_read_bwd_kernel(
   const In* phb = phr + b * q_sb;
   const float* dYb = dY + b * y_sb;
   CbGather<In, float> ga;
-  if (beg < end) ga.load(ent, beg, beg, end, L, phb, q_st, dYb, y_st, tid);
+  if (beg < end) {
+    ga.peek(ent, beg, beg, end, tid);
+    ga.load(beg, end, L, phb, q_st, dYb, y_st, tid);
+    ga.peek(ent, beg + cw::kStep, beg, end, tid);
+  }
   cb_stage_rp(sF, F + b * f_sb + (int64_t)x * cw::kRP);
   __syncthreads();
 
@@ -77,17 +85,19 @@ __global__ __launch_bounds__(cw::kThreads, 4) void cell_read_bwd_kernel(
 #pragma unroll
   for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) fa[kc][j] = sF[(16 * w + r16) * kS + 32 * kc + 4 * j + g];
-  const float fat = g == 0 ? sF[(16 * w + r16) * kS + 64] : 0.f;
+    for (int j = 0; j < 8; ++j) fa[kc][j] = sF[(16 * w + r16) * kS + 32 * kc + 8 * g + j];
+  f32x4 ft;                                          // column 64 of rows 16w + 4g + i
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ft[i] = sF[(16 * w + 4 * g + i) * kS + 64];
 
   Out* dPb = dPhi + b * d_sb;
   float* dwb = dw + b * w_sb;
-  f32x4 acc[4], acc4[4];
+  f32x4 acc[4];
+  float c64[8];
 #pragma unroll
-  for (int at = 0; at < 4; ++at) {
-    acc[at] = zero4();
-    acc4[at] = zero4();
-  }
+  for (int at = 0; at < 4; ++at) acc[at] = zero4();
+#pragma unroll
+  for (int e = 0; e < 8; ++e) c64[e] = 0.f;
   for (int64_t s0 = beg; s0 < end; s0 += cw::kStep) {
     const int par = (int)(((s0 - beg) / cw::kStep) & 1);
     float (*sDot)[cw::kStep] = sDotB[par];
@@ -95,34 +105,35 @@ __global__ __launch_bounds__(cw::kThreads, 4) void cell_read_bwd_kernel(
     int* sPair = sPairB[par];
     {
       const int slot = tid >> 3, sub = tid & 7;
-      sPh[cb_slot(slot, sub)] = ga.ok ? ga.r64 : make_uint4(0, 0, 0, 0);
+      if (s0 + cw::kStep > end) ga.mask();
+      sPh[cb_slot(slot, sub)] = __builtin_bit_cast(uint4, ga.r64);
+      f32x4* y = reinterpret_cast<f32x4*>(sY + slot * kS + 8 * sub);
+      y[0] = __builtin_shufflevector(ga.r65, ga.r65, 0, 1, 2, 3);
+      y[1] = __builtin_shufflevector(ga.r65, ga.r65, 4, 5, 6, 7);
+      const float y64 = ga.pair == 0 ? ga.c65 : 0.f;
 #pragma unroll
-      for (int u = 0; u < CbGather<In, float>::kU; ++u) {
-        const int col = sub + 8 * u;
-        if (col < kP) sY[slot * kS + col] = ga.ok ? ga.r65[u] : 0.f;
-      }
+      for (int e = 0; e < 8; ++e) c64[e] += to_f32(ga.r64[e]) * y64;
       if (sub == 0) {
+        sY[slot * kS + 64] = ga.c65;
         sTok[slot] = ga.ok ? ga.tok : -1;
         sPair[slot] = ga.pair;
       }
     }
     __syncthreads();
-    if (s0 + cw::kStep < end) ga.load(ent, s0 + cw::kStep, beg, end, L, phb, q_st, dYb, y_st, tid);
+    if (s0 + cw::kStep < end) {
+      ga.load(s0 + cw::kStep, end, L, phb, q_st, dYb, y_st, tid);
+      ga.peek(ent, s0 + 2 * cw::kStep, beg, end, tid);
+    }
     const bool has0 = sPair[0] == 0;                 // uniform: entry 0 of the step is valid
 
     // v = F dy for the two 16-entry tiles; dPhi (pair 0) and Phi . v
 #pragma unroll
     for (int et = 0; et < 2; ++et) {
       const int es = 16 * et + r16;
-      f32x4 v = zero4();
+      f32x4 v = ft * sY[es * kS + 64];
 #pragma unroll
-      for (int kc = 0; kc < 2; ++kc) {
-        f32x8 yb;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) yb[j] = sY[es * kS + 32 * kc + 4 * j + g];
-        v = mma(v, fa[kc], yb);
-      }
-      v = __builtin_amdgcn_mfma_f32_16x16x4f32(fat, g == 0 ? sY[es * kS + 64] : 0.f, v, 0, 0, 0);
+      for (int kc = 0; kc < 2; ++kc)
+        v = mma(v, fa[kc], CbRow8<float>::load(sY + es * kS + 32 * kc + 8 * g));
       // lane (es, g) holds v[16w + 4g + i]; Phi of the entry at the same columns
       const Half ph = *reinterpret_cast<const Half*>(
           reinterpret_cast<const char*>(sPh + cb_slot(es, 2 * w + (g >> 1))) + 8 * (g & 1));
@@ -136,43 +147,29 @@ __global__ __launch_bounds__(cw::kThreads, 4) void cell_read_bwd_kernel(
     }
 
     // dF += Phi^T dy over the pair-0 entries of the step
-    auto bfrag = [&](int ct, Frag& hi, Frag& lo) {
-      const int col = 16 * ct + r16;
-      const bool okc = col < kP;
-      const int cc = okc ? col : 0;
-#pragma unroll
-      for (int e8 = 0; e8 < 8; ++e8) {
-        const int es = 8 * g + e8;
-        const bool use = okc && sTok[es] >= 0 && sPair[es] == 0;
-        const float v = use ? sY[es * kS + cc] : 0.f;
-        In hh, ll;
-        split2<In>(v, hh, ll);
-        hi[e8] = hh;
-        lo[e8] = ll;
-      }
-    };
     if (has0) {                                      // steps past the pair-0 entries add nothing
+      const uint32_t use =
+          (uint32_t)__ballot(sTok[lane & 31] >= 0 && sPair[lane & 31] == 0) >> (8 * g);
       Frag bh, bl;
-      bfrag(w, bh, bl);
 #pragma unroll
-      for (int at = 0; at < 4; ++at) {
-        const int k = 2 * at + ((r16 & 3) >> 1), half = r16 & 1;
-        const Half lo4 = cb_tr<In>(sPh, 8 * g + (r16 >> 2), k, half);
-        const Half hi4 = cb_tr<In>(sPh, 8 * g + 4 + (r16 >> 2), k, half);
-        Frag pa;
+      for (int h = 0; h < 2; ++h) {
+        f32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          v[i] = (use >> (4 * h + i)) & 1 ? sY[(8 * g + 4 * h + i) * kS + 16 * w + r16] : 0.f;
+        Half hh, ll;
+        split4<In>(v, hh, ll);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          pa[i] = lo4[i];
-          pa[4 + i] = hi4[i];
+          bh[4 * h + i] = hh[i];
+          bl[4 * h + i] = ll[i];
         }
+      }
+#pragma unroll
+      for (int at = 0; at < 4; ++at) {
+        const Frag pa = cb_col32<In>(sPh, at, lane);
         acc[at] = mma(acc[at], pa, bh);
         acc[at] = mma(acc[at], pa, bl);
-        if (w == 0) {
-          Frag b4h, b4l;
-          bfrag(4, b4h, b4l);
-          acc4[at] = mma(acc4[at], pa, b4h);
-          acc4[at] = mma(acc4[at], pa, b4l);
-        }
       }
     }
     __syncthreads();                                 // sDot complete; LDS free for the next step
@@ -186,19 +183,14 @@ __global__ __launch_bounds__(cw::kThreads, 4) void cell_read_bwd_kernel(
   for (int at = 0; at < 4; ++at)
 #pragma unroll
     for (int i = 0; i < 4; ++i) out[(16 * at + 4 * g + i) * kP + 16 * w + r16] = acc[at][i];
-  if (w == 0 && r16 == 0) {
-#pragma unroll
-    for (int at = 0; at < 4; ++at)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) out[(16 * at + 4 * g + i) * kP + 64] = acc4[at][i];
-  }
+  cb_store_col64(c64, sY, out);
 }
 
 // ---------------------------------------------------------------------------
 // Pool backward.  dF[x] staged once; per step of 32 entries, their Psi and Vb
 // rows are staged as fp32 rows of kS (LDS).  Wave w forms feature tile w of
 // v^T = dF Vb^T (A = dF rows) and value-column tile w of dVb^T = dF^T Psi^T
-// (A = dF columns; wave 0 also column 64) for two 16-entry tiles, stores dPsi
+// (A = dF columns) for two 16-entry tiles, stores dPsi
 // and dVb for pair-0 entries and Psi . v for every entry.
 // ---------------------------------------------------------------------------
 template <typename In, typename Out>
@@ -223,7 +215,9 @@ __global__ __launch_bounds__(cw::kThreads, 4) void cell_pool_bwd_kernel(
   const In* psib = psi + b * k_sb;
   const In* vbb = vb + b * v_sb;
   CbGather<In, In> ga;
-  ga.load(ent, beg, beg, end, L, psib, k_st, vbb, v_st, tid);
+  ga.peek(ent, beg, beg, end, tid);
+  ga.load(beg, end, L, psib, k_st, vbb, v_st, tid);
+  ga.peek(ent, beg + cw::kStep, beg, end, tid);
   cb_stage_rp(sF, dF + b * f_sb + (int64_t)x * cw::kRP);
   __syncthreads();
 
@@ -236,10 +230,12 @@ __global__ __launch_bounds__(cw::kThreads, 4) void cell_pool_bwd_kernel(
   for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      fr[kc][j] = sF[(16 * w + r16) * kS + 32 * kc + 4 * j + g];
-      fc[kc][j] = sF[(32 * kc + 4 * j + g) * kS + 16 * w + r16];
+      fr[kc][j] = sF[(16 * w + r16) * kS + 32 * kc + 8 * g + j];
+      fc[kc][j] = sF[(32 * kc + 8 * g + j) * kS + 16 * w + r16];
     }
-  const float frt = g == 0 ? sF[(16 * w + r16) * kS + 64] : 0.f;
+  f32x4 ft;                                          // column 64 of rows 16w + 4g + i
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ft[i] = sF[(16 * w + 4 * g + i) * kS + 64];
 
   Out* dPb = dPsi + b * d_sb;
   Out* dVbb = dVb + b * e_sb;
@@ -251,39 +247,54 @@ __global__ __launch_bounds__(cw::kThreads, 4) void cell_pool_bwd_kernel(
     int* sPair = sPairB[par];
     {
       const int slot = tid >> 3, sub = tid & 7;
-      const typename Traits<In>::frag pv = __builtin_bit_cast(typename Traits<In>::frag, ga.r64);
+      if (s0 + cw::kStep > end) ga.mask();
+      f32x4* ps = reinterpret_cast<f32x4*>(sP + slot * kS + 8 * sub);
+      f32x4* vs = reinterpret_cast<f32x4*>(sV + slot * kS + 8 * sub);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) sP[slot * kS + 8 * sub + i] = ga.ok ? to_f32(pv[i]) : 0.f;
+      for (int h = 0; h < 2; ++h) {
+        f32x4 pf, vf;
 #pragma unroll
-      for (int u = 0; u < CbGather<In, In>::kU; ++u) {
-        const int col = sub + 8 * u;
-        if (col < kP) sV[slot * kS + col] = ga.ok ? to_f32(ga.r65[u]) : 0.f;
+        for (int i = 0; i < 4; ++i) {
+          pf[i] = to_f32(ga.r64[4 * h + i]);
+          vf[i] = to_f32(ga.r65[4 * h + i]);
+        }
+        ps[h] = pf;
+        vs[h] = vf;
+      }
+      const bool first = ga.ok && ga.pair == 0;
+      if (__any(first)) {
+        // column 64 of dVb: Psi . dF's column 64, over the entry's eight threads
+        float d = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) d += to_f32(ga.r64[i]) * sF[(8 * sub + i) * kS + 64];
+        d += __shfl_xor(d, 1);
+        d += __shfl_xor(d, 2);
+        d += __shfl_xor(d, 4);
+        if (first && sub == 0) dVbb[(int64_t)ga.tok * e_st + 64] = from_f32<Out>(d);
       }
       if (sub == 0) {
+        sV[slot * kS + 64] = to_f32(ga.c65);
         sTok[slot] = ga.ok ? ga.tok : -1;
         sPair[slot] = ga.pair;
       }
     }
     __syncthreads();
-    if (s0 + cw::kStep < end) ga.load(ent, s0 + cw::kStep, beg, end, L, psib, k_st, vbb, v_st, tid);
+    if (s0 + cw::kStep < end) {
+      ga.load(s0 + cw::kStep, end, L, psib, k_st, vbb, v_st, tid);
+      ga.peek(ent, s0 + 2 * cw::kStep, beg, end, tid);
+    }
     const bool has0 = sPair[0] == 0;                 // uniform: entry 0 of the step is valid
 
 #pragma unroll
     for (int et = 0; et < 2; ++et) {
       const int es = 16 * et + r16;
-      f32x4 v = zero4(), dv = zero4();
+      f32x4 v = ft * sV[es * kS + 64], dv = zero4();
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc) {
-        f32x8 vbf, psf;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          vbf[j] = sV[es * kS + 32 * kc + 4 * j + g];
-          psf[j] = sP[es * kS + 32 * kc + 4 * j + g];
-        }
-        v = mma(v, fr[kc], vbf);
-        if (has0) dv = mma(dv, fc[kc], psf);         // dVb: pair-0 entries only
+        const int o = es * kS + 32 * kc + 8 * g;
+        v = mma(v, fr[kc], CbRow8<float>::load(sV + o));
+        if (has0) dv = mma(dv, fc[kc], CbRow8<float>::load(sP + o));   // dVb: pair-0 entries only
       }
-      v = __builtin_amdgcn_mfma_f32_16x16x4f32(frt, g == 0 ? sV[es * kS + 64] : 0.f, v, 0, 0, 0);
       // lane (es, g): v[16w + 4g + i] (dPsi), dv[16w + 4g + i] (dVb columns)
       float pd = 0.f;
 #pragma unroll
@@ -294,23 +305,7 @@ __global__ __launch_bounds__(cw::kThreads, 4) void cell_pool_bwd_kernel(
       if (t >= 0 && sPair[es] == 0) {
         store_grad4(dPb + (int64_t)t * d_st + 16 * w + 4 * g, v);
         Out* ov = dVbb + (int64_t)t * e_st + 16 * w + 4 * g;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ov[i] = from_f32<Out>(dv[i]);
-      }
-      if (w == 0 && has0) {
-        // column 64 of dVb: sum_a dF[a][64] Psi[a] (lane group 0, slot 0)
-        f32x4 d4 = zero4();
-#pragma unroll
-        for (int kc = 0; kc < 2; ++kc) {
-          f32x8 a4, psf;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            a4[j] = r16 == 0 ? sF[(32 * kc + 4 * j + g) * kS + 64] : 0.f;
-            psf[j] = sP[es * kS + 32 * kc + 4 * j + g];
-          }
-          d4 = mma(d4, a4, psf);
-        }
-        if (g == 0 && t >= 0 && sPair[es] == 0) dVbb[(int64_t)t * e_st + 64] = from_f32<Out>(d4[0]);
+        cb_store4(ov, dv);
       }
     }
     __syncthreads();                                 // sDot complete; LDS free for the next step

@@ -86,8 +86,6 @@ struct ChunkBwdArgs {
 // value each of the columns 64: fp32 of dH (tid < 128), Sin (128 .. 191) or
 // Q (192 .. 255), and Vb's.  The fp32 rows lie at any float stride: their
 // sixteen-byte loads need only the floats' own alignment.
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-
 template <typename In>
 struct ChunkBwdStage {
   typedef typename Traits<In>::frag Frag;
@@ -107,9 +105,7 @@ struct ChunkBwdStage {
       const int row = (tid >> 3) + 64 * u;
       phi[u] = *reinterpret_cast<const Frag*>(phib + row * a.q_st + 8 * k);
       psi[u] = *reinterpret_cast<const Frag*>(psib + row * a.k_st + 8 * k);
-      const In* v = vbb + row * a.v_st + 8 * k;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vb[u][e] = v[e];   // one 16-byte load
+      vb[u] = cb_load8(vbb + row * a.v_st + 8 * k);
       const float* y = dHb + row * a.h_st + 8 * k;
       dh[2 * u] = *reinterpret_cast<const f32x4u*>(y);
       dh[2 * u + 1] = *reinterpret_cast<const f32x4u*>(y + 4);
@@ -159,22 +155,6 @@ __global__ __launch_bounds__(cb::kThreads, 1) void chunk_bwd_kernel(
             vb + b * a.v_sb + t0 * a.v_st, dH + b * a.h_sb + t0 * a.h_st, Sin + so, Qs + so, a,
             tid);
   };
-  auto split8 = [](const f32x4& x, const f32x4& y, uint4& hi, uint4& lo) {
-    Half h0, l0, h1, l1;
-    split4<In>(x, h0, l0);
-    split4<In>(y, h1, l1);
-    Frag h, l;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      h[e] = h0[e];
-      h[4 + e] = h1[e];
-      l[e] = l0[e];
-      l[4 + e] = l1[e];
-    }
-    hi = __builtin_bit_cast(uint4, h);
-    lo = __builtin_bit_cast(uint4, l);
-  };
-
   const int w = __builtin_amdgcn_readfirstlane(wave_id());
   // the chunks blockIdx.x, + gridDim.x, ... of the (sequence, chunk) list
   const int step_b = (int)gridDim.x / a.nc, step_c = (int)gridDim.x - step_b * a.nc;
@@ -218,14 +198,6 @@ __global__ __launch_bounds__(cb::kThreads, 1) void chunk_bwd_kernel(
                     (lds4)(__attribute__((address_space(3))) char*)(p + 2048 * t1)));
       return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
     };
-    // B operand hi/lo from two accumulator tiles (k-slot 4h + e <- tile h, entry e)
-    auto split_pair = [](const f32x4& x, const f32x4& y, Frag& hi, Frag& lo) {
-      Half h0, l0, h1, l1;
-      split4<In>(x, h0, l0);
-      split4<In>(y, h1, l1);
-      hi = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-      lo = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
-    };
     auto four = [](const float* t, int row) { return *reinterpret_cast<const f32x4*>(t + row); };
     // A operand down 8 consecutive rows row0 + 8g .. +7 of a 16-bit tile: lane
     // (m = 16 ct + lane % 16, g), k-slot e <- column m of row row0 + 8g + e
@@ -251,11 +223,11 @@ __global__ __launch_bounds__(cb::kThreads, 1) void chunk_bwd_kernel(
         sPhi[s] = __builtin_bit_cast(uint4, sg.phi[u]);
         sPsi[s] = __builtin_bit_cast(uint4, sg.psi[u]);
         sVb[s] = __builtin_bit_cast(uint4, sg.vb[u]);
-        split8(sg.dh[2 * u], sg.dh[2 * u + 1], sdHh[s], sdHl[s]);
+        cb_split8<In>(sg.dh[2 * u], sg.dh[2 * u + 1], sdHh[s], sdHl[s]);
       }
       const int s = cb_slot(tid >> 3, k);
-      split8(sg.sn[0], sg.sn[1], sSinh[s], sSinl[s]);
-      split8(sg.qq[0], sg.qq[1], sQh[s], sQl[s]);
+      cb_split8<In>(sg.sn[0], sg.sn[1], sSinh[s], sSinl[s]);
+      cb_split8<In>(sg.qq[0], sg.qq[1], sQh[s], sQl[s]);
       if (tid < 128) {
         sdH64[tid] = sg.c64;
         sVb64[tid] = to_f32(sg.v64);
@@ -349,7 +321,7 @@ __global__ __launch_bounds__(cb::kThreads, 1) void chunk_bwd_kernel(
             for (int e = 0; e < 4; ++e) dat[h][e] = 16 * h + 4 * g + e <= t ? dat[h][e] : 0.f;
         }
         Frag bh, bl;
-        split_pair(dat[0], dat[1], bh, bl);
+        cb_split_pair<In>(dat[0], dat[1], bh, bl);
 #pragma unroll
         for (int at = 0; at < 4; ++at) {
           const Frag pa = tr_op(sPsi, 2 * sp, 2 * sp + 1, at);
@@ -444,8 +416,8 @@ __global__ __launch_bounds__(cb::kThreads, 1) void chunk_bwd_kernel(
           aa[h] = s;
         }
         Frag dah, dal, aah, aal;
-        split_pair(da[0], da[1], dah, dal);
-        split_pair(aa[0], aa[1], aah, aal);
+        cb_split_pair<In>(da[0], da[1], dah, dal);
+        cb_split_pair<In>(aa[0], aa[1], aah, aal);
         // dPsi^T += Phi^T dA
 #pragma unroll
         for (int at = 0; at < 4; ++at) {
@@ -478,13 +450,7 @@ __global__ __launch_bounds__(cb::kThreads, 1) void chunk_bwd_kernel(
       for (int at = 0; at < 4; ++at) store_grad4(op + 16 * at + 4 * g, accq[at]);
       Out* ov = dVb + b * a.e_sb + row * a.e_st;
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) {
-        typedef Out out4u __attribute__((ext_vector_type(4), aligned(sizeof(Out))));
-        out4u o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = from_f32<Out>(accv[ct][e]);
-        *reinterpret_cast<out4u*>(ov + 16 * ct + 4 * g) = o;
-      }
+      for (int ct = 0; ct < 4; ++ct) cb_store4(ov + 16 * ct + 4 * g, accv[ct]);
       if (g == 0) ov[64] = from_f32<Out>(v64);
     }
     b = nxt_b;

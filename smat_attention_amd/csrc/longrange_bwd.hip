@@ -14,11 +14,16 @@
 //
 // Each launch streams one r x p fp32 matrix per item (U_h, dF_x) against the
 // few token rows of that item -- bandwidth kernels whose waves mostly wait
-// on their loads: the list gram and the pool backward cap their registers
-// so five workgroups share a CU (a few spilled values; 245 -> 232 and
-// 171 -> 163 us at C4 d = 3).  The products run on bf16
+// on their loads, so the list gram and the pool backward cap their registers
+// for five workgroups a CU, every launch has its token rows in flight while the
+// matrix is staged, and rows are read eight values at a time wherever they
+// start.  At 96 sequences of 4096 tokens, d = 3 (T_R = 2048): the query's dPhi
+// 107 -> 91 us (its 390 MB at a copy's rate: 80), the list gram 226 -> 140
+// (1 GB of rows from L2; the split of dY once per gathered row instead of by
+// every wave, and column 64 off one wave, took it from the LDS and the VALU),
+// the pool backward 164 -> 97 (420 MB: 86).  The products run on 16-bit
 // MFMA with fp32 operands split hi/lo, except the query's dPhi (fp32 MFMA, see
-// there).  The reference differentiates
+// there) and the terms of value column 64, which are fp32.  The reference differentiates
 // the query and incidence with torch and fuses the pool backward in
 // src/smat/kernels/triton_bwd.py:203-237 ("dF_x loaded once"); the
 // incidence backward there is the forward kernel over C^T (:262-276).
@@ -35,11 +40,12 @@ constexpr int kStep = 32;           // tokens per K step of the list gram
 // ---------------------------------------------------------------------------
 // dPhi[n + h + kB] += dY[n + h + kB] U_h^T, one workgroup per (h, sequence).
 // Wave w forms feature tile w of the transposed product, dPhi^T = U_h dY^T:
-// A = U_h rows (LDS, loaded once), B = dY^T from the token rows, 16 at a time;
-// lane (row, g) ends with dPhi[row][16w + 4g .. +3].
+// A = U_h rows (LDS, loaded once), B = dY^T from the token rows, 16 at a time
+// (the first sixteen in flight while U_h is staged); lane (row, g) ends with
+// dPhi[row][16w + 4g .. +3].
 //
-// This product runs on fp32 MFMA (v_mfma_f32_16x16x4_f32, k = 4j + g for
-// frag element j): its sum over value columns cancels the normaliser column
+// This product runs on fp32 MFMA (v_mfma_f32_16x16x4_f32, column 32 kc + 8g + j
+// for frag element j): its sum over value columns cancels the normaliser column
 // against the values (the quotient rule of the final division), and U_h holds
 // large pooled sums, so hi/lo 16-bit operands (~2^-16) would leave an error
 // of order 1e-3 of the result.
@@ -55,36 +61,43 @@ __global__ __launch_bounds__(lr::kThreads) void lr_dphi_kernel(
   const int64_t b = blockIdx.y;
   const int cnt = h < T_R ? (T_R - h + B - 1) / B : 0;
   if (cnt == 0) return;                              // uniform over the workgroup
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const int lane = lane_id(), r16 = lane & 15, g = lane >> 4;
+  const float* dHb = dH + b * h_sb;
+  float* dPb = dPhi + b * d_sb;
+  // this lane's row of row tile rt (a row past the end reads the first one and
+  // is not stored): columns 32 kc + 8g .. +7, and 64
+  f32x8 yb[2];
+  float yt;
+  auto load = [&](int rt) {
+    const int k = 16 * rt + r16;
+    const float* y = dHb + (n + h + (int64_t)(k < cnt ? k : 0) * B) * h_st;
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) yb[kc] = CbRow8<float>::load(y + 32 * kc + 8 * g);
+    yt = y[64];
+  };
+  load(0);
   cb_stage_rp(sU, U + b * u_sb + (int64_t)h * lr::kRP);
   __syncthreads();
 
-  const int w = __builtin_amdgcn_readfirstlane(wave_id());
-  const int lane = lane_id(), r16 = lane & 15, g = lane >> 4;
   const int arow = 16 * w + r16;
   f32x8 ua[2];
 #pragma unroll
   for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) ua[kc][j] = sU[arow * kS + 32 * kc + 4 * j + g];
-  const float ut = g == 0 ? sU[arow * kS + 64] : 0.f;   // column 64: k-slot 0 of the tail
+    for (int j = 0; j < 8; ++j) ua[kc][j] = sU[arow * kS + 32 * kc + 8 * g + j];
+  f32x4 ut;                                          // column 64 of rows 16w + 4g + i
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ut[i] = sU[(16 * w + 4 * g + i) * kS + 64];
 
-  const float* dHb = dH + b * h_sb;
-  float* dPb = dPhi + b * d_sb;
   for (int rt = 0; 16 * rt < cnt; ++rt) {
     const int k = 16 * rt + r16;
     const bool ok = k < cnt;
     const int64_t row = n + h + (int64_t)(ok ? k : 0) * B;
-    const float* y = dHb + row * h_st;
-    f32x4 acc = zero4();
+    f32x4 acc = ut * yt;
 #pragma unroll
-    for (int kc = 0; kc < 2; ++kc) {
-      f32x8 yb;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) yb[j] = ok ? y[32 * kc + 4 * j + g] : 0.f;
-      acc = mma(acc, ua[kc], yb);
-    }
-    const float yt = ok && g == 0 ? y[64] : 0.f;
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ut, yt, acc, 0, 0, 0);
+    for (int kc = 0; kc < 2; ++kc) acc = mma(acc, ua[kc], yb[kc]);
+    if (16 * (rt + 1) < cnt) load(rt + 1);
     if (ok) {
       float4* o = reinterpret_cast<float4*>(dPb + row * d_st + 16 * w + 4 * g);
       float4 cur = accumulate ? *o : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -99,12 +112,12 @@ __global__ __launch_bounds__(lr::kThreads) void lr_dphi_kernel(
 
 // ---------------------------------------------------------------------------
 // dF[x] = sum over the token list of item x of Phi_t^T dY_t, one workgroup
-// per (item, sequence): 32 tokens a step are gathered into LDS (Phi rows
-// swizzled, dY rows of kS floats; eight threads a token, the next step's
-// gather in flight during the products), then D[a][c] += Phi^T dY with
-// A = Phi^T by transposing reads (k-slot 8g + e = token slot) and B = dY
-// columns split hi/lo.  Wave w owns value-column tile w for all four feature
-// tiles; wave 0 also tile 4 (column 64).
+// per (item, sequence): 32 tokens a step are gathered into LDS as 16-bit rows
+// (Phi, and dY split hi/lo once; eight threads a token, the next step's gather
+// in flight during the products, two buffers and one barrier a step), then
+// D[a][c] += Phi^T dY with both operands by transposing reads (k-slot 8g + e =
+// token slot).  Wave w owns value-column tile w for all four feature tiles;
+// column 64 is summed in fp32 by the threads that gather.
 // ---------------------------------------------------------------------------
 template <typename In>
 __global__ __launch_bounds__(lr::kThreads, 5) void lr_dfeat_kernel(
@@ -113,9 +126,7 @@ __global__ __launch_bounds__(lr::kThreads, 5) void lr_dfeat_kernel(
     int64_t h_sb, int64_t h_st, int64_t f_sb) {
   using namespace cb;
   typedef typename Traits<In>::frag Frag;
-  typedef typename Traits<In>::half_frag Half;
-  __shared__ __attribute__((aligned(16))) uint4 sPh[lr::kStep * kRowChunks];
-  __shared__ __attribute__((aligned(16))) float sY[lr::kStep * kS];
+  __shared__ __attribute__((aligned(16))) uint4 sT[2][3][lr::kStep * kRowChunks];
   int x;
   int64_t b;
   xcd_item_seq(x, b);
@@ -126,69 +137,42 @@ __global__ __launch_bounds__(lr::kThreads, 5) void lr_dfeat_kernel(
   const int w = __builtin_amdgcn_readfirstlane(wave_id());
   const int lane = lane_id(), r16 = lane & 15, g = lane >> 4;
 
-  f32x4 acc[4], acc4[4];
+  f32x4 acc[4];
+  float c64[8];
 #pragma unroll
-  for (int at = 0; at < 4; ++at) {
-    acc[at] = zero4();
-    acc4[at] = zero4();
-  }
+  for (int at = 0; at < 4; ++at) acc[at] = zero4();
+#pragma unroll
+  for (int e = 0; e < 8; ++e) c64[e] = 0.f;
   CbGather<In, float> ga;
-  // plain token ids: an L above every id decodes each as (pair 0, token id)
-  constexpr int kNoPair = 0x7fffffff;
-  if (beg < end) ga.load(tok, beg, beg, end, kNoPair, phib, q_st, dHb, h_st, tid);
+  if (beg < end) {
+    ga.peek(tok, beg, beg, end, tid);
+    ga.load(beg, end, 0, phib, q_st, dHb, h_st, tid);
+    ga.peek(tok, beg + lr::kStep, beg, end, tid);
+  }
   for (int64_t s0 = beg; s0 < end; s0 += lr::kStep) {
-    if (s0 > beg) __syncthreads();                   // the last step's readers are done
+    uint4 (*buf)[lr::kStep * kRowChunks] = sT[((s0 - beg) / lr::kStep) & 1];
+    if (s0 + lr::kStep > end) ga.mask();
     {
-      const int slot = tid >> 3, sub = tid & 7;
-      sPh[cb_slot(slot, sub)] = ga.ok ? ga.r64 : make_uint4(0, 0, 0, 0);
+      const int s = cb_slot(tid >> 3, tid & 7);
+      buf[0][s] = __builtin_bit_cast(uint4, ga.r64);
+      cb_split8<In>(__builtin_shufflevector(ga.r65, ga.r65, 0, 1, 2, 3),
+                    __builtin_shufflevector(ga.r65, ga.r65, 4, 5, 6, 7), buf[1][s], buf[2][s]);
 #pragma unroll
-      for (int u = 0; u < CbGather<In, float>::kU; ++u) {
-        const int col = sub + 8 * u;
-        if (col < kP) sY[slot * kS + col] = ga.ok ? ga.r65[u] : 0.f;
-      }
+      for (int e = 0; e < 8; ++e) c64[e] += to_f32(ga.r64[e]) * ga.c65;
     }
+    // a wave writes the other buffer only after this barrier, which every wave
+    // reaches after its products of the step before
     __syncthreads();
-    if (s0 + lr::kStep < end)
-      ga.load(tok, s0 + lr::kStep, beg, end, kNoPair, phib, q_st, dHb, h_st, tid);
-
-    // B = dY (k = token slot 8g + e, n = column c)
-    auto bfrag = [&](int ct, Frag& hi, Frag& lo) {
-      const int col = 16 * ct + r16;
-      const bool okc = col < kP;
-      const int cc = okc ? col : 0;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = okc ? sY[(8 * g + e) * kS + cc] : 0.f;
-        In hh, ll;
-        split2<In>(v, hh, ll);
-        hi[e] = hh;
-        lo[e] = ll;
-      }
-    };
-    Frag bh, bl;
-    bfrag(w, bh, bl);
+    if (s0 + lr::kStep < end) {
+      ga.load(s0 + lr::kStep, end, 0, phib, q_st, dHb, h_st, tid);
+      ga.peek(tok, s0 + 2 * lr::kStep, beg, end, tid);
+    }
+    const Frag bh = cb_col32<In>(buf[1], w, lane), bl = cb_col32<In>(buf[2], w, lane);
 #pragma unroll
     for (int at = 0; at < 4; ++at) {
-      // A = Phi^T: lane (a = 16 at + r16, g), k-slot 4h + e = token slot
-      // 8g + 4h + e; lane 4e + q addresses slot 8g + 4h + e, columns
-      // 16 at + 4q .. +3
-      const int k = 2 * at + ((r16 & 3) >> 1), half = r16 & 1;
-      const Half lo4 = cb_tr<In>(sPh, 8 * g + (r16 >> 2), k, half);
-      const Half hi4 = cb_tr<In>(sPh, 8 * g + 4 + (r16 >> 2), k, half);
-      Frag pa;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        pa[e] = lo4[e];
-        pa[4 + e] = hi4[e];
-      }
+      const Frag pa = cb_col32<In>(buf[0], at, lane);
       acc[at] = mma(acc[at], pa, bh);
       acc[at] = mma(acc[at], pa, bl);
-      if (w == 0) {
-        Frag b4h, b4l;
-        bfrag(4, b4h, b4l);
-        acc4[at] = mma(acc4[at], pa, b4h);
-        acc4[at] = mma(acc4[at], pa, b4l);
-      }
     }
   }
   // lane (c = 16 w + r16, g) holds dF[16 at + 4g + e][c]
@@ -197,12 +181,8 @@ __global__ __launch_bounds__(lr::kThreads, 5) void lr_dfeat_kernel(
   for (int at = 0; at < 4; ++at)
 #pragma unroll
     for (int e = 0; e < 4; ++e) out[(16 * at + 4 * g + e) * kP + 16 * w + r16] = acc[at][e];
-  if (w == 0 && r16 == 0) {
-#pragma unroll
-    for (int at = 0; at < 4; ++at)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) out[(16 * at + 4 * g + e) * kP + 64] = acc4[at][e];
-  }
+  __syncthreads();
+  cb_store_col64(c64, reinterpret_cast<float*>(sT), out);
 }
 
 // ---------------------------------------------------------------------------
@@ -212,7 +192,8 @@ __global__ __launch_bounds__(lr::kThreads, 5) void lr_dfeat_kernel(
 // wave w forms
 //   dPsi^T tile w = dF_x Vb^T       (A = dF rows, B = Vb rows)
 //   dVb^T  tile w = dF_x^T Psi^T    (A = dF columns, B = Psi rows)
-// (wave 0 also column tile 4) for the tokens, 16 at a time, and adds them in.
+// for the tokens, 16 at a time, and stores them or adds them in; dVb's column
+// 64 is an fp32 sum by one wave.
 // ---------------------------------------------------------------------------
 template <typename In>
 __global__ __launch_bounds__(lr::kThreads, 5) void lr_pool_bwd_kernel(
@@ -222,7 +203,6 @@ __global__ __launch_bounds__(lr::kThreads, 5) void lr_pool_bwd_kernel(
     int64_t e_sb, int64_t e_st, int accumulate) {
   using namespace cb;
   typedef typename Traits<In>::frag Frag;
-  typedef typename Traits<In>::half_frag Half;
   __shared__ __attribute__((aligned(16))) float sF[kR * kS];
   int x;
   int64_t b;
@@ -232,77 +212,82 @@ __global__ __launch_bounds__(lr::kThreads, 5) void lr_pool_bwd_kernel(
   const int nX = n - n_P;
   const int cnt = x < N0 ? (x < nX ? (nX - x + N0 - 1) / N0 : 0) : n_P;
   if (cnt == 0) return;                              // uniform over the workgroup
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const int lane = lane_id(), r16 = lane & 15, g = lane >> 4;
+  const In* psib = psi + b * k_sb;
+  const In* vbb = vb + b * v_sb;
+  // B operands along this lane's token row of row tile rt (a row past the end
+  // reads the first one and is not stored)
+  Frag vf[2], pf[2];
+  In vt;
+  auto load = [&](int rt) {
+    const int k = 16 * rt + r16;
+    const int64_t j = start + (int64_t)(k < cnt ? k : 0) * stride;
+    const In* vrow = vbb + j * v_st;
+    const In* prow = psib + j * k_st;
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+      pf[kc] = *reinterpret_cast<const Frag*>(prow + 32 * kc + 8 * g);
+      vf[kc] = cb_load8(vrow + 32 * kc + 8 * g);
+    }
+    vt = vrow[64];
+  };
+  load(0);
   cb_stage_rp(sF, dF + b * f_sb + (int64_t)x * lr::kRP);
   __syncthreads();
 
-  const int w = __builtin_amdgcn_readfirstlane(wave_id());
-  const int lane = lane_id(), r16 = lane & 15, g = lane >> 4;
-  // dPsi: A = dF rows a = 16w + r16 (hi/lo), columns 32 kc + 8g + e and 64
+  // dPsi: A = dF rows a = 16w + r16 (hi/lo), columns 32 kc + 8g + e, and
+  // column 64 of rows 16w + 4g + i
   Frag fh[2], fl[2];
-  Half fth, ftl;
 #pragma unroll
   for (int kc = 0; kc < 2; ++kc) cb_row32<In>(sF, 16 * w + r16, kc, g, fh[kc], fl[kc]);
-  cb_tail32<In>(sF, 16 * w + r16, g, fth, ftl);
+  f32x4 ft;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ft[i] = sF[(16 * w + 4 * g + i) * kS + 64];
   // dVb: A = dF^T rows c (value column), k = feature 32 ka + 8g + e
-  auto colfrag = [&](int ct, Frag (&hi)[2], Frag (&lo)[2]) {
-    const int col = 16 * ct + r16;
-    const bool okc = col < kP;
-    const int cc = okc ? col : 0;
+  Frag ch[2], cl[2];
 #pragma unroll
-    for (int ka = 0; ka < 2; ++ka)
+  for (int ka = 0; ka < 2; ++ka)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = okc ? sF[(32 * ka + 8 * g + e) * kS + cc] : 0.f;
-        In hh, ll;
-        split2<In>(v, hh, ll);
-        hi[ka][e] = hh;
-        lo[ka][e] = ll;
+    for (int h = 0; h < 2; ++h) {
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = sF[(32 * ka + 8 * g + 4 * h + e) * kS + 16 * w + r16];
+      typename Traits<In>::half_frag hh, ll;
+      split4<In>(v, hh, ll);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        ch[ka][4 * h + e] = hh[e];
+        cl[ka][4 * h + e] = ll[e];
       }
-  };
-  Frag ch[2], cl[2], c4h[2], c4l[2];
-  colfrag(w, ch, cl);
-  if (w == 0) colfrag(4, c4h, c4l);
+    }
 
-  const In* psib = psi + b * k_sb;
-  const In* vbb = vb + b * v_sb;
   float* dPb = dPsi + b * d_sb;
   float* dVbb = dVb + b * e_sb;
   for (int rt = 0; 16 * rt < cnt; ++rt) {
     const int k = 16 * rt + r16;
     const bool ok = k < cnt;
     const int64_t j = start + (int64_t)(ok ? k : 0) * stride;
-    // B operands along this lane's token row j
-    Frag vf[2], pf[2];
-    Half vt;
-    const In* vrow = vbb + j * v_st;
-    const In* prow = psib + j * k_st;
-#pragma unroll
-    for (int kc = 0; kc < 2; ++kc) {
-      const Frag pv = *reinterpret_cast<const Frag*>(prow + 32 * kc + 8 * g);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        vf[kc][e] = ok ? vrow[32 * kc + 8 * g + e] : from_f32<In>(0.f);
-        pf[kc][e] = ok ? pv[e] : from_f32<In>(0.f);
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) vt[e] = from_f32<In>(0.f);
-    if (ok && g == 0) vt[0] = vrow[64];
-
-    f32x4 ap = zero4(), av = zero4(), av4 = zero4();
+    f32x4 ap = ft * to_f32(vt), av = zero4();
 #pragma unroll
     for (int kc = 0; kc < 2; ++kc) {
       ap = mma(ap, fh[kc], vf[kc]);
       ap = mma(ap, fl[kc], vf[kc]);
       av = mma(av, ch[kc], pf[kc]);
       av = mma(av, cl[kc], pf[kc]);
-      if (w == 0) {
-        av4 = mma(av4, c4h[kc], pf[kc]);
-        av4 = mma(av4, c4l[kc], pf[kc]);
-      }
     }
-    ap = mma_k16(ap, fth, vt);
-    ap = mma_k16(ap, ftl, vt);
+    // dVb's column 64, a sum over the features in fp32, by one wave of the four
+    const bool mine = (rt & 3) == w;
+    float v64 = 0.f;
+    if (mine) {
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          v64 += sF[(32 * kc + 8 * g + e) * kS + 64] * to_f32(pf[kc][e]);
+      v64 = cb_sum_groups(v64);
+    }
+    if (16 * (rt + 1) < cnt) load(rt + 1);
     if (ok) {
       // lane (j, g): dPsi[j][16w + 4g + e], dVb[j][16w + 4g + e] (and dVb[j][64])
       float4* o = reinterpret_cast<float4*>(dPb + j * d_st + 16 * w + 4 * g);
@@ -312,10 +297,9 @@ __global__ __launch_bounds__(lr::kThreads, 5) void lr_pool_bwd_kernel(
       cur.z += ap[2];
       cur.w += ap[3];
       *o = cur;
-      float* ov = dVbb + j * e_st + 16 * w + 4 * g;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ov[e] = (accumulate ? ov[e] : 0.f) + av[e];
-      if (w == 0 && g == 0) dVbb[j * e_st + 64] = (accumulate ? dVbb[j * e_st + 64] : 0.f) + av4[0];
+      f32x4u* ov = reinterpret_cast<f32x4u*>(dVbb + j * e_st + 16 * w + 4 * g);
+      *ov = accumulate ? *ov + av : av;
+      if (mine && g == 0) dVbb[j * e_st + 64] = (accumulate ? dVbb[j * e_st + 64] : 0.f) + v64;
     }
   }
 }

@@ -470,6 +470,122 @@ def test_chunk_backward_walks_every_chunk(nb, nc, pad, split):
             assert err < 2e-5, (name, i, err)
 
 
+@pytest.mark.parametrize("counts", [[0, 1, 31, 32, 33], [64, 65, 2, 127, 0]])
+def test_long_range_gradients_at_step_edges(counts):
+    """smat_lr_dfeat over token lists that end at and beside its 32-token steps:
+    dF against fp64 within 2e-5 of its largest entry (dY enters split hi/lo)."""
+    from smat_attention_amd.kernels.hip_fwd import call, stream_of
+    nb, T, r, p = 9, 200, 64, 65                      # a sequence past the eight of one XCD round
+    gen = torch.Generator().manual_seed(96)
+    Ph = (torch.rand(nb, T, r, generator=gen) + 0.1).to(torch.bfloat16)
+    dH = torch.randn(nb, T, p, generator=gen)
+    lists = [torch.randint(0, T, (c,), generator=gen) for c in counts]
+    tptr = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
+    tok = torch.cat(lists).int().to(DEV)
+    x, y = Ph.to(DEV), dH.to(DEV)
+    ni = len(counts)
+    dF = torch.full((nb, ni, r, p), float("nan"), device=DEV)
+    call("smat_lr_dfeat", 0, x.data_ptr(), y.data_ptr(), tptr.data_ptr(), tok.data_ptr(),
+         dF.data_ptr(), nb, ni, r, p, T * r, r, T * p, p, ni * r * p, stream_of(dF))
+    ref = torch.stack([Ph.double()[:, t].transpose(1, 2) @ dH.double()[:, t] for t in lists], 1)
+    assert (dF.cpu().double() - ref).abs().max() < 2e-5 * ref.abs().max()
+    assert (dF[:, counts.index(0)] == 0).all()
+
+
+@pytest.mark.parametrize("per", [1, 15, 16, 17, 33])
+def test_long_range_gradients_at_row_tile_edges(per):
+    """smat_lr_dphi and smat_pool_backward with ``per`` tokens (and one fewer in the
+    later half) for each row type or profile and a global channel of ``per``:
+    against fp64, within 1e-5 (dPhi: fp32 products) and 2e-5 (dPsi, dVb: dF split
+    hi/lo) of the largest entry, added to what the rows held or stored."""
+    from smat_attention_amd.kernels.hip_fwd import call, stream_of
+    nb, B, r, p = 3, 6, 64, 65
+    gen = torch.Generator().manual_seed(97)
+    T_R, n_P = B * per - B // 2, per
+    n = n_P + T_R
+    bf = torch.bfloat16
+    Ps = (torch.rand(nb, n, r, generator=gen) + 0.1).to(bf)
+    Vv = torch.randn(nb, n, p, generator=gen).to(bf)
+    dH = torch.randn(nb, n, p, generator=gen)
+    U = torch.randn(nb, B + 1, r, p, generator=gen)
+    kind = [B] * n_P + [i % B for i in range(T_R)]
+    Ut = U.double()[:, kind]                          # the matrix of every row
+    refs = [torch.einsum("btap,btp->bta", Ut, dH.double()),
+            torch.einsum("btap,btp->bta", Ut, Vv.double()),
+            torch.einsum("btap,bta->btp", Ut, Ps.double())]
+    ps, v, y, u = (t.to(DEV) for t in (Ps, Vv, dH, U))
+    for acc in (0, 1):
+        g = [torch.full((nb, n, w), 0.5 if acc else float("nan"), device=DEV) for w in (r, r, p)]
+        call("smat_lr_dphi", 0, y.data_ptr(), u.data_ptr(), g[0].data_ptr(), nb, T_R, B, n_P, r, p,
+             n * p, p, (B + 1) * r * p, n * r, r, acc, stream_of(g[0]))
+        call("smat_pool_backward", 0, ps.data_ptr(), v.data_ptr(), u.data_ptr(), g[1].data_ptr(),
+             g[2].data_ptr(), nb, B, n, n_P, r, p, n * r, r, n * p, p, (B + 1) * r * p, n * r, r,
+             n * p, p, acc, stream_of(g[1]))
+        for name, a, b, lo, tol in zip(("dPhi", "dPsi", "dVb"), g, refs, (n_P, 0, 0),
+                                       (1e-5, 2e-5, 2e-5)):
+            e = (a.cpu().double() - 0.5 * acc - b)[:, lo:].abs().max() / b.abs().max()
+            assert e < tol, (name, acc, e)
+
+
+@pytest.mark.parametrize("out_dtype", [2, 0])
+def test_cell_gradients_at_step_edges(out_dtype):
+    """smat_cell_read_backward and smat_cell_pool_backward over cells whose entry
+    lists, and the pair-0 entries at their head, end at and beside the 32-entry
+    steps (one list empty, one without pair 0): against fp64 within 2e-5 of the
+    largest entry (bf16 rows: 2^-8 more, the rounding of eight significand bits)."""
+    from smat_attention_amd.kernels.hip_fwd import call, stream_of
+    nb, L, K, r, p = 9, 160, 4, 64, 65
+    cells = [(0, 0), (1, 0), (31, 2), (32, 0), (0, 33), (20, 45), (33, 31), (2, 62)]
+    N0 = len(cells)
+    gen = torch.Generator().manual_seed(98)
+    bf = torch.bfloat16
+    X = (torch.rand(nb, L, r, generator=gen) + 0.1).to(bf)     # Phi, then Psi
+    V = torch.randn(nb, L, p, generator=gen).to(bf)
+    Y = torch.randn(nb, L, p, generator=gen)
+    F = torch.randn(nb, N0, r, p, generator=gen)
+    ent, offs, lists = [], [0], []
+    for b in range(nb):
+        t0 = torch.randperm(L, generator=gen)
+        tk = torch.randperm(L * (K - 1), generator=gen) + L
+        i = j = 0
+        for c0, ck in cells:
+            e = torch.cat([t0[i:i + c0].sort().values, tk[j:j + ck].sort().values])
+            i, j = i + c0, j + ck
+            ent.append(e)
+            offs.append(offs[-1] + len(e))
+    lists = [ent[b * N0:(b + 1) * N0] for b in range(nb)]
+    od = torch.float32 if out_dtype == 2 else bf
+    x, v, y, f = (t.to(DEV) for t in (X, V, Y, F))
+    en, of = torch.cat(ent).int().to(DEV), torch.tensor(offs).to(DEV)
+    dPhi, dPsi = (torch.zeros(nb, L, r, device=DEV, dtype=od) for _ in range(2))
+    dVb = torch.zeros(nb, L, p, device=DEV, dtype=od)
+    dF = torch.full((nb, N0, r, p), float("nan"), device=DEV)
+    dw = [torch.zeros(nb, L, K, device=DEV) for _ in range(2)]
+    call("smat_cell_read_backward", 0, out_dtype, x.data_ptr(), y.data_ptr(), f.data_ptr(),
+         en.data_ptr(), of.data_ptr(), dPhi.data_ptr(), dF.data_ptr(), dw[0].data_ptr(), nb, N0, K,
+         L, r, p, L * r, r, L * p, p, N0 * r * p, L * r, r, L * K, stream_of(dF))
+    call("smat_cell_pool_backward", 0, out_dtype, x.data_ptr(), v.data_ptr(), f.data_ptr(),
+         en.data_ptr(), of.data_ptr(), dPsi.data_ptr(), dVb.data_ptr(), dw[1].data_ptr(), nb, N0, K,
+         L, r, p, L * r, r, L * p, p, N0 * r * p, L * r, r, L * p, p, L * K, stream_of(dF))
+    R = [torch.zeros_like(t, device="cpu", dtype=torch.float64) for t in (dPhi, dF, dw[0], dPsi, dVb, dw[1])]
+    for b in range(nb):
+        for c, e in enumerate(lists[b]):
+            t, k = e % L, e // L
+            M, xt = F[b, c].double(), X[b, t].double()
+            for rows, out, w in ((Y[b, t].double(), R[0], R[2]), (V[b, t].double(), R[3], R[5])):
+                g = rows @ M.T
+                out[b, t[k == 0]] = g[k == 0]
+                w[b, t, k] = (xt * g).sum(1)
+            t0 = t[k == 0]
+            R[1][b, c] = X[b, t0].double().T @ Y[b, t0].double()
+            R[4][b, t0] = X[b, t0].double() @ M
+    for name, a, b in zip(("dPhi", "dF", "dw read", "dPsi", "dVb", "dw pool"),
+                          (dPhi, dF, dw[0], dPsi, dVb, dw[1]), R):
+        tol = 2e-5 + (2.0 ** -8 if a.dtype == bf else 0)
+        err = (a.cpu().double() - b).abs().max() / b.abs().max()
+        assert err < tol, (name, err)
+
+
 @pytest.mark.parametrize("vb_pad", [False, True])
 def test_chunk_state_gradients(vb_pad):
     """smat_chunk_dstates: Dr_c = Phi_c^T dH_c for every (sequence, chunk), bf16
