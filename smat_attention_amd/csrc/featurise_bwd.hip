@@ -15,9 +15,15 @@
 //     feeds the two-tile pairs, split hi/lo, as the B operand of
 //     dx^T = W^T g^T (A = W^T by transposing reads); lane (t, g) ends with
 //     dx[t][16 dt + 4g .. +3];
-//   * forms y for feature tile w over the tile's 64 tokens (A = x rows,
-//     B = W rows; lane (f, g) holds tokens 4g + i) and adds
-//     dW^T = x^T g (A = x^T by transposing reads) to its accumulators.
+//   * leaves g's hi and lo parts in LDS (hi over G, which only that lane
+//     reads), and after a barrier adds dW^T = x^T g for feature tile w (A = x^T
+//     and B = g by transposing reads) to its accumulators.
+//
+// Bound by VALU work per value (the map's exponential, the splits) and by the
+// latency of its passes: with y, e^y and G formed once per value instead of
+// once for dx and once for dW, and four workgroups a CU instead of two, one map
+// at 96 sequences of 4096 tokens takes 45 us (75 before; its 384 bytes a token
+// at a copy's rate: 31).
 //
 // The per-workgroup dW partials go to a buffer that a second launch sums.
 // y is fp32 from exact 16-bit products; g is split hi/lo (~2^-17) against
@@ -35,7 +41,7 @@ constexpr int kD = 64;             // d_qk = r
 }  // namespace fb
 
 template <typename In>
-__global__ __launch_bounds__(fb::kThreads) void featurise_bwd_kernel(
+__global__ __launch_bounds__(fb::kThreads, 4) void featurise_bwd_kernel(
     const In* __restrict__ x, const In* __restrict__ G, const In* __restrict__ W,
     const In* __restrict__ h, In* __restrict__ dx, float* __restrict__ dWp, In* __restrict__ dh,
     int T, int kind, int64_t ntiles, int64_t x_sb, int64_t x_st, int64_t g_sb, int64_t g_st,
@@ -45,7 +51,8 @@ __global__ __launch_bounds__(fb::kThreads) void featurise_bwd_kernel(
   typedef typename Traits<In>::half_frag Half;
   __shared__ __attribute__((aligned(16))) uint4 sW[fb::kD * kRowChunks];
   __shared__ __attribute__((aligned(16))) uint4 sX[fb::kTile * kRowChunks];
-  __shared__ __attribute__((aligned(16))) uint4 sG[fb::kTile * kRowChunks];
+  __shared__ __attribute__((aligned(16))) uint4 sG[fb::kTile * kRowChunks];   // G, then g hi
+  __shared__ __attribute__((aligned(16))) uint4 sL[fb::kTile * kRowChunks];   // g lo
   __shared__ float sH[fb::kTile];
   const int tid = threadIdx.x;
   for (int i = tid; i < fb::kD * kRowChunks; i += fb::kThreads)
@@ -108,7 +115,7 @@ __global__ __launch_bounds__(fb::kThreads) void featurise_bwd_kernel(
     {
       const int trow = 16 * w + r16;
       const float hv = sH[trow];
-      f32x4 gq[4];
+      Frag gh[2], gl[2];                             // g of feature tiles 2 fp, 2 fp + 1
       float dhs = 0.f;
 #pragma unroll
       for (int ft = 0; ft < 4; ++ft) {
@@ -117,13 +124,24 @@ __global__ __launch_bounds__(fb::kThreads) void featurise_bwd_kernel(
         for (int kd = 0; kd < 2; ++kd)
           y = mma(y, cb_row<In>(sW, ft, kd, lane), cb_row<In>(sX, w, kd, lane));
         // lane (t, g) holds y[t][16 ft + 4g + i]; G at the same features
-        const Half gv = *reinterpret_cast<const Half*>(
-            reinterpret_cast<const char*>(sG + cb_slot(trow, 2 * ft + (g >> 1))) + 8 * (g & 1));
+        const int at = 16 * cb_slot(trow, 2 * ft + (g >> 1)) + 8 * (g & 1);
+        Half* gp = reinterpret_cast<Half*>(reinterpret_cast<char*>(sG) + at);
+        const Half gv = *gp;
+        f32x4 gq;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float gi = to_f32(gv[i]);
           if (h) dhs += gi * fmap(y[i]);
-          gq[ft][i] = gi * hv * dmap(y[i]);
+          gq[i] = gi * hv * dmap(y[i]);
+        }
+        Half hi, lo;
+        split4<In>(gq, hi, lo);
+        *gp = hi;
+        *reinterpret_cast<Half*>(reinterpret_cast<char*>(sL) + at) = lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          gh[ft >> 1][4 * (ft & 1) + i] = hi[i];
+          gl[ft >> 1][4 * (ft & 1) + i] = lo[i];
         }
       }
       if (h) {
@@ -136,13 +154,11 @@ __global__ __launch_bounds__(fb::kThreads) void featurise_bwd_kernel(
       for (int dt = 0; dt < 4; ++dt) ax[dt] = zero4();
 #pragma unroll
       for (int fp = 0; fp < 2; ++fp) {
-        Frag bh, bl;
-        cb_split_pair<In>(gq[2 * fp], gq[2 * fp + 1], bh, bl);
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) {
           const Frag wa = cb_tr_pair<In>(sW, 2 * fp, 2 * fp + 1, dt, lane);
-          ax[dt] = mma(ax[dt], wa, bh);
-          ax[dt] = mma(ax[dt], wa, bl);
+          ax[dt] = mma(ax[dt], wa, gh[fp]);
+          ax[dt] = mma(ax[dt], wa, gl[fp]);
         }
       }
       if (t0 + trow < T) {
@@ -158,33 +174,16 @@ __global__ __launch_bounds__(fb::kThreads) void featurise_bwd_kernel(
     }
 
     // ---- dW for features 16w .. 16w+15 over the tile's 64 tokens -----------
-    {
-      const int frow = 16 * w + r16;
-      f32x4 gt[4];
+    __syncthreads();                                 // every wave's g written
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt) {
-        f32x4 y = zero4();
+    for (int tp = 0; tp < 2; ++tp) {
+      const Frag bh = cb_tr_pair<In>(sG, 2 * tp, 2 * tp + 1, w, lane);
+      const Frag bl = cb_tr_pair<In>(sL, 2 * tp, 2 * tp + 1, w, lane);
 #pragma unroll
-        for (int kd = 0; kd < 2; ++kd)
-          y = mma(y, cb_row<In>(sX, tt, kd, lane), cb_row<In>(sW, w, kd, lane));
-        // lane (f, g) holds y[t = 16 tt + 4g + i][f]
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int t = 16 * tt + 4 * g + i;
-          const In gv = reinterpret_cast<const In*>(sG + cb_slot(t, frow >> 3))[frow & 7];
-          gt[tt][i] = to_f32(gv) * sH[t] * dmap(y[i]);
-        }
-      }
-#pragma unroll
-      for (int tp = 0; tp < 2; ++tp) {
-        Frag bh, bl;
-        cb_split_pair<In>(gt[2 * tp], gt[2 * tp + 1], bh, bl);
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          const Frag xa = cb_tr_pair<In>(sX, 2 * tp, 2 * tp + 1, dt, lane);
-          accW[dt] = mma(accW[dt], xa, bh);
-          accW[dt] = mma(accW[dt], xa, bl);
-        }
+      for (int dt = 0; dt < 4; ++dt) {
+        const Frag xa = cb_tr_pair<In>(sX, 2 * tp, 2 * tp + 1, dt, lane);
+        accW[dt] = mma(accW[dt], xa, bh);
+        accW[dt] = mma(accW[dt], xa, bl);
       }
     }
   }
