@@ -7,14 +7,20 @@
 // dtype, elu rounded, + 1 rounded, the gate product rounded (fp32 math in
 // between, as torch does for 16-bit tensors).
 //
-// One wave computes a 16-row tile of X (Q or K) against all r features as
-// C = W X^T on MFMA (W is the A operand from LDS, rows padded by 16 bytes so
-// the sixteen feature rows a fragment reads fall in distinct banks; the X rows
-// are the B operand, loaded straight from HBM as 16-byte rows).  Each lane
-// then holds four consecutive features of one row and stores them as one
-// 8-byte (16-bit types) or 16-byte (fp32) write.  The [V, 1] rows are copied
-// by the same launch.  HBM-bound: 2 (T d_qk + T r) + T (d_v + p) elements per
-// sequence.
+// One wave computes two 16-row tiles of X (Q or K) at a time against all r
+// features as C = W X^T on MFMA (W is the A operand from LDS, rows padded by 16
+// bytes so the sixteen feature rows a fragment reads fall in distinct banks;
+// the X rows are the B operand, loaded straight from HBM as 16-byte rows).  A
+// lane then holds four consecutive features of a row in each feature tile; W's
+// rows are ordered so that two tiles give it eight, one 16-byte store (16-bit
+// types, r a multiple of 32).  The [V, 1] rows are copied by the same launch.
+//
+// HBM-bound: 2 (T d_qk + T r) + T (d_v + p) elements per sequence, so what
+// counts is bytes in flight against the number of places written at once: at 96
+// sequences of 4096 tokens, all widths 64, 79 us (the bytes at a copy's rate:
+// 63) with four workgroups a CU resident and none waiting; 85 with three of
+// them, 84 with twelve in turn, 93 with six resident; 99 with one row tile a
+// wave, 8-byte stores and W's LDS sized for 128 features.
 #include <math.h>
 
 #include "feat_map.hpp"
@@ -27,29 +33,45 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 constexpr int kMaxDqk = 128;       // d_qk
 constexpr int kMaxRank = 128;      // feature rank
+constexpr int kTiles = 2;          // 16-row tiles a wave takes at a time
+constexpr int kRows = 16 * kTiles;
+// W rows in LDS: whole 32-wide k-steps and 16 bytes, so the sixteen rows a
+// fragment reads start four banks apart
+template <typename In>
+__host__ __device__ constexpr int w_stride(int dqk) {
+  return (dqk + 31) / 32 * 32 + 16 / (int)sizeof(In);
+}
 }  // namespace ft
 
 template <typename In>
-__global__ __launch_bounds__(ft::kThreads) void featurise_kernel(
+__global__ __launch_bounds__(ft::kThreads, sizeof(In) == 2 ? 4 : 2) void featurise_kernel(
     const In* __restrict__ q, const In* __restrict__ k, const In* __restrict__ v,
     const In* __restrict__ W, const In* __restrict__ h, In* __restrict__ phi,
     In* __restrict__ psi, In* __restrict__ vb, int nb, int T, int dqk, int r, int dv, int kind,
     int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb, int64_t v_st,
-    int64_t h_sb, int64_t o_sb, int64_t o_st, int64_t vb_sb, int64_t vb_st, int64_t ntiles,
-    int vec) {
+    int64_t h_sb, int64_t o_sb, int64_t o_st, int64_t vb_sb, int64_t vb_st, int vec) {
   // vec: bit 0 = Q/K rows and W 16-byte aligned (vector loads), bit 1 = Phi/Psi
   // rows aligned to four elements (one store per lane and tile), bit 2 = V and
-  // Vb rows 16-byte aligned.
+  // Vb rows 16-byte aligned, bit 3 = Phi/Psi rows 16-byte aligned and r a
+  // multiple of 32 (16-bit types: one 16-byte store per lane and two tiles).
   using namespace ft;
   typedef typename Traits<In>::frag Frag;
   typedef typename Traits<In>::half_frag Quad;
   constexpr int kE = 16 / (int)sizeof(In);                   // elements per 16 bytes
-  constexpr int kWst = kMaxDqk + kE;                           // padded W row (elements)
-  __shared__ __attribute__((aligned(16))) In w_lds[kMaxRank * kWst];
+  const int nks = (dqk + 31) / 32;
+  const int nft = (r + 15) / 16;
+  const int wst = w_stride<In>(dqk);                           // padded W row (elements)
+  extern __shared__ __attribute__((aligned(16))) char w_raw[];
+  In* w_lds = reinterpret_cast<In*>(w_raw);
 
-  // W (r x dqk) -> LDS, zero beyond r and dqk
-  for (int i = threadIdx.x; i < kMaxRank * (kMaxDqk / kE); i += kThreads) {
-    const int f = i / (kMaxDqk / kE), c = (i - f * (kMaxDqk / kE)) * kE;
+  // W (r x dqk) -> LDS, zero beyond r and dqk.  With bit 3 of vec, feature tiles
+  // 2 j and 2 j + 1 hold the features of [32 j, 32 j + 32) in the order that
+  // leaves a lane eight consecutive ones, four in each tile.
+  const bool pair = sizeof(In) == 2 && (vec & 8);
+  const int wch = 32 * nks / kE;
+  for (int i = threadIdx.x; i < 16 * nft * wch; i += kThreads) {
+    const int m = i / wch, c = (i - m * wch) * kE;
+    const int f = pair ? (m & ~31) + 8 * ((m >> 2) & 3) + 4 * ((m >> 4) & 1) + (m & 3) : m;
     In tmp[kE];
     if ((vec & 1) && f < r && c + kE <= dqk) {
       *reinterpret_cast<uint4*>(tmp) = *reinterpret_cast<const uint4*>(W + (int64_t)f * dqk + c);
@@ -58,41 +80,59 @@ __global__ __launch_bounds__(ft::kThreads) void featurise_kernel(
       for (int e = 0; e < kE; ++e)
         tmp[e] = (f < r && c + e < dqk) ? W[(int64_t)f * dqk + c + e] : from_f32<In>(0.f);
     }
-    *reinterpret_cast<uint4*>(w_lds + f * kWst + c) = *reinterpret_cast<const uint4*>(tmp);
+    *reinterpret_cast<uint4*>(w_lds + m * wst + c) = *reinterpret_cast<const uint4*>(tmp);
   }
   __syncthreads();
 
   const int lane = lane_id();
   const int r16 = lane & 15, grp = lane >> 4;
-  const int64_t tiles_per = (int64_t)nb * ((T + 15) / 16);
-  const int nks = (dqk + 31) / 32;
-  const int nft = (r + 15) / 16;
-  const int64_t gwave = (int64_t)blockIdx.x * kWaves + wave_id();
-  const int64_t nwaves = (int64_t)gridDim.x * kWaves;
-
-  for (int64_t tile = gwave; tile < ntiles; tile += nwaves) {
-    const int which = (int)(tile / tiles_per);               // 0: Q, 1: K, 2: V
-    const int64_t rem = tile - which * tiles_per;
-    const int64_t b = rem / ((T + 15) / 16);
-    const int t0 = (int)(rem - b * ((T + 15) / 16)) * 16;
-    const int row = t0 + r16;
-    const bool live = row < T;
+  // tiles gwave, + nwaves, ... of the (Q / K / V, sequence, 32 rows) list, as
+  // a pair (which * nb + b, tile of the sequence) that each step advances
+  const int per = (T + kRows - 1) / kRows;
+  const int gwave = (int)blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(wave_id());
+  const int nwaves = (int)gridDim.x * kWaves;
+  const int step_s = nwaves / per, step_t = nwaves - step_s * per;
+  int seq = gwave / per, tile = gwave - seq * per;
+  for (; seq < 3 * nb; seq += step_s, tile += step_t) {
+    if (tile >= per) {
+      tile -= per;
+      if (++seq >= 3 * nb) break;
+    }
+    const int which = seq >= 2 * nb ? 2 : seq >= nb ? 1 : 0;  // 0: Q, 1: K, 2: V
+    const int64_t b = seq - which * nb;
+    const int t0 = tile * kRows;
     if ((which == 1 && !k) || (which == 2 && !v)) continue;   // wave-uniform
     if (which == 2) {
-      // [V, 1]: lane r16 copies row t0 + r16 in chunks of kE, four lanes per row
-      if (live) {
-        const In* src = v + b * v_sb + (int64_t)row * v_st;
-        In* dst = vb + b * vb_sb + (int64_t)row * vb_st;
-        for (int c = grp; c * kE < dv + 1; c += 4) {
-          if ((vec & 4) && (c + 1) * kE <= dv) {
-            *reinterpret_cast<uint4*>(dst + c * kE) = *reinterpret_cast<const uint4*>(src + c * kE);
-          } else {
+      // [V, 1]: four lanes a row, 16-byte pieces; a tile's loads before its stores
+      const In* src = v + b * v_sb;
+      In* dst = vb + b * vb_sb;
+      const int npc = dv / kE;
+      for (int c = lane & 3; c * kE < dv + 1; c += 4) {
+        if ((vec & 4) && c < npc) {
+          typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+          u32x4 y[kTiles];
 #pragma unroll
-            for (int e = 0; e < kE; ++e) {
-              const int col = c * kE + e;
-              if (col < dv) dst[col] = src[col];
-              else if (col == dv) dst[col] = from_f32<In>(1.f);
-            }
+          for (int u = 0; u < kTiles; ++u) {
+            const int row = t0 + 16 * u + (lane >> 2);
+            y[u] = *reinterpret_cast<const u32x4*>(src + (int64_t)(row < T ? row : t0) * v_st +
+                                                   c * kE);
+          }
+#pragma unroll
+          for (int u = 0; u < kTiles; ++u) {
+            const int row = t0 + 16 * u + (lane >> 2);
+            if (row < T) *reinterpret_cast<u32x4*>(dst + (int64_t)row * vb_st + c * kE) = y[u];
+          }
+          continue;
+        }
+#pragma unroll
+        for (int u = 0; u < kTiles; ++u) {
+          const int row = t0 + 16 * u + (lane >> 2);
+          if (row >= T) continue;
+#pragma unroll
+          for (int e = 0; e < kE; ++e) {
+            const int col = c * kE + e;
+            if (col < dv) dst[(int64_t)row * vb_st + col] = src[(int64_t)row * v_st + col];
+            else if (col == dv) dst[(int64_t)row * vb_st + col] = from_f32<In>(1.f);
           }
         }
       }
@@ -100,57 +140,87 @@ __global__ __launch_bounds__(ft::kThreads) void featurise_kernel(
     }
     const In* X = (which == 0 ? q + b * q_sb : k + b * k_sb);
     const int64_t x_st = which == 0 ? q_st : k_st;
-    // B operand: row r16 of the tile, k-slots 32 ks + 8 grp .. + 8
-    Frag xb[kMaxDqk / 32];
-    const In* xr = X + (int64_t)(live ? row : t0) * x_st;
+    // B operands: row r16 of each 16-row tile, k-slots 32 ks + 8 grp .. + 8
+    Frag xb[kTiles][kMaxDqk / 32];
+    float hv[kTiles];
 #pragma unroll
-    for (int ks = 0; ks < kMaxDqk / 32; ++ks) {
-      if (ks < nks) {
-        const int c0 = 32 * ks + 8 * grp;
-        if ((vec & 1) && c0 + 8 <= dqk) {
-          xb[ks] = *reinterpret_cast<const Frag*>(xr + c0);
-          if (!live) xb[ks] = Frag{};
-        } else {
+    for (int u = 0; u < kTiles; ++u) {
+      const int row = t0 + 16 * u + r16;
+      const bool live = row < T;
+      const In* xr = X + (int64_t)(live ? row : t0) * x_st;
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            xb[ks][e] = (live && c0 + e < dqk) ? xr[c0 + e] : from_f32<In>(0.f);
+      for (int ks = 0; ks < kMaxDqk / 32; ++ks) {
+        if (ks < nks) {
+          const int c0 = 32 * ks + 8 * grp;
+          if ((vec & 1) && c0 + 8 <= dqk) {
+            xb[u][ks] = *reinterpret_cast<const Frag*>(xr + c0);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) xb[u][ks][e] = c0 + e < dqk ? xr[c0 + e] : from_f32<In>(0.f);
+          }
         }
       }
+      hv[u] = which == 1 && h ? to_f32(h[b * h_sb + (live ? row : t0)]) : 1.f;
     }
-    float hv = 1.f;
-    if (which == 1 && h) hv = live ? to_f32(h[b * h_sb + row]) : 0.f;
-    In* O = (which == 0 ? phi : psi) + b * o_sb + (int64_t)row * o_st;
-#pragma unroll 1
-    for (int f = 0; f < nft; ++f) {
-      f32x4 acc = zero4();
+    In* O = (which == 0 ? phi : psi) + b * o_sb;
+    // the lane's four features of feature tile f, for each row tile (a row past
+    // the end computes the tile's first row and stores nothing)
+    auto features = [&](int f, Quad (&out)[kTiles]) {
+      f32x4 acc[kTiles];
+#pragma unroll
+      for (int u = 0; u < kTiles; ++u) acc[u] = zero4();
 #pragma unroll
       for (int ks = 0; ks < kMaxDqk / 32; ++ks) {
         if (ks < nks) {
           Frag wa;
-          const In* wp = w_lds + (16 * f + r16) * kWst + 32 * ks + 8 * grp;
+          const In* wp = w_lds + (16 * f + r16) * wst + 32 * ks + 8 * grp;
 #pragma unroll
           for (int e = 0; e < 8; ++e) wa[e] = wp[e];
-          acc = mma(acc, wa, xb[ks]);
+#pragma unroll
+          for (int u = 0; u < kTiles; ++u) acc[u] = mma(acc[u], wa, xb[u][ks]);
         }
       }
-      if (live) {
-        const int c0 = 16 * f + 4 * grp;
-        Quad outv;
+#pragma unroll
+      for (int u = 0; u < kTiles; ++u)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          float y = feature_map<In>(acc[i], kind);
-          if (which == 1 && h) y = to_f32(from_f32<In>(y * hv));
-          outv[i] = from_f32<In>(y);
+          float y = feature_map<In>(acc[u][i], kind);
+          if (which == 1 && h) y = to_f32(from_f32<In>(y * hv[u]));
+          out[u][i] = from_f32<In>(y);
         }
-        if ((vec & 2) && c0 + 3 < r) {
-          *reinterpret_cast<Quad*>(O + c0) = outv;
-        } else if (c0 + 3 < r) {
+    };
+    if (pair) {
+#pragma unroll 1
+      for (int f = 0; f < nft; f += 2) {
+        Quad a[kTiles], c[kTiles];
+        features(f, a);
+        features(f + 1, c);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) O[c0 + i] = outv[i];
+        for (int u = 0; u < kTiles; ++u) {
+          const int row = t0 + 16 * u + r16;
+          if (row < T)
+            *reinterpret_cast<Frag*>(O + (int64_t)row * o_st + 16 * f + 8 * grp) =
+                __builtin_shufflevector(a[u], c[u], 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+      }
+      continue;
+    }
+#pragma unroll 1
+    for (int f = 0; f < nft; ++f) {
+      Quad out[kTiles];
+      features(f, out);
+      const int c0 = 16 * f + 4 * grp;
+#pragma unroll
+      for (int u = 0; u < kTiles; ++u) {
+        const int row = t0 + 16 * u + r16;
+        if (row >= T) continue;
+        In* o = O + (int64_t)row * o_st + c0;
+        if ((vec & 2) && c0 + 3 < r) {
+          *reinterpret_cast<Quad*>(o) = out[u];
         } else {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (c0 + i < r) O[c0 + i] = outv[i];
+            if (c0 + i < r) o[i] = out[u][i];
         }
       }
     }
@@ -181,7 +251,7 @@ extern "C" int smat_featurise(int dtype, const void* q, const void* k, const voi
                    o_st >= r,
                SMAT_EINVAL, "smat_featurise: row stride too short");
   if (nb == 0 || T == 0) return SMAT_OK;
-  const int64_t ntiles = 3 * (int64_t)nb * ((T + 15) / 16);
+  const int64_t ntiles = 3 * (int64_t)nb * ((T + ft::kRows - 1) / ft::kRows);
   const int64_t e16 = 16 / elem_bytes(dtype);
   if (!k) { k = q; k_sb = q_sb; k_st = q_st; psi = phi; }      // alignment checks only
   if (!v) { v = q; vb = phi; v_st = d_v; vb_st = d_v + 1; v_sb = vb_sb = 0; }
@@ -192,20 +262,23 @@ extern "C" int smat_featurise(int dtype, const void* q, const void* k, const voi
                   ((((uintptr_t)phi | (uintptr_t)psi) % (4 * elem_bytes(dtype)) == 0 &&
                     o_st % 4 == 0 && o_sb % 4 == 0) ? 2 : 0) |
                   ((aligned16(v) && aligned16(vb) && v_st % e16 == 0 && v_sb % e16 == 0 &&
-                    vb_st % e16 == 0 && vb_sb % e16 == 0) ? 4 : 0);
+                    vb_st % e16 == 0 && vb_sb % e16 == 0) ? 4 : 0) |
+                  ((aligned16(phi) && aligned16(psi) && o_st % 8 == 0 && o_sb % 8 == 0 &&
+                    r % 32 == 0) ? 8 : 0);
   int dev = 0, ncu = 256;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   const int64_t want = (ntiles + ft::kWaves - 1) / ft::kWaves;
-  const unsigned grid = (unsigned)std::min<int64_t>(want, (int64_t)ncu * 8);
+  const unsigned grid = (unsigned)std::min<int64_t>(want, (int64_t)ncu * 4);
   hipStream_t st = (hipStream_t)stream;
   const void* kk = have_k ? k : nullptr;
   const void* vv = have_v ? v : nullptr;
 #define SMAT_FT(T_)                                                                            \
-  smat::launch(featurise_kernel<T_>, dim3(grid), dim3(ft::kThreads), 0, st, (const T_*)q, \
+  smat::launch(featurise_kernel<T_>, dim3(grid), dim3(ft::kThreads),                           \
+                     (r + 15) / 16 * 16 * ft::w_stride<T_>(d_qk) * sizeof(T_), st, (const T_*)q, \
                      (const T_*)kk, (const T_*)vv, (const T_*)W, (const T_*)h, (T_*)phi, (T_*)psi, \
                      (T_*)vb, nb, T, d_qk, r, d_v, kind, q_sb, q_st, k_sb, k_st, v_sb, v_st,     \
-                     h_sb, o_sb, o_st, vb_sb, vb_st, ntiles, vec)
+                     h_sb, o_sb, o_st, vb_sb, vb_st, vec)
   switch (dtype) {
     case SMAT_BF16: SMAT_FT(bf16); break;
     case SMAT_F16: SMAT_FT(f16); break;

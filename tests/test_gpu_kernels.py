@@ -1183,3 +1183,33 @@ def test_stage_events_time_the_one_call_forward(fused):
     run()
     torch.cuda.synchronize()
     assert ev[0].elapsed_time(ev[4]) == stamp
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("dqk,r,dv", [(64, 64, 64), (128, 128, 128), (40, 96, 33), (64, 48, 8)])
+def test_featurise_store_forms_agree(dt, dqk, r, dv):
+    """The feature rows stored 16 bytes a lane (16-byte aligned rows, r a multiple of
+    32) and value by value (rows at an odd stride) are bitwise the same, at
+    lengths beside the 32-row tiles, and no row past the end is written."""
+    from smat_attention_amd.kernels.hip_fwd import DTYPE_CODE, call, stream_of
+    for T in (1, 15, 16, 31, 32, 33, 65, 200):
+        nb = 3
+        gen = torch.Generator().manual_seed(T)
+        q, k = (torch.randn(nb, T, dqk, generator=gen).to(dt).to(DEV) for _ in range(2))
+        v = torch.randn(nb, T, dv, generator=gen).to(dt).to(DEV)
+        W = (torch.randn(r, dqk, generator=gen) / dqk ** 0.5).to(dt).to(DEV)
+        h = torch.rand(nb, T, generator=gen).to(dt).to(DEV)
+        got = []
+        for pad, vpad in ((0, (dv + 8) // 8 * 8 - dv), (3, 1)):
+            phi, psi = (torch.full((nb, T + 1, r + pad), 7.0, device=DEV, dtype=dt) for _ in range(2))
+            vb = torch.full((nb, T + 1, dv + vpad), 7.0, device=DEV, dtype=dt)
+            call("smat_featurise", DTYPE_CODE[dt], q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                 W.data_ptr(), h.data_ptr(), phi.data_ptr(), psi.data_ptr(), vb.data_ptr(), nb, T, dqk,
+                 r, dv, 0, T * dqk, dqk, T * dqk, dqk, T * dv, dv, T, phi.stride(0), phi.stride(1),
+                 vb.stride(0), vb.stride(1), stream_of(phi))
+            for t, w in ((phi, r), (psi, r), (vb, dv + 1)):
+                assert (t[:, T:] == 7).all() and (t[..., w:] == 7).all()
+            got.append((phi[:, :T, :r], psi[:, :T, :r], vb[:, :T, :dv + 1]))
+        for a, b in zip(*got):
+            assert torch.equal(a, b), T
+        assert torch.equal(got[0][2][..., :dv], v) and (got[0][2][..., dv] == 1).all()
