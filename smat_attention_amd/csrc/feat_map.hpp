@@ -16,56 +16,62 @@
 
 namespace smat {
 
-// expm1(v) for v <= 0 in a few instructions: the degree-6 Taylor polynomial
-// on (-0.25, 0] (truncation under 2e-8 relative there) and exp(v) - 1 below,
-// where |expm1| > 0.22 and the hardware exp2 keeps the error under 1e-5
-// relative.  Rounded to bf16, it equals the correctly rounded expm1 (and the
-// fp32 libm expm1f) for every negative bf16 input -- an exhaustive check --
-// at a fraction of expm1f's cost, which dominates the feature map's VALU time.
-// Both forms are computed and one selected: no divergent branch, so the
-// feature map's instructions interleave with the MFMAs around them.  (For
-// v > 0 the exp2 form may be inf; callers select v there.)
-__device__ __forceinline__ float expm1_neg(float v) {
-  float r = 1.f / 720.f;
-  r = fmaf(v, r, 1.f / 120.f);
-  r = fmaf(v, r, 1.f / 24.f);
-  r = fmaf(v, r, 1.f / 6.f);
-  r = fmaf(v, r, 0.5f);
-  r = fmaf(v, r, 1.f);
-  const float near = v * r;
-  const float far = __builtin_amdgcn_exp2f(v * 1.4426950408889634f) - 1.f;
-  return v > -0.25f ? near : far;
-}
-
-// expm1 of a non-positive argument for input type In: the short form where the
-// result is rounded to bf16 (where it is exact after rounding, above), libm's
-// expm1f for fp16 (whose 11-bit significand the short form's 1e-5 error could
-// round differently) and for fp32 (where nothing rounds afterwards).
-template <typename In>
-__device__ __forceinline__ float expm1_nonpos(float v) {
-  if constexpr (std::is_same<In, bf16>::value) return expm1_neg(v);
-  else return expm1f(v);
-}
-
+// map() of four values of the product, each step rounded to In.  bf16's elu is
+// exp2 minus one: its error (1e-7, absolute) only matters where |expm1| is so
+// small that the roundings after it, to steps of 2^-8 of 1 + expm1, discard it,
+// and map() equals the one on the correctly rounded expm1 for every
+// non-positive bf16 input -- an exhaustive check.  It is formed for every lane
+// and selected, so no branch keeps the map from interleaving with the MFMAs
+// around it (for v > 0 exp2 may be inf), and the conversions go two values to
+// an instruction: half the vector work of a form that holds expm1's relative
+// error (a polynomial near zero), and the map's vector work weighs on the kernels
+// that form their features (the forward from q, k, v at 8 sequences of 131072
+// tokens: 1780 -> 1734 us; the feature map alone at 96 of 4096, widths 64:
+// 79 -> 71).  fp16, whose 11-bit significand could round that error differently,
+// and fp32, where nothing rounds afterwards, take libm's expm1f.
 template <typename In, int KIND>
-__device__ __forceinline__ float feature_map_k(float acc) {
-  const float v = to_f32(from_f32<In>(acc));                 // torch's matmul output
-  if constexpr (KIND == 0) {
-    float e;
-    if constexpr (std::is_same<In, bf16>::value) {
-      const float m = expm1_neg(v);                            // computed for every lane
-      e = to_f32(from_f32<In>(v > 0.f ? v : m));
+__device__ __forceinline__ typename Traits<In>::half_frag feature_map4(const f32x4& acc) {
+  typedef typename Traits<In>::half_frag Half;
+  if constexpr (std::is_same<In, bf16>::value) {
+    auto rounded = [](const f32x4& x) {
+      return __builtin_convertvector(__builtin_convertvector(x, Half), f32x4);
+    };
+    const f32x4 v = rounded(acc);                              // torch's matmul output
+    f32x4 y;
+    if constexpr (KIND == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float m = __builtin_amdgcn_exp2f(v[i] * 1.4426950408889634f) - 1.f;
+        y[i] = v[i] > 0.f ? v[i] : m;
+      }
+      y = rounded(y) + 1.0f;
     } else {
-      e = to_f32(from_f32<In>(v > 0.f ? v : expm1_nonpos<In>(v)));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = fmaxf(v[i], 0.f) + 1e-3f;
     }
-    return to_f32(from_f32<In>(e + 1.0f));
+    return __builtin_convertvector(y, Half);
+  } else {
+    Half out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float v = to_f32(from_f32<In>(acc[i]));
+      float y;
+      if constexpr (KIND == 0) y = to_f32(from_f32<In>(v > 0.f ? v : expm1f(v))) + 1.0f;
+      else y = fmaxf(v, 0.f) + 1e-3f;
+      out[i] = from_f32<In>(y);
+    }
+    return out;
   }
-  return to_f32(from_f32<In>(fmaxf(v, 0.f) + 1e-3f));
 }
 
+// Four mapped values times their row's gate, rounded.
 template <typename In>
-__device__ __forceinline__ float feature_map(float acc, int kind) {
-  return kind == 0 ? feature_map_k<In, 0>(acc) : feature_map_k<In, 1>(acc);
+__device__ __forceinline__ typename Traits<In>::half_frag feature_gate4(
+    const typename Traits<In>::half_frag& y, float gate) {
+  typename Traits<In>::half_frag out;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) out[i] = from_f32<In>(to_f32(y[i]) * gate);
+  return out;
 }
 
 // The feature map handed to a consumer kernel: W (128 x 128, features x d_qk,
@@ -136,13 +142,8 @@ __device__ __forceinline__ void feat_rows(const uint4* src, uint4* dst, int rt0,
 #pragma unroll
     for (int rt = 0; rt < NRT; ++rt) {
       const int t = 16 * (rt0 + rt) + r16;
-      Half hv;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float y = feature_map_k<In, KIND>(acc[rt][i]);
-        if (use_gate) y = to_f32(from_f32<In>(y * gate[rt]));
-        hv[i] = from_f32<In>(y);
-      }
+      Half hv = feature_map4<In, KIND>(acc[rt]);
+      if (use_gate) hv = feature_gate4<In>(hv, gate[rt]);
       char* p = reinterpret_cast<char*>(dst + t * 16 + ((2 * wf + (g >> 1)) ^ swz(t)));
       *reinterpret_cast<Half*>(p + 8 * (g & 1)) = hv;
     }

@@ -17,8 +17,8 @@
 //
 // HBM-bound: 2 (T d_qk + T r) + T (d_v + p) elements per sequence, so what
 // counts is bytes in flight against the number of places written at once: at 96
-// sequences of 4096 tokens, all widths 64, 79 us (the bytes at a copy's rate:
-// 63) with four workgroups a CU resident and none waiting; 85 with three of
+// sequences of 4096 tokens, all widths 64, 71 us (the bytes at a copy's rate:
+// 63); with the longer elu it then had, 79 with four workgroups a CU resident and none waiting; 85 with three of
 // them, 84 with twelve in turn, 93 with six resident; 99 with one row tile a
 // wave, 8-byte stores and W's LDS sized for 128 features.
 #include <math.h>
@@ -181,13 +181,10 @@ __global__ __launch_bounds__(ft::kThreads, sizeof(In) == 2 ? 4 : 2) void featuri
         }
       }
 #pragma unroll
-      for (int u = 0; u < kTiles; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float y = feature_map<In>(acc[u][i], kind);
-          if (which == 1 && h) y = to_f32(from_f32<In>(y * hv[u]));
-          out[u][i] = from_f32<In>(y);
-        }
+      for (int u = 0; u < kTiles; ++u) {
+        out[u] = kind == 0 ? feature_map4<In, 0>(acc[u]) : feature_map4<In, 1>(acc[u]);
+        if (which == 1 && h) out[u] = feature_gate4<In>(out[u], hv[u]);
+      }
     };
     if (pair) {
 #pragma unroll 1
