@@ -45,8 +45,15 @@ int pool_dispatch(int dtype, const void* psi, const void* vb, float* F, float* F
 int64_t pool_workspace_bytes(int nb, int n_P, int n, int N0, int r, int p, bool glob);
 int chunk_states_dispatch(int dtype, const void* psi, const void* vb, float* D, int nb, int T,
                           int C, int K, int n, int r, int p, int64_t k_sb, int64_t k_st,
-                          int64_t v_sb, int64_t v_st, float* partials, int64_t partial_bytes,
-                          hipStream_t stream, int* ngroups_out, int* ng0_out);
+                          int64_t v_sb, int64_t v_st, hipStream_t stream);
+GramPart pool_part(float* F, float* F_glob, int nb, int n_P, int n, int N0, int r, int p,
+                   int64_t f_ld);
+int gram_pair_dispatch(int dtype, const void* psi, const void* vb, const GramPart& A,
+                       const GramPart& B, int nb, int r, int p, int64_t k_sb, int64_t k_st,
+                       int64_t v_sb, int64_t v_st, hipStream_t stream, const char* who,
+                       bool* done);
+GramPart causal_scan_part(int dtype, int nb, int T, int n, int C, int r, int p, int kmax,
+                          void* ws);
 int segment_scan_dispatch(const float* D, float* Sin, int nb, int nc, int nc0, int64_t rp,
                           hipStream_t stream);
 int chunk_local_dispatch(int dtype, const void* phi, const void* psi, const void* vb,
@@ -90,7 +97,7 @@ int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void
                          int C, int r, int p, int64_t q_sb, int64_t q_st, int64_t k_sb,
                          int64_t k_st, int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st,
                          int64_t o_sb, int64_t o_st, int64_t g_sb, int write_H, void* ws,
-                         int64_t ws_bytes, int kmax, hipStream_t stream);
+                         int64_t ws_bytes, int kmax, bool have_G, hipStream_t stream);
 
 // Workspace carve-up, each region 256-byte aligned.  The fused causal pass
 // (chunk <= 128, no H requested) needs only its group states; the staged one
@@ -255,10 +262,11 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
     StageScope stage(3);
     return causal_scan_dispatch(dtype, phi, psi, vb, nullptr, g, out, nb, T, 0, C, r, p, q_sb,
                                 q_st, k_sb, k_st, v_sb, v_st, 0, 0, o_sb, o_st, g_sb, 0,
-                                ws + L.scan, L.part - L.scan, kForwardK, st);
+                                ws + L.scan, L.part - L.scan, kForwardK, false, st);
   }
 
   // ---- long range: S^T, then C, then R ---------------------------------
+  bool have_G = false;                               // the causal pass's chunk-group summaries
   if (T_R > 0) {
     // With no profiled landmark columns (n == n_P) every U_h is the global
     // channel alone (or zero): the incidence runs with an empty row.
@@ -268,8 +276,16 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
     const int64_t ld = idx && plane_code && profiled ? incidence_plane_ld(q, N0, B, rp) : rp;
     {
       StageScope stage(0);
-      rc = pool_dispatch(dtype, psi, vb, F, Fg, nb, n_P, n, N0, r, p, k_sb, k_st, v_sb, v_st,
-                         part, part_bytes, st, ld);
+      // a small problem's profile sums and chunk-group summaries in one launch
+      rc = SMAT_OK;
+      if (L.fused)
+        rc = gram_pair_dispatch(
+            dtype, psi, vb, pool_part(F, Fg, nb, n_P, n, N0, r, p, ld),
+            causal_scan_part(dtype, nb, T, n, C, r, p, kForwardK, ws + L.scan), nb, r, p, k_sb,
+            k_st, v_sb, v_st, st, "smat_forward", &have_G);
+      if (!rc && !have_G)
+        rc = pool_dispatch(dtype, psi, vb, F, Fg, nb, n_P, n, N0, r, p, k_sb, k_st, v_sb, v_st,
+                           part, part_bytes, st, ld);
     }
     if (rc) return rc;
     const float* Uq = U;
@@ -298,7 +314,8 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
     // one kernel: segmented scan, + Y on recent rows, normalise, gate
     return causal_scan_dispatch(dtype, phi, psi, vb, T_R > 0 ? Y : nullptr, g, out, nb, T, n, C,
                                 r, p, q_sb, q_st, k_sb, k_st, v_sb, v_st, (int64_t)T_R * yst, yst,
-                                o_sb, o_st, g_sb, 0, ws + L.scan, L.part - L.scan, kForwardK, st);
+                                o_sb, o_st, g_sb, 0, ws + L.scan, L.part - L.scan, kForwardK,
+                                have_G, st);
   }
   // staged: chunk summaries, segmented scan, chunk-local pass into H, normalise
   float* D = (float*)(ws + L.D);
@@ -306,8 +323,7 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
   // H in (nb, nc*C, p) fp32: the caller's H_out is (nb, T, p), which is the
   // same layout for every row the chunk pass writes (rows >= T are skipped).
   float* H = H_out ? H_out : (float*)(ws + L.H);
-  rc = chunk_states_dispatch(dtype, psi, vb, D, nb, T, C, 1, n, r, p, k_sb, k_st, v_sb, v_st,
-                             nullptr, 0, st, nullptr, nullptr);
+  rc = chunk_states_dispatch(dtype, psi, vb, D, nb, T, C, 1, n, r, p, k_sb, k_st, v_sb, v_st, st);
   if (rc) return rc;
   rc = segment_scan_dispatch(D, Sin, nb, nc, n / C, rp, st);
   if (rc) return rc;

@@ -33,11 +33,15 @@ template <typename In> constexpr int bt() { return sizeof(In) == 4 ? 32 : 64; }
 // in LDS transposed (Psi^T[a][t], Vb^T[c][t]) from 8 x 8 tiles; the next
 // block's tiles are loaded into registers while the current block is
 // multiplied, so one memory latency per block overlaps the MFMAs.
+//
+// A launch holds one part (gram_kernel), or two over the same keys and values
+// (gram_pair_kernel, part A's workgroups first): a small problem's profile sums and its chunk-group
+// summaries read nothing of each other, and each alone leaves most of the
+// device idle for the length of one workgroup.
 template <typename In, bool VEC, int kTW, int kNCT>
-__global__ __launch_bounds__(gr::kThreads, kTW == 1 ? 4 : 2) void gram_kernel(
-    const In* __restrict__ psi, const In* __restrict__ vb, float* __restrict__ G,
-    float* __restrict__ G_last, GramItems it, int r, int p, int64_t k_sb, int64_t k_st,
-    int64_t v_sb, int64_t v_st, int64_t g_sb, int64_t g_si, int64_t gl_sb) {
+__device__ __forceinline__ void gram_body(const In* __restrict__ psi, const In* __restrict__ vb,
+                                          const GramPart& P, int part_wg, int r, int p,
+                                          int64_t k_sb, int64_t k_st, int64_t v_sb, int64_t v_st) {
   using namespace gr;
   typedef typename Traits<In>::frag Frag;
   constexpr int kB = bt<In>();
@@ -47,8 +51,9 @@ __global__ __launch_bounds__(gr::kThreads, kTW == 1 ? 4 : 2) void gram_kernel(
   __shared__ __attribute__((aligned(16))) In psiT[kRows * kTPad];
   __shared__ __attribute__((aligned(16))) In vbT[kCols * kTPad];
 
-  const int item = blockIdx.x / it.nsplit;
-  const int sp = blockIdx.x - item * it.nsplit;
+  const GramItems& it = P.it;
+  const int item = part_wg / it.nsplit;
+  const int sp = part_wg - item * it.nsplit;
   const int64_t b = blockIdx.y;
   const int lane = lane_id(), w = wave_id();
   const int row16 = lane & 15, grp = lane >> 4;
@@ -148,12 +153,12 @@ __global__ __launch_bounds__(gr::kThreads, kTW == 1 ? 4 : 2) void gram_kernel(
 
   // nsplit > 1: G is the partial buffer (nb, nitems, nsplit, r, p) and G_last
   // is unused; otherwise item nitems-1 goes to G_last when that is given.
-  const int nitems = gridDim.x / it.nsplit;
   float* Gb;
   if (it.nsplit > 1)
-    Gb = G + ((b * nitems + item) * it.nsplit + sp) * (int64_t)r * p;
+    Gb = P.G + ((b * P.nitems + item) * it.nsplit + sp) * (int64_t)r * p;
   else
-    Gb = (G_last != nullptr && item == nitems - 1) ? G_last + b * gl_sb : G + b * g_sb + item * g_si;
+    Gb = (P.G_last != nullptr && item == P.nitems - 1) ? P.G_last + b * P.gl_sb
+                                                       : P.G + b * P.g_sb + item * P.g_si;
 #pragma unroll
   for (int t = 0; t < kTW; ++t) {
     const int rt = kTW * w + t;
@@ -169,6 +174,21 @@ __global__ __launch_bounds__(gr::kThreads, kTW == 1 ? 4 : 2) void gram_kernel(
       }
     }
   }
+}
+
+template <typename In, bool VEC, int kTW, int kNCT>
+__global__ __launch_bounds__(gr::kThreads, kTW == 1 ? 4 : 2) void gram_kernel(
+    const In* __restrict__ psi, const In* __restrict__ vb, GramPart A, int r, int p, int64_t k_sb,
+    int64_t k_st, int64_t v_sb, int64_t v_st) {
+  gram_body<In, VEC, kTW, kNCT>(psi, vb, A, blockIdx.x, r, p, k_sb, k_st, v_sb, v_st);
+}
+template <typename In, bool VEC, int kTW, int kNCT>
+__global__ __launch_bounds__(gr::kThreads, kTW == 1 ? 4 : 2) void gram_pair_kernel(
+    const In* __restrict__ psi, const In* __restrict__ vb, GramPart A, GramPart B, int r, int p,
+    int64_t k_sb, int64_t k_st, int64_t v_sb, int64_t v_st) {
+  const bool second = (int)blockIdx.x >= A.nitems;   // neither is split
+  gram_body<In, VEC, kTW, kNCT>(psi, vb, second ? B : A, blockIdx.x - (second ? A.nitems : 0), r,
+                                p, k_sb, k_st, v_sb, v_st);
 }
 
 // Sum the nsplit partials of every (b, item) in run order into G / G_last.
@@ -189,56 +209,66 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(const float* __restric
   dst[e] = acc;
 }
 
+// Part A and, where B.nitems > 0, part B (neither split).
 template <typename In, int TW, int NCT>
-static int launch_gram_shape(const void* psi, const void* vb, float* G, float* G_last,
-                       const GramItems& it, int nitems, int nb, int r, int p, int64_t k_sb,
-                       int64_t k_st, int64_t v_sb, int64_t v_st, int64_t g_sb, int64_t g_si,
-                       int64_t gl_sb, float* partials, hipStream_t stream, const char* who) {
-  const int64_t gx = (int64_t)nitems * it.nsplit;
-  const int vk = rows_vec8_ok(psi, k_sb, k_st);
-  const int vv = rows_vec8_ok(vb, v_sb, v_st);
+static int launch_gram_shape(const void* psi, const void* vb, const GramPart& A, const GramPart& B,
+                             int nb, int r, int p, int64_t k_sb, int64_t k_st, int64_t v_sb,
+                             int64_t v_st, float* partials, hipStream_t stream, const char* who) {
+  const int64_t gx = (int64_t)A.nitems * A.it.nsplit + B.nitems;
   if (gx >= (1ll << 31) || nb >= 65536) {
     set_error("%s: problem too large", who);
     return SMAT_EUNSUPPORTED;
   }
-  if (it.nsplit > 1) {
-    if (vk && vv)
-      smat::launch((gram_kernel<In, true, TW, NCT>), dim3((unsigned)gx, (unsigned)nb),
-                         dim3(gr::kThreads), 0, stream, (const In*)psi, (const In*)vb, partials,
-                         nullptr, it, r, p, k_sb, k_st, v_sb, v_st, 0, 0, 0);
-    else
-      smat::launch((gram_kernel<In, false, TW, NCT>), dim3((unsigned)gx, (unsigned)nb),
-                         dim3(gr::kThreads), 0, stream, (const In*)psi, (const In*)vb, partials,
-                         nullptr, it, r, p, k_sb, k_st, v_sb, v_st, 0, 0, 0);
-    int st = launch_status(who);
-    if (st != SMAT_OK) return st;
-    const int64_t rp = (int64_t)r * p;
-    smat::launch(gram_reduce_kernel, dim3((unsigned)((rp + 255) / 256), nitems, nb),
-                       dim3(256), 0, stream, partials, G, G_last, nitems, it.nsplit, rp, g_sb,
-                       g_si, gl_sb);
-    return launch_status(who);
+  const bool vec = rows_vec8_ok(psi, k_sb, k_st) && rows_vec8_ok(vb, v_sb, v_st);
+  GramPart a = A;
+  if (A.it.nsplit > 1) {
+    a.G = partials;
+    a.G_last = nullptr;
   }
-  if (vk && vv)
-    smat::launch((gram_kernel<In, true, TW, NCT>), dim3((unsigned)gx, (unsigned)nb),
-                       dim3(gr::kThreads), 0, stream, (const In*)psi, (const In*)vb, G, G_last,
-                       it, r, p, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb);
+  const dim3 grid((unsigned)gx, (unsigned)nb), block(gr::kThreads);
+  if (B.nitems > 0)
+    smat::launch(vec ? gram_pair_kernel<In, true, TW, NCT> : gram_pair_kernel<In, false, TW, NCT>,
+                 grid, block, 0, stream, (const In*)psi, (const In*)vb, a, B, r, p, k_sb, k_st,
+                 v_sb, v_st);
   else
-    smat::launch((gram_kernel<In, false, TW, NCT>), dim3((unsigned)gx, (unsigned)nb),
-                       dim3(gr::kThreads), 0, stream, (const In*)psi, (const In*)vb, G, G_last,
-                       it, r, p, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb);
+    smat::launch(vec ? gram_kernel<In, true, TW, NCT> : gram_kernel<In, false, TW, NCT>, grid,
+                 block, 0, stream, (const In*)psi, (const In*)vb, a, r, p, k_sb, k_st, v_sb, v_st);
+  const int st = launch_status(who);
+  if (st != SMAT_OK || A.it.nsplit <= 1) return st;
+  const int64_t rp = (int64_t)r * p;
+  smat::launch(gram_reduce_kernel, dim3((unsigned)((rp + 255) / 256), A.nitems, nb), dim3(256), 0,
+               stream, partials, A.G, A.G_last, A.nitems, A.it.nsplit, rp, A.g_sb, A.g_si, A.gl_sb);
   return launch_status(who);
 }
 
 template <typename In>
-static int launch_gram(const void* psi, const void* vb, float* G, float* G_last,
-                       const GramItems& it, int nitems, int nb, int r, int p, int64_t k_sb,
-                       int64_t k_st, int64_t v_sb, int64_t v_st, int64_t g_sb, int64_t g_si,
-                       int64_t gl_sb, float* partials, hipStream_t stream, const char* who) {
+static int launch_gram(const void* psi, const void* vb, const GramPart& A, const GramPart& B,
+                       int nb, int r, int p, int64_t k_sb, int64_t k_st, int64_t v_sb,
+                       int64_t v_st, float* partials, hipStream_t stream, const char* who) {
   if (r <= 64 && p <= 80)
-    return launch_gram_shape<In, 1, 5>(psi, vb, G, G_last, it, nitems, nb, r, p, k_sb, k_st, v_sb,
-                                       v_st, g_sb, g_si, gl_sb, partials, stream, who);
-  return launch_gram_shape<In, 2, 9>(psi, vb, G, G_last, it, nitems, nb, r, p, k_sb, k_st, v_sb,
-                                     v_st, g_sb, g_si, gl_sb, partials, stream, who);
+    return launch_gram_shape<In, 1, 5>(psi, vb, A, B, nb, r, p, k_sb, k_st, v_sb, v_st, partials,
+                                       stream, who);
+  return launch_gram_shape<In, 2, 9>(psi, vb, A, B, nb, r, p, k_sb, k_st, v_sb, v_st, partials,
+                                     stream, who);
+}
+
+static int gram_general(int dtype, const void* psi, const void* vb, const GramPart& A,
+                        const GramPart& B, int nb, int r, int p, int64_t k_sb, int64_t k_st,
+                        int64_t v_sb, int64_t v_st, float* partials, hipStream_t stream,
+                        const char* who) {
+  switch (dtype) {
+    case SMAT_BF16:
+      return launch_gram<bf16>(psi, vb, A, B, nb, r, p, k_sb, k_st, v_sb, v_st, partials, stream,
+                               who);
+    case SMAT_F16:
+      return launch_gram<f16>(psi, vb, A, B, nb, r, p, k_sb, k_st, v_sb, v_st, partials, stream,
+                              who);
+    case SMAT_F32:
+      return launch_gram<float>(psi, vb, A, B, nb, r, p, k_sb, k_st, v_sb, v_st, partials, stream,
+                                who);
+  }
+  set_error("%s: unknown dtype %d", who, dtype);
+  return SMAT_EINVAL;
 }
 
 // Choose the split of the longest progression so that a launch has enough
@@ -433,26 +463,34 @@ int gram_dispatch(int dtype, const void* psi, const void* vb, float* G, float* G
     set_error("%s: split-K needs a workspace", who);
     return SMAT_EINVAL;
   }
-  switch (dtype) {
-    case SMAT_BF16:
-      return launch_gram<bf16>(psi, vb, G, G_last, it, nitems, nb, r, p, k_sb, k_st, v_sb, v_st,
-                               g_sb, g_si, gl_sb, partials, stream, who);
-    case SMAT_F16:
-      return launch_gram<f16>(psi, vb, G, G_last, it, nitems, nb, r, p, k_sb, k_st, v_sb, v_st,
-                              g_sb, g_si, gl_sb, partials, stream, who);
-    case SMAT_F32:
-      return launch_gram<float>(psi, vb, G, G_last, it, nitems, nb, r, p, k_sb, k_st, v_sb,
-                                v_st, g_sb, g_si, gl_sb, partials, stream, who);
-  }
-  set_error("%s: unknown dtype %d", who, dtype);
-  return SMAT_EINVAL;
+  return gram_general(dtype, psi, vb, GramPart{G, G_last, it, nitems, g_sb, g_si, gl_sb},
+                      GramPart{}, nb, r, p, k_sb, k_st, v_sb, v_st, partials, stream, who);
 }
 
-// Chunk summaries for chunks of width C (K = 1) or groups of K chunks.
-int chunk_states_dispatch(int dtype, const void* psi, const void* vb, float* D, int nb, int T,
-                          int C, int K, int n, int r, int p, int64_t k_sb, int64_t k_st,
-                          int64_t v_sb, int64_t v_st, float* partials, int64_t partial_bytes,
-                          hipStream_t stream, int* ngroups_out, int* ng0_out) {
+// Two parts in one launch, where both would take the general kernel unsplit and
+// fit the device together (four workgroups a CU at the narrow tile shape, two at
+// the wide one): *done says whether they were launched.  The forward of four
+// fp32 sequences of 1024 tokens of head size 64, d = 2, takes 34.2 us; with the
+// two launches of 6.3 us one after the other, 39.4.
+int gram_pair_dispatch(int dtype, const void* psi, const void* vb, const GramPart& A,
+                       const GramPart& B, int nb, int r, int p, int64_t k_sb, int64_t k_st,
+                       int64_t v_sb, int64_t v_st, hipStream_t stream, const char* who,
+                       bool* done) {
+  *done = false;
+  if (nb < 1 || A.nitems < 1 || B.nitems < 1 || A.it.nsplit != 1 || B.it.nsplit != 1)
+    return SMAT_OK;
+  const int64_t fit = 256 * (r <= 64 && p <= 80 ? 4 : 2);
+  if (((int64_t)A.nitems + B.nitems) * nb > fit) return SMAT_OK;
+  for (const GramPart* P : {&A, &B})
+    if (gram64_ok(dtype, psi, r, p, k_sb, k_st, P->nitems, nb) ||
+        gram_stream_ok(dtype, psi, vb, r, p, k_sb, k_st, v_sb, v_st, P->it, P->nitems, nb))
+      return SMAT_OK;
+  *done = true;
+  return gram_general(dtype, psi, vb, A, B, nb, r, p, k_sb, k_st, v_sb, v_st, nullptr, stream, who);
+}
+
+// Chunk summaries for chunks of width C (K = 1) or groups of K chunks, unsplit.
+GramPart chunk_part(float* D, int T, int C, int K, int n, int r, int p) {
   GramItems it{};
   it.mode = 0;
   it.T = T;
@@ -461,17 +499,19 @@ int chunk_states_dispatch(int dtype, const void* psi, const void* vb, float* D, 
   it.nc = (T + C - 1) / C;
   it.nc0 = n / C;
   it.ng0 = (it.nc0 + K - 1) / K;
+  it.nsplit = 1;
+  it.per = K * C;
   const int ng = it.ng0 + (it.nc - it.nc0 + K - 1) / K;
-  if (ngroups_out) *ngroups_out = ng;
-  if (ng0_out) *ng0_out = it.ng0;
-  const int64_t need = plan_split(it, ng, nb, K * C, r, p);
-  if (need > partial_bytes) {   // not enough scratch: run unsplit
-    it.nsplit = 1;
-    it.per = K * C;
-  }
   const int64_t rp = (int64_t)r * p;
-  return gram_dispatch(dtype, psi, vb, D, nullptr, it, ng, nb, r, p, k_sb, k_st, v_sb, v_st,
-                       (int64_t)ng * rp, rp, 0, partials, stream, "smat_chunk_states");
+  return GramPart{D, nullptr, it, ng, (int64_t)ng * rp, rp, 0};
+}
+
+int chunk_states_dispatch(int dtype, const void* psi, const void* vb, float* D, int nb, int T,
+                          int C, int K, int n, int r, int p, int64_t k_sb, int64_t k_st,
+                          int64_t v_sb, int64_t v_st, hipStream_t stream) {
+  const GramPart P = chunk_part(D, T, C, K, n, r, p);
+  return gram_dispatch(dtype, psi, vb, D, nullptr, P.it, P.nitems, nb, r, p, k_sb, k_st, v_sb,
+                       v_st, P.g_sb, P.g_si, 0, nullptr, stream, "smat_chunk_states");
 }
 
 static GramItems pool_items(int n_P, int n, int N0, bool glob, int nb, int r, int p,
@@ -492,6 +532,16 @@ int64_t pool_workspace_bytes(int nb, int n_P, int n, int N0, int r, int p, bool 
   int64_t need = 0;
   pool_items(n_P, n, N0, glob, nb, r, p, &need);
   return need;
+}
+
+// The profile sums as one part (split-K as pool_dispatch would).
+GramPart pool_part(float* F, float* F_glob, int nb, int n_P, int n, int N0, int r, int p,
+                   int64_t f_ld) {
+  const bool glob = (F_glob != nullptr && n_P > 0);
+  int64_t need = 0;
+  const GramItems it = pool_items(n_P, n, N0, glob, nb, r, p, &need);
+  return GramPart{F,  glob ? F_glob : nullptr, it, N0 + (glob ? 1 : 0), (int64_t)N0 * f_ld, f_ld,
+                  (int64_t)r * p};
 }
 
 // F: (nb, N0) rows of r * p floats, f_ld floats apart.
@@ -565,7 +615,7 @@ extern "C" int smat_chunk_states(int dtype, const void* psi, const void* vb, flo
                "smat_chunk_states: r=%d p=%d beyond r<=%d, p<=%d", r, p, kMaxR, kMaxP);
   SMAT_REQUIRE(k_st >= r && v_st >= p, SMAT_EINVAL, "smat_chunk_states: row stride too short");
   return chunk_states_dispatch(dtype, psi, vb, D, nb, T, C, 1, 0, r, p, k_sb, k_st, v_sb, v_st,
-                               nullptr, 0, (hipStream_t)stream, nullptr, nullptr);
+                               (hipStream_t)stream);
 }
 
 extern "C" int64_t smat_pool_workspace_bytes(int nb, int n_P, int n, int N0, int r, int p) {

@@ -444,8 +444,8 @@ static int launch_scan_fused(const void* phi, const void* psi, const void* vb, c
 
 int chunk_states_dispatch(int dtype, const void* psi, const void* vb, float* D, int nb, int T,
                           int C, int K, int n, int r, int p, int64_t k_sb, int64_t k_st,
-                          int64_t v_sb, int64_t v_st, float* partials, int64_t partial_bytes,
-                          hipStream_t stream, int* ngroups_out, int* ng0_out);
+                          int64_t v_sb, int64_t v_st, hipStream_t stream);
+GramPart chunk_part(float* D, int T, int C, int K, int n, int r, int p);
 int segment_scan_dispatch(const float* D, float* Sin, int nb, int nc, int nc0, int64_t rp,
                           hipStream_t stream);
 bool scan_stream_ok(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
@@ -522,7 +522,8 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
                     const float* gate, float* out, int nb, int T, int n, int C, int K, int r, int p,
                     int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st,
                     int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb,
-                    int64_t o_st, int64_t g_sb, int write_H, void* ws, hipStream_t stream);
+                    int64_t o_st, int64_t g_sb, int write_H, void* ws, bool have_G,
+                    hipStream_t stream);
 
 // The most any input type's chunk needs (the type is not an argument).
 int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, int kmax) {
@@ -541,7 +542,7 @@ int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void
                          int C, int r, int p, int64_t q_sb, int64_t q_st, int64_t k_sb,
                          int64_t k_st, int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st,
                          int64_t o_sb, int64_t o_st, int64_t g_sb, int write_H, void* ws,
-                         int64_t ws_bytes, int kmax, hipStream_t stream) {
+                         int64_t ws_bytes, int kmax, bool have_G, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
   const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, kmax);
   C = scan_chunk(dtype, nb, T, C, r, p);
@@ -553,23 +554,34 @@ int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void
   }
   return causal_scan_run(dtype, phi, psi, vb, Y, gate, out, nb, T, n, C, K, r, p,
                          q_sb, q_st, k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb, o_st, g_sb,
-                         write_H, ws, stream);
+                         write_H, ws, have_G, stream);
+}
+
+// The summaries that causal_scan_dispatch begins with, for a caller that forms
+// them itself in the launch of something else and then passes have_G.
+GramPart causal_scan_part(int dtype, int nb, int T, int n, int C, int r, int p, int kmax,
+                          void* ws) {
+  C = scan_chunk(dtype, nb, T, C, r, p);
+  return chunk_part((float*)ws, T, C, scan_group_chunks(nb, (T + C - 1) / C, r, p, kmax), n, r, p);
 }
 
 // The causal pass with groups of K chunks; ws holds twice group_bytes: the
-// summaries, then the states.
+// summaries (already there with have_G), then the states.
 int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
                     const float* gate, float* out, int nb, int T, int n, int C, int K, int r, int p,
                     int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st,
                     int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb,
-                    int64_t o_st, int64_t g_sb, int write_H, void* ws, hipStream_t stream) {
+                    int64_t o_st, int64_t g_sb, int write_H, void* ws, bool have_G,
+                    hipStream_t stream) {
   const int nc = (T + C - 1) / C;
   float* G = (float*)ws;
   float* Sg = (float*)((char*)ws + group_bytes(nb, nc, K, r, p));
   // groups over [0, n), then over [n, T)
-  int ng = 0, ng0 = 0;
-  int rc = chunk_states_dispatch(dtype, psi, vb, G, nb, T, C, K, n, r, p, k_sb, k_st, v_sb, v_st,
-                                 nullptr, 0, stream, &ng, &ng0);
+  const GramPart P = chunk_part(G, T, C, K, n, r, p);
+  const int ng = P.nitems, ng0 = P.it.ng0;
+  int rc = have_G ? SMAT_OK
+                  : chunk_states_dispatch(dtype, psi, vb, G, nb, T, C, K, n, r, p, k_sb, k_st,
+                                          v_sb, v_st, stream);
   if (rc) return rc;
   rc = segment_scan_dispatch(G, Sg, nb, ng, ng0, (int64_t)r * p, stream);
   if (rc) return rc;
@@ -772,7 +784,7 @@ extern "C" int smat_causal_scan_noalloc(int dtype, const void* phi, const void* 
   int rc = scratch_for_current_device(&ws);
   if (rc) return rc;
   return causal_scan_run(dtype, phi, psi, vb, Y, gate, out, nb, T, n, C, K, r, p, q_sb, q_st,
-                         k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb, o_st, g_sb, write_H, ws,
+                         k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb, o_st, g_sb, write_H, ws, false,
                          (hipStream_t)stream);
 }
 
@@ -804,5 +816,5 @@ extern "C" int smat_causal_scan(int dtype, const void* phi, const void* psi, con
                "smat_causal_scan: workspace must be 256-byte aligned");
   return causal_scan_dispatch(dtype, phi, psi, vb, Y, gate, out, nb, T, n, C, r, p, q_sb, q_st,
                               k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb, o_st, g_sb, write_H,
-                              workspace, workspace_bytes, kScanK, (hipStream_t)stream);
+                              workspace, workspace_bytes, kScanK, false, (hipStream_t)stream);
 }

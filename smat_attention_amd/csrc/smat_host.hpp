@@ -117,6 +117,16 @@ struct GramItems {
   const int64_t* offs;
 };
 
+// One launch's Gram sums: item i of sequence b goes to G + b g_sb + i g_si, the
+// last item to G_last + b gl_sb when that is given.
+struct GramPart {
+  float* G;
+  float* G_last;
+  GramItems it;
+  int nitems;
+  int64_t g_sb, g_si, gl_sb;
+};
+
 __device__ __forceinline__ void gram_item(const GramItems& it, int i, int64_t& start,
                                           int64_t& stride, int& count) {
   if (it.mode == 0) {

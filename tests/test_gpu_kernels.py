@@ -1213,3 +1213,20 @@ def test_featurise_store_forms_agree(dt, dqk, r, dv):
         for a, b in zip(*got):
             assert torch.equal(a, b), T
         assert torch.equal(got[0][2][..., :dv], v) and (got[0][2][..., dv] == 1).all()
+
+
+@pytest.mark.parametrize("dt,hd", [(torch.float32, 64), (torch.float32, 96), (torch.bfloat16, 64),
+                                   (torch.float16, 40)])
+@pytest.mark.parametrize("T,d,n_P", [(1024, 2, 0), (1000, 3, 0), (2048, 2, 128), (300, 2, 0)])
+def test_forward_profile_and_chunk_sums_in_one_launch(dt, hd, T, d, n_P):
+    """The one-call forward of a small problem sums its profiles and its chunk groups
+    in one launch, a larger one in two: at batch sizes on both sides of that line
+    (1024 workgroups at head size 64, 512 above) against the schedule's separate
+    launches, whose sums differ only in the order of fp32 additions."""
+    _say("pool and prepass", dt, hd, T, d, n_P)
+    spec = A.to_device(build_mask(T, d, chunk=128, n_P=n_P), DEV)
+    for nb in (1, 3, 7, 12, 24):
+        Phi, Psi, Vb = (t.to(DEV) for t in _feats(nb, T, hd, dt, seed=73))
+        one = A.smat_attention(Phi, Psi, Vb, spec)
+        parts, _ = A.smat_attention(Phi, Psi, Vb, spec, return_parts=True)
+        assert _rel(one, parts.double().cpu()) < (2e-5 if dt == torch.float32 else 2.0 ** -7), nb
