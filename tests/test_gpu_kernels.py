@@ -1230,3 +1230,34 @@ def test_forward_profile_and_chunk_sums_in_one_launch(dt, hd, T, d, n_P):
         one = A.smat_attention(Phi, Psi, Vb, spec)
         parts, _ = A.smat_attention(Phi, Psi, Vb, spec, return_parts=True)
         assert _rel(one, parts.double().cpu()) < (2e-5 if dt == torch.float32 else 2.0 ** -7), nb
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("p", [2, 3, 4, 5, 8, 33, 64, 65, 66, 67, 129])
+def test_combine_normalise_row_widths(dt, p):
+    """The division and its backward at row widths beside the four-value accesses and
+    the 64 columns of a pass, rows starting at every alignment, the long-range
+    term from row n on: against fp64 (fp32 arithmetic; 2^-8 or 2^-11 more where the
+    output is rounded), the floor reached on one row."""
+    nb, T, n = 2, 37, 13
+    gen = torch.Generator().manual_seed(p)
+    H = torch.randn(nb, T, p, generator=gen)
+    H[..., -1] = torch.rand(nb, T, generator=gen) + 0.5
+    H[0, 3, -1] = -1.0
+    Y = torch.rand(nb, T - n, p, generator=gen)
+    do = torch.randn(nb, T, p - 1, generator=gen).to(dt)
+    Hd, Yd = H.to(DEV).requires_grad_(True), Y.to(DEV).requires_grad_(True)
+    out = A.combine_normalise(Hd, Yd, n, out_dtype=dt)
+    out.backward(do.to(DEV))
+    H64, Y64 = H.double().requires_grad_(True), Y.double().requires_grad_(True)
+    N = torch.cat([H64[:, :n], H64[:, n:] + Y64], 1)
+    ref = N[..., :-1] / N[..., -1:].clamp_min(1e-6)
+    ref.backward(do.double())
+    keep = torch.ones(nb, T, dtype=torch.bool)
+    keep[0, 3] = False                                # 1e6 times larger: compared by itself
+    eps = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10}[dt]
+    got, want = out.detach().cpu().double(), ref.detach()
+    assert ((got - want).abs()[keep] <= (1e-5 + eps) * want.abs()[keep] + 1e-5).all()
+    for a, b, m in ((Hd.grad, H64.grad, keep), (Yd.grad, Y64.grad, keep[:, n:])):
+        assert _rel(a.cpu()[m].to(DEV), b[m]) < 1e-5
+    assert _rel(Hd.grad[0, 3, :-1], H64.grad[0, 3, :-1]) < 1e-5 and Hd.grad[0, 3, -1] == 0
