@@ -184,10 +184,15 @@ template <int RC>
 __device__ __forceinline__ int swz(int t) { return RC == 16 ? t & 15 : (t >> 1) & 7; }
 }  // namespace qt
 
-template <typename In, int NW>
+// LIST: the rows of type h are rows[roffs[h] .. roffs[h + 1]) (one sequence), in
+// row blocks rb, rb + nrb, ... -- a list longer than the grid was sized for is
+// still covered; Y rows at any alignment.  The content-addressed read at 96
+// sequences of 4096 tokens, d = 2, r = 64: 55 us, the general kernel 80.
+template <typename In, int NW, bool LIST>
 __global__ __launch_bounds__(64 * (NW + 1)) void query_tile_kernel(
     const In* __restrict__ phi, const float* __restrict__ U, float* __restrict__ Y, int T_R, int B,
-    int64_t u_ld, int64_t q_sb, int64_t q_st, int64_t y_sb, int64_t y_st, int nrb) {
+    int64_t u_ld, int64_t q_sb, int64_t q_st, int64_t y_sb, int64_t y_st, int nrb,
+    const int32_t* __restrict__ rows, const int64_t* __restrict__ roffs) {
   typedef qt::Shape<NW> Sh;
   typedef typename Traits<In>::frag Frag;
   typedef typename Traits<In>::half_frag Half;
@@ -195,15 +200,19 @@ __global__ __launch_bounds__(64 * (NW + 1)) void query_tile_kernel(
   __shared__ __attribute__((aligned(16))) float us[Sh::kULoads * 256];
   __shared__ __attribute__((aligned(16))) uint4 ps[Sh::kPLoads * 64];
   const int h = blockIdx.x / nrb;
-  const int k0 = (blockIdx.x - h * nrb) * qy::kRowsPerWG;
+  int k0 = (blockIdx.x - h * nrb) * qy::kRowsPerWG;
   const int64_t b = blockIdx.y;
-  const int cnt = (h < T_R ? (T_R - h + B - 1) / B : 0) - k0;   // rows of this block
-  if (cnt <= 0) return;
+  const int all = LIST ? (int)(roffs[h + 1] - roffs[h]) : h < T_R ? (T_R - h + B - 1) / B : 0;
+  if (k0 >= all) return;
+  const int32_t* hrows = LIST ? rows + roffs[h] : nullptr;
   const int w = __builtin_amdgcn_readfirstlane(wave_id());
   __builtin_assume(w >= 0 && w < Sh::kWaves);
   const int lane = lane_id();
   const float* Uh = U + (b * B + h) * u_ld;
-  const In* phih = phi + b * q_sb + ((int64_t)h + (int64_t)k0 * B) * q_st;
+  const In* phib = phi + b * q_sb;
+  float* Yb = Y + b * y_sb;
+  // the row of term k of the type
+  auto row_of = [&](int k) { return LIST ? (int64_t)hrows[k] : (int64_t)h + (int64_t)k * B; };
 #pragma unroll
   for (int u = 0; u < (Sh::kULoads + Sh::kWaves - 1) / Sh::kWaves; ++u) {
     const int I = w + Sh::kWaves * u;
@@ -212,86 +221,91 @@ __global__ __launch_bounds__(64 * (NW + 1)) void query_tile_kernel(
       lds_dma16<true>(Uh + 4 * (c < Sh::kUChunks ? c : 0), us + 256 * I);
     }
   }
+  do {
+    const int cnt = all - k0;                          // rows of this block, or more
 #pragma unroll
-  for (int u = 0; u < (Sh::kPLoads + Sh::kWaves - 1) / Sh::kWaves; ++u) {
-    const int I = w + Sh::kWaves * u;
-    if (I < Sh::kPLoads) {
-      const int row = (64 / RC) * I + lane / RC;
-      int k = (lane % RC) ^ qt::swz<RC>(row);
-      if (2 * NW < RC && k >= 2 * NW) k -= 8;        // past the row: one of its own
-      lds_dma16<true>(phih + (int64_t)(row < cnt ? row : 0) * B * q_st + 8 * k, ps + 64 * I);
-    }
-  }
-  wait_vmcnt<0>();
-  lds_barrier();
-
-  const int r16 = lane & 15, g = lane >> 4;
-  const int c = 16 * w + r16;
-  // Lane group g takes the k-slots of feature group pg of each 32, as in the
-  // streaming kernel (rows of U_h 16 apart fall on disjoint banks: 16 p is 16
-  // modulo the 64 banks at every one of these widths).
-  const int pg = (g >> 1) | ((g & 1) << 1);
-  f32x4 acc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = zero4();
-  // the hi and lo parts of n <= 8 rows of U_h from row a
-  auto u_frag = [&](Frag& ah, Frag& al, int a, int n) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float uv = e < n && c < kP ? us[(a + e) * kP + c] : 0.f;
-      In hh, ll;
-      split2<In>(uv, hh, ll);
-      ah[e] = hh;
-      al[e] = ll;
-    }
-  };
-#pragma unroll
-  for (int kb = 0; kb < NW / 2; ++kb) {
-    Frag ah, al;
-    u_frag(ah, al, 32 * kb + 8 * pg, 8);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int row = 16 * t + r16;
-      const Frag pb =
-          *reinterpret_cast<const Frag*>(ps + row * RC + ((4 * kb + pg) ^ qt::swz<RC>(row)));
-      acc[t] = mma(acc[t], ah, pb);
-      acc[t] = mma(acc[t], al, pb);
-    }
-  }
-  if constexpr (NW % 2 != 0) {
-    // the last 16 features: a k-block whose upper halves are zero
-    Frag ah, al;
-    u_frag(ah, al, 16 * (NW - 1) + 4 * g, 4);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int row = 16 * t + r16;
-      const char* src = reinterpret_cast<const char*>(
-          ps + row * RC + ((2 * (NW - 1) + (g >> 1)) ^ qt::swz<RC>(row)));
-      const Half ph = *reinterpret_cast<const Half*>(src + 8 * (g & 1));
-      Frag pb;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        pb[e] = ph[e];
-        pb[4 + e] = from_f32<In>(0.f);
+    for (int u = 0; u < (Sh::kPLoads + Sh::kWaves - 1) / Sh::kWaves; ++u) {
+      const int I = w + Sh::kWaves * u;
+      if (I < Sh::kPLoads) {
+        const int row = (64 / RC) * I + lane / RC;
+        int k = (lane % RC) ^ qt::swz<RC>(row);
+        if (2 * NW < RC && k >= 2 * NW) k -= 8;        // past the row: one of its own
+        lds_dma16<true>(phib + row_of(k0 + (row < cnt ? row : 0)) * q_st + 8 * k, ps + 64 * I);
       }
-      acc[t] = mma(acc[t], ah, pb);
-      acc[t] = mma(acc[t], al, pb);
     }
-  }
-  float* Yb = Y + b * y_sb;
-  const int c0 = 16 * w + 4 * g;
+    wait_vmcnt<0>();
+    lds_barrier();
+
+    const int r16 = lane & 15, g = lane >> 4;
+    const int c = 16 * w + r16;
+    // Lane group g takes the k-slots of feature group pg of each 32, as in the
+    // streaming kernel (rows of U_h 16 apart fall on disjoint banks: 16 p is 16
+    // modulo the 64 banks at every one of these widths).
+    const int pg = (g >> 1) | ((g & 1) << 1);
+    f32x4 acc[4];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int k = 16 * t + r16;
-    if (k < cnt) {
-      float* yrow = Yb + ((int64_t)h + (int64_t)(k0 + k) * B) * y_st;
-      if (w < NW)
-        *reinterpret_cast<float4*>(yrow + c0) =
-            make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
-      else if (g == 0)
-        yrow[c0] = acc[t][0];
+    for (int t = 0; t < 4; ++t) acc[t] = zero4();
+    // the hi and lo parts of n <= 8 rows of U_h from row a
+    auto u_frag = [&](Frag& ah, Frag& al, int a, int n) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float uv = e < n && c < kP ? us[(a + e) * kP + c] : 0.f;
+        In hh, ll;
+        split2<In>(uv, hh, ll);
+        ah[e] = hh;
+        al[e] = ll;
+      }
+    };
+#pragma unroll
+    for (int kb = 0; kb < NW / 2; ++kb) {
+      Frag ah, al;
+      u_frag(ah, al, 32 * kb + 8 * pg, 8);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int row = 16 * t + r16;
+        const Frag pb =
+            *reinterpret_cast<const Frag*>(ps + row * RC + ((4 * kb + pg) ^ qt::swz<RC>(row)));
+        acc[t] = mma(acc[t], ah, pb);
+        acc[t] = mma(acc[t], al, pb);
+      }
     }
-  }
+    if constexpr (NW % 2 != 0) {
+      // the last 16 features: a k-block whose upper halves are zero
+      Frag ah, al;
+      u_frag(ah, al, 16 * (NW - 1) + 4 * g, 4);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int row = 16 * t + r16;
+        const char* src = reinterpret_cast<const char*>(
+            ps + row * RC + ((2 * (NW - 1) + (g >> 1)) ^ qt::swz<RC>(row)));
+        const Half ph = *reinterpret_cast<const Half*>(src + 8 * (g & 1));
+        Frag pb;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          pb[e] = ph[e];
+          pb[4 + e] = from_f32<In>(0.f);
+        }
+        acc[t] = mma(acc[t], ah, pb);
+        acc[t] = mma(acc[t], al, pb);
+      }
+    }
+    const int c0 = 16 * w + 4 * g;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int k = 16 * t + r16;
+      if (k < cnt) {
+        typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));   // list rows start anywhere
+        float* yrow = Yb + row_of(k0 + k) * y_st;
+        if (w < NW)
+          *reinterpret_cast<f4*>(yrow + c0) = acc[t];
+        else if (g == 0)
+          yrow[c0] = acc[t][0];
+      }
+    }
+    if (!LIST) break;
+    k0 += nrb * qy::kRowsPerWG;
+    if (k0 < all) lds_barrier();                       // every wave is done with the rows
+  } while (k0 < all);
 }
 
 // ---------------------------------------------------------------------------
@@ -587,6 +601,16 @@ static int launch_query_lists(const void* phi, const float* U, float* Y, const i
     return SMAT_EUNSUPPORTED;
   }
   if (gx == 0) return SMAT_OK;
+  if constexpr (sizeof(In) == 2) {
+    // the tile kernel's one list width: the training shape
+    if (r == 64 && p == 65 && rows_vec_ok(phi, 0, q_st, 2) && aligned16(U) &&
+        variant(SMAT_VARIANT_QUERY) == 0) {
+      smat::launch((query_tile_kernel<In, 4, true>), dim3((unsigned)gx, 1u), dim3(64 * 5), 0,
+                   stream, (const In*)phi, U, Y, 0, ntypes, (int64_t)r * p, (int64_t)0, q_st,
+                   (int64_t)0, y_st, nrb, rows, roffs);
+      return launch_status("smat_query_lists");
+    }
+  }
   const int vq = rows_vec_ok(phi, 0, q_st, sizeof(In));
   if (r <= 64 && p <= 80)
     smat::launch((query_kernel<In, 2, 5, true>), dim3((unsigned)gx, 1u), dim3(qy::kThreads), 0,
@@ -678,8 +702,9 @@ static int launch_query_tile(const void* phi, const float* U, float* Y, int nb, 
   const dim3 grid((unsigned)gx, (unsigned)nb);
 #define SMAT_QT(NWV)                                                                           \
   case NWV:                                                                                    \
-    smat::launch((query_tile_kernel<In, NWV>), grid, dim3(64 * (NWV + 1)), 0, stream,          \
-                 (const In*)phi, U, Y, T_R, B, u_ld, q_sb, q_st, y_sb, y_st, nrb);             \
+    smat::launch((query_tile_kernel<In, NWV, false>), grid, dim3(64 * (NWV + 1)), 0, stream,   \
+                 (const In*)phi, U, Y, T_R, B, u_ld, q_sb, q_st, y_sb, y_st, nrb, nullptr,     \
+                 nullptr);                                                                     \
     break;
   switch (r / 16) {
     SMAT_QT(4)

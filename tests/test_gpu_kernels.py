@@ -1261,3 +1261,32 @@ def test_combine_normalise_row_widths(dt, p):
     for a, b, m in ((Hd.grad, H64.grad, keep), (Yd.grad, Y64.grad, keep[:, n:])):
         assert _rel(a.cpu()[m].to(DEV), b[m]) < 1e-5
     assert _rel(Hd.grad[0, 3, :-1], H64.grad[0, 3, :-1]) < 1e-5 and Hd.grad[0, 3, -1] == 0
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("maxcnt", [0, 64, 100, 400])
+def test_query_lists_at_row_block_edges(dt, maxcnt):
+    """smat_query_lists at the training shape over lists that end at and beside its
+    64-row blocks (empty ones too), with grids sized too small and too large, Y
+    rows 65 floats apart: against fp64 within 2e-5 of the largest entry (U enters
+    split hi/lo), rows in no list untouched."""
+    from smat_attention_amd.kernels.hip_fwd import DTYPE_CODE, call, stream_of
+    r, p = 64, 65
+    counts = [0, 1, 15, 16, 63, 64, 65, 0, 127, 128, 129, 200]
+    L = sum(counts) + 9
+    gen = torch.Generator().manual_seed(maxcnt)
+    rows = torch.randperm(L, generator=gen)[:sum(counts)]
+    X = (torch.rand(L, r, generator=gen) + 0.1).to(dt)
+    U = torch.randn(len(counts), r, p, generator=gen)
+    Y = torch.full((L, p), 3.0, device=DEV)
+    x, u, rw = X.to(DEV), U.to(DEV), rows.int().to(DEV)
+    offs = torch.tensor([0] + counts).cumsum(0).to(DEV)
+    call("smat_query_lists", DTYPE_CODE[dt], x.data_ptr(), u.data_ptr(), Y.data_ptr(),
+         rw.data_ptr(), offs.data_ptr(), len(counts), maxcnt, r, p, r, p, stream_of(Y))
+    want = torch.full((L, p), 3.0, dtype=torch.float64)
+    kind = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))
+    want[rows] = (X.double()[rows].unsqueeze(1) @ U.double()[kind]).squeeze(1)
+    assert _rel(Y, want) < 2e-5
+    left = torch.ones(L, dtype=torch.bool)
+    left[rows] = False
+    assert (Y.cpu()[left] == 3).all()
