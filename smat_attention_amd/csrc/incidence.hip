@@ -353,11 +353,21 @@ constexpr int kQMax = 41;         // largest q whose four planes fit the LDS
 // and more items' loads are in flight: 193 -> 149 us at q = 13 (96 sequences,
 // head size 64), 160 -> 150 us at q = 23 (8 of 128).  Two workgroups at q = 29
 // (the panels fill the LDS exactly) ran as one does, 234 us.
-template <int Q>
+// Between q = 17 and 23 that turns around where F and U outgrow the memory-side
+// cache several times over: an item takes as many times longer as there are
+// workgroups, so the other half of a 128-byte line, which the neighbouring item
+// reads or writes, more often finds the line gone from the L2.  At 12 and 16
+// sequences of head size 128 (0.5-0.65 GB) 118 and 154 us against 128 and 166 at
+// q = 17; at 32 to 64 (2.3-2.9 GB) 719 against 615 at q = 17, 845 against 661 at
+// q = 19, 642 against 582 at q = 23.  One workgroup of 1024 threads runs those
+// (WIDE; at q <= 13 the smaller ones win at every size).
+constexpr int64_t kWideBytes = 768ll << 20;
+constexpr bool has_wide(int q) { return q >= 17 && q <= 23; }
+template <int Q, bool WIDE = false>
 struct Shape {
-  static constexpr int kThreads = Q <= 19 ? 256 : Q <= 23 ? 512 : 1024;
+  static constexpr int kThreads = WIDE ? 1024 : Q <= 19 ? 256 : Q <= 23 ? 512 : 1024;
   static constexpr int kWaves = kThreads / 64;
-  static constexpr int kWgs = Q <= 17 ? 4 : Q <= 19 ? 3 : Q <= 23 ? 2 : 1;   // on a CU
+  static constexpr int kWgs = WIDE ? 1 : Q <= 17 ? 4 : Q <= 19 ? 3 : Q <= 23 ? 2 : 1;   // on a CU
   static constexpr int kPF = (Q * Q * kPlanes + kThreads - 1) / kThreads;   // chunks a thread
   static constexpr int kCW = (Q + 15 + 1) / 2 * 2;       // entries per column: even, >= q + 15
   static constexpr int kPlane = (kCW * Q + 15) / 16 * 16;
@@ -517,8 +527,8 @@ struct LgGroup {
 // consecutive entries of one plane.  Its F offset in bytes (4 N0 rp < 2^32,
 // checked on the host) is 4 (x*rp + 4*kx) for the point x = x0*q + x1; its LDS
 // entry is kx*kPlane + kCW*x1 + x0, with copies at + q, + 2q, ... below q + 15.
-template <int Q>
-using LgSlot = LgDiv<Q, 16 * iw::Shape<Q>::kWaves * iw::Shape<Q>::kPF>;
+template <int Q, bool WIDE>
+using LgSlot = LgDiv<Q, 16 * iw::Shape<Q, WIDE>::kWaves * iw::Shape<Q, WIDE>::kPF>;
 
 // Byte offsets into one sequence's F panel rows and U type rows are 32-bit;
 // ld is their row stride in floats.
@@ -618,15 +628,15 @@ __device__ __forceinline__ LrLane own_lane(int li, int& code) {
   return ln;
 }
 
-template <int Q, bool HasG>
-__global__ __launch_bounds__(iw::Shape<Q>::kThreads,
-                             iw::Shape<Q>::kWgs * iw::Shape<Q>::kWaves / 4)
+template <int Q, bool HasG, bool WIDE>
+__global__ __launch_bounds__((iw::Shape<Q, WIDE>::kThreads),
+                             (iw::Shape<Q, WIDE>::kWgs * iw::Shape<Q, WIDE>::kWaves / 4))
 void incidence_wave_kernel(
     const float* __restrict__ F, const float* __restrict__ Fg, const int* __restrict__ code,
     float* __restrict__ U, int B, int64_t rp, int64_t ld, int nslices, int64_t total,
     int64_t per_xcd) {
   using namespace iw;
-  typedef Shape<Q> Sh;
+  typedef Shape<Q, WIDE> Sh;
   constexpr int kThreads = Sh::kThreads, kWaves = Sh::kWaves, kPF = Sh::kPF, kCW = Sh::kCW;
   constexpr int kPlane = Sh::kPlane, kPlaneBytes = Sh::kPlaneBytes;
   constexpr uint32_t kSlots = kThreads / 4;          // slots from one chunk to the next
@@ -673,7 +683,7 @@ void incidence_wave_kernel(
   float4 pf[kPF];
   uint32_t src[kPF];
   auto chunk_src = [&](uint32_t ps) {
-    const uint32_t x1 = LgSlot<Q>::div(ps), x0 = ps - Q * x1;
+    const uint32_t x1 = LgSlot<Q, WIDE>::div(ps), x0 = ps - Q * x1;
     return __umul24(x0 * Q + x1, ld4) + 16u * kx;   // 4 (x ld + 4 kx)
   };
   auto prefetch = [&](int64_t item) {
@@ -771,7 +781,7 @@ void incidence_wave_kernel(
 #pragma unroll
       for (int u = 0; u < kPF; ++u) {
         const uint32_t ps = p0 + kSlots * u;
-        const uint32_t x1 = LgSlot<Q>::div(ps), x0 = ps - Q * x1;
+        const uint32_t x1 = LgSlot<Q, WIDE>::div(ps), x0 = ps - Q * x1;
         if (ps < (uint32_t)N0) {
           float4* e = smem + (kx * kPlane + kCW * x1 + x0);
 #pragma unroll
@@ -841,28 +851,34 @@ void incidence_wave_kernel(
   }
 }
 
-template <int Q>
+template <int Q, bool WIDE = false>
 static int launch_wave_q(const float* F, const float* F_glob, const int* code, float* U, int nb,
                          int B, int64_t rp, int64_t ld, hipStream_t stream) {
   using namespace iw;
+  if constexpr (has_wide(Q) && !WIDE) {
+    if ((int64_t)nb * (Q * Q + B) * ld * 4 > kWideBytes)
+      return launch_wave_q<Q, true>(F, F_glob, code, U, nb, B, rp, ld, stream);
+  }
   const int nslices = (int)((rp + kE - 1) / kE);
   const int64_t total = (int64_t)nb * nslices;
   int dev = 0, ncu = 256;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   const int64_t per_xcd = (total + inc::kXCD - 1) / inc::kXCD;
-  const int64_t per_xcd_wgs = std::max<int64_t>(1, std::min<int64_t>((int64_t)ncu * Shape<Q>::kWgs / inc::kXCD, per_xcd));
+  const int64_t per_xcd_wgs = std::max<int64_t>(
+      1, std::min<int64_t>((int64_t)ncu * Shape<Q, WIDE>::kWgs / inc::kXCD, per_xcd));
   const unsigned grid = (unsigned)(per_xcd_wgs * inc::kXCD);
-  const size_t smem = (size_t)Shape<Q>::kLdsBytes;
+  const size_t smem = (size_t)Shape<Q, WIDE>::kLdsBytes;
   static bool attr_set[2] = {false, false};
-  auto kern = F_glob ? incidence_wave_kernel<Q, true> : incidence_wave_kernel<Q, false>;
+  auto kern = F_glob ? incidence_wave_kernel<Q, true, WIDE>
+                     : incidence_wave_kernel<Q, false, WIDE>;
   if (!attr_set[F_glob ? 1 : 0]) {
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                               inc::kPlaneLdsBudget);
     attr_set[F_glob ? 1 : 0] = true;
   }
-  smat::launch(kern, dim3(grid), dim3(Shape<Q>::kThreads), smem, stream, F, F_glob, code, U, B, rp, ld,
-                     nslices, total, per_xcd);
+  smat::launch(kern, dim3(grid), dim3(Shape<Q, WIDE>::kThreads), smem, stream, F, F_glob, code, U,
+               B, rp, ld, nslices, total, per_xcd);
   return launch_status("smat_incidence_plane");
 }
 

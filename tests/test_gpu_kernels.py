@@ -1290,3 +1290,24 @@ def test_query_lists_at_row_block_edges(dt, maxcnt):
     left = torch.ones(L, dtype=torch.bool)
     left[rows] = False
     assert (Y.cpu()[left] == 3).all()
+
+
+@pytest.mark.parametrize("T,q,nb", [(5000, 17, 24), (10007, 19, 20), (16384, 23, 14)])
+@pytest.mark.parametrize("glob", [False, True])
+def test_incidence_line_groups_above_the_cache(T, q, nb, glob):
+    """Between q = 17 and 23 F and U of more than 768 MB take one workgroup of 1024
+    threads a CU: the first, a middle and the last sequence are bitwise those of a
+    launch of one sequence, which takes the small workgroups (the same sums in the
+    same order)."""
+    _say("incidence line groups, large", T, q, nb, glob)
+    spec = A.to_device(build_mask(T, 3, chunk=128), DEV)
+    assert spec.q == q and nb * (spec.N0 + spec.B) * 128 * 129 * 4 > 768 << 20
+    assert (nb // 2) * (spec.N0 + spec.B) * 128 * 129 * 4 < 768 << 20
+    g = torch.Generator(device=DEV).manual_seed(q)
+    F = torch.randn(nb, spec.N0, 128, 129, device=DEV, generator=g)
+    Fg = torch.randn(nb, 128, 129, device=DEV, generator=g) if glob else None
+    U = K.incidence_plane(F, spec.plane_code_t, spec.q, F_glob=Fg)
+    for i in (0, nb // 2, nb - 1):
+        one = K.incidence_plane(F[i:i + 1], spec.plane_code_t, spec.q,
+                                F_glob=Fg[i:i + 1] if glob else None)
+        assert torch.equal(U[i:i + 1], one), i

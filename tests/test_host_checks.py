@@ -352,22 +352,22 @@ def test_line_group_incidence_reads_each_line_once_in_bounds(q):
     assert sorted(stored) == list(range(q * (q + 1))) and set(stored.values()) == {1}
 
 
-def _line_group_shape(q):
-    """(threads, workgroups a CU, chunks a thread, kCW, kPlane) of iw::Shape<q>."""
-    threads = 256 if q <= 19 else 512 if q <= 23 else 1024
-    wgs = 4 if q <= 17 else 3 if q <= 19 else 2 if q <= 23 else 1
+def _line_group_shape(q, wide):
+    """(threads, workgroups a CU, chunks a thread, kCW, kPlane) of iw::Shape<q, wide>."""
+    threads = 1024 if wide else 256 if q <= 19 else 512 if q <= 23 else 1024
+    wgs = 1 if wide else 4 if q <= 17 else 3 if q <= 19 else 2 if q <= 23 else 1
     cw = (q + 15 + 1) // 2 * 2
     return threads, wgs, -(-q * q * 4 // threads), cw, -(-cw * q // 16) * 16
 
 
-@pytest.mark.parametrize("q", _WAVE_Q)
-def test_line_group_incidence_shapes_by_field_size(q, monkeypatch):
+@pytest.mark.parametrize("q,wide", [(q, False) for q in _WAVE_Q] + [(q, True) for q in (17, 19, 23)])
+def test_line_group_incidence_shapes_by_field_size(q, wide, monkeypatch):
     """The panel shape and thread count of each field size: the panels of a CU's
     workgroups fit its 160 KB of LDS and the 16-bit read offset, the line table
     (which shares the panel's first bytes before the first item) fits a panel,
     the staging covers every (point, plane) once, and every read lands on a
     staged entry, each line on its own q points."""
-    threads, wgs, pf, cw, plane = _line_group_shape(q)
+    threads, wgs, pf, cw, plane = _line_group_shape(q, wide)
     waves = threads // 64
     monkeypatch.setitem(globals(), "_KCW", cw)
     monkeypatch.setitem(globals(), "_KPLANE", plane)
