@@ -51,11 +51,13 @@ const char* smat_version(void);
  * the two on the same inputs.  value 1 selects the general kernel, 0 (the
  * default) the specialised one; returns the previous value, or SMAT_EINVAL.
  *   SMAT_VARIANT_SCAN             general fused causal scan instead of the
- *                                 head_dim-128 streaming scan
+ *                                 streaming scan (head sizes 64 to 128)
  *   SMAT_VARIANT_GRAM             general Gram kernel instead of the
- *                                 head_dim-128 streaming pool / prepass
+ *                                 streaming pool / prepass (80 to 128) and
+ *                                 the one at 64
  *   SMAT_VARIANT_QUERY            general query kernel instead of the
- *                                 head_dim-128 streaming query
+ *                                 streaming query (128) and the tile one
+ *                                 (64 to 112, row lists at 64)
  *   SMAT_VARIANT_INCIDENCE        L2 gather kernel instead of the LDS panel
  *   SMAT_VARIANT_INCIDENCE_PLANE  line-per-lane generated-line kernel instead
  *                                 of the line-group one
@@ -468,8 +470,9 @@ int64_t smat_forward_workspace_bytes(int nb, int T, int n, int N0, int B, int n_
  * dispatch gaps between them (stage 0: from an event the caller records
  * before the call).  The device-side counterpart of the timer argument of
  * smat_attention (src/smat/attention.py:391-455, whose phases lr_pool,
- * lr_incidence, lr_query and scan + normalise these stages are).  Stages a
- * call does not run (no recent rows) record nothing.  n = 0 clears them; at
+ * lr_incidence, lr_query and scan + normalise these stages are).  A small
+ * problem's chunk-group summaries share the pool's launch and count to stage 0.
+ * Stages a call does not run (no recent rows) record nothing.  n = 0 clears them; at
  * most 8.  The caller keeps the events alive while they are set.
  */
 int smat_set_stage_events(void* const* events, int n);
