@@ -470,7 +470,9 @@ int gram_stream_launch_feat(int dtype, const void* k, const void* v, float* G, f
 // x (K + 1), the smallest such K.  The rounds: a workgroup a CU at head size 128
 // (8 sequences of 32768 tokens: forward 641 -> 599 us with 256 groups in place
 // of 1024, 613 with 512), four for the narrow shape (8192 tokens, 32 sequences:
-// 164.0 us with 1024 groups, 166.2 with 512).  n is not an argument (the
+// 164.0 us with 1024 groups, 166.2 with 512; eight at r <= 48 gained 4 % on 4 x
+// 41344 tokens of 32 and lost 4 % on 8 x 65536, 8 % on 8 x 32768 of 48).  n is
+// not an argument (the
 // workspace is sized without it): the groups are counted as if it split the
 // chunks in half, where build_mask puts it.
 //
