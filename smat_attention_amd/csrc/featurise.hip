@@ -18,9 +18,10 @@
 // HBM-bound: 2 (T d_qk + T r) + T (d_v + p) elements per sequence, so what
 // counts is bytes in flight against the number of places written at once: at 96
 // sequences of 4096 tokens, all widths 64, 71 us (the bytes at a copy's rate:
-// 63); with the longer elu it then had, 79 with four workgroups a CU resident and none waiting; 85 with three of
-// them, 84 with twelve in turn, 93 with six resident; 99 with one row tile a
-// wave, 8-byte stores and W's LDS sized for 128 features.
+// 63).  With the longer elu it then had: 79 with four workgroups a CU resident
+// and none waiting, 85 with three of them, 84 with twelve in turn, 93 with six
+// resident; 99 with one row tile a wave, 8-byte stores and W's LDS sized for 128
+// features.
 #include <math.h>
 
 #include "feat_map.hpp"

@@ -472,9 +472,8 @@ int gram_stream_launch_feat(int dtype, const void* k, const void* v, float* G, f
 // of 1024, 613 with 512), four for the narrow shape (8192 tokens, 32 sequences:
 // 164.0 us with 1024 groups, 166.2 with 512; eight at r <= 48 gained 4 % on 4 x
 // 41344 tokens of 32 and lost 4 % on 8 x 65536, 8 % on 8 x 32768 of 48).  n is
-// not an argument (the
-// workspace is sized without it): the groups are counted as if it split the
-// chunks in half, where build_mask puts it.
+// not an argument (the workspace is sized without it): the groups are counted
+// as if it split the chunks in half, where build_mask puts it.
 //
 // The one-call forward takes up to kForwardK: past 32 the uneven halves (only
 // recent rows read Y) cost more than the states (524288 tokens: 5810 us at 32,
