@@ -687,6 +687,7 @@ def _fused_ok(Q, K, V, phi, spec, C, h) -> bool:
     # 256 of them the unfused pool's split-K reduction is the faster path --
     # except for one profile holding every landmark token (d = 1, no global
     # channel), whose forward is the causal pass without its reset and no pool
+    # (fp16: its pool is summed from that pass's chunk-group summaries)
     one_profile = spec.N0 == 1 and spec.B == 1 and spec.n_P == 0
     if T > spec.n and spec.n > spec.n_P and nb * spec.N0 < 256 and not one_profile:
         return False
@@ -711,7 +712,8 @@ def smat_attention_fused(Q, K, V, phi, spec: MaskSpec, *, g=None, h=None, chunk:
     chunk groups, up to the order of the fp32 state sums) while Phi, Psi and Vb
     never reach memory (where a row type has more than 64 recent rows, the recent rows'
     Phi alone is featurised for the general query kernel; at d = 1 the causal
-    pass without its reset is the whole forward).  Other inputs --
+    pass without its reset is the whole forward, in fp16 with its reset and a pool
+    summed from its chunk-group summaries).  Other inputs --
     other widths and dtypes, fewer than 256 (sequence, profile) pools with
     more than one profile or a global channel -- and inputs that require grad
     run :func:`featurise` then :func:`smat_attention`.  Returns fp32 (nb, T, d_v).

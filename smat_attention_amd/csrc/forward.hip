@@ -90,7 +90,14 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
                          int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb,
                          int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb, int64_t o_st,
                          int64_t g_sb, const FeatArgs& fa, void* ws, int64_t ws_bytes,
-                         void* psi_buf, hipStream_t stream);
+                         void* psi_buf, bool have_G, hipStream_t stream);
+int causal_scan_feat_summaries(int dtype, const void* k, const void* v, int nb, int T, int n,
+                               int C, int64_t k_sb, int64_t k_st, int64_t v_sb, int64_t v_st,
+                               const FeatArgs& fa, void* ws, void* psi_buf, float* F,
+                               int64_t f_sb, hipStream_t stream);
+int causal_scan_pool(int dtype, const void* psi, const void* vb, const GramPart& P, float* F,
+                     int64_t f_sb, int nb, int r, int p, int64_t k_sb, int64_t k_st, int64_t v_sb,
+                     int64_t v_st, hipStream_t stream);
 int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, int kmax);
 int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void* vb,
                          const float* Y, const float* gate, float* out, int nb, int T, int n,
@@ -112,9 +119,22 @@ static inline int64_t al256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 static inline int64_t y_stride(int p) { return (p + 3) & ~3; }
 
 // Every recent row reads the state of all landmark tokens: the identity
-// incidence (no table) over one profile, no global channel.
-static bool one_state(const void* idx, int N0, int B, int n_P) {
-  return !idx && N0 == 1 && B == 1 && n_P == 0;
+// incidence (no table) over one profile, no global channel (d = 1).  U = F is
+// then the state at n, and adding Phi F to the recent rows is the scan carried
+// on past n without its reset: the causal pass over one segment is the whole
+// forward, with no pool, no query (198 us at 8 x 131072 tokens of head size 128)
+// and no Y (0.55 GB there); 701 -> 407 us.
+// Not in fp16, whose states and tables enter the products as hi + lo parts up to
+// 65504 an entry: the one segment's state sums twice the tokens F or either of two
+// segments' does, so a sum that fits those can overflow there.
+static bool one_segment(const void* idx, int N0, int B, int n_P, int dtype) {
+  return !idx && N0 == 1 && B == 1 && n_P == 0 && dtype != SMAT_F16;
+}
+// The same single profile where the segments stay apart: F is the sum of the
+// causal pass's summaries of the tokens [0, n), added as float4, and no pool pass
+// is made.
+static bool pool_from_summaries(const void* idx, int N0, int n_P, int T, int n, int64_t rp) {
+  return !idx && N0 == 1 && n_P == 0 && n > 0 && T > n && rp % 4 == 0;
 }
 
 // kmax: the causal pass's largest group, kForwardK or kFeatK.
@@ -252,13 +272,7 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
   const int64_t yst = y_stride(p);
   int rc;
 
-  // One profile holding every landmark token and one row type reading it (d = 1,
-  // no global channel, the identity incidence): U = F is the state at n, so
-  // adding Phi F to the recent rows is the scan carried on past n without its
-  // reset.  The causal pass over one segment is the whole forward: no pool, no
-  // query (198 us at 8 x 131072 tokens of head size 128) and no Y (0.55 GB
-  // there): 699 -> 459 us.
-  if (L.fused && one_state(idx, N0, B, n_P)) {
+  if (L.fused && one_segment(idx, N0, B, n_P, dtype)) {
     StageScope stage(3);
     return causal_scan_dispatch(dtype, phi, psi, vb, nullptr, g, out, nb, T, 0, C, r, p, q_sb,
                                 q_st, k_sb, k_st, v_sb, v_st, 0, 0, o_sb, o_st, g_sb, 0,
@@ -278,7 +292,12 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
       StageScope stage(0);
       // a small problem's profile sums and chunk-group summaries in one launch
       rc = SMAT_OK;
-      if (L.fused)
+      if (L.fused && pool_from_summaries(idx, N0, n_P, T, n, rp)) {
+        have_G = true;
+        rc = causal_scan_pool(
+            dtype, psi, vb, causal_scan_part(dtype, nb, T, n, C, r, p, kForwardK, ws + L.scan), F,
+            ld, nb, r, p, k_sb, k_st, v_sb, v_st, st);
+      } else if (L.fused)
         rc = gram_pair_dispatch(
             dtype, psi, vb, pool_part(F, Fg, nb, n_P, n, N0, r, p, ld),
             causal_scan_part(dtype, nb, T, n, C, r, p, kForwardK, ws + L.scan), nb, r, p, k_sb,
@@ -461,19 +480,24 @@ extern "C" int smat_forward_fused(int dtype, const void* q, const void* k, const
   int rc;
 
   void* psi_rows = ws + L.total + fused_phi_bytes(nb, T, n, B);
-  // One state (d = 1): the causal pass without its reset, as in smat_forward.
-  if (one_state(idx, N0, B, n_P)) {
+  if (one_segment(idx, N0, B, n_P, dtype)) {         // as in smat_forward
     StageScope stage(3);
     return causal_scan_run_feat(dtype, q, k, v, nullptr, g, out, nb, T, 0, C, q_sb, q_st, k_sb,
                                 k_st, v_sb, v_st, 0, 0, o_sb, o_st, g_sb, fa, ws + L.scan,
-                                L.part - L.scan, psi_rows, st);
+                                L.part - L.scan, psi_rows, false, st);
   }
+  bool have_G = false;                               // the causal pass's chunk-group summaries
   if (T_R > 0) {
     const bool profiled = n > n_P;
     // row stride of F and U
     const int64_t ld =
         idx && plane_code && profiled ? incidence_plane_ld(field_q, N0, B, rp) : rp;
-    {
+    if (pool_from_summaries(idx, N0, n_P, T, n, rp)) {
+      StageScope stage(0);
+      have_G = true;
+      rc = causal_scan_feat_summaries(dtype, k, v, nb, T, n, C, k_sb, k_st, v_sb, v_st, fa,
+                                      ws + L.scan, psi_rows, F, ld, st);
+    } else {
       GramItems it{};
       it.mode = 1;
       it.n_P = n_P;
@@ -520,5 +544,5 @@ extern "C" int smat_forward_fused(int dtype, const void* q, const void* k, const
   StageScope stage(3);
   return causal_scan_run_feat(dtype, q, k, v, T_R > 0 ? Y : nullptr, g, out, nb, T, n, C, q_sb,
                               q_st, k_sb, k_st, v_sb, v_st, (int64_t)T_R * yst, yst, o_sb, o_st,
-                              g_sb, fa, ws + L.scan, L.part - L.scan, psi_rows, st);
+                              g_sb, fa, ws + L.scan, L.part - L.scan, psi_rows, have_G, st);
 }

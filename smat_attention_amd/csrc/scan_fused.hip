@@ -446,6 +446,10 @@ int chunk_states_dispatch(int dtype, const void* psi, const void* vb, float* D, 
                           int C, int K, int n, int r, int p, int64_t k_sb, int64_t k_st,
                           int64_t v_sb, int64_t v_st, hipStream_t stream);
 GramPart chunk_part(float* D, int T, int C, int K, int n, int r, int p);
+int gram_dispatch(int dtype, const void* psi, const void* vb, float* G, float* G_last,
+                  const GramItems& it, int nitems, int nb, int r, int p, int64_t k_sb,
+                  int64_t k_st, int64_t v_sb, int64_t v_st, int64_t g_sb, int64_t g_si,
+                  int64_t gl_sb, float* partials, hipStream_t stream, const char* who);
 int segment_scan_dispatch(const float* D, float* Sin, int nb, int nc, int nc0, int64_t rp,
                           hipStream_t stream);
 bool scan_stream_ok(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
@@ -566,6 +570,66 @@ GramPart causal_scan_part(int dtype, int nb, int T, int n, int C, int r, int p, 
   return chunk_part((float*)ws, T, C, scan_group_chunks(nb, (T + C - 1) / C, r, p, kmax), n, r, p);
 }
 
+// F[b] = sum of the group sums G[b][g], g < ng0 (the tokens [0, n)).  A
+// block takes 64 float4 columns of the r*p floats; its four waves sum every
+// fourth group (each wave's loads independent of one another), then wave 0
+// adds the other three partial sums in wave order.
+__global__ __launch_bounds__(256) void group_sum_kernel(const float* __restrict__ G,
+                                                        float* __restrict__ F, int ng0,
+                                                        int64_t rp4, int64_t g_sb,
+                                                        int64_t f_sb) {
+  __shared__ float4 part[3][64];
+  const int64_t b = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6;
+  const int64_t e = (int64_t)blockIdx.x * 64 + lane;
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (e < rp4) {
+    const float4* Gb = reinterpret_cast<const float4*>(G + b * g_sb) + e;
+#pragma unroll 4
+    for (int g = w; g < ng0; g += 4) {
+      const float4 x = Gb[(int64_t)g * rp4];
+      acc.x += x.x;
+      acc.y += x.y;
+      acc.z += x.z;
+      acc.w += x.w;
+    }
+  }
+  if (w > 0) part[w - 1][lane] = acc;
+  __syncthreads();
+  if (w == 0 && e < rp4) {
+    for (int k = 0; k < 3; ++k) {
+      const float4 x = part[k][lane];
+      acc.x += x.x;
+      acc.y += x.y;
+      acc.z += x.z;
+      acc.w += x.w;
+    }
+    reinterpret_cast<float4*>(F + b * f_sb)[e] = acc;
+  }
+}
+
+// One profile's pool from the summaries P of the causal pass (r * p and f_sb
+// multiples of four floats).
+static int group_sum(const GramPart& P, float* F, int64_t f_sb, int nb, int64_t rp,
+                     hipStream_t stream, const char* who) {
+  SMAT_REQUIRE(rp % 4 == 0 && f_sb % 4 == 0, SMAT_EINVAL,
+               "%s: group sums need r*p and the row stride of F a multiple of 4", who);
+  smat::launch(group_sum_kernel, dim3((unsigned)((rp / 4 + 63) / 64), (unsigned)nb), dim3(256), 0,
+               stream, (const float*)P.G, F, P.it.ng0, rp / 4, P.g_sb, f_sb);
+  return launch_status(who);
+}
+
+// The summaries of causal_scan_part formed by themselves, and F[b], the sum over
+// the tokens [0, n) of Psi^T Vb, from them.
+int causal_scan_pool(int dtype, const void* psi, const void* vb, const GramPart& P, float* F,
+                     int64_t f_sb, int nb, int r, int p, int64_t k_sb, int64_t k_st, int64_t v_sb,
+                     int64_t v_st, hipStream_t stream) {
+  const int rc = gram_dispatch(dtype, psi, vb, P.G, nullptr, P.it, P.nitems, nb, r, p, k_sb, k_st,
+                               v_sb, v_st, P.g_sb, P.g_si, 0, nullptr, stream, "smat_forward");
+  return rc ? rc : group_sum(P, F, f_sb, nb, (int64_t)r * p, stream, "smat_forward");
+}
+
 // The causal pass with groups of K chunks; ws holds twice group_bytes: the
 // summaries (already there with have_G), then the states.
 int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
@@ -622,50 +686,57 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
   return SMAT_EINVAL;
 }
 
+// The summaries of the causal pass with the feature map computed inside the
+// kernels (k and v the K and V rows): Psi tiles formed in LDS from the DMA'd K
+// rows, Vb = [V, 1] from V, into ws; the Psi rows also go to psi_buf (nb x T rows
+// of 128, 16-bit).  With F, F[b] is the sum over the tokens [0, n) of Psi^T Vb.
+int causal_scan_feat_summaries(int dtype, const void* k, const void* v, int nb, int T, int n,
+                               int C, int64_t k_sb, int64_t k_st, int64_t v_sb, int64_t v_st,
+                               const FeatArgs& fa, void* ws, void* psi_buf, float* F,
+                               int64_t f_sb, hipStream_t stream) {
+  if (nb == 0 || T == 0) return SMAT_OK;
+  constexpr int r = 128, p = 129;
+  const GramPart P = causal_scan_part(dtype, nb, T, n, C, r, p, kFeatK, ws);
+  FeatArgs fp = fa;
+  fp.psi_out = psi_buf;
+  fp.psi_sb = (int64_t)T * 128;
+  const int rc = gram_stream_launch_feat(dtype, k, v, P.G, nullptr, P.it, P.nitems, nb, k_sb,
+                                         k_st, v_sb, v_st, P.g_sb, P.g_si, 0, fp, stream,
+                                         "smat_forward_fused");
+  if (rc || !F) return rc;
+  return group_sum(P, F, f_sb, nb, (int64_t)r * p, stream, "smat_forward_fused");
+}
+
 // The streaming causal pass with the feature map computed inside the kernels:
-// q, k, v are the Q, K, V rows (r = d_qk = d_v = 128); the prepass Gram sums
-// and the scan form Psi (and Phi) tiles in LDS from the DMA'd K (and Q) rows,
-// and Vb = [V, 1] from V.  The workspace is
-// causal_scan_workspace_bytes' at kFeatK.  The prepass also stores the Psi
-// tiles it forms to psi_buf (nb x T rows of 128, 16-bit) and the scan reads
-// them, forming only Phi.
+// q, k, v are the Q, K, V rows (r = d_qk = d_v = 128).  The summaries as above
+// (already there with have_G); the scan reads their Psi rows from psi_buf and forms
+// only Phi.  The workspace is causal_scan_workspace_bytes' at kFeatK.
 int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v, const float* Y,
                          const float* gate, float* out, int nb, int T, int n, int C,
                          int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb,
                          int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb, int64_t o_st,
                          int64_t g_sb, const FeatArgs& fa, void* ws, int64_t ws_bytes,
-                         void* psi_buf, hipStream_t stream) {
+                         void* psi_buf, bool have_G, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
   constexpr int r = 128, p = 129;
   const int64_t rp = (int64_t)r * p;
   const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, kFeatK);
-  C = scan_chunk(dtype, nb, T, C, r, p);
-  const int nc = (T + C - 1) / C;
-  const int K = scan_group_chunks(nb, nc, r, p, kFeatK);
   if (ws_bytes < need) {
     set_error("smat_forward_fused: causal-pass workspace of %lld bytes needed, %lld given",
               (long long)need, (long long)ws_bytes);
     return SMAT_EINVAL;
   }
-  float* G = (float*)ws;
-  float* Sg = (float*)((char*)ws + group_bytes(nb, nc, K, r, p));
-  GramItems it{};
-  it.mode = 0;
-  it.T = T;
-  it.C = C;
-  it.K = K;
-  it.nc = nc;
-  it.nc0 = n / C;
-  it.ng0 = (it.nc0 + K - 1) / K;
-  it.nsplit = 1;
-  it.per = K * C;
-  const int ng = it.ng0 + (nc - it.nc0 + K - 1) / K;
-  FeatArgs fp = fa;
-  fp.psi_out = psi_buf;
-  fp.psi_sb = (int64_t)T * 128;
-  int rc = gram_stream_launch_feat(dtype, k, v, G, nullptr, it, ng, nb, k_sb, k_st, v_sb, v_st,
-                                   (int64_t)ng * rp, rp, 0, fp, stream, "smat_forward_fused");
+  int rc = have_G ? SMAT_OK
+                  : causal_scan_feat_summaries(dtype, k, v, nb, T, n, C, k_sb, k_st, v_sb, v_st,
+                                               fa, ws, psi_buf, nullptr, 0, stream);
   if (rc) return rc;
+  const GramPart P = causal_scan_part(dtype, nb, T, n, C, r, p, kFeatK, ws);
+  const GramItems& it = P.it;
+  const int ng = P.nitems;
+  C = it.C;
+  const int nc = it.nc, K = it.K;
+  float* G = P.G;
+  float* Sg = (float*)((char*)ws + group_bytes(nb, nc, K, r, p));
   rc = segment_scan_dispatch(G, Sg, nb, ng, it.ng0, rp, stream);
   if (rc) return rc;
   ScanArgs a{};
@@ -680,7 +751,7 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
   a.p = p;
   a.q_sb = q_sb;
   a.q_st = q_st;
-  a.k_sb = fp.psi_sb;
+  a.k_sb = (int64_t)T * 128;
   a.k_st = 128;
   a.v_sb = v_sb;
   a.v_st = v_st;

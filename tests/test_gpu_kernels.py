@@ -641,6 +641,41 @@ def test_forward_one_state(T, hd, dt, gate):
     assert e < tol * (1.5 if gate else 1.0)
 
 
+@pytest.mark.parametrize("hd,fused", [(32, False), (64, False), (96, False), (128, False),
+                                      (128, True)])
+def test_forward_d1_fp16_keeps_its_range(hd, fused):
+    """d = 1 in fp16, whose states and tables enter the products as hi + lo parts up to
+    65504: landmark sums of 51200 and sums of all tokens of 102400 (features near
+    100) give the attention of the same values in fp64, scores rounded once to
+    fp16 (2^-12 each, at most doubled by the division)."""
+    _say("forward d=1 fp16 range", hd, fused)
+    T, dt = 1024, torch.float16
+    spec = build_mask(T, 1, chunk=128)
+    gen = torch.Generator().manual_seed(51)
+    u = lambda *s: torch.rand(*s, generator=gen)
+    if fused:
+        phi = A.FeatureMap(torch.eye(hd, device=DEV, dtype=dt), "elu1")
+        Q, Kk, V = ((-7 + 2 * u(2, T, hd)).to(dt), (90 + 20 * u(2, T, hd)).to(dt),
+                    torch.randn(2, T, hd, generator=gen).to(dt))
+        x = [t.to(DEV) for t in (Q, Kk, V)]
+        assert A._fused_ok(*x, phi, spec, 128, None)
+        got = A.smat_attention_fused(*x, phi, spec)
+        Phi, Psi, Vb = (t.cpu() for t in A.featurise(*x, phi))
+    else:
+        Phi, Psi = (2.0 ** -9 + 2.0 ** -7 * u(2, T, hd)).to(dt), (90 + 20 * u(2, T, hd)).to(dt)
+        Vb = torch.ones(2, T, hd + 8, dtype=dt)
+        Vb[..., :hd] = torch.randn(2, T, hd, generator=gen).to(dt)
+        Vb = Vb[..., :hd + 1]
+        got = A.smat_attention(Phi.to(DEV), Psi.to(DEV),
+                               torch.nn.functional.pad(Vb, (0, 7)).to(DEV)[..., :hd + 1], spec)
+    S = Phi.double() @ Psi.double().transpose(1, 2).contiguous()
+    H = S.tril() @ Vb.double()
+    want = H[..., :-1] / H[..., -1:]
+    e = (got.double().cpu() - want).abs().max().item() / Vb[..., :-1].abs().max().item()
+    _say(f"  rel {e:.2e}")
+    assert torch.isfinite(got).all() and e < 2.0 ** -10
+
+
 def test_forward_single_gpu_d2_bf16():
     """nb=32 (B=4, H=8), T=8192, d=2, head_dim=64, bf16, q,k,v ~ N(0,1)/sqrt(64)."""
     _say("forward T=8192 d=2 nb=32 hd=64 bf16")
