@@ -171,7 +171,8 @@ __global__ __launch_bounds__(256) void normalise_bwd_kernel(
     const f32x4 dc = dv * gate * inv;
     nrm::store4(dh, c, p - 1, dc);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {                    // columns past the end: zeros
+    for (int i = 0; i < 4; ++i) {
+      if (c + i >= p - 1) break;                     // not 0 * inv, which may be NaN
       sh += dc[i] * o[i];
       sg += dv[i] * o[i];
     }

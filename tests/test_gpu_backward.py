@@ -425,6 +425,27 @@ def test_fused_chunk_backward(T, n):
         assert a.dtype == bf and torch.equal(a, b.to(bf)), name
 
 
+@pytest.mark.parametrize("p", [2, 3, 4, 5, 6, 65, 66, 68])
+def test_normalise_backward_of_an_infinite_reciprocal(p):
+    """Rows whose normaliser is zero, infinite or NaN beside an ordinary one: every
+    gradient is fp64's, infinities and NaN included, at row widths whose last
+    access of four values is full and partly empty."""
+    from smat_attention_amd.kernels.hip_fwd import call, stream_of
+    _say("normalise backward, special normalisers", p)
+    H = torch.rand(1, 4, p, generator=torch.Generator().manual_seed(61)) + 1
+    H[0, :3, -1] = torch.tensor([0.0, float("inf"), float("nan")])
+    do, g = torch.full((1, 4, p - 1), 0.75), torch.full((1, 4), 1.5)
+    H64, g64 = H.double().requires_grad_(True), g.double().requires_grad_(True)
+    (H64[..., :-1] / H64[..., -1:] * g64.unsqueeze(-1)).backward(do.double())
+    Hd, dod, gd = H.to(DEV), do.to(DEV), g.to(DEV)
+    dH, dg = torch.empty_like(Hd), torch.empty_like(gd)
+    call("smat_normalise_backward", dod.data_ptr(), Hd.data_ptr(), gd.data_ptr(), dH.data_ptr(),
+         dg.data_ptr(), 1, 4, p, dod.stride(0), dod.stride(1), Hd.stride(0), Hd.stride(1),
+         dH.stride(0), dH.stride(1), gd.stride(0), stream_of(Hd))
+    for got, want in ((dH, H64.grad), (dg, g64.grad)):
+        assert torch.allclose(got.cpu().double(), want, rtol=1e-5, atol=0, equal_nan=True)
+
+
 @pytest.mark.parametrize("nb,nc,pad,split", [(1, 1, 0, 0), (5, 77, 0, 77 * 128), (3, 129, 7, 4130),
                                              (257, 2, 3, 100)])
 def test_chunk_backward_walks_every_chunk(nb, nc, pad, split):
