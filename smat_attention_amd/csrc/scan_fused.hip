@@ -845,8 +845,8 @@ extern "C" int smat_causal_scan_noalloc(int dtype, const void* phi, const void* 
   SMAT_REQUIRE(q_st >= r && k_st >= r && v_st >= p && o_st >= (write_H ? p : p - 1),
                SMAT_EINVAL, "smat_causal_scan_noalloc: a row stride is shorter than its row");
   if (nb == 0 || T == 0) return SMAT_OK;
-  const int nc = (T + C - 1) / C;
-  const int K = noalloc_group_chunks(nb, nc, r, p);
+  C = scan_chunk(dtype, nb, T, C, r, p);             // smat_causal_scan's: the same scores rounded
+  const int K = noalloc_group_chunks(nb, (T + C - 1) / C, r, p);
   SMAT_REQUIRE(K > 0, SMAT_EUNSUPPORTED,
                "smat_causal_scan_noalloc: nb=%d sequences of r=%d x p=%d states need more "
                "than the %lld-byte scratch array even with one group per segment; use "

@@ -92,6 +92,20 @@ def test_noalloc_matches_workspace_entry_point_twice():
     assert torch.isfinite(got).all() and e2 < 1e-5
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("nb,T,n,hd", [(2, 4096, 2048, 40), (1, 1000, 512, 32), (3, 2048, 0, 64),
+                                       (40, 1024, 512, 16)])
+@pytest.mark.parametrize("write_H", [False, True])
+def test_noalloc_small_16bit_inputs(nb, T, n, hd, dt, write_H):
+    """Few chunks of 16-bit inputs, whose scores are rounded inside a chunk: the two
+    entry points run the same chunks, so they agree to the fp32 bar here too (head
+    sizes of the general kernel, and 64, which streams)."""
+    ref, got, _ = _both(nb, T, n, hd, dt, write_H, seed=5)
+    e = _rel(got, ref)
+    print(f"  rel diff {e:.2e}", flush=True)
+    assert torch.isfinite(got).all() and e < 1e-5
+
+
 def test_noalloc_refuses_what_does_not_fit():
     """255 sequences of 128 x 129 states exceed the array even with one group
     per segment (254 fit): a clear error before any launch."""
