@@ -509,18 +509,53 @@ static int64_t group_bytes(int nb, int nc, int K, int r, int p) {
   return al256((int64_t)nb * ((nc + K - 1) / K + 1) * r * p * 4);
 }
 
-// The chunk a small causal pass runs at: C halved while fewer than 256 chunks
-// would leave CUs without one, down to 32 tokens (64 for the streaming kernel's
-// widths in 16 bits: its step).  A group is then the smaller part of a longer
-// chain, and a 16-bit score that falls outside its chunk is not rounded.
-// Forward of 4 x 1024 tokens of 64: fp32 62 -> 40 us, bf16 43 -> 28 us; of 8 x
-// 1024 of 128 at d = 3 121 -> 88 us; of 32 x 4096 of 64 in fp32 (1024 chunks: as
-// before) 175 -> 165 us, from the last update that is now left out.
-static int scan_chunk(int dtype, int nb, int T, int C, int r, int p) {
-  const bool steps = dtype != SMAT_F32 && r % 16 == 0 && r >= 64 && p == r + 1;
-  const int least = steps ? 64 : 32;
+// C halved while fewer than 256 chunks would leave CUs without one, down to
+// `least` tokens: a group is then the smaller part of a longer chain.
+static int halve_chunk(int nb, int T, int C, int least) {
   while (C % (2 * least) == 0 && (int64_t)nb * ((T + C - 1) / C) < 256) C /= 2;
   return C;
+}
+constexpr int kLeastF32 = 32, kLeastStream = 64;
+
+static ScanArgs scan_args(int T, int n, int C, int r, int p, int64_t q_sb, int64_t q_st,
+                          int64_t k_sb, int64_t k_st, int64_t v_sb, int64_t v_st, int64_t y_sb,
+                          int64_t y_st, int64_t o_sb, int64_t o_st, int64_t g_sb, int write_H) {
+  ScanArgs a{};
+  a.T = T;
+  a.n = n;
+  a.C = C;
+  a.r = r;
+  a.p = p;
+  a.q_sb = q_sb;
+  a.q_st = q_st;
+  a.k_sb = k_sb;
+  a.k_st = k_st;
+  a.v_sb = v_sb;
+  a.v_st = v_st;
+  a.y_sb = y_sb;
+  a.y_st = y_st;
+  a.o_sb = o_sb;
+  a.o_st = o_st;
+  a.g_sb = g_sb;
+  a.write_H = write_H;
+  return a;
+}
+
+// The chunk a causal pass runs at: the caller's, halved in a small call where
+// that rounds no other value.  fp32 scores are not rounded (down to 32 tokens:
+// forward of 4 x 1024 tokens of 64 62 -> 34 us), and the streaming kernel rounds
+// its scores inside 64-token steps at any chunk (down to those: 43 -> 26 us in
+// bf16; 8 x 1024 of 128 at d = 3 121 -> 88).  The general kernel rounds 16-bit
+// scores inside the chunk, so there a halved one would make a sequence's
+// rounding depend on the batch beside it.
+int causal_scan_chunk(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
+                      const float* out, int nb, int T, int n, int C, int r, int p, int64_t q_sb,
+                      int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb, int64_t v_st,
+                      int64_t y_sb, int64_t y_st, int64_t o_sb, int64_t o_st, int write_H) {
+  if (dtype == SMAT_F32) return halve_chunk(nb, T, C, kLeastF32);
+  const ScanArgs a = scan_args(T, n, C, r, p, q_sb, q_st, k_sb, k_st, v_sb, v_st, y_sb, y_st,
+                               o_sb, o_st, 0, write_H);
+  return scan_stream_ok(dtype, phi, psi, vb, Y, out, a) ? halve_chunk(nb, T, C, kLeastStream) : C;
 }
 
 int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
@@ -530,11 +565,12 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
                     int64_t o_st, int64_t g_sb, int write_H, void* ws, bool have_G,
                     hipStream_t stream);
 
-// The most any input type's chunk needs (the type is not an argument).
+// The most any chunk that causal_scan_chunk may give needs (neither the type nor
+// the rows are arguments).
 int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, int kmax) {
   int64_t most = 0;
-  for (const int dtype : {SMAT_F32, SMAT_BF16}) {
-    const int c = scan_chunk(dtype, nb, T, C, r, p);
+  for (const int least : {kLeastF32, kLeastStream, C}) {
+    const int c = halve_chunk(nb, T, C, least);
     const int nc = (T + c - 1) / c;
     const int K = scan_group_chunks(nb, nc, r, p, kmax);
     most = std::max(most, 2 * group_bytes(nb, nc, K, r, p));
@@ -550,7 +586,8 @@ int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void
                          int64_t ws_bytes, int kmax, bool have_G, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
   const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, kmax);
-  C = scan_chunk(dtype, nb, T, C, r, p);
+  C = causal_scan_chunk(dtype, phi, psi, vb, Y, out, nb, T, n, C, r, p, q_sb, q_st, k_sb, k_st,
+                        v_sb, v_st, y_sb, y_st, o_sb, o_st, write_H);
   const int K = scan_group_chunks(nb, (T + C - 1) / C, r, p, kmax);
   if (ws_bytes < need) {
     set_error("smat_causal_scan: workspace of %lld bytes needed, %lld given", (long long)need,
@@ -562,11 +599,10 @@ int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void
                          write_H, ws, have_G, stream);
 }
 
-// The summaries that causal_scan_dispatch begins with, for a caller that forms
-// them itself in the launch of something else and then passes have_G.
-GramPart causal_scan_part(int dtype, int nb, int T, int n, int C, int r, int p, int kmax,
-                          void* ws) {
-  C = scan_chunk(dtype, nb, T, C, r, p);
+// The summaries that causal_scan_dispatch begins with, C the chunk that
+// causal_scan_chunk gives for its arguments, for a caller that forms them itself
+// and then passes have_G.
+GramPart causal_scan_part(int nb, int T, int n, int C, int r, int p, int kmax, void* ws) {
   return chunk_part((float*)ws, T, C, scan_group_chunks(nb, (T + C - 1) / C, r, p, kmax), n, r, p);
 }
 
@@ -650,28 +686,12 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
   if (rc) return rc;
   rc = segment_scan_dispatch(G, Sg, nb, ng, ng0, (int64_t)r * p, stream);
   if (rc) return rc;
-  ScanArgs a{};
-  a.T = T;
-  a.n = n;
-  a.C = C;
+  ScanArgs a = scan_args(T, n, C, r, p, q_sb, q_st, k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb,
+                         o_st, g_sb, write_H);
   a.K = K;
   a.nc = nc;
   a.nc0 = n / C;
   a.ng0 = ng0;
-  a.r = r;
-  a.p = p;
-  a.q_sb = q_sb;
-  a.q_st = q_st;
-  a.k_sb = k_sb;
-  a.k_st = k_st;
-  a.v_sb = v_sb;
-  a.v_st = v_st;
-  a.y_sb = y_sb;
-  a.y_st = y_st;
-  a.o_sb = o_sb;
-  a.o_st = o_st;
-  a.g_sb = g_sb;
-  a.write_H = write_H;
   if (scan_stream_ok(dtype, phi, psi, vb, Y, out, a))
     return scan_stream_launch(dtype, phi, psi, vb, Sg, Y, gate, out, nb, ng, a, stream);
   switch (dtype) {
@@ -696,7 +716,8 @@ int causal_scan_feat_summaries(int dtype, const void* k, const void* v, int nb, 
                                int64_t f_sb, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
   constexpr int r = 128, p = 129;
-  const GramPart P = causal_scan_part(dtype, nb, T, n, C, r, p, kFeatK, ws);
+  const GramPart P =
+      causal_scan_part(nb, T, n, halve_chunk(nb, T, C, kLeastStream), r, p, kFeatK, ws);
   FeatArgs fp = fa;
   fp.psi_out = psi_buf;
   fp.psi_sb = (int64_t)T * 128;
@@ -730,37 +751,19 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
                   : causal_scan_feat_summaries(dtype, k, v, nb, T, n, C, k_sb, k_st, v_sb, v_st,
                                                fa, ws, psi_buf, nullptr, 0, stream);
   if (rc) return rc;
-  const GramPart P = causal_scan_part(dtype, nb, T, n, C, r, p, kFeatK, ws);
+  const GramPart P =
+      causal_scan_part(nb, T, n, halve_chunk(nb, T, C, kLeastStream), r, p, kFeatK, ws);
   const GramItems& it = P.it;
   const int ng = P.nitems;
-  C = it.C;
-  const int nc = it.nc, K = it.K;
-  float* G = P.G;
-  float* Sg = (float*)((char*)ws + group_bytes(nb, nc, K, r, p));
-  rc = segment_scan_dispatch(G, Sg, nb, ng, it.ng0, rp, stream);
+  float* Sg = (float*)((char*)ws + group_bytes(nb, it.nc, it.K, r, p));
+  rc = segment_scan_dispatch(P.G, Sg, nb, ng, it.ng0, rp, stream);
   if (rc) return rc;
-  ScanArgs a{};
-  a.T = T;
-  a.n = n;
-  a.C = C;
-  a.K = K;
-  a.nc = nc;
-  a.nc0 = n / C;
+  ScanArgs a = scan_args(T, n, it.C, r, p, q_sb, q_st, (int64_t)T * 128, 128, v_sb, v_st, y_sb,
+                         y_st, o_sb, o_st, g_sb, 0);
+  a.K = it.K;
+  a.nc = it.nc;
+  a.nc0 = it.nc0;
   a.ng0 = it.ng0;
-  a.r = r;
-  a.p = p;
-  a.q_sb = q_sb;
-  a.q_st = q_st;
-  a.k_sb = (int64_t)T * 128;
-  a.k_st = 128;
-  a.v_sb = v_sb;
-  a.v_st = v_st;
-  a.y_sb = y_sb;
-  a.y_st = y_st;
-  a.o_sb = o_sb;
-  a.o_st = o_st;
-  a.g_sb = g_sb;
-  a.write_H = 0;
   return scan_stream_launch_feat(dtype, q, psi_buf, v, Sg, Y, gate, out, nb, ng, a, fa, stream);
 }
 
@@ -845,7 +848,9 @@ extern "C" int smat_causal_scan_noalloc(int dtype, const void* phi, const void* 
   SMAT_REQUIRE(q_st >= r && k_st >= r && v_st >= p && o_st >= (write_H ? p : p - 1),
                SMAT_EINVAL, "smat_causal_scan_noalloc: a row stride is shorter than its row");
   if (nb == 0 || T == 0) return SMAT_OK;
-  C = scan_chunk(dtype, nb, T, C, r, p);             // smat_causal_scan's: the same scores rounded
+  // smat_causal_scan's chunk, so that the same scores are rounded
+  C = causal_scan_chunk(dtype, phi, psi, vb, Y, out, nb, T, n, C, r, p, q_sb, q_st, k_sb, k_st,
+                        v_sb, v_st, y_sb, y_st, o_sb, o_st, write_H);
   const int K = noalloc_group_chunks(nb, (T + C - 1) / C, r, p);
   SMAT_REQUIRE(K > 0, SMAT_EUNSUPPORTED,
                "smat_causal_scan_noalloc: nb=%d sequences of r=%d x p=%d states need more "

@@ -493,6 +493,33 @@ def test_causal_scan_small_batches(dt, nb, T, n, hd):
     assert _rel(H, ref) < (1e-5 if dt == torch.float32 else 2.0 ** -8)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hd,stride", [(32, 40), (40, 48), (64, 65), (64, 72), (128, 129),
+                                       (128, 136)])
+def test_causal_scan_of_one_sequence_and_of_a_batch(hd, stride, dt):
+    """A sequence gives the same rows alone, among 64 (more than 256 chunks) and, up to
+    its length, in a longer one: in 16 bits the same scores are rounded whatever the
+    call's size, on the general kernel (narrow heads, value rows that are not
+    16-byte aligned) and the streaming one; what may differ is the order of the
+    states' fp32 sums."""
+    _say("causal scan, one and a batch", hd, stride, dt)
+    nb, T, n = 64, 1024, 512
+    gen = torch.Generator().manual_seed(81)
+    Phi, Psi = (torch.rand(nb, T, hd, generator=gen).to(dt).to(DEV) for _ in range(2))
+    Vb = torch.randn(nb, T, stride, generator=gen).to(dt).to(DEV)
+    Vb[..., hd] = 1.0
+    Vb = Vb[..., :hd + 1]
+    for wh in (False, True):
+        many = K.causal_scan(Phi, Psi, Vb, n, 128, write_H=wh)
+        one = K.causal_scan(Phi[:1], Psi[:1], Vb[:1], n, 128, write_H=wh)
+        short = K.causal_scan(Phi[:1, :640], Psi[:1, :640], Vb[:1, :640], n, 128, write_H=wh)
+        for got, want in ((one, many[:1]), (short, many[:1, :640])):
+            assert _rel(got, want) < 2e-6
+    spec = A.to_device(build_mask(T, 2, chunk=128), DEV)
+    many = A.smat_attention(Phi, Psi, Vb, spec)
+    assert _rel(A.smat_attention(Phi[:1], Psi[:1], Vb[:1], spec), many[:1]) < 2e-6
+
+
 @pytest.mark.parametrize("hd", [80, 96, 112])
 @pytest.mark.parametrize("T,n_P,n,N0,nb", [(2048, 0, 1024, 121, 3), (2048, 16, 1000, 90, 3),
                                            (9000, 64, 8000, 50, 6), (640, 0, 640, 640, 1)])
