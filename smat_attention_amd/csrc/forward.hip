@@ -52,11 +52,12 @@ int gram_pair_dispatch(int dtype, const void* psi, const void* vb, const GramPar
                        const GramPart& B, int nb, int r, int p, int64_t k_sb, int64_t k_st,
                        int64_t v_sb, int64_t v_st, hipStream_t stream, const char* who,
                        bool* done);
-GramPart causal_scan_part(int nb, int T, int n, int C, int r, int p, int kmax, void* ws);
-int causal_scan_chunk(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
-                      const float* out, int nb, int T, int n, int C, int r, int p, int64_t q_sb,
-                      int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb, int64_t v_st,
-                      int64_t y_sb, int64_t y_st, int64_t o_sb, int64_t o_st, int write_H);
+GramPart causal_scan_part(int T, int n, const ScanPlan& plan, int r, int p, void* ws);
+ScanPlan causal_scan_plan(int dtype, const void* phi, const void* psi, const void* vb,
+                          const float* Y, const float* out, int nb, int T, int n, int C, int r,
+                          int p, int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st,
+                          int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb,
+                          int64_t o_st, int write_H, int kmax);
 int segment_scan_dispatch(const float* D, float* Sin, int nb, int nc, int nc0, int64_t rp,
                           hipStream_t stream);
 int chunk_local_dispatch(int dtype, const void* phi, const void* psi, const void* vb,
@@ -297,10 +298,10 @@ extern "C" int smat_forward(int dtype, const void* phi, const void* psi, const v
       rc = SMAT_OK;
       GramPart sums{};                               // the causal pass's summaries
       if (L.fused) {
-        const int c = causal_scan_chunk(dtype, phi, psi, vb, Y, out, nb, T, n, C, r, p, q_sb, q_st,
-                                        k_sb, k_st, v_sb, v_st, (int64_t)T_R * yst, yst, o_sb,
-                                        o_st, 0);
-        sums = causal_scan_part(nb, T, n, c, r, p, kForwardK, ws + L.scan);
+        const ScanPlan plan = causal_scan_plan(
+            dtype, phi, psi, vb, Y, out, nb, T, n, C, r, p, q_sb, q_st, k_sb, k_st, v_sb, v_st,
+            (int64_t)T_R * yst, yst, o_sb, o_st, 0, kForwardK);
+        sums = causal_scan_part(T, n, plan, r, p, ws + L.scan);
       }
       if (L.fused && pool_from_summaries(idx, N0, n_P, T, n, rp)) {
         have_G = true;

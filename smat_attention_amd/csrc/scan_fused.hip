@@ -433,11 +433,14 @@ static int launch_scan_fused_shape(const void* phi, const void* psi, const void*
   return launch_status("smat_causal_scan");
 }
 
+// The sizes of the narrow tile shape (2, 5), several workgroups a CU.
+static bool narrow_shape(int r, int p) { return r <= 64 && p <= 80; }
+
 template <typename In>
 static int launch_scan_fused(const void* phi, const void* psi, const void* vb, const float* Sg,
                              const float* Y, const float* gate, float* out, int nb, int ng,
                              const ScanArgs& a, hipStream_t stream) {
-  if (a.r <= 64 && a.p <= 80)
+  if (narrow_shape(a.r, a.p))
     return launch_scan_fused_shape<In, 2, 5>(phi, psi, vb, Sg, Y, gate, out, nb, ng, a, stream);
   return launch_scan_fused_shape<In, 4, 9>(phi, psi, vb, Sg, Y, gate, out, nb, ng, a, stream);
 }
@@ -467,39 +470,73 @@ int gram_stream_launch_feat(int dtype, const void* k, const void* v, float* G, f
                             int64_t gl_sb, const FeatArgs& fa, hipStream_t stream,
                             const char* who);
 
-// Chunks a group, at most kmax.  A group costs its chunks plus the summary it
-// writes, the two passes of the scan over groups and the state it loads -- four
-// r x p tables, about what one of its chunks moves in all -- and the launch runs
-// in rounds of as many groups as the GPU works on at once, so K minimises rounds
+// Chunks a group.  The launch runs in rounds of as many groups as the GPU works on
+// at once, and n is not an argument (the workspace is sized without it): groups
+// are counted as if it split the chunks in half, where build_mask puts it.
+static int64_t scan_groups(int nb, int nc, int K) {
+  return (int64_t)nb * 2 * (((nc + 1) / 2 + K - 1) / K);
+}
+
+// The streaming kernel, at most kmax.  A group costs its chunks plus the summary
+// it writes, the two passes of the scan over groups and the state it loads -- four
+// r x p tables, about what one of its chunks moves in all -- so K minimises rounds
 // x (K + 1), the smallest such K.  The rounds: a workgroup a CU at head size 128
 // (8 sequences of 32768 tokens: forward 641 -> 599 us with 256 groups in place
 // of 1024, 613 with 512), four for the narrow shape (8192 tokens, 32 sequences:
-// 164.0 us with 1024 groups, 166.2 with 512; eight at r <= 48 gained 4 % on 4 x
-// 41344 tokens of 32 and lost 4 % on 8 x 65536, 8 % on 8 x 32768 of 48).  n is
-// not an argument (the workspace is sized without it): the groups are counted
-// as if it split the chunks in half, where build_mask puts it.
+// 164.0 us with 1024 groups, 166.2 with 512).
 //
 // The one-call forward takes up to kForwardK: past 32 the uneven halves (only
 // recent rows read Y) cost more than the states (524288 tokens: 5810 us at 32,
 // 5850 at 64; 8 x 131072 tokens at d = 1: 408 us at 32, 428 at 16).  The forward
 // from q, k, v keeps to kFeatK, whose 512 groups there let two workgroups of the
 // prepass share a CU and hide each other's feature map (1776 us at 16, 1809 at
-// 32); the scan called alone to kScanK: it also serves the H-writing general
-// kernel, whose groups overlap less.
+// 32); the scan called alone to kScanK.
 constexpr int kScanK = 16;
-static int scan_group_chunks(int nb, int nc, int r, int p, int kmax) {
-  const int64_t slots = r <= 64 && p <= 80 ? 1024 : 256;
+static int stream_group_chunks(int nb, int nc, int r, int p, int kmax) {
+  const int64_t slots = narrow_shape(r, p) ? 1024 : 256;
   int best = 1;
   int64_t best_cost = INT64_MAX;
   for (int K = 1; K <= kmax && K <= nc; ++K) {
-    const int64_t groups = (int64_t)nb * 2 * (((nc + 1) / 2 + K - 1) / K);
-    const int64_t cost = (groups + slots - 1) / slots * (K + 1);
+    const int64_t cost = (scan_groups(nb, nc, K) + slots - 1) / slots * (K + 1);
     if (cost < best_cost) {
       best_cost = cost;
       best = K;
     }
   }
   return best;
+}
+
+// The general kernel, whose chunk costs several times the tables of its group, at
+// most kGeneralK.  Wide shape, a workgroup a CU: a round takes K chunks and about
+// 0.15 of one (64 sequences of 4096 tokens of 128, bf16: 565, 519, 490 and 529 us
+// at K = 1, 2, 4 and 8), and a launch of one round a tenth more, with nothing to
+// fill in where a group ends early (56 of 2048: 256 us at K = 2, 270 at 4; 96 of
+// 1024: 212 at K = 1, 268 at 4, which rounds x (K + 1) would take).  Narrow shape,
+// several a CU: groups are worth more than the rounds they end in, so K is the
+// largest power of two that leaves 1024 of them (96 of 4096 tokens of 64: 254 us
+// at K = 2, 274 at 4; 48 of 4096: 139 at K = 1, 146 at 2).
+constexpr int kGeneralK = 8;
+static int general_group_chunks(int nb, int nc, int r, int p) {
+  if (narrow_shape(r, p)) {
+    int K = kGeneralK;
+    while (K > 1 && (int64_t)nb * ((nc + K - 1) / K) < 1024) K >>= 1;
+    return K;
+  }
+  int best = 1;
+  int64_t best_cost = INT64_MAX;
+  for (int K = 1; K <= kGeneralK && K <= nc; ++K) {
+    const int64_t rounds = (scan_groups(nb, nc, K) + 255) / 256;
+    const int64_t cost = rounds * (100 * K + 15) * (rounds == 1 ? 11 : 10);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = K;
+    }
+  }
+  return best;
+}
+
+static int scan_group_chunks(int nb, int nc, int r, int p, bool streams, int kmax) {
+  return streams ? stream_group_chunks(nb, nc, r, p, kmax) : general_group_chunks(nb, nc, r, p);
 }
 
 static int64_t al256(int64_t x) { return (x + 255) & ~(int64_t)255; }
@@ -509,13 +546,22 @@ static int64_t group_bytes(int nb, int nc, int K, int r, int p) {
   return al256((int64_t)nb * ((nc + K - 1) / K + 1) * r * p * 4);
 }
 
-// C halved while fewer than 256 chunks would leave CUs without one, down to
-// `least` tokens: a group is then the smaller part of a longer chain.
-static int halve_chunk(int nb, int T, int C, int least) {
-  while (C % (2 * least) == 0 && (int64_t)nb * ((T + C - 1) / C) < 256) C /= 2;
+// C halved, down to `least` tokens, while there are fewer than `want` chunks: a
+// group is then the smaller part of a longer chain.
+static int halve_chunk(int nb, int T, int C, int least, int want) {
+  while (C % (2 * least) == 0 && (int64_t)nb * ((T + C - 1) / C) < want) C /= 2;
   return C;
 }
-constexpr int kLeastF32 = 32, kLeastStream = 64;
+// Streaming, until every CU has a chunk.  The general kernel's wide shape runs one
+// a CU, so past 128 a halved chunk is a second round: 24 sequences of 1024 tokens
+// of 128 in fp32 101 us as they are, 114 halved.
+constexpr int kLeastF32 = 32, kLeastStream = 64, kWantStream = 256;
+static int f32_chunk(int nb, int T, int C, int r, int p) {
+  return halve_chunk(nb, T, C, kLeastF32, narrow_shape(r, p) ? 256 : 129);
+}
+static int stream_chunk(int nb, int T, int C) {
+  return halve_chunk(nb, T, C, kLeastStream, kWantStream);
+}
 
 static ScanArgs scan_args(int T, int n, int C, int r, int p, int64_t q_sb, int64_t q_st,
                           int64_t k_sb, int64_t k_st, int64_t v_sb, int64_t v_st, int64_t y_sb,
@@ -541,21 +587,27 @@ static ScanArgs scan_args(int T, int n, int C, int r, int p, int64_t q_sb, int64
   return a;
 }
 
-// The chunk a causal pass runs at: the caller's, halved in a small call where
-// that rounds no other value.  fp32 scores are not rounded (down to 32 tokens:
-// forward of 4 x 1024 tokens of 64 62 -> 34 us), and the streaming kernel rounds
-// its scores inside 64-token steps at any chunk (down to those: 43 -> 26 us in
-// bf16; 8 x 1024 of 128 at d = 3 121 -> 88).  The general kernel rounds 16-bit
-// scores inside the chunk, so there a halved one would make a sequence's
+// The chunk and group a causal pass runs at.  The chunk is the caller's, halved in
+// a small call where that rounds no other value.  fp32 scores are not rounded (down
+// to 32 tokens: forward of 4 x 1024 tokens of 64 62 -> 34 us), and the streaming
+// kernel rounds its scores inside 64-token steps at any chunk (down to those: 43 ->
+// 26 us in bf16; 8 x 1024 of 128 at d = 3 121 -> 88).  The general kernel rounds
+// 16-bit scores inside the chunk, so there a halved one would make a sequence's
 // rounding depend on the batch beside it.
-int causal_scan_chunk(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
-                      const float* out, int nb, int T, int n, int C, int r, int p, int64_t q_sb,
-                      int64_t q_st, int64_t k_sb, int64_t k_st, int64_t v_sb, int64_t v_st,
-                      int64_t y_sb, int64_t y_st, int64_t o_sb, int64_t o_st, int write_H) {
-  if (dtype == SMAT_F32) return halve_chunk(nb, T, C, kLeastF32);
-  const ScanArgs a = scan_args(T, n, C, r, p, q_sb, q_st, k_sb, k_st, v_sb, v_st, y_sb, y_st,
-                               o_sb, o_st, 0, write_H);
-  return scan_stream_ok(dtype, phi, psi, vb, Y, out, a) ? halve_chunk(nb, T, C, kLeastStream) : C;
+ScanPlan causal_scan_plan(int dtype, const void* phi, const void* psi, const void* vb,
+                          const float* Y, const float* out, int nb, int T, int n, int C, int r,
+                          int p, int64_t q_sb, int64_t q_st, int64_t k_sb, int64_t k_st,
+                          int64_t v_sb, int64_t v_st, int64_t y_sb, int64_t y_st, int64_t o_sb,
+                          int64_t o_st, int write_H, int kmax) {
+  const bool streams =
+      scan_stream_ok(dtype, phi, psi, vb, Y, out,
+                     scan_args(T, n, C, r, p, q_sb, q_st, k_sb, k_st, v_sb, v_st, y_sb, y_st,
+                               o_sb, o_st, 0, write_H));
+  if (streams)
+    C = stream_chunk(nb, T, C);
+  else if (dtype == SMAT_F32)
+    C = f32_chunk(nb, T, C, r, p);
+  return ScanPlan{C, scan_group_chunks(nb, (T + C - 1) / C, r, p, streams, kmax)};
 }
 
 int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
@@ -565,17 +617,15 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
                     int64_t o_st, int64_t g_sb, int write_H, void* ws, bool have_G,
                     hipStream_t stream);
 
-// The most any chunk that causal_scan_chunk may give needs (neither the type nor
-// the rows are arguments).
+// The most any plan of causal_scan_plan needs (neither the type nor the rows are
+// arguments).
 int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, int kmax) {
-  int64_t most = 0;
-  for (const int least : {kLeastF32, kLeastStream, C}) {
-    const int c = halve_chunk(nb, T, C, least);
+  auto bytes = [&](int c, bool streams) {
     const int nc = (T + c - 1) / c;
-    const int K = scan_group_chunks(nb, nc, r, p, kmax);
-    most = std::max(most, 2 * group_bytes(nb, nc, K, r, p));
-  }
-  return most;
+    return 2 * group_bytes(nb, nc, scan_group_chunks(nb, nc, r, p, streams, kmax), r, p);
+  };
+  return std::max({bytes(C, false), bytes(f32_chunk(nb, T, C, r, p), false),
+                   bytes(stream_chunk(nb, T, C), true)});
 }
 
 int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void* vb,
@@ -586,24 +636,28 @@ int causal_scan_dispatch(int dtype, const void* phi, const void* psi, const void
                          int64_t ws_bytes, int kmax, bool have_G, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
   const int64_t need = causal_scan_workspace_bytes(nb, T, C, r, p, kmax);
-  C = causal_scan_chunk(dtype, phi, psi, vb, Y, out, nb, T, n, C, r, p, q_sb, q_st, k_sb, k_st,
-                        v_sb, v_st, y_sb, y_st, o_sb, o_st, write_H);
-  const int K = scan_group_chunks(nb, (T + C - 1) / C, r, p, kmax);
+  const ScanPlan plan =
+      causal_scan_plan(dtype, phi, psi, vb, Y, out, nb, T, n, C, r, p, q_sb, q_st, k_sb, k_st,
+                       v_sb, v_st, y_sb, y_st, o_sb, o_st, write_H, kmax);
   if (ws_bytes < need) {
     set_error("smat_causal_scan: workspace of %lld bytes needed, %lld given", (long long)need,
               (long long)ws_bytes);
     return SMAT_EINVAL;
   }
-  return causal_scan_run(dtype, phi, psi, vb, Y, gate, out, nb, T, n, C, K, r, p,
+  return causal_scan_run(dtype, phi, psi, vb, Y, gate, out, nb, T, n, plan.C, plan.K, r, p,
                          q_sb, q_st, k_sb, k_st, v_sb, v_st, y_sb, y_st, o_sb, o_st, g_sb,
                          write_H, ws, have_G, stream);
 }
 
-// The summaries that causal_scan_dispatch begins with, C the chunk that
-// causal_scan_chunk gives for its arguments, for a caller that forms them itself
-// and then passes have_G.
-GramPart causal_scan_part(int nb, int T, int n, int C, int r, int p, int kmax, void* ws) {
-  return chunk_part((float*)ws, T, C, scan_group_chunks(nb, (T + C - 1) / C, r, p, kmax), n, r, p);
+// The summaries that causal_scan_dispatch begins with, for a caller that forms them
+// itself (with the plan of its arguments) and then passes have_G.
+GramPart causal_scan_part(int T, int n, const ScanPlan& plan, int r, int p, void* ws) {
+  return chunk_part((float*)ws, T, plan.C, plan.K, n, r, p);
+}
+// The plan of the pass with the feature map, which always streams.
+static ScanPlan feat_plan(int nb, int T, int C) {
+  C = stream_chunk(nb, T, C);
+  return ScanPlan{C, stream_group_chunks(nb, (T + C - 1) / C, 128, 129, kFeatK)};
 }
 
 // F[b] = sum of the group sums G[b][g], g < ng0 (the tokens [0, n)).  A
@@ -716,8 +770,7 @@ int causal_scan_feat_summaries(int dtype, const void* k, const void* v, int nb, 
                                int64_t f_sb, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
   constexpr int r = 128, p = 129;
-  const GramPart P =
-      causal_scan_part(nb, T, n, halve_chunk(nb, T, C, kLeastStream), r, p, kFeatK, ws);
+  const GramPart P = causal_scan_part(T, n, feat_plan(nb, T, C), r, p, ws);
   FeatArgs fp = fa;
   fp.psi_out = psi_buf;
   fp.psi_sb = (int64_t)T * 128;
@@ -751,8 +804,7 @@ int causal_scan_run_feat(int dtype, const void* q, const void* k, const void* v,
                   : causal_scan_feat_summaries(dtype, k, v, nb, T, n, C, k_sb, k_st, v_sb, v_st,
                                                fa, ws, psi_buf, nullptr, 0, stream);
   if (rc) return rc;
-  const GramPart P =
-      causal_scan_part(nb, T, n, halve_chunk(nb, T, C, kLeastStream), r, p, kFeatK, ws);
+  const GramPart P = causal_scan_part(T, n, feat_plan(nb, T, C), r, p, ws);
   const GramItems& it = P.it;
   const int ng = P.nitems;
   float* Sg = (float*)((char*)ws + group_bytes(nb, it.nc, it.K, r, p));
@@ -810,11 +862,10 @@ static int scratch_for_current_device(void** out) {
   return SMAT_OK;
 }
 
-// The group size of the allocating entry point when its scratch fits the
+// The group size of the allocating entry point, K, when its scratch fits the
 // array, else the least power-of-two multiple of it that fits (larger groups,
 // fewer summaries; 0 when not even one group per segment fits).
-static int noalloc_group_chunks(int nb, int nc, int r, int p) {
-  int K = scan_group_chunks(nb, nc, r, p, kScanK);
+static int noalloc_group_chunks(int nb, int nc, int K, int r, int p) {
   while (2 * group_bytes(nb, nc, K, r, p) > kNoAllocScratchBytes) {
     if (K >= nc) return 0;
     K *= 2;
@@ -849,9 +900,11 @@ extern "C" int smat_causal_scan_noalloc(int dtype, const void* phi, const void* 
                SMAT_EINVAL, "smat_causal_scan_noalloc: a row stride is shorter than its row");
   if (nb == 0 || T == 0) return SMAT_OK;
   // smat_causal_scan's chunk, so that the same scores are rounded
-  C = causal_scan_chunk(dtype, phi, psi, vb, Y, out, nb, T, n, C, r, p, q_sb, q_st, k_sb, k_st,
-                        v_sb, v_st, y_sb, y_st, o_sb, o_st, write_H);
-  const int K = noalloc_group_chunks(nb, (T + C - 1) / C, r, p);
+  const ScanPlan plan =
+      causal_scan_plan(dtype, phi, psi, vb, Y, out, nb, T, n, C, r, p, q_sb, q_st, k_sb, k_st,
+                       v_sb, v_st, y_sb, y_st, o_sb, o_st, write_H, kScanK);
+  C = plan.C;
+  const int K = noalloc_group_chunks(nb, (T + C - 1) / C, plan.K, r, p);
   SMAT_REQUIRE(K > 0, SMAT_EUNSUPPORTED,
                "smat_causal_scan_noalloc: nb=%d sequences of r=%d x p=%d states need more "
                "than the %lld-byte scratch array even with one group per segment; use "

@@ -92,9 +92,13 @@ struct ScanArgs {
   int write_H;          // 1: out is H (nb, T, p) unnormalised, no Y / gate
 };
 
-// Most chunks a group of the causal pass takes in smat_forward and in
-// smat_forward_fused (scan_group_chunks, scan_fused.hip).
+// Most chunks a group of the streaming causal pass takes in smat_forward and in
+// smat_forward_fused (stream_group_chunks, scan_fused.hip).
 constexpr int kForwardK = 32, kFeatK = 16;
+// The tokens a chunk and the chunks a group of a causal pass (causal_scan_plan).
+struct ScanPlan {
+  int C, K;
+};
 
 // Token progressions summed by the Gram kernels (gram.hip, scan_stream.hip).
 struct GramItems {

@@ -477,6 +477,34 @@ def _check_forward(spec, Phi, Psi, Vb, *, dt, g=None, label=""):
     return out
 
 
+@pytest.mark.parametrize("dt,nb,T,n,hd,K", [
+    (torch.bfloat16, 96, 1024, 512, 80, 1), (torch.float32, 96, 1024, 512, 128, 1),
+    (torch.float32, 24, 1024, 512, 128, 1), (torch.bfloat16, 56, 2048, 1024, 72, 2),
+    (torch.bfloat16, 48, 4096, 2048, 64, 1), (torch.float32, 96, 4096, 2048, 16, 2),
+    (torch.bfloat16, 8, 10007, 4992, 80, 3)])
+def test_causal_scan_general_groups(dt, nb, T, n, hd, K):
+    """The general kernel (fp32, and 16-bit value rows that are not 16-byte aligned)
+    takes the group of K chunks that measured fastest, not the streaming kernel's
+    larger one: the workspace holds the groups of K and the pass stays inside it,
+    with its values as in fp64 (a few sequences; 16 bits: scores rounded once)."""
+    from smat_attention_amd.kernels.hip_fwd import DTYPE_CODE, _lib, call, stream_of
+    _say("causal scan general groups", dt, nb, T, n, hd, K)
+    P, nc = hd + 1, -(-T // 128)
+    Phi, Psi, Vb = (t.to(DEV) for t in _feats(nb, T, hd, dt, seed=91))
+    wsb = _lib.query("smat_causal_scan_workspace_bytes", nb, T, 128, hd, P)
+    assert wsb >= 2 * nb * (-(-nc // K)) * hd * P * 4
+    ws = torch.full((wsb + 512,), 0x5A, device=DEV, dtype=torch.uint8)
+    off = -ws.data_ptr() % 256
+    H = torch.empty(nb, T, P, device=DEV)
+    call("smat_causal_scan", DTYPE_CODE[dt], Phi.data_ptr(), Psi.data_ptr(), Vb.data_ptr(), 0, 0,
+         H.data_ptr(), nb, T, n, 128, hd, P, T * hd, hd, T * hd, hd, T * P, P, 0, 0, T * P, P, 0, 1,
+         ws.data_ptr() + off, wsb, stream_of(H))
+    assert (ws[:off] == 0x5A).all() and (ws[off + wsb:] == 0x5A).all()
+    some = [0, nb // 2, nb - 1]
+    ref = O.segmented_causal_scan(*(t[some].double().cpu() for t in (Phi, Psi, Vb)), n, chunk=128)
+    assert _rel(H[some], ref) < (1e-5 if dt == torch.float32 else 2.0 ** -8)
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nb,T,n,hd", [(64, 600, 256, 16), (31, 1000, 512, 16), (63, 130, 128, 64),
                                        (128, 256, 128, 64), (1, 127, 0, 64), (2, 4096, 2048, 64)])
