@@ -137,6 +137,24 @@ __device__ __forceinline__ typename Traits<In>::frag row_chunk(const uint4* tile
   return *reinterpret_cast<const typename Traits<In>::frag*>(tile + t * RC + (k ^ swz_row<RC>(t)));
 }
 
+// The state's hi and lo parts.  In fp16 hi ends at the largest value and lo holds
+// what is left: the state is read every 64 tokens, so a segment's last state sums 64
+// tokens more than the general kernel's last one does, and a sum that fits there
+// up to 65504 may pass that here (rounded then, up to twice it, to 2^-12 of it).
+template <typename In>
+__device__ __forceinline__ void split_state(const f32x4& x, typename Traits<In>::half_frag& hi,
+                                            typename Traits<In>::half_frag& lo) {
+  if constexpr (__is_same(In, f16)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      hi[i] = from_f32<f16>(__builtin_amdgcn_fmed3f(x[i], -65504.f, 65504.f));
+      lo[i] = from_f32<f16>(x[i] - to_f32(hi[i]));
+    }
+  } else {
+    split4<In>(x, hi, lo);
+  }
+}
+
 template <typename In>
 __device__ __forceinline__ typename Traits<In>::half_frag tr_read(const char* addr) {
   short4v v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
@@ -616,8 +634,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
     for (int kk = 0; kk < NKB; ++kk) {
       if (kk + 1 < NKB) read_bf(bfs[(kk + 1) & 1], kk + 1);
       Half h0, l0, h1, l1;
-      split4<In>(accS[2 * kk], h0, l0);
-      split4<In>(accS[2 * kk + 1], h1, l1);
+      split_state<In>(accS[2 * kk], h0, l0);
+      split_state<In>(accS[2 * kk + 1], h1, l1);
       const Frag shi = join<In>(h0, h1), slo = join<In>(l0, l1);
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) accO[tt] = mma(accO[tt], shi, bfs[kk & 1][tt]);
@@ -630,7 +648,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt)
         bh[tt] = join<In>(phi_half(tt, 2 * (NW - 1) + (g >> 1)), Half{});
-      split4<In>(accS[NW - 1], hi, lo);
+      split_state<In>(accS[NW - 1], hi, lo);
       const Frag shi = join<In>(hi, Half{}), slo = join<In>(lo, Half{});
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) accO[tt] = mma(accO[tt], shi, bh[tt]);
@@ -642,7 +660,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
       Half s8hi, s8lo, bfn[4];
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) bfn[tt] = phi_half(tt, 2 * w + (g >> 1));
-      split4<In>(accS8, s8hi, s8lo);
+      split_state<In>(accS8, s8hi, s8lo);
       f32x4 pn[4];
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) pn[tt] = mma16(zero4(), s8hi, bfn[tt]);

@@ -10,6 +10,7 @@ with the fp64 oracle.  Tolerances:
   * pooled tables / chunk summaries from bf16 inputs are exact products summed
     in fp32, so they are held to 1e-5 relative against fp64 as well.
 """
+import contextlib
 import math
 
 import pytest
@@ -546,6 +547,31 @@ def test_causal_scan_of_one_sequence_and_of_a_batch(hd, stride, dt):
     spec = A.to_device(build_mask(T, 2, chunk=128), DEV)
     many = A.smat_attention(Phi, Psi, Vb, spec)
     assert _rel(A.smat_attention(Phi[:1], Psi[:1], Vb[:1], spec), many[:1]) < 2e-6
+
+
+@pytest.mark.parametrize("hd", [64, 80, 96, 112])
+def test_causal_scan_fp16_last_states(hd):
+    """fp16 segments whose state passes 65504 only in their last chunk, which the
+    streaming kernel reads there and the general one never forms: both give the
+    pass in fp64 (scores rounded once to fp16, 2^-12 each; the states within that)."""
+    _say("causal scan, last states of fp16", hd)
+    nb, T, n, dt = 2, 1024, 512, torch.float16
+    gen = torch.Generator().manual_seed(53)
+    u = lambda *s: torch.rand(*s, generator=gen)
+    Phi, Psi = (2.0 ** -9 + 2.0 ** -7 * u(nb, T, hd)).to(dt), (150 + 10 * u(nb, T, hd)).to(dt)
+    sums = Psi.double().reshape(nb, 2, 8, 64, hd).sum(3).cumsum(2)
+    assert (sums[:, :, 5] < 65504).all() and (sums[:, :, 6] > 65520).all()
+    Vb = torch.ones(nb, T, hd + 8, dtype=dt)
+    Vb[..., :hd] = torch.randn(nb, T, hd, generator=gen).to(dt)
+    ref = O.segmented_causal_scan(Phi.double(), Psi.double(), Vb[..., :hd + 1].double(), n,
+                                  chunk=128)
+    x = (Phi.to(DEV), Psi.to(DEV), Vb.to(DEV)[..., :hd + 1])
+    for which in (general_kernel("scan"), contextlib.nullcontext()):
+        with which:
+            H = K.causal_scan(*x, n, 128, write_H=True)
+            o = K.causal_scan(*x, n, 128, write_H=False)
+        for got, want in ((H, ref), (o, ref[..., :-1] / ref[..., -1:])):
+            assert torch.isfinite(got).all() and _rel(got, want) < 2.0 ** -10
 
 
 @pytest.mark.parametrize("hd", [80, 96, 112])
