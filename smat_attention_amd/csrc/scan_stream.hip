@@ -346,6 +346,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
   constexpr bool kOdd = NW % 2 != 0;
   constexpr int kSteps = NKB + (kOdd ? 1 : 0);
   constexpr int kBase = Sh::kBase, kExtra = Sh::kExtra;
+  constexpr bool kRcp = NW == 8 && !RAG;
   static_assert(!FEAT || (NW == 8 && !RAG && !WH), "the feature map is 128 x 128");
   static_assert(!(WH && TERMS), "H carries no Y and no gate");
   __shared__ __attribute__((aligned(16))) uint4 phi0[Sh::kTile];
@@ -778,14 +779,21 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
         o.z += yr.y[tt][2];
         o.w += yr.y[tt][3];
       }
-      const float num = TERMS && gb ? yr.gv[tt] : 1.f;   // the gate (1 without)
-      // the reciprocal (1 ulp) in place of the IEEE division's ten-instruction
-      // sequence; the product below rounds once more either way
-      const float inv = num * __builtin_amdgcn_rcpf(den);
+      // At r = 128 and whole steps the gate (1 without) times the reciprocal (1 ulp,
+      // zero past 2^126) in place of the IEEE division's ten instructions; the
+      // others divide as the general kernel does, whole range, the gate last.
+      const float num = TERMS && gb ? yr.gv[tt] : 1.f;
+      const float inv = kRcp ? num * __builtin_amdgcn_rcpf(den) : 1.f / den;
       o.x *= inv;
       o.y *= inv;
       o.z *= inv;
       o.w *= inv;
+      if (!kRcp && TERMS && gb) {
+        o.x *= num;
+        o.y *= num;
+        o.z *= num;
+        o.w *= num;
+      }
       if (!RAG || t < left)
         *reinterpret_cast<float4*>(reinterpret_cast<char*>(outb + ts * a.o_st) + rof.o[tt]) = o;
     }

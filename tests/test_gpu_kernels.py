@@ -549,18 +549,19 @@ def test_causal_scan_of_one_sequence_and_of_a_batch(hd, stride, dt):
     assert _rel(A.smat_attention(Phi[:1], Psi[:1], Vb[:1], spec), many[:1]) < 2e-6
 
 
-@pytest.mark.parametrize("hd", [64, 80, 96, 112])
-def test_causal_scan_fp16_last_states(hd):
+@pytest.mark.parametrize("hd,T", [(64, 1024), (80, 1024), (96, 1000), (112, 1024), (128, 1000)])
+def test_causal_scan_fp16_last_states(hd, T):
     """fp16 segments whose state passes 65504 only in their last chunk, which the
     streaming kernel reads there and the general one never forms: both give the
     pass in fp64 (scores rounded once to fp16, 2^-12 each; the states within that)."""
-    _say("causal scan, last states of fp16", hd)
-    nb, T, n, dt = 2, 1024, 512, torch.float16
+    _say("causal scan, last states of fp16", hd, T)
+    nb, n, dt = 2, 512, torch.float16
     gen = torch.Generator().manual_seed(53)
     u = lambda *s: torch.rand(*s, generator=gen)
     Phi, Psi = (2.0 ** -9 + 2.0 ** -7 * u(nb, T, hd)).to(dt), (150 + 10 * u(nb, T, hd)).to(dt)
-    sums = Psi.double().reshape(nb, 2, 8, 64, hd).sum(3).cumsum(2)
-    assert (sums[:, :, 5] < 65504).all() and (sums[:, :, 6] > 65520).all()
+    for a in (0, n):
+        S = Psi[:, a:a + n].double().cumsum(1)
+        assert (S[:, 383] < 65504).all() and (S[:, 447] > 65520).all()
     Vb = torch.ones(nb, T, hd + 8, dtype=dt)
     Vb[..., :hd] = torch.randn(nb, T, hd, generator=gen).to(dt)
     ref = O.segmented_causal_scan(Phi.double(), Psi.double(), Vb[..., :hd + 1].double(), n,
@@ -572,6 +573,27 @@ def test_causal_scan_fp16_last_states(hd):
             o = K.causal_scan(*x, n, 128, write_H=False)
         for got, want in ((H, ref), (o, ref[..., :-1] / ref[..., -1:])):
             assert torch.isfinite(got).all() and _rel(got, want) < 2.0 ** -10
+
+
+@pytest.mark.parametrize("gate", [False, True])
+@pytest.mark.parametrize("hd", [64, 80, 96, 112, 128])
+def test_causal_scan_divides_large_normalisers(hd, gate):
+    """bf16 normalisers past 2^126, whose reciprocals are below the smallest normal
+    value, and gates times reciprocals that are: the running mean of the values,
+    as the general kernel gives it (scores exact; 2^-20 for a subnormal reciprocal)."""
+    _say("causal scan, large normalisers", hd, gate)
+    T, bf = 31, torch.bfloat16
+    Phi = torch.full((1, T, hd), 2.0 ** 58, dtype=bf, device=DEV)
+    Vb = torch.ones(1, T, hd + 8, dtype=bf, device=DEV)
+    Vb[..., :hd] = torch.rand(1, T, hd, generator=torch.Generator().manual_seed(57)).to(bf)
+    Vb = Vb[..., :hd + 1]
+    V = Vb[..., :hd].double()
+    want = V.cumsum(1) / torch.arange(1, T + 1, device=DEV).view(1, T, 1)
+    g = torch.full((1, T), 2.0 ** -30, device=DEV) if gate else None
+    for which in (general_kernel("scan"), contextlib.nullcontext()):
+        with which:
+            o = K.causal_scan(Phi, Phi, Vb, 0, 128, g=g)
+        assert _rel(o, want * (2.0 ** -30 if gate else 1.0)) < 2.0 ** -20
 
 
 @pytest.mark.parametrize("hd", [80, 96, 112])
