@@ -107,33 +107,49 @@ __global__ __launch_bounds__(256) void segment_scan_rev_kernel(const float* __re
 }
 
 // Rows of the normalisation: sixteen lanes a row, four rows a wave, sixteen
-// a workgroup; lane l of a row's group takes columns 4 l .. +3, 4 l + 64 .. in
-// loads and stores of four values at the element's own alignment (rows of 65
-// floats start anywhere).  Bound by HBM: at 96 sequences of 4096 rows of 65, a
-// value a lane left 64-byte pieces and the backward took 76 us with fp32 and 84
-// with bf16 gradients and a long-range term, the forward 41 and 54; now 55, 54,
-// 36 and 36.
+// a workgroup; lane l of a row's group takes columns V l .. + V - 1, V (l + 16) ..,
+// V = 4 at the element's own alignment (rows of 65 floats start anywhere).  Bound
+// by HBM: at 96 sequences of 4096 rows of 65, a value a lane left 64-byte pieces
+// and the backward took 76 us with fp32 and 84 with bf16 gradients and a
+// long-range term, the forward 41 and 54; four values 55, 54, 36 and 36.
+// Narrow rows leave lanes without a column then, and the last, partly filled four
+// of a row goes value by value: V = 1 up to 32 value columns forward and 16
+// backward.  1.6 million rows, forward, V = 1 and 4: 3 columns 58 and 124 us,
+// 16 69 and 89, 32 125 and 130, 40 173 and 143; backward 3 81 and 158, 16 125 and
+// 140, 24 152 and 150.
 namespace nrm {
 constexpr int kLanes = 16;
 constexpr int kRows = 256 / kLanes;
-// Four values at c (the last up to three of a row one by one; zeros past `end`).
-template <typename T>
-__device__ __forceinline__ f32x4 load4(const T* x, int c, int end) {
-  typedef T t4u __attribute__((ext_vector_type(4), aligned(sizeof(T))));
-  if (c + 4 <= end)
-    return __builtin_convertvector(*reinterpret_cast<const t4u*>(x + c), f32x4);
-  f32x4 v = zero4();
-  for (int i = 0; c + i < end; ++i) v[i] = to_f32(x[c + i]);
-  return v;
-}
-template <typename T>
-__device__ __forceinline__ void store4(T* x, int c, int end, const f32x4& v) {
-  typedef T t4u __attribute__((ext_vector_type(4), aligned(sizeof(T))));
-  if (c + 4 <= end) {
-    *reinterpret_cast<t4u*>(x + c) = __builtin_convertvector(v, t4u);
-    return;
+constexpr int kNarrow = 32, kNarrowBwd = 16;
+template <int V> struct Vec {
+  typedef float type __attribute__((ext_vector_type(V)));
+};
+// V values at c (V = 4: the last up to three of a row one by one; zeros past `end`).
+template <int V, typename T>
+__device__ __forceinline__ typename Vec<V>::type load(const T* x, int c, int end) {
+  typedef typename Vec<V>::type F;
+  if constexpr (V == 1) {
+    return F(to_f32(x[c]));
+  } else {
+    typedef T tu __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+    if (c + V <= end) return __builtin_convertvector(*reinterpret_cast<const tu*>(x + c), F);
+    F v = F(0.f);
+    for (int i = 0; c + i < end; ++i) v[i] = to_f32(x[c + i]);
+    return v;
   }
-  for (int i = 0; c + i < end; ++i) x[c + i] = from_f32<T>(v[i]);
+}
+template <int V, typename T>
+__device__ __forceinline__ void store(T* x, int c, int end, const typename Vec<V>::type& v) {
+  if constexpr (V == 1) {
+    x[c] = from_f32<T>(v[0]);
+  } else {
+    typedef T tu __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+    if (c + V <= end) {
+      *reinterpret_cast<tu*>(x + c) = __builtin_convertvector(v, tu);
+      return;
+    }
+    for (int i = 0; c + i < end; ++i) x[c + i] = from_f32<T>(v[i]);
+  }
 }
 }  // namespace nrm
 
@@ -144,7 +160,7 @@ __device__ __forceinline__ void store4(T* x, int c, int end, const f32x4& v) {
 //   dN_{p-1} = -sum_c dN_c N_c / den (0 where the floor is active),
 //   dg = sum_c dout_c N_c / den.
 // dN is the gradient of H and, from row n on, of Y as well.
-template <bool kFloor, typename Din>
+template <bool kFloor, int V, typename Din>
 __global__ __launch_bounds__(256) void normalise_bwd_kernel(
     const Din* __restrict__ dout, const float* __restrict__ H, const float* __restrict__ Y,
     const float* __restrict__ g, float* __restrict__ dH, float* __restrict__ dg, int T, int n,
@@ -163,15 +179,16 @@ __global__ __launch_bounds__(256) void normalise_bwd_kernel(
   const float inv = 1.f / den;
   const float gate = g ? g[b * g_sb + row] : 1.f;
   float sh = 0.f, sg = 0.f;
-  for (int c = 4 * l; c < p - 1; c += 4 * nrm::kLanes) {
-    f32x4 o = nrm::load4(h, c, p - 1);
-    if (y) o += nrm::load4(y, c, p - 1);
+  typedef typename nrm::Vec<V>::type F;
+  for (int c = V * l; c < p - 1; c += V * nrm::kLanes) {
+    F o = nrm::load<V>(h, c, p - 1);
+    if (y) o += nrm::load<V>(y, c, p - 1);
     o *= inv;
-    const f32x4 dv = nrm::load4(d, c, p - 1);
-    const f32x4 dc = dv * gate * inv;
-    nrm::store4(dh, c, p - 1, dc);
+    const F dv = nrm::load<V>(d, c, p - 1);
+    const F dc = dv * gate * inv;
+    nrm::store<V>(dh, c, p - 1, dc);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < V; ++i) {
       if (c + i >= p - 1) break;                     // not 0 * inv, which may be NaN
       sh += dc[i] * o[i];
       sg += dv[i] * o[i];
@@ -200,7 +217,7 @@ int segment_scan_dispatch(const float* D, float* Sin, int nb, int nc, int nc0, i
 // Sixteen lanes per output row: the normaliser is read once, every column
 // divided; with kFloor (eps >= 0 at dispatch) the normaliser is floored at
 // eps first.
-template <bool kFloor, typename Out>
+template <bool kFloor, int V, typename Out>
 __global__ __launch_bounds__(256) void normalise_kernel(
     const float* __restrict__ H, const float* __restrict__ Y, const float* __restrict__ g,
     Out* __restrict__ out, int T, int n, int p, float eps, int64_t h_sb, int64_t h_st,
@@ -216,13 +233,13 @@ __global__ __launch_bounds__(256) void normalise_kernel(
   if (kFloor) den = fmaxf(den, eps);
   const float gate = g ? g[b * g_sb + row] : 1.f;
   Out* o = out + b * o_sb + row * o_st;
-  for (int c = 4 * lane; c < p - 1; c += 4 * nrm::kLanes) {
-    f32x4 v = nrm::load4(h, c, p - 1);
-    if (y) v += nrm::load4(y, c, p - 1);
+  for (int c = V * lane; c < p - 1; c += V * nrm::kLanes) {
+    auto v = nrm::load<V>(h, c, p - 1);
+    if (y) v += nrm::load<V>(y, c, p - 1);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = v[i] / den;
+    for (int i = 0; i < V; ++i) v[i] = v[i] / den;
     if (g) v *= gate;
-    nrm::store4(o, c, p - 1, v);
+    nrm::store<V>(o, c, p - 1, v);
   }
 }
 
@@ -233,12 +250,11 @@ static int launch_normalise(const float* H, const float* Y, const float* g, Out*
                             float eps) {
   if (nb == 0 || T == 0) return SMAT_OK;
   dim3 grid((unsigned)((T + nrm::kRows - 1) / nrm::kRows), (unsigned)nb);
-  if (eps >= 0.f)
-    smat::launch((normalise_kernel<true, Out>), grid, dim3(256), 0, stream, H, Y, g, out, T,
-                       n, p, eps, h_sb, h_st, y_sb, y_st, o_sb, o_st, g_sb);
-  else
-    smat::launch((normalise_kernel<false, Out>), grid, dim3(256), 0, stream, H, Y, g, out, T,
-                       n, p, 0.f, h_sb, h_st, y_sb, y_st, o_sb, o_st, g_sb);
+  const bool narrow = p - 1 <= nrm::kNarrow, floored = eps >= 0.f;
+  auto kern = floored ? (narrow ? normalise_kernel<true, 1, Out> : normalise_kernel<true, 4, Out>)
+                      : (narrow ? normalise_kernel<false, 1, Out> : normalise_kernel<false, 4, Out>);
+  smat::launch(kern, grid, dim3(256), 0, stream, H, Y, g, out, T, n, p, floored ? eps : 0.f, h_sb,
+               h_st, y_sb, y_st, o_sb, o_st, g_sb);
   return launch_status("smat_normalise");
 }
 
@@ -258,14 +274,12 @@ static int launch_normalise_bwd(const Din* dout, const float* H, const float* Y,
                                 int64_t g_sb, hipStream_t stream) {
   if (nb == 0 || T == 0) return SMAT_OK;
   dim3 grid((unsigned)((T + nrm::kRows - 1) / nrm::kRows), (unsigned)nb);
-  if (eps >= 0.f)
-    smat::launch((normalise_bwd_kernel<true, Din>), grid, dim3(256), 0, stream, dout, H, Y,
-                       g, dH, dg, T, n, p, eps, o_sb, o_st, h_sb, h_st, y_sb, y_st, d_sb, d_st,
-                       g_sb);
-  else
-    smat::launch((normalise_bwd_kernel<false, Din>), grid, dim3(256), 0, stream, dout, H, Y,
-                       g, dH, dg, T, n, p, 0.f, o_sb, o_st, h_sb, h_st, y_sb, y_st, d_sb, d_st,
-                       g_sb);
+  const bool narrow = p - 1 <= nrm::kNarrowBwd, floored = eps >= 0.f;
+  auto kern =
+      floored ? (narrow ? normalise_bwd_kernel<true, 1, Din> : normalise_bwd_kernel<true, 4, Din>)
+              : (narrow ? normalise_bwd_kernel<false, 1, Din> : normalise_bwd_kernel<false, 4, Din>);
+  smat::launch(kern, grid, dim3(256), 0, stream, dout, H, Y, g, dH, dg, T, n, p,
+               floored ? eps : 0.f, o_sb, o_st, h_sb, h_st, y_sb, y_st, d_sb, d_st, g_sb);
   return launch_status("smat_normalise_backward");
 }
 

@@ -446,6 +446,34 @@ def test_normalise_backward_of_an_infinite_reciprocal(p):
         assert torch.allclose(got.cpu().double(), want, rtol=1e-5, atol=0, equal_nan=True)
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("p", [2, 5, 17, 18, 33, 34, 36])
+def test_combine_normalise_widths(p, dt):
+    """The division and its backward on both sides of the widths where a lane takes
+    one value and four (16 value columns backward, 32 forward), rows that a
+    workgroup does not fill, a long-range term on half of them: fp64's values
+    (bf16 outputs rounded once), gradients in fp32."""
+    _say("combine normalise widths", p, dt)
+    T, n = 37, 18
+    gen = torch.Generator().manual_seed(67)
+    H = torch.rand(2, T, p, generator=gen) + 1
+    Y = torch.rand(2, T - n, p, generator=gen)
+    dO = torch.randn(2, T, p - 1, generator=gen).to(dt)
+    x64 = [t.double().requires_grad_(True) for t in (H, Y)]
+    N = torch.cat([x64[0][:, :n], x64[0][:, n:] + x64[1]], 1)
+    o64 = N[..., :-1] / N[..., -1:]
+    o64.backward(dO.double())
+    x = [t.to(DEV).requires_grad_(True) for t in (H, Y)]
+    o = A.combine_normalise(x[0], x[1], n, out_dtype=dt)
+    o.backward(dO.to(DEV))
+    assert o.dtype == dt
+    tol = 2.0 ** -8 if dt == torch.bfloat16 else 1e-6
+    assert torch.allclose(o.detach().cpu().double(), o64.detach(), rtol=tol, atol=0)
+    for got, want in zip(x, x64):
+        e = (got.grad.cpu().double() - want.grad).abs().max() / want.grad.abs().max()
+        assert e < 2e-6
+
+
 @pytest.mark.parametrize("nb,nc,pad,split", [(1, 1, 0, 0), (5, 77, 0, 77 * 128), (3, 129, 7, 4130),
                                              (257, 2, 3, 100)])
 def test_chunk_backward_walks_every_chunk(nb, nc, pad, split):
