@@ -7,8 +7,8 @@
 // dtype, elu rounded, + 1 rounded, the gate product rounded (fp32 math in
 // between, as torch does for 16-bit tensors).
 //
-// One wave computes two 16-row tiles of X (Q or K) at a time against all r
-// features as C = W X^T on MFMA (W is the A operand from LDS, rows padded by 16
+// One wave computes two 16-row tiles of X (Q or K; one in a small call) at a time
+// against all r features as C = W X^T on MFMA (W is the A operand from LDS, rows padded by 16
 // bytes so the sixteen feature rows a fragment reads fall in distinct banks;
 // the X rows are the B operand, loaded straight from HBM as 16-byte rows).  A
 // lane then holds four consecutive features of a row in each feature tile; W's
@@ -34,17 +34,15 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 constexpr int kMaxDqk = 128;       // d_qk
 constexpr int kMaxRank = 128;      // feature rank
-constexpr int kTiles = 2;          // 16-row tiles a wave takes at a time
-constexpr int kRows = 16 * kTiles;
 // W rows in LDS: whole 32-wide k-steps and 16 bytes, so the sixteen rows a
 // fragment reads start four banks apart
-template <typename In>
-__host__ __device__ constexpr int w_stride(int dqk) {
-  return (dqk + 31) / 32 * 32 + 16 / (int)sizeof(In);
+__host__ __device__ constexpr int w_stride(int dqk, int elem_bytes) {
+  return (dqk + 31) / 32 * 32 + 16 / elem_bytes;
 }
 }  // namespace ft
 
-template <typename In>
+// kTiles: 16-row tiles a wave takes at a time.
+template <typename In, int kTiles>
 __global__ __launch_bounds__(ft::kThreads, sizeof(In) == 2 ? 4 : 2) void featurise_kernel(
     const In* __restrict__ q, const In* __restrict__ k, const In* __restrict__ v,
     const In* __restrict__ W, const In* __restrict__ h, In* __restrict__ phi,
@@ -56,12 +54,13 @@ __global__ __launch_bounds__(ft::kThreads, sizeof(In) == 2 ? 4 : 2) void featuri
   // Vb rows 16-byte aligned, bit 3 = Phi/Psi rows 16-byte aligned and r a
   // multiple of 32 (16-bit types: one 16-byte store per lane and two tiles).
   using namespace ft;
+  constexpr int kRows = 16 * kTiles;
   typedef typename Traits<In>::frag Frag;
   typedef typename Traits<In>::half_frag Quad;
   constexpr int kE = 16 / (int)sizeof(In);                   // elements per 16 bytes
   const int nks = (dqk + 31) / 32;
   const int nft = (r + 15) / 16;
-  const int wst = w_stride<In>(dqk);                           // padded W row (elements)
+  const int wst = w_stride(dqk, (int)sizeof(In));              // padded W row (elements)
   extern __shared__ __attribute__((aligned(16))) char w_raw[];
   In* w_lds = reinterpret_cast<In*>(w_raw);
 
@@ -249,7 +248,6 @@ extern "C" int smat_featurise(int dtype, const void* q, const void* k, const voi
                    o_st >= r,
                SMAT_EINVAL, "smat_featurise: row stride too short");
   if (nb == 0 || T == 0) return SMAT_OK;
-  const int64_t ntiles = 3 * (int64_t)nb * ((T + ft::kRows - 1) / ft::kRows);
   const int64_t e16 = 16 / elem_bytes(dtype);
   if (!k) { k = q; k_sb = q_sb; k_st = q_st; psi = phi; }      // alignment checks only
   if (!v) { v = q; vb = phi; v_st = d_v; vb_st = d_v + 1; v_sb = vb_sb = 0; }
@@ -266,14 +264,25 @@ extern "C" int smat_featurise(int dtype, const void* q, const void* k, const voi
   int dev = 0, ncu = 256;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-  const int64_t want = (ntiles + ft::kWaves - 1) / ft::kWaves;
+  // Workgroups a CU: four, or as many as W's LDS leaves room for.  Up to a 16-row
+  // tile for each of their waves (a third of it where only Q is mapped), two a wave
+  // would only be a longer chain: a sequence of 1000, widths 128, fp32 14.5 us
+  // against 22.0, fp16 9.2 against 13.1; past it 16 of 2048 in fp32 57 and 48 us.
+  const int eb = elem_bytes(dtype);
+  const int64_t lds = (int64_t)((r + 15) / 16 * 16) * ft::w_stride(d_qk, eb) * eb;
+  const int64_t wgs = ncu * std::min<int64_t>(4, (160 << 10) / lds);
+  const int64_t lists = (int64_t)nb * (have_v ? 3 : have_k ? 2 : 1);
+  const bool two = lists * ((T + 15) / 16) > wgs * ft::kWaves;
+  const int64_t tiles = lists * (two ? (T + 31) / 32 : (T + 15) / 16);
+  const int64_t want = (tiles + ft::kWaves - 1) / ft::kWaves;
   const unsigned grid = (unsigned)std::min<int64_t>(want, (int64_t)ncu * 4);
   hipStream_t st = (hipStream_t)stream;
   const void* kk = have_k ? k : nullptr;
   const void* vv = have_v ? v : nullptr;
 #define SMAT_FT(T_)                                                                            \
-  smat::launch(featurise_kernel<T_>, dim3(grid), dim3(ft::kThreads),                           \
-                     (r + 15) / 16 * 16 * ft::w_stride<T_>(d_qk) * sizeof(T_), st, (const T_*)q, \
+  smat::launch(two ? featurise_kernel<T_, 2> : featurise_kernel<T_, 1>, dim3(grid),            \
+                     dim3(ft::kThreads),                                                         \
+                     (uint32_t)lds, st, (const T_*)q,                                            \
                      (const T_*)kk, (const T_*)vv, (const T_*)W, (const T_*)h, (T_*)phi, (T_*)psi, \
                      (T_*)vb, nb, T, d_qk, r, d_v, kind, q_sb, q_st, k_sb, k_st, v_sb, v_st,     \
                      h_sb, o_sb, o_st, vb_sb, vb_st, vec)

@@ -1201,6 +1201,28 @@ def test_feature_map_every_negative_16_bit_input(dt):
         assert step.max().item() <= 1 and (step > 0).double().mean().item() <= 1e-3
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("dqk,r,dv", [(128, 128, 128), (64, 64, 64), (40, 48, 33)])
+def test_featurise_of_a_sequence_and_of_a_batch(dqk, r, dv, dt):
+    """A call of more row tiles than the GPU has waves (two to a wave) gives, bit for
+    bit, the rows of its sequences mapped alone (one to a wave), at a length that
+    ends inside a tile and inside a pair; Q, K and V together and Q alone."""
+    _say("featurise, one and a batch", dqk, r, dv, dt)
+    gen = torch.Generator(device=DEV).manual_seed(93)
+    u = lambda *s: torch.randn(*s, device=DEV, generator=gen).to(dt)
+    W = (u(r, dqk).float() / dqk ** 0.5).to(dt)
+    nb, T = 24, 997
+    Q, Kk, V, h = u(nb, T, dqk), u(nb, T, dqk), u(nb, T, dv), u(nb, T)
+    many = K.featurise(W, "elu1", Q, Kk, V, h)
+    for b in (0, 11, nb - 1):
+        one = K.featurise(W, "elu1", Q[b:b + 1], Kk[b:b + 1], V[b:b + 1], h[b:b + 1])
+        assert all(torch.equal(x, y[b:b + 1]) for x, y in zip(one, many))
+    Q = u(70, T, dqk)
+    many = K.featurise(W, "relu", Q)[0]
+    for b in (0, 69):
+        assert torch.equal(K.featurise(W, "relu", Q[b:b + 1])[0], many[b:b + 1])
+
+
 def test_featurise_rejects_mixed_dtypes():
     phi = A.make_phi(32, 32, device=DEV, dtype=torch.float32)
     Q = torch.randn(1, 16, 32, device=DEV, dtype=torch.bfloat16)
