@@ -354,14 +354,19 @@ constexpr int kQMax = 41;         // largest q whose four planes fit the LDS
 // head size 64), 160 -> 150 us at q = 23 (8 of 128).  Two workgroups at q = 29
 // (the panels fill the LDS exactly) ran as one does, 234 us.
 // Between q = 17 and 23 that turns around where F and U outgrow the memory-side
-// cache several times over: an item takes as many times longer as there are
-// workgroups, so the other half of a 128-byte line, which the neighbouring item
-// reads or writes, more often finds the line gone from the L2.  At 12 and 16
-// sequences of head size 128 (0.5-0.65 GB) 118 and 154 us against 128 and 166 at
-// q = 17; at 32 to 64 (2.3-2.9 GB) 719 against 615 at q = 17, 845 against 661 at
-// q = 19, 642 against 582 at q = 23.  One workgroup of 1024 threads runs those
-// (WIDE; at q <= 13 the smaller ones win at every size).
-constexpr int64_t kWideBytes = 768ll << 20;
+// cache: an item takes as many times longer as there are workgroups, so the other
+// half of a 128-byte line, which the neighbouring item reads or writes, more often
+// finds the line gone from the L2.  One workgroup of 1024 threads runs those (WIDE;
+// at q <= 13 the smaller ones win, but for 4 % at 265 MB).  Rows r*p apart, us,
+// smaller / WIDE: q = 17 151 MB 31 / 44, 253 MB 79 / 71, 599 MB 203 / 193; q = 19
+// 188 MB 45 / 49, 280 MB 102 / 88; q = 23 153 MB 40 / 42, 204 MB 62 / 57, 544 MB 200
+// / 190.  The forward's rows share few lines and turn later: q = 17 599 MB 154 / 160
+// (head size 64, 604 MB: 186 / 178), 899 MB 243 / 236; q = 23 557 MB 148 / 154,
+// 1089 MB 304 / 297.  q = 19 turns early there too: 191 MB 49 / 52, 280 MB 75 / 74,
+// 752 MB 234 / 202.
+constexpr int64_t wide_bytes(int q, bool spread) {
+  return (spread && q != 19 ? 600ll : 200ll) << 20;
+}
 constexpr bool has_wide(int q) { return q >= 17 && q <= 23; }
 template <int Q, bool WIDE = false>
 struct Shape {
@@ -856,7 +861,7 @@ static int launch_wave_q(const float* F, const float* F_glob, const int* code, f
                          int B, int64_t rp, int64_t ld, hipStream_t stream) {
   using namespace iw;
   if constexpr (has_wide(Q) && !WIDE) {
-    if ((int64_t)nb * (Q * Q + B) * ld * 4 > kWideBytes)
+    if ((int64_t)nb * (Q * Q + B) * ld * 4 > wide_bytes(Q, ld > rp))
       return launch_wave_q<Q, true>(F, F_glob, code, U, nb, B, rp, ld, stream);
   }
   const int nslices = (int)((rp + kE - 1) / kE);
