@@ -137,14 +137,15 @@ __device__ __forceinline__ typename Traits<In>::frag row_chunk(const uint4* tile
   return *reinterpret_cast<const typename Traits<In>::frag*>(tile + t * RC + (k ^ swz_row<RC>(t)));
 }
 
-// The state's hi and lo parts.  In fp16 hi ends at the largest value and lo holds
-// what is left: the state is read every 64 tokens, so a segment's last state sums 64
-// tokens more than the general kernel's last one does, and a sum that fits there
-// up to 65504 may pass that here (rounded then, up to twice it, to 2^-12 of it).
-template <typename In>
+// The state's hi and lo parts.  WIDE, in fp16: hi ends at the largest value and lo
+// holds what is left.  The state is read every 64 tokens, so a segment's last state
+// sums 64 tokens more than the general kernel's last one does, and a sum that fits
+// there up to 65504 may pass that here (rounded then, up to twice it, to 2^-12 of
+// it).  One instruction a value, 3 % of a pass over 128 features.
+template <typename In, bool WIDE>
 __device__ __forceinline__ void split_state(const f32x4& x, typename Traits<In>::half_frag& hi,
                                             typename Traits<In>::half_frag& lo) {
-  if constexpr (__is_same(In, f16)) {
+  if constexpr (WIDE && __is_same(In, f16)) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       hi[i] = from_f32<f16>(__builtin_amdgcn_fmed3f(x[i], -65504.f, 65504.f));
@@ -346,7 +347,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
   constexpr bool kOdd = NW % 2 != 0;
   constexpr int kSteps = NKB + (kOdd ? 1 : 0);
   constexpr int kBase = Sh::kBase, kExtra = Sh::kExtra;
-  constexpr bool kRcp = NW == 8 && !RAG;
+  // The shape that has always streamed.  The others took the general kernel's place
+  // and keep its range: the whole division, and in fp16 the states it never forms.
+  constexpr bool kFirst = NW == 8 && !RAG;
   static_assert(!FEAT || (NW == 8 && !RAG && !WH), "the feature map is 128 x 128");
   static_assert(!(WH && TERMS), "H carries no Y and no gate");
   __shared__ __attribute__((aligned(16))) uint4 phi0[Sh::kTile];
@@ -635,8 +638,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
     for (int kk = 0; kk < NKB; ++kk) {
       if (kk + 1 < NKB) read_bf(bfs[(kk + 1) & 1], kk + 1);
       Half h0, l0, h1, l1;
-      split_state<In>(accS[2 * kk], h0, l0);
-      split_state<In>(accS[2 * kk + 1], h1, l1);
+      split_state<In, !kFirst>(accS[2 * kk], h0, l0);
+      split_state<In, !kFirst>(accS[2 * kk + 1], h1, l1);
       const Frag shi = join<In>(h0, h1), slo = join<In>(l0, l1);
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) accO[tt] = mma(accO[tt], shi, bfs[kk & 1][tt]);
@@ -649,7 +652,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt)
         bh[tt] = join<In>(phi_half(tt, 2 * (NW - 1) + (g >> 1)), Half{});
-      split_state<In>(accS[NW - 1], hi, lo);
+      split_state<In, !kFirst>(accS[NW - 1], hi, lo);
       const Frag shi = join<In>(hi, Half{}), slo = join<In>(lo, Half{});
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) accO[tt] = mma(accO[tt], shi, bh[tt]);
@@ -661,7 +664,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
       Half s8hi, s8lo, bfn[4];
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) bfn[tt] = phi_half(tt, 2 * w + (g >> 1));
-      split_state<In>(accS8, s8hi, s8lo);
+      split_state<In, !kFirst>(accS8, s8hi, s8lo);
       f32x4 pn[4];
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) pn[tt] = mma16(zero4(), s8hi, bfn[tt]);
@@ -779,16 +782,15 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void scan_stream_kernel(
         o.z += yr.y[tt][2];
         o.w += yr.y[tt][3];
       }
-      // At r = 128 and whole steps the gate (1 without) times the reciprocal (1 ulp,
-      // zero past 2^126) in place of the IEEE division's ten instructions; the
-      // others divide as the general kernel does, whole range, the gate last.
+      // The gate (1 without) times the reciprocal (1 ulp, zero past 2^126) in place
+      // of the IEEE division's ten instructions, or that division, the gate last.
       const float num = TERMS && gb ? yr.gv[tt] : 1.f;
-      const float inv = kRcp ? num * __builtin_amdgcn_rcpf(den) : 1.f / den;
+      const float inv = kFirst ? num * __builtin_amdgcn_rcpf(den) : 1.f / den;
       o.x *= inv;
       o.y *= inv;
       o.z *= inv;
       o.w *= inv;
-      if (!kRcp && TERMS && gb) {
+      if (!kFirst && TERMS && gb) {
         o.x *= num;
         o.y *= num;
         o.z *= num;
