@@ -472,7 +472,7 @@ int gram_stream_launch_feat(int dtype, const void* k, const void* v, float* G, f
 
 // Chunks a group.  The launch runs in rounds of as many groups as the GPU works on
 // at once, and n is not an argument (the workspace is sized without it): groups
-// are counted as if it split the chunks in half, where build_mask puts it.
+// are counted as if it lay in the middle, where build_mask puts it.
 static int64_t scan_groups(int nb, int nc, int K) {
   return (int64_t)nb * 2 * (((nc + 1) / 2 + K - 1) / K);
 }
@@ -515,17 +515,26 @@ static int stream_group_chunks(int nb, int nc, int r, int p, int kmax) {
 // several a CU: groups are worth more than the rounds they end in, so K is the
 // largest power of two that leaves 1024 of them (96 of 4096 tokens of 64: 254 us
 // at K = 2, 274 at 4; 48 of 4096: 139 at K = 1, 146 at 2).
+//
+// A round too many costs as much as a larger K saves, so the chunks are counted as
+// they are worked: n at the last whole chunk before T / 2, a last chunk of less
+// than half of one for nothing (36 sequences of 8913 of 80, bf16: 582 us at K = 5,
+// whose 504 groups of two equal halves are 540 there, 441 at K = 2; 88 of 1795 of
+// 72, fp32: 370 at K = 1, 411 at 2).
 constexpr int kGeneralK = 8;
-static int general_group_chunks(int nb, int nc, int r, int p) {
+static int general_group_chunks(int nb, int T, int C, int r, int p) {
+  const int nc = (T + C - 1) / C;
   if (narrow_shape(r, p)) {
     int K = kGeneralK;
     while (K > 1 && (int64_t)nb * ((nc + K - 1) / K) < 1024) K >>= 1;
     return K;
   }
+  const int nc0 = T / 2 / C, nc1 = (int)(((int64_t)T + C / 2) / C) - nc0;
   int best = 1;
   int64_t best_cost = INT64_MAX;
   for (int K = 1; K <= kGeneralK && K <= nc; ++K) {
-    const int64_t rounds = (scan_groups(nb, nc, K) + 255) / 256;
+    const int64_t groups = (int64_t)nb * ((nc0 + K - 1) / K + (nc1 + K - 1) / K);
+    const int64_t rounds = std::max<int64_t>(1, (groups + 255) / 256);
     const int64_t cost = rounds * (100 * K + 15) * (rounds == 1 ? 11 : 10);
     if (cost < best_cost) {
       best_cost = cost;
@@ -535,8 +544,9 @@ static int general_group_chunks(int nb, int nc, int r, int p) {
   return best;
 }
 
-static int scan_group_chunks(int nb, int nc, int r, int p, bool streams, int kmax) {
-  return streams ? stream_group_chunks(nb, nc, r, p, kmax) : general_group_chunks(nb, nc, r, p);
+static int scan_group_chunks(int nb, int T, int C, int r, int p, bool streams, int kmax) {
+  return streams ? stream_group_chunks(nb, (T + C - 1) / C, r, p, kmax)
+                 : general_group_chunks(nb, T, C, r, p);
 }
 
 static int64_t al256(int64_t x) { return (x + 255) & ~(int64_t)255; }
@@ -607,7 +617,7 @@ ScanPlan causal_scan_plan(int dtype, const void* phi, const void* psi, const voi
     C = stream_chunk(nb, T, C);
   else if (dtype == SMAT_F32)
     C = f32_chunk(nb, T, C, r, p);
-  return ScanPlan{C, scan_group_chunks(nb, (T + C - 1) / C, r, p, streams, kmax)};
+  return ScanPlan{C, scan_group_chunks(nb, T, C, r, p, streams, kmax)};
 }
 
 int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb, const float* Y,
@@ -622,7 +632,7 @@ int causal_scan_run(int dtype, const void* phi, const void* psi, const void* vb,
 int64_t causal_scan_workspace_bytes(int nb, int T, int C, int r, int p, int kmax) {
   auto bytes = [&](int c, bool streams) {
     const int nc = (T + c - 1) / c;
-    return 2 * group_bytes(nb, nc, scan_group_chunks(nb, nc, r, p, streams, kmax), r, p);
+    return 2 * group_bytes(nb, nc, scan_group_chunks(nb, T, c, r, p, streams, kmax), r, p);
   };
   return std::max({bytes(C, false), bytes(f32_chunk(nb, T, C, r, p), false),
                    bytes(stream_chunk(nb, T, C), true)});

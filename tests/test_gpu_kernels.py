@@ -482,7 +482,8 @@ def _check_forward(spec, Phi, Psi, Vb, *, dt, g=None, label=""):
     (torch.bfloat16, 96, 1024, 512, 80, 1), (torch.float32, 96, 1024, 512, 128, 1),
     (torch.float32, 24, 1024, 512, 128, 1), (torch.bfloat16, 56, 2048, 1024, 72, 2),
     (torch.bfloat16, 48, 4096, 2048, 64, 1), (torch.float32, 96, 4096, 2048, 16, 2),
-    (torch.bfloat16, 8, 10007, 4992, 80, 3)])
+    (torch.bfloat16, 8, 10007, 4992, 80, 3), (torch.bfloat16, 36, 8913, 4352, 80, 2),
+    (torch.float32, 88, 1795, 896, 72, 1)])
 def test_causal_scan_general_groups(dt, nb, T, n, hd, K):
     """The general kernel (fp32, and 16-bit value rows that are not 16-byte aligned)
     takes the group of K chunks that measured fastest, not the streaming kernel's
