@@ -165,11 +165,13 @@ def test_fused_forward_long_prefill_T524288():
 
 
 @pytest.mark.parametrize("T,nb,gates", [(4096, 2, False), (8192, 3, True), (131072, 8, False)])
-def test_fused_forward_d1_pools_from_the_causal_pass(T, nb, gates):
-    """d = 1 (one profile holding every landmark token, the identity incidence):
-    the fused forward takes the profile's pool from the causal pass's group
-    sums over the tokens [0, n) instead of a pool pass; against featurise +
-    smat_attention (1e-5 of the largest entry; the pool sums in another order)."""
+def test_fused_forward_d1_is_plain_causal_attention(T, nb, gates):
+    """d = 1 (one profile holding every landmark token, the identity incidence): the
+    forward is the causal pass over the whole sequence, with no pool and no query.
+    The fused call against featurise + smat_attention (1e-5 of the largest entry;
+    other chunk groups) and, up to 8192 tokens, against causal linear attention of
+    the same features in fp64, which neither takes a shortcut in (scores rounded
+    once to bf16, 2^-9 each, in the numerator and in the normaliser)."""
     spec = build_mask(T, 1, chunk=128)
     assert (spec.N0, spec.B, spec.n_P) == (1, 1, 0)
     _say(f"fused forward d=1 T={T} nb={nb} gates={gates}")
@@ -178,6 +180,18 @@ def test_fused_forward_d1_pools_from_the_causal_pass(T, nb, gates):
     e = _rel(fused, unfused)
     _say(f"  vs featurise + smat_attention: {e:.2e}")
     assert torch.isfinite(fused).all() and e < 1e-5
+    if T > 8192:
+        return
+    phi = A.FeatureMap(O.phi_weight(128, 128, dtype=BF, seed=0).to(DEV), "elu1")
+    hd = h.to(DEV) if gates else None
+    Phi, Psi, Vb = A.featurise(Q.to(DEV), K.to(DEV), V.to(DEV), phi, h=hd)
+    for b in range(nb):
+        H = (Phi[b].double() @ Psi[b].double().T.contiguous()).tril() @ Vb[b].double()
+        want = H[:, :-1] / H[:, -1:]
+        tol = 2.0 ** -8 * V[b].abs().max().item()
+        if gates:
+            want, tol = want * g[b].to(DEV).double()[:, None], tol * g[b].max().item()
+        assert (fused[b].double() - want).abs().max().item() < tol
 
 
 def test_fused_forward_falls_back_outside_its_shape_and_under_grad():
