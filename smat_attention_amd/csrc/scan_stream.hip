@@ -899,6 +899,7 @@ __global__ __launch_bounds__(64 * NW, (ONE && !FEAT) ? 3 : 2) void gram_stream_k
   constexpr int kP = 16 * NW + 1;                    // = p
   constexpr int kL = kPhiLoads + kVbLoads - (FEAT ? 1 : 0);
   static_assert(!FEAT || NW == 8, "the feature map is 128 x 128");
+  static_assert(!(ONE && LIST), "a list's length is not known to the launch");
   // psi0 and vb0 are one array: after the last step it stages the output
   __shared__ __attribute__((aligned(16))) uint4 stage0[kTileChunks + kVbTileChunks];
   static_assert((kTileChunks + kVbTileChunks) * 16 >= 64 * kP * 4, "stage holds 64 rows of G");
@@ -1115,12 +1116,8 @@ static void gram_stream_kernel_launch(const void* psi, const void* vb, float* G,
   // lists (r = 128) have no form with the feature map
   if constexpr (!FEAT && NW == 8) {
     if (it.mode == 2) {
-      if (one)
-        smat::launch((gram_stream_kernel<In, 8, true, false, true>), grid, blk, 0, stream, k, v,
-                     G, G_last, it, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
-      else
-        smat::launch((gram_stream_kernel<In, 8, false, false, true>), grid, blk, 0, stream, k, v,
-                     G, G_last, it, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
+      smat::launch((gram_stream_kernel<In, 8, false, false, true>), grid, blk, 0, stream, k, v, G,
+                   G_last, it, k_sb, k_st, v_sb, v_st, g_sb, g_si, gl_sb, fa);
       return;
     }
   }
@@ -1205,8 +1202,11 @@ bool scan_stream_ok(int dtype, const void* phi, const void* psi, const void* vb,
   if (!rows_vec_ok(phi, a.q_sb, a.q_st, 2) || !rows_vec_ok(psi, a.k_sb, a.k_st, 2) ||
       !rows_vec_ok(vb, a.v_sb, a.v_st, 2) || a.v_st < a.r + 8)
     return false;
-  // H only at r = 64, the width of the fused backward; the wider general kernel
-  // gives a training step the same bits for every row stride of Vb
+  // H only at r = 64, the width of the fused backward.  There a training step's bits
+  // depend on Vb's rows, as a forward's do at every width here: those that are not
+  // 16-byte aligned take the general kernel, which rounds 16-bit scores inside its
+  // chunk of 128 tokens instead of inside steps of 64.  Wider H takes the general
+  // kernel for every row stride.
   if (a.write_H ? a.r != 64 : !rows_vec_ok(out, a.o_sb, a.o_st, 4)) return false;
   if (Y && !rows_vec_ok(Y, a.y_sb, a.y_st, 4)) return false;
   // per-lane row offsets are 32-bit bytes over 64 rows
