@@ -148,6 +148,10 @@ int smat_chunk_local_decay(int dtype, const void* phi, const void* psi, const vo
  * y_st apart), g optional.  Reads Phi, Psi, Vb once; H never reaches memory in
  * the normalised mode.  Replaces segmented_causal_scan
  * (src/smat/attention.py:134-192) plus the cat/normalise of :446-453.
+ * 16-bit inputs: the scores of tokens of one chunk are rounded to the input type;
+ * of one 64-token step where r = 64, 80 .. 128, p = r + 1, n and C are multiples of
+ * 64, rows are 16-byte aligned and v_st >= r + 8 (write_H = 1: at r = 64).  Which
+ * scores those are depends on neither nb nor T.
  * workspace: smat_causal_scan_workspace_bytes(...) bytes, 256-byte aligned.
  */
 int64_t smat_causal_scan_workspace_bytes(int nb, int T, int C, int r, int p);
@@ -303,8 +307,8 @@ int smat_bgemm(int dtype_a, int dtype_b, const void* A, const void* B, float* C,
                int64_t cn, int beta, int mask, void* stream);
 
 /*
- * Fused backward of the intra-chunk causal scan, one workgroup per
- * (sequence, chunk) with the C x C scores A = tril(Phi Psi^T) and
+ * Fused backward of the intra-chunk causal scan, persistent workgroups that walk
+ * the (sequence, chunk) list with the C x C scores A = tril(Phi Psi^T) and
  * dA = tril(dH Vb^T) kept on chip:
  *   dPhi = dA Psi + dH Sin^T,  dPsi = dA^T Phi + Vb Q^T,  dVb = A^T dH + Psi Q
  * for 16-bit Phi, Psi, Vb (nb x nc*C rows; dtype SMAT_BF16 or SMAT_F16), fp32
@@ -472,8 +476,10 @@ int64_t smat_forward_workspace_bytes(int nb, int T, int n, int N0, int B, int n_
  * smat_attention (src/smat/attention.py:391-455, whose phases lr_pool,
  * lr_incidence, lr_query and scan + normalise these stages are).  A small
  * problem's chunk-group summaries share the pool's launch and count to stage 0.
- * Stages a call does not run (no recent rows) record nothing.  n = 0 clears them; at
- * most 8.  The caller keeps the events alive while they are set.
+ * Stages a call does not run record nothing: without recent rows 0 to 2; with one
+ * profile, the identity incidence and no global channel (d = 1), bf16 and fp32 run
+ * the causal pass alone (stage 3) and fp16 the pool, the query and the causal pass.
+ * n = 0 clears them; at most 8.  The caller keeps the events alive while they are set.
  */
 int smat_set_stage_events(void* const* events, int n);
 int smat_forward(int dtype, const void* phi, const void* psi, const void* vb,

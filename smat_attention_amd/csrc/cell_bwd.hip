@@ -223,8 +223,7 @@ __global__ __launch_bounds__(cw::kThreads, 4) void cell_pool_bwd_kernel(
 
   const int w = __builtin_amdgcn_readfirstlane(wave_id());
   const int lane = lane_id(), r16 = lane & 15, g = lane >> 4;
-  // A operands: dF rows a = 16w + r16 (for v) and dF columns c = 16w + r16
-  // (for dVb; wave 0 also c = 64 + r16, of which only 64 exists)
+  // A operands: dF rows a = 16w + r16 (for v) and dF columns c = 16w + r16 (for dVb)
   f32x8 fr[2], fc[2];
 #pragma unroll
   for (int kc = 0; kc < 2; ++kc)

@@ -1175,8 +1175,7 @@ def test_feature_map_every_negative_16_bit_input(dt):
     """The elu + 1 map on every finite non-positive 16-bit input, through the
     featurise launch with W = I (so the product is the input itself), against
     expm1 in fp64 rounded to the dtype, then + 1 rounded (torch's rounding
-    steps).  bf16 runs the short expm1 form and must be bit-exact on all 32 641
-    inputs; fp16 runs libm's expm1f (about 1 ulp of fp32), which may land one
+    steps).  bf16 takes exp2 minus one and must be bit-exact on all 32 641 inputs; fp16 runs libm's expm1f (about 1 ulp of fp32), which may land one
     fp16 step off where the exact value sits within that ulp of a rounding
     boundary: at most 1e-3 of the inputs, by one step."""
     _say("feature map exhaustive", dt)
