@@ -363,7 +363,9 @@ constexpr int kQMax = 41;         // largest q whose four planes fit the LDS
 // / 190.  The forward's rows share few lines and turn later: q = 17 599 MB 154 / 160
 // (head size 64, 604 MB: 186 / 178), 899 MB 243 / 236; q = 23 557 MB 148 / 154,
 // 1089 MB 304 / 297.  q = 19 turns early there too: 191 MB 49 / 52, 280 MB 75 / 74,
-// 752 MB 234 / 202.
+// 752 MB 234 / 202.  With a global channel, whose row each line starts from, the
+// smaller ones win at every size (alone, q = 19 1493 MB 444 / 520, q = 23 544 MB 183
+// / 203; forward, q = 19 315 MB 93 / 109).
 constexpr int64_t wide_bytes(int q, bool spread) {
   return (spread && q != 19 ? 600ll : 200ll) << 20;
 }
@@ -861,7 +863,7 @@ static int launch_wave_q(const float* F, const float* F_glob, const int* code, f
                          int B, int64_t rp, int64_t ld, hipStream_t stream) {
   using namespace iw;
   if constexpr (has_wide(Q) && !WIDE) {
-    if ((int64_t)nb * (Q * Q + B) * ld * 4 > wide_bytes(Q, ld > rp))
+    if (!F_glob && (int64_t)nb * (Q * Q + B) * ld * 4 > wide_bytes(Q, ld > rp))
       return launch_wave_q<Q, true>(F, F_glob, code, U, nb, B, rp, ld, stream);
   }
   const int nslices = (int)((rp + kE - 1) / kE);
@@ -875,8 +877,10 @@ static int launch_wave_q(const float* F, const float* F_glob, const int* code, f
   const unsigned grid = (unsigned)(per_xcd_wgs * inc::kXCD);
   const size_t smem = (size_t)Shape<Q, WIDE>::kLdsBytes;
   static bool attr_set[2] = {false, false};
-  auto kern = F_glob ? incidence_wave_kernel<Q, true, WIDE>
-                     : incidence_wave_kernel<Q, false, WIDE>;
+  auto kern = incidence_wave_kernel<Q, false, WIDE>;
+  if constexpr (!WIDE) {
+    if (F_glob) kern = incidence_wave_kernel<Q, true, false>;
+  }
   if (!attr_set[F_glob ? 1 : 0]) {
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                               inc::kPlaneLdsBudget);

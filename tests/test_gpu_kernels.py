@@ -1456,9 +1456,9 @@ def test_query_lists_at_row_block_edges(dt, maxcnt):
 @pytest.mark.parametrize("glob", [False, True])
 def test_incidence_line_groups_above_the_cache(T, q, nb, glob):
     """Between q = 17 and 23 F and U of more than 200 MB (600 MB where the forward
-    spreads its rows) take one workgroup of 1024 threads a CU: the first, a middle and
-    the last sequence are bitwise those of a launch of one sequence, which takes the
-    small workgroups (the same sums in the same order)."""
+    spreads its rows) take one workgroup of 1024 threads a CU, without a global channel:
+    the first, a middle and the last sequence are bitwise those of a launch of one
+    sequence, which takes the small workgroups (the same sums in the same order)."""
     _say("incidence line groups, large", T, q, nb, glob)
     spec = A.to_device(build_mask(T, 3, chunk=128), DEV)
     assert spec.q == q and nb * (spec.N0 + spec.B) * 128 * 129 * 4 > 768 << 20
